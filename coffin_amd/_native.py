@@ -101,6 +101,16 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+def load_host():
+    """The compiled host path of the table entries (``csrc/host_adapters.cpp``); raises like :func:`load`."""
+    load()
+    try:
+        from coffin_amd import _host
+    except ImportError as exc:
+        raise RuntimeError(f"coffin_amd host extension unusable: {exc}; build it with `python -m coffin_amd.build`") from exc
+    return _host
+
+
 def available() -> bool:
     """True when the shared library loads (says nothing about a GPU being present)."""
     try:

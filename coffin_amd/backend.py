@@ -534,6 +534,41 @@ def _rows_w4a16(rec: _Record, act: torch.Tensor, rows: int, out: torch.Tensor) -
             _native.check(rc, "gemv_w4a16")
 
 
+# ----------------------------------------------------------------- compiled calls
+
+# What an entry does on every call is compiled (csrc/host_adapters.cpp): at one row the Python adapters
+# below cost 7 us per call in front of kernels of 2.5 .. 10 us.  A compiled call reads the switches, records and
+# scratch of this module, does the whole entry for plain bf16 tensors on the current device and a weight
+# that has been seen before, and answers ``None`` for anything else, which the adapters below then do
+# (first uses, other dtypes and layouts, errors).  Loaded by the first call that holds a GPU tensor.
+
+_HOST_CALLS = ("project", "rms_norm", "add_rms_norm", "silu_mul", "kv_quant", "embed_rows")
+
+
+def _bind_host() -> None:
+    host = _native.load_host()
+    host.bind(globals(), _native.check, _rows_quantised)
+    for name in _HOST_CALLS:
+        globals()["_host_" + name] = getattr(host, name)
+
+
+def _until_bound(name: str):
+    def first(*args):
+        if not any(isinstance(a, torch.Tensor) and a.is_cuda for a in args):
+            return None
+        _bind_host()
+        return globals()["_host_" + name](*args)
+    return first
+
+
+for _name in _HOST_CALLS:
+    globals()["_host_" + _name] = _until_bound(_name)
+
+#: Flags of the compiled ``project``: the entry may quantise from ``PREFILL_MIN_ROWS`` rows / may use
+#: the matrix-pipe family from ``MFMA_MIN_ROWS`` rows.
+_PREFILL, _MFMA = 1, 2
+
+
 # ------------------------------------------------------------------ dispatch
 
 def _dense(w, x: torch.Tensor) -> torch.Tensor:
@@ -607,13 +642,15 @@ def _project(w, x: torch.Tensor, prefill: bool, min_rows: int = PREFILL_MIN_ROWS
 
 def linear(w, x: torch.Tensor) -> torch.Tensor:
     """``linear(w, x) -> y``: ``x`` ``[K]`` or ``[C, K]``, ``y`` ``[N]`` or ``[C, N]``, dtype of ``x``."""
-    return _project(w, x, prefill=False)
+    y = _host_project(w, x, 0)
+    return y if y is not None else _project(w, x, prefill=False)
 
 
 def linear_m(w, x: torch.Tensor) -> torch.Tensor:
     """``linear_m(w, x[M, K]) -> [M, N]``: one weight read serves all rows; row r carries the bits
     of ``linear(w, x[r])`` (in either kernel family: both entries switch together, see :func:`configure`)."""
-    return _project(w, x, prefill=False)
+    y = _host_project(w, x, 0)
+    return y if y is not None else _project(w, x, prefill=False)
 
 
 def linear_m_verify(w, x: torch.Tensor) -> torch.Tensor:
@@ -625,6 +662,9 @@ def linear_m_verify(w, x: torch.Tensor) -> torch.Tensor:
     backends/corex/__init__.py:462-485: ``QWeight`` only, rows >= 2).  int4 weights: as
     ``linear_m`` (exact integer sums, one summation order everywhere).
     """
+    y = _host_project(w, x, _MFMA)
+    if y is not None:
+        return y
     if (W8A8_VERIFY and _is_q8(w) and x.dim() == 2 and x.shape[0] >= 2 and _on_gpu(x)
             and x.dtype == torch.bfloat16 and int(w.k) % 16 == 0 and x.shape[-1] == int(w.k)):
         return _project(w, x, prefill=True, min_rows=2)
@@ -634,7 +674,18 @@ def linear_m_verify(w, x: torch.Tensor) -> torch.Tensor:
 def linear_prefill(w, x: torch.Tensor) -> torch.Tensor:
     """``linear_prefill(w, x[C, K]) -> [C, N]``: the GEMM regime (W8A8 from 64 rows up; shorter
     chunks of int8 weights stay weight-only, on the matrix-pipe GEMV)."""
-    return _project(w, x, prefill=True, mfma=True)
+    y = _host_project(w, x, _PREFILL | _MFMA)
+    return y if y is not None else _project(w, x, prefill=True, mfma=True)
+
+
+_ROLE_FLAGS = {"linear": 0, "linear_m": 0, "linear_m_verify": _MFMA, "linear_prefill": _PREFILL | _MFMA}
+
+
+def linear_parts(entry: str, w, x: torch.Tensor, sizes) -> tuple:
+    """The table entry named ``entry`` on a weight that holds several projections along its output axis:
+    ``entry(w, x).split(sizes, dim=-1)`` in one call."""
+    parts = _host_project(w, x, _ROLE_FLAGS[entry], sizes)
+    return parts if parts is not None else globals()[entry](w, x).split(sizes, dim=-1)
 
 
 def linear_quantized(w, xq: torch.Tensor, xs: torch.Tensor) -> torch.Tensor:
@@ -688,6 +739,8 @@ def kv_quant(x: torch.Tensor, out_q: torch.Tensor, out_s: torch.Tensor) -> torch
     (backends/reference/__init__.py:386-389).  bf16 rows on the GPU run the
     kernel; other inputs take the same formula in torch.
     """
+    if _host_kv_quant(x, out_q, out_s) is not None:
+        return out_q
     if x.dim() != 2 or tuple(out_q.shape) != tuple(x.shape) or out_s.numel() != x.shape[0]:
         raise ValueError("kv_quant expects x [M, N], out_q [M, N], out_s [M]")
     native_ok = (_on_gpu(x) and x.dtype == torch.bfloat16 and x.is_contiguous()
@@ -760,6 +813,8 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor) -> torch.T
     that may alias ``up`` (backends/protocol.py:265-273, backends/reference/__init__.py:253-268).
     Registered together with :func:`silu_mul_quant` so that the two share one arithmetic.  Any
     leading shape (``[...]`` in the contract): layouts the kernel does not take go to torch."""
+    if _host_silu_mul(gate, up, out) is not None:
+        return out
     if gate.shape != up.shape or out.shape != gate.shape:
         raise ValueError("silu_mul needs gate, up and out of one shape")
     _drop_handed()
@@ -774,6 +829,8 @@ def silu_mul_quant(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor, out_
     and, in the same pass, quantised per row to int8 (``out_q`` + ``out_s``) -- bit for bit what
     ``silu_mul`` followed by ``kv_quant`` gives, because the absmax is taken over the stored bf16
     values (backends/protocol.py:274-278, backends/corex/__init__.py:1038-1071)."""
+    if _host_silu_mul(gate, up, out, out_q, out_s) is not None:
+        return out
     if gate.shape != up.shape or gate.dim() != 2:
         raise ValueError("silu_mul_quant needs two same-shaped [rows, K] inputs")
     if tuple(out.shape) != tuple(gate.shape) or tuple(out_q.shape) != tuple(gate.shape) \
@@ -846,6 +903,9 @@ def rms_norm(x: torch.Tensor, w: torch.Tensor, stride: int = 0, eps: float = 1e-
     the same, with and without the quantised outputs).  ``stride`` is informational, as in the
     reference: the row pitch is read from ``x``."""
     del stride
+    y = _host_rms_norm(x, w, eps)
+    if y is not None:
+        return y
     if not _norm_native(x, w):
         xf = x.to(torch.float32)
         scale = torch.rsqrt(xf.pow(2).mean(dim=-1, keepdim=True) + eps)
@@ -874,6 +934,8 @@ def add_rms_norm(x: torch.Tensor, add: torch.Tensor, w: torch.Tensor, out: torch
     """``add_rms_norm(x, add, w, out, stride=0, eps=1e-6) -> out``: ``x += add`` in place, then the
     RMSNorm of the sum into ``out`` (backends/protocol.py:244-248, backends/reference/__init__.py:224-250)."""
     del stride
+    if _host_add_rms_norm(x, add, w, out, eps) is not None:
+        return out
     ok = (_norm_native(x, w) and add.shape == x.shape and add.dtype == torch.bfloat16 and add.device == x.device
           and (add.shape[1] == 1 or add.stride(1) == 1) and out.shape == x.shape and out.dtype == torch.bfloat16
           and out.device == x.device and (out.shape[1] == 1 or out.stride(1) == 1))
@@ -904,6 +966,9 @@ def embed_rows(w, ids: torch.Tensor) -> torch.Tensor:
     """Rows ``ids`` of a quantized embedding matrix as bf16 ``[T, K]``: only the gathered rows are
     dequantised (ops/embed.py:64-81; ``QWeight.rows`` int8_weights.py:361-372,
     ``W4A8Weight.rows`` w4a8_weights.py:84-94).  Ids outside the vocabulary give NaN rows."""
+    y = _host_embed_rows(w, ids)
+    if y is not None:
+        return y
     rec = _lookup(w)
     if rec is None:
         if not (_is_w4(w) or _is_q8(w)):

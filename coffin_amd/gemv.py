@@ -111,24 +111,31 @@ class GEMVGroup:
                 fused[at:at + w.shape[0]].copy_(w)
                 at += w.shape[0]
         self.g = GEMV(fused, bench, ops)
+        # this package's adapters answer the projection and its parts in one call
+        self._parts = _backend.linear_parts if self.g.ops is _backend and not isinstance(fused, torch.Tensor) else None
+
+    def _split(self, entry: str, x: torch.Tensor):
+        if self._parts is not None:
+            return self._parts(entry, self.g.w, x, self.sizes)
+        return getattr(self.g.ops, entry)(self.g.w, x).split(self.sizes, dim=-1)
 
     def __call__(self, x: torch.Tensor):
-        return self.g(x).split(self.sizes, dim=-1)
+        return self._split("linear", x)
 
     def linear_m(self, x: torch.Tensor):
         if x.shape[0] == 1:
             return [part.unsqueeze(0) for part in self(x[0])]
-        return self.g.linear_m(x).split(self.sizes, dim=1)
+        return self._split("linear_m", x)
 
     def linear_m_verify(self, x: torch.Tensor):
         if x.shape[0] == 1:
             return [part.unsqueeze(0) for part in self(x[0])]
-        return self.g.linear_m_verify(x).split(self.sizes, dim=1)
+        return self._split("linear_m_verify", x)
 
     def prefill(self, x: torch.Tensor):
         if x.shape[0] == 1:
             return [part.unsqueeze(0) for part in self(x[0])]
-        return self.g.prefill(x).split(self.sizes, dim=1)
+        return self._split("linear_m" if x.shape[0] <= SMALL_BATCH_ROWS else "linear_prefill", x)
 
 
 def _proj(sd: dict, prefixes: list[str], bench: bool = True):
