@@ -1,8 +1,8 @@
 // Per-token symmetric int8 activation quantiser (bf16 in, int8 + fp32 scale out).
 //
-// One workgroup per row.  The row is read once from HBM with 16-byte loads and
-// kept in registers across the absmax reduction when it fits (VPT vectors per
-// thread), so HBM traffic is the algorithmic 2 B in + 1 B out per element.
+// One workgroup per row, or a part of a wavefront per short row.  The row is read once from
+// HBM with 16-byte loads and kept in registers across the absmax reduction when it fits (VPT
+// vectors per thread), so HBM traffic is the algorithmic 2 B in + 1 B out per element.
 // The scale and the rounding follow the torch spec bit for bit: IEEE fp32
 // division by the scale (not a reciprocal multiply), round-half-even, clamp.
 #include "quant_math.hpp"
@@ -68,6 +68,67 @@ quant_act_i8_vec(const uint4 *__restrict__ x, uint2 *__restrict__ q, float *__re
     }
 }
 
+// Max over the LANES lanes of a row's group; every lane of the group returns it.
+template <int LANES>
+__device__ __forceinline__ float group_max(float v) {
+    static_assert(LANES == 8 || LANES == 16 || LANES == 32 || LANES == 64, "a power of two from 8");
+    v = fmaxf(v, dpp_f32<0xB1, 0xf>(v));   // l ^ 1
+    v = fmaxf(v, dpp_f32<0x4E, 0xf>(v));   // l ^ 2
+    v = fmaxf(v, dpp_f32<0x141, 0xf>(v));  // the other quad of the half row
+    if constexpr (LANES >= 16) v = fmaxf(v, dpp_f32<0x140, 0xf>(v));  // the other half of the row
+    typedef unsigned u32x2_swap __attribute__((ext_vector_type(2)));
+    if constexpr (LANES >= 32) {
+        const u32x2_swap r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = fmaxf(__uint_as_float(r.x), __uint_as_float(r.y));
+    }
+    if constexpr (LANES == 64) {
+        const u32x2_swap r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = fmaxf(__uint_as_float(r.x), __uint_as_float(r.y));
+    }
+    return v;
+}
+
+// Short rows (cache rows of 64 .. 576 elements): LANES lanes own a row, VPT vectors each, so a wavefront
+// carries 64 / LANES rows at a time, R times, and reduces them without LDS or a barrier.  A workgroup per
+// row left 15 of 16 lanes idle at 128 elements and was bound by the rate at which workgroups are started.
+// Cold operands in a graph: 16384 x 128 13.1 -> 3.6 us (1.7 TB/s; 1.6 us of it are the launch), 65536 x 128
+// 45.9 -> 7.8 us (3.2 TB/s), 8192 x 512 9.0 -> 5.6 us, 3000 x 1024 6.1 -> 4.5 us.  Same arithmetic, same bits.
+template <int LANES, int VPT, int R>
+__global__ void __launch_bounds__(QUANT_THREADS)
+quant_act_i8_rows(const uint4 *__restrict__ x, uint2 *__restrict__ q, float *__restrict__ s, int nvec, int rows,
+                  int *__restrict__ zero, int n_zero) {
+    constexpr int STEP = QUANT_THREADS / LANES;
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < n_zero; i += QUANT_THREADS) zero[i] = 0;
+    const int l = threadIdx.x % LANES;
+    const int row0 = blockIdx.x * (STEP * R) + threadIdx.x / LANES;
+    uint4 v[R][VPT];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const size_t at = (size_t)min(row0 + r * STEP, rows - 1) * nvec;
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) {
+            const int idx = l + i * LANES;
+            v[r][i] = idx < nvec ? x[at + idx] : make_uint4(0, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int row = row0 + r * STEP;
+        float amax = 0.f;
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) amax = absmax8(v[r][i], amax);
+        const RowScale rs = row_scale(group_max<LANES>(amax));
+        if (row >= rows) continue;  // a whole group of lanes; the next rows lie further on
+        if (l == 0) s[row] = rs.sc;
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) {
+            const int idx = l + i * LANES;
+            if (idx < nvec) q[(size_t)row * nvec + idx] = quant8(v[r][i], rs);
+        }
+    }
+}
+
 // Any K, any alignment; q rows have pitch ldq >= K and the tail K .. ldq-1 is cleared.
 __global__ void __launch_bounds__(QUANT_THREADS)
 quant_act_i8_scalar(const uint16_t *__restrict__ x, int8_t *__restrict__ q,
@@ -104,7 +165,19 @@ int cmi::quant_act_i8_and_clear(const void *x, int8_t *q, float *s, int M, int K
         const uint4 *xv = static_cast<const uint4 *>(x);
         uint2 *qv = reinterpret_cast<uint2 *>(q);
         const int vpt = (nvec + QUANT_THREADS - 1) / QUANT_THREADS;
-        if (vpt <= 1) quant_act_i8_vec<1><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);
+        const auto rows_launch = [&](auto kernel, int rows_per_block) {
+            kernel<<<dim3((M + rows_per_block - 1) / rows_per_block), block, 0, st>>>(xv, qv, s, nvec, M, zero, n_zero);
+        };
+        // Up to 1024 elements a wavefront or less owns a row.  Two rows per lane group once one each would
+        // be more than two workgroups per CU: twice the bytes in flight per wavefront (65536 x 128: 9.8 ->
+        // 7.8 us; below that the second row only lengthens the launch, 2048 x 576: 3.3 -> 3.9 us).
+        const auto many = [&](int rows_per_block) { return M > 512 * rows_per_block; };
+        if (nvec <= 8) many(32) ? rows_launch(quant_act_i8_rows<8, 1, 2>, 64) : rows_launch(quant_act_i8_rows<8, 1, 1>, 32);
+        else if (nvec <= 16) many(16) ? rows_launch(quant_act_i8_rows<16, 1, 2>, 32) : rows_launch(quant_act_i8_rows<16, 1, 1>, 16);
+        else if (nvec <= 32) many(8) ? rows_launch(quant_act_i8_rows<32, 1, 2>, 16) : rows_launch(quant_act_i8_rows<32, 1, 1>, 8);
+        else if (nvec <= 64) many(4) ? rows_launch(quant_act_i8_rows<64, 1, 2>, 8) : rows_launch(quant_act_i8_rows<64, 1, 1>, 4);
+        else if (nvec <= 128) rows_launch(quant_act_i8_rows<64, 2, 1>, 4);
+        else if (vpt <= 1) quant_act_i8_vec<1><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);
         else if (vpt <= 2) quant_act_i8_vec<2><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);
         else if (vpt <= 4) quant_act_i8_vec<4><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);
         else if (vpt <= 8) quant_act_i8_vec<8><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);
