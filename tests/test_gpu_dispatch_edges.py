@@ -19,3 +19,42 @@ def test_quantiser_of_short_rows(orc, m, k):
     q_ref, s_ref = orc.quant_act_i8(G.bits(x))
     q, s = G.quant(x.to(G.DEV))
     assert (q.cpu().numpy() == q_ref).all() and (s.cpu().numpy() == s_ref).all()
+
+
+@pytest.mark.parametrize("m,k", [(256, 8192), (257, 8192), (2, 8200), (257, 1032), (258, 16392), (3, 24584), (257, 32768), (2, 32776)])
+def test_silu_mul_quant_at_the_edges_of_a_thread_s_share(orc, m, k):
+    g = synth.generator(m + k)
+    gate, up = (torch.randn((m, 2 * k), generator=g) * 3).to(torch.bfloat16).split(k, dim=1)
+    gd, ud = (torch.cat([gate, up], dim=1).to(G.DEV)).split(k, dim=1)
+    out = torch.empty((m, k), dtype=torch.bfloat16, device=G.DEV)
+    q = torch.empty((m, k), dtype=torch.int8, device=G.DEV)
+    s = torch.empty(m, dtype=torch.float32, device=G.DEV)
+    lib = _native.load()
+    rows = [0, 1, m - 1]
+    o_ref, q_ref, s_ref = orc.silu_mul_quant(G.bits(gate[rows].contiguous()), G.bits(up[rows].contiguous()))
+    for quantised in (True, False):
+        out.zero_()
+        _native.check(lib.cmi_silu_mul_quant(G.ptr(gd), G.ptr(ud), G.ptr(out), G.ptr(q if quantised else None),
+                                             G.ptr(s if quantised else None), m, k, 2 * k, 2 * k, k, G.stream()), "silu")
+        assert (G.bits(out[rows]) == o_ref).all()
+    assert (q[rows].cpu().numpy() == q_ref).all() and (s[rows].cpu().numpy() == s_ref).all()
+
+
+@pytest.mark.parametrize("m,n", [(256, 1024), (257, 512), (259, 520), (257, 1024), (2, 1032), (300, 8192), (3, 8200), (2, 16392),
+                                 (257, 32768), (2, 32776)])
+def test_add_rms_norm_i8_at_the_edges_of_a_row_s_wavefronts(orc, m, n):
+    g = synth.generator(m + n)
+    x, add = synth.activations(m, n, g), synth.activations(m, n, g)
+    gain = (1 + 0.1 * torch.randn(n, generator=g)).to(torch.bfloat16)
+    xd, y = x.to(G.DEV), torch.empty((m, n), dtype=torch.bfloat16, device=G.DEV)
+    q = torch.empty((m, n), dtype=torch.int8, device=G.DEV)
+    s = torch.empty(m, dtype=torch.float32, device=G.DEV)
+    ad, gd = add.to(G.DEV), gain.to(G.DEV)
+    _native.check(_native.load().cmi_add_rms_norm_i8(G.ptr(xd), G.ptr(ad), G.ptr(gd), G.ptr(y), G.ptr(q), G.ptr(s), m, n,
+                                                     n, n, n, 1e-6, G.stream()), "add_rms_norm_i8")
+    rows = [0, 1, m - 1]
+    total = (x.float() + add.float()).to(torch.bfloat16)[rows].contiguous()
+    y_ref, _ = orc.rms_norm(G.bits(total), G.bits(gain))
+    q_ref, s_ref = orc.quant_act_i8(y_ref)
+    assert (G.bits(xd[rows]) == G.bits(total)).all() and (G.bits(y[rows]) == y_ref).all()
+    assert (q[rows].cpu().numpy() == q_ref).all() and (s[rows].cpu().numpy() == s_ref).all()
