@@ -50,8 +50,8 @@ __device__ __forceinline__ void widen_w4_piece(uint32_t w0, uint32_t w1, uint32_
 // third slower than from the memory-side cache (Infinity Cache, 256 MiB, shared by all CUs).  The
 // CUs that have no tile therefore read the weight front to back at memory speed and drop it:
 // after a few microseconds the tiles' requests are answered by that cache.  (W8A8 tiles: -15..-25 %
-// on cold weights.  The W4A8 ring kernels, whose step is set by the widening and the per-group
-// flush rather than by the operand stream, measured the same with and without: not used there.)
+// on cold weights.  The W4A8 tiles, whose step is set by the widening and the per-group flush rather
+// than by the operand stream, do not use it.)
 // Workgroup `part` of `parts` (256 threads each) reads its share of `bytes` (a multiple of 16,
 // p 16-byte aligned), eight 16-byte requests in flight per thread.
 __device__ __forceinline__ void warm_caches(const void *p, size_t bytes, int part, int parts) {

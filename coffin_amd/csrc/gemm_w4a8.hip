@@ -1,29 +1,20 @@
-// W4A8 prefill GEMM for CDNA4 int8 MFMA on the re-laid-out int4 weight (group size 128).
+// cmi_gemm_w4a8: the choice of route, and the kernel for calls that ask for the integer group sums.
 //
 //   sum_g  = sum_{k in group g} xq[m,k] * (code(n,k) - 8)     int32, exact
 //   total  = fma((float)sum_g, ws[n,g], total)                 g = 0,1,.. from 0.f
 //   y[m,n] = bf16(total * xs[m])
 //
-// Same bits as the W4A8 GEMV for every m: the integer part is exact and the
-// fp32 part is the one chain over the groups in ascending order.
+// Same bits from every route: the integer part is exact and the fp32 part is the one chain over the groups in
+// ascending order.  The product alone runs the tile kernels of gemm_w4a8_tile.hip or, for a few rows, the GEMV.
 //
-// Block tile 128(m) x 128(n), 4 wavefronts (2 x 2) of 64 x 64, v_mfma_i32_32x32x32_i8,
-// K walked one scale group (128) per step, two LDS stages, two workgroups per CU.
-//   - activations go global -> LDS directly (global_load_lds_dwordx4, chunk
-//     index XOR-swizzled on the global side, as in the W8A8 kernel);
-//   - the packed weight (64 B per row and step) is fetched into registers one
-//     step ahead, widened there to int8 code-8 (no cross-byte borrow), and
-//     written to LDS once per workgroup, so the inner loop is the int8 one;
-//   - the activation is the MFMA row operand and the weight the column operand:
-//     a lane then owns ONE n per MFMA tile (and 16 m), so the per-group flush
-//     total = fma((float)sum, ws[n,g], total) needs one scale per tile and lane,
-//     fetched from memory a step ahead;
-//   - the integer accumulators restart every step (first MFMA of a group takes
-//     C = 0); the flush is 64 converts + 64 fmas per lane and step, which is why
-//     two workgroups share a CU: one flushes while the other multiplies.
-#include <cmath>
-#include <cstdlib>
-
+// With group sums (parity checks): block tile 128(m) x 128(n), 4 wavefronts (2 x 2) of 64 x 64,
+// v_mfma_i32_32x32x32_i8, K walked 128 per step, two LDS stages, two workgroups per CU.
+//   - activations go global -> LDS directly (global_load_lds_dwordx4, chunk index XOR-swizzled on the global side);
+//   - the packed weight (64 B per row and step) is fetched into registers one step ahead, widened there to int8
+//     code-8 (no cross-byte borrow), and written to LDS once per workgroup;
+//   - the activation is the MFMA row operand and the weight the column operand: a lane owns ONE n per MFMA tile (and
+//     16 m), so the flush needs one scale per tile and lane, fetched from memory a step ahead;
+//   - the integer accumulators restart every group (first MFMA takes C = 0) and are written out before the flush.
 #include "common.hpp"
 #include "gemm_tiles.hpp"
 
@@ -45,22 +36,18 @@ struct Args {
     const float *xs;
     const float *ws;  // [N, G]
     uint16_t *y;
-    int32_t *group_acc;  // [M, G, N], nullable
+    int32_t *group_acc;  // [M, G, N]
     int M, N, K, G;
-    int ldy;  // row pitch of y (elements), >= N
     int tiles_m, tiles_n;
 };
 
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
 
-// DUMP: also write the int32 group sums (parity checks); a separate instantiation, the
-// 64 extra store addresses per lane would otherwise be carried through the hot loop.
-// LG: log2(group size / 32).  2: a K step is a group (what the kernel is tuned for).  3: a group is
-// two steps, the integer accumulators run on over the odd step and flush behind it.  1: a step holds
-// two groups, flushed behind the second and the fourth k quarter.
-template <bool DUMP, int LG = 2>
+// LG: log2(group size / 32).  2: a K step is a group.  3: a group is two steps, the integer accumulators run on over
+// the odd step and flush behind it.  1: a step holds two groups, flushed behind the second and the fourth k quarter.
+template <int LG>
 __global__ void __launch_bounds__(THREADS, 2)
-gemm_w4a8_kernel(const Args a) {
+gemm_w4a8_group_sums_kernel(const Args a) {
     static_assert(LG >= 1 && LG <= 3, "group sizes 64, 128, 256");
     extern __shared__ __align__(16) int8_t lds[];
     const int lane = threadIdx.x & 63;
@@ -213,7 +200,7 @@ gemm_w4a8_kernel(const Args a) {
         mma_q(f1, false);
         pace_quarter();
         if constexpr (LG == 1) {  // the step's first group is complete
-            if constexpr (DUMP) dump(2 * ks);
+            dump(2 * ks);
             flush(sc);
         }
         read_q(cur, 3, f1);
@@ -248,7 +235,7 @@ gemm_w4a8_kernel(const Args a) {
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
         if (closes) {
-            if constexpr (DUMP) dump(LG == 3 ? ks >> 1 : LG == 1 ? 2 * ks + 1 : ks);
+            dump(LG == 3 ? ks >> 1 : LG == 1 ? 2 * ks + 1 : ks);
             if constexpr (LG == 1) flush(sc_b);
             else flush(sc);
         }
@@ -296,14 +283,12 @@ gemm_w4a8_kernel(const Args a) {
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int n = nb + j * 32 + (lane & 31);
-                if (n < a.N) a.y[(size_t)m * a.ldy + n] = (uint16_t)f32_to_bf16_bits(total[i][j][v] * xm);
+                if (n < a.N) a.y[(size_t)m * a.N + n] = (uint16_t)f32_to_bf16_bits(total[i][j][v] * xm);
             }
         }
 }
 
 }  // namespace
-
-static inline int a_ceil(int a, int b) { return (a + b - 1) / b; }
 
 extern "C" int cmi_gemm_w4a8(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs,
                              void *y, int32_t *group_acc, int M, int N, int K, int gs,
@@ -317,39 +302,21 @@ extern "C" int cmi_gemm_w4a8(const uint8_t *w4, const float *ws, const int8_t *x
                 "cmi_gemm_w4a8: K=%d is not a multiple of 128 and of the group size %d (pad the rows with zeros)", K, gs);
     CMI_REQUIRE(aligned(xq, 16) && aligned(w4, 16), CMI_E_ARG,
                 "cmi_gemm_w4a8: xq and w4 must be 16-byte aligned");
-    // Which kernel: with few tiles a launch is a chain of K/128 dependent steps and the kernels differ
-    // in the length of a step (two-stage 128 x 128 tiles: 1.15 us and up; ring of stages with
-    // 64 x 64 tiles 0.44 us, with 128 x 64 tiles 0.6 us), with many tiles in how a step's time grows
-    // with the tiles per CU, and up to 256 rows the matrix-pipe GEMV reads the weight once per 128
-    // rows at memory speed and pays per 16-row chunk.  Same integer sums, same fp32 chain, same
-    // bits from all of them.  Cost models (us) fitted to cold-weight measurements on ten layer
-    // shapes x eleven batch sizes.  The ring kernels do not write the group sums.
     const int forced = option_gemm_tile();
-    int ring = !group_acc && gs == BK && (forced == 64 || forced == 6464) ? forced : 0;
-    // groups of 64 and 256: the two-stage tile kernel (and, up to 16 rows, the general GEMV)
+    // Which kernel.  Up to 256 rows of groups of 128 the matrix-pipe GEMV reads the weight once per 128 rows at memory
+    // speed and pays per 16-row chunk (K <= 10240: it keeps the weight in registers; longer rows run in passes, 16
+    // rows per launch, at about half the speed); beyond, the tile kernels, whose cost model stands with them.
+    // Same integer sums, same fp32 chain, same bits from all of them.
     if (gs != BK && M <= 16 && !forced) return cmi_gemv_w4a8(w4, ws, xq, xs, y, group_acc, M, N, K, gs, stream);
-    if (!forced && gs == BK) {
+    int tile = 0;
+    const double t_tile = forced ? 0.0 : gemm_w4a8_tile_us(M, N, K, gs, &tile);
+    if (!forced && gs == BK && M <= 256) {
         const double steps = K / 128.0, wn = (double)N * K;
-        const double tiles = (double)a_ceil(M, BM) * a_ceil(N, BN);
-        const double t_tiled = 3.0 + steps * (tiles <= 512 ? 1.15 + 0.0013 * tiles : 1.6 * ceil(tiles / 512.0));
-        // up to 10240 elements per row the GEMV keeps the weight in registers for 128 rows per launch
-        // and pays per 16-row chunk only the chunk's sums and chain; longer rows run it in passes,
-        // 16 rows per launch, at about half the speed
-        const double t_rows16 =
-            M > 256 ? 1e30
-            : K <= 10240 ? a_ceil(M, 128) * (2.0 + wn / 2 / 4.2e6) + a_ceil(M, 16) * (0.6 + wn / 1.3e7 + steps * 0.012)
-                         : a_ceil(M, 16) * (3.6 + wn / 2 / 2.1e6);
-        const double tiles_h = (double)a_ceil(M, 64) * a_ceil(N, 64), tiles_g = (double)a_ceil(M, 128) * a_ceil(N, 64);
-        // a step of the ring kernels: flat while every tile has a CU to itself, a second level up to
-        // two tiles per CU, then linear in the tiles
-        const double s_h = tiles_h <= 256 ? 0.44 + 6e-6 * N : tiles_h <= 512 ? 0.65 + 1e-5 * N : 0.4 + 0.00137 * tiles_h;
-        const double s_g = tiles_g <= 256 ? 0.60 + 1.4e-5 * N : tiles_g <= 512 ? 1.0 + 4e-6 * N : 0.4 + 0.00205 * tiles_g;
-        const double t_h = group_acc ? 1e30 : 2.5 + steps * s_h;
-        const double t_g = group_acc ? 1e30 : 2.5 + steps * s_g;
-        // (the GEMV's model is the optimistic one of the four at four chunks and more: it has to win by 10 %)
-        if (t_rows16 <= t_tiled && t_rows16 <= 0.9 * t_h && t_rows16 <= 0.9 * t_g) {
+        const int chunks = (M + 15) / 16, step = K <= 10240 ? 128 : 16;
+        const double t_rows16 = K <= 10240 ? (M + 127) / 128 * (2.0 + wn / 2 / 4.2e6) + chunks * (0.6 + wn / 1.3e7 + steps * 0.012)
+                                           : chunks * (3.6 + wn / 2 / 2.1e6);
+        if (t_rows16 <= t_tile) {
             const int G = K / BK;
-            const int step = K <= 10240 ? 128 : 16;
             for (int lo = 0; lo < M; lo += step) {
                 const int m = M - lo < step ? M - lo : step;
                 const int rc = gemv_w4a8_rows16(w4, ws, xq + (size_t)lo * K, xs + lo, nullptr,
@@ -360,10 +327,9 @@ extern "C" int cmi_gemm_w4a8(const uint8_t *w4, const float *ws, const int8_t *x
             }
             return CMI_OK;
         }
-        if (t_h <= t_tiled && t_h <= t_g) ring = 6464;
-        else if (t_g <= t_tiled) ring = 64;
     }
-    if (ring) return gemm_w4a8_ring(w4, ws, xq, xs, y, M, N, K, ring, stream);
+    if (!group_acc)
+        return gemm_w4a8_tile(w4, ws, xq, xs, y, M, N, K, gs, forced ? gemm_w4a8_forced_tile(forced, gs) : tile, stream);
     Args a;
     a.xq = xq;
     a.w4 = w4;
@@ -375,45 +341,15 @@ extern "C" int cmi_gemm_w4a8(const uint8_t *w4, const float *ws, const int8_t *x
     a.N = N;
     a.K = K;
     a.G = K / gs;
-    a.ldy = N;
     a.tiles_m = (M + BM - 1) / BM;
     a.tiles_n = (N + BN - 1) / BN;
-    // Whole rounds.  Two workgroups share a CU, so a launch runs in rounds of 512 tiles and a last
-    // round that is nearly empty costs as much as a full one (1024 x 25600: 1600 tiles = 3.125
-    // rounds, 252 us against 211 us for the 3.000 rounds of N = 24576).  The n tiles of such a
-    // remainder (at most half a round) go to a second launch of 64 x 64 tiles with a ring of
-    // stages, whose step is 0.44 us instead of 1.15 us and which spreads them over all CUs:
-    // same arithmetic, same bits.  (Not when the group sums are asked for: the ring kernels do not
-    // write them.)
-    int ring_n = 0;  // columns handed to the second launch
-    if (!forced && gs == BK && !group_acc) {
-        const int slots = 512, tiles = a.tiles_m * a.tiles_n, rest = tiles % slots;
-        if (tiles > slots && rest > 0 && rest <= slots / 2 && rest % a.tiles_m == 0) {
-            const int rest_n = rest / a.tiles_m;             // n tiles of the remainder
-            const int cols = N - (a.tiles_n - rest_n) * BN;  // their columns (the last tile may be ragged)
-            const double steps = K / 128.0, tiles_h = (double)a_ceil(M, 64) * a_ceil(cols, 64);
-            const double s_h = tiles_h <= 256 ? 0.44 + 6e-6 * cols : tiles_h <= 512 ? 0.65 + 1e-5 * cols : 0.4 + 0.00137 * tiles_h;
-            if (2.5 + steps * s_h < steps * 1.15) {
-                ring_n = cols;
-                a.N = N - cols;
-                a.tiles_n -= rest_n;
-            }
-        }
-    }
-    const dim3 grid(a.tiles_m * a.tiles_n), block(THREADS);
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    static std::atomic<uint64_t> devices[6];
+    static std::atomic<uint64_t> devices[3];
     auto run = [&](auto kernel, int slot) {
         if (const int rc = reserve_lds(reinterpret_cast<const void *>(kernel), LDS_BYTES, devices[slot], "cmi_gemm_w4a8"))
             return rc;
-        kernel<<<grid, block, LDS_BYTES, st>>>(a);
+        kernel<<<dim3(a.tiles_m * a.tiles_n), dim3(THREADS), LDS_BYTES, static_cast<hipStream_t>(stream)>>>(a);
         return check_launch("cmi_gemm_w4a8");
     };
-    if (gs == 64) return group_acc ? run(gemm_w4a8_kernel<true, 1>, 0) : run(gemm_w4a8_kernel<false, 1>, 1);
-    if (gs == 256) return group_acc ? run(gemm_w4a8_kernel<true, 3>, 2) : run(gemm_w4a8_kernel<false, 3>, 3);
-    if (const int rc = group_acc ? run(gemm_w4a8_kernel<true, 2>, 4) : run(gemm_w4a8_kernel<false, 2>, 5)) return rc;
-    if (!ring_n) return CMI_OK;
-    const int n1 = N - ring_n;
-    return gemm_w4a8_ring(w4 + (size_t)n1 * (K / 2), ws + (size_t)n1 * a.G, xq, xs, static_cast<uint16_t *>(y) + n1, M, ring_n,
-                          K, 6464, stream, N);
+    if (gs == 64) return run(gemm_w4a8_group_sums_kernel<1>, 0);
+    return gs == 256 ? run(gemm_w4a8_group_sums_kernel<3>, 1) : run(gemm_w4a8_group_sums_kernel<2>, 2);
 }

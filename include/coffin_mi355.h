@@ -42,8 +42,10 @@ int cmi_abi_version(void);
  *                   tile: what the library runs where it chooses that tile; 320 names the older
  *                   two-stage kernel) | 322 (321 as one workgroup per CU that walks its tiles one
  *                   after the other; measures the same as 321 and is never the library's choice):
- *                   block tile of cmi_gemm_w8a8 / cmi_gemm_w4a8 (non-zero also
- *                   bypasses their few-row routes);
+ *                   block tile of cmi_gemm_w8a8 (non-zero also bypasses its few-row routes).
+ *                   cmi_gemm_w4a8 has tiles of its own under the same values (m x n): 64 32 x 64,
+ *                   128 128 x 128, 192 64 x 96, 128192 64 x 128, 256 32 x 128, 320 128 x 160, 321
+ *                   16 x 32, 322 and 6464 64 x 64 (groups of 64 and 256: the nearest it is built for);
  *   "gemv_wholerow" -1 (the library chooses) | 0 (never) | 1: the one-wavefront-per-weight-row
  *                   kernel of cmi_gemv_w8a16;
  *   "w4_decode_waves" 0 (the library chooses) | 4 | 16: wavefronts per workgroup of the W4A8
@@ -182,8 +184,8 @@ int cmi_gemm_w8a8(const int8_t *xq, const int8_t *wq, const float *xs, const flo
                   void *y, int32_t *acc_out, int M, int N, int K, int ldy, void *stream);
 
 /* W4A8 GEMM on the re-laid-out weight; same arithmetic as cmi_gemv_w4a8 for
- * any M.  K % 128 == 0 and K % gs == 0, gs in {64, 128, 256} (the tile-count and few-row routes
- * are built for 128; other group sizes take the two-stage tile kernel).  Replaces w4a8_gemm_tcu
+ * any M.  K % 128 == 0 and K % gs == 0, gs in {64, 128, 256} (some tiles and the few-row
+ * route are built for 128 only).  Replaces w4a8_gemm_tcu
  * (backends/corex/kernels/w8a8_tcu.cu:453-574, called from
  * backends/corex/__init__.py:647). group_acc as in cmi_gemv_w4a8. */
 int cmi_gemm_w4a8(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs,

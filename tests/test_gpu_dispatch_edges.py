@@ -58,3 +58,35 @@ def test_add_rms_norm_i8_at_the_edges_of_a_row_s_wavefronts(orc, m, n):
     q_ref, s_ref = orc.quant_act_i8(y_ref)
     assert (G.bits(xd[rows]) == G.bits(total)).all() and (G.bits(y[rows]) == y_ref).all()
     assert (q[rows].cpu().numpy() == q_ref).all() and (s[rows].cpu().numpy() == s_ref).all()
+
+
+@pytest.mark.parametrize("gs", [128, 64, 256])
+@pytest.mark.parametrize("tile", [64, 128, 192, 128192, 256, 320, 321, 6464])
+@pytest.mark.parametrize("m,n,k", [(17, 33, 256), (129, 161, 256), (65, 97, 512), (130, 264, 768), (33, 129, 1024), (257, 40, 1280)])
+def test_w4a8_tiles_at_their_edges(orc, tile, m, n, k, gs):
+    """Every tile with a remainder in both directions, one to ten steps (fewer than it has stages, and whole chunks of
+    four and not), odd and 16-byte rows of results."""
+    g = synth.generator(m + n + k)
+    w = synth.int4_weight(n, k, g, group_size=gs)
+    x = synth.activations(m, k, g, outliers=True)
+    xq, xs = orc.quant_act_i8(G.bits(x))
+    _, y_ref = orc.linear_w4a8(xq, xs, w.packed.numpy(), w.scale.numpy(), k, gs)
+    w4, ws = G.w4_repack(w.packed.to(G.DEV), w.scale.to(G.DEV), k, gs)
+    G.set_option("gemm_tile", tile)
+    _, y = G.w4a8(w4, ws, G.dev(xq), G.dev(xs), k, gemm=True, want_acc=False, gs=gs)
+    assert (G.bits(y) == y_ref).all()
+
+
+@pytest.mark.parametrize("k", [128, 384, 640])
+def test_w4a8_tiles_with_a_step_count_that_is_no_whole_chunk(orc, k):
+    g = synth.generator(k)
+    n, m = 200, 70
+    w = synth.int4_weight(n, k, g)
+    x = synth.activations(m, k, g)
+    xq, xs = orc.quant_act_i8(G.bits(x))
+    _, y_ref = orc.linear_w4a8(xq, xs, w.packed.numpy(), w.scale.numpy(), k, 128)
+    w4, ws = G.w4_repack(w.packed.to(G.DEV), w.scale.to(G.DEV), k, 128)
+    for tile in (64, 128, 192, 128192, 256, 320, 321, 6464):
+        G.set_option("gemm_tile", tile)
+        _, y = G.w4a8(w4, ws, G.dev(xq), G.dev(xs), k, gemm=True, want_acc=False)
+        assert (G.bits(y) == y_ref).all(), tile
