@@ -40,8 +40,7 @@ int cmi_abi_version(void);
  *   "gemm_tile"     0 (the library chooses) | 64 | 128 | 192 | 256 | 320 (tile along n) | 6464 (64 x 64)
  *                   | 128192 (128 n x 192 m) | 321 (the 256 x 320 tile walked weight tile by weight
  *                   tile: what the library runs where it chooses that tile; 320 names the older
- *                   two-stage kernel) | 322 (321 as one workgroup per CU that walks its tiles one
- *                   after the other; measures the same as 321 and is never the library's choice):
+ *                   two-stage kernel; 322 is taken as 321):
  *                   block tile of cmi_gemm_w8a8 (non-zero also bypasses its few-row routes).
  *                   cmi_gemm_w4a8 has tiles of its own under the same values (m x n): 64 32 x 64,
  *                   128 128 x 128, 192 64 x 96, 128192 64 x 128, 256 32 x 128, 320 128 x 160, 321
