@@ -3,9 +3,13 @@
 //   acc[m,n] = sum_k xq[m,k] * wq[n,k]           int32, exact
 //   y[m,n]   = bf16((float)acc * xs[m] * ws[n])   left to right, one narrowing
 //
-// v_mfma_i32_32x32x32_i8 with the weight on the MFMA rows and the activation on
-// the MFMA columns, both K-contiguous in memory (16 consecutive k per lane), so
-// a lane ends with groups of four consecutive n of one m.
+// The weight is on the MFMA rows and the activation on the MFMA columns, both
+// K-contiguous in memory (16 consecutive k per lane), so a lane ends with groups
+// of four consecutive n of one m.  v_mfma_i32_16x16x64_i8 in the 8-wavefront kernels
+// the library chooses (256 x 256 and the tile-wise 256 x 320): they are bound by power,
+// and under random operands it sustains 12 % more than 32x32x32 for the same LDS
+// reads.  The 4-wavefront kernels keep 32x32x32: with one wavefront per SIMD the
+// shorter MFMAs measured 0..20 % slower (9728 -> 2560, 500 rows, 128 x 128 tile 35.4 -> 41.1 us).
 //
 // Common to both kernels below: K is walked in steps of 128 (one whole cache
 // line per row and request: with 64-byte steps every line is fetched from L2
@@ -514,12 +518,15 @@ int launch_split(Args &a, hipStream_t st) {
 // X tile of successive k steps (unit 2s = W of step s, unit 2s+1 = X of step s),
 // so that beside the two units being computed from, up to three are in flight or
 // landed -- with whole two-operand stages only two would fit and the memory
-// pipe would drain at every step.  Fragments are double-buffered per k quarter
-// (32 k), not per step, to stay within 256 registers.  One barrier per step:
+// pipe would drain at every step.  Fragments are double-buffered per quarter
+// step, not per step, to stay within 256 registers.  One barrier per step:
 // when the last quarter's fragments have been read the step's two slots are
 // free and take units 2s+5, 2s+6, while units 2s+2, 2s+3 must have landed (only
 // unit 2s+4 may still be in flight); those loads and the first fragments of
-// step s+1 are issued under the last quarter's MFMAs.
+// step s+1 are issued under the last quarter's MFMAs.  A quarter is two weight tiles
+// against both activation tiles in one k half (16x16x64 MFMAs want 64 k at a time).
+// With 32x32x32 MFMAs and quarters of 32 k: 8192 x 6144 x 2560 125.6 -> 115.0 us,
+// 8192 x 19456 404 -> 379, 2048 x 6144 37.7 -> 36.3, 500 x 19456 36.5 -> 36.6.
 namespace big {
 constexpr int BM = 256, BN = 256, TN = 4, TM = 2;
 constexpr int SLOT_BYTES = 256 * BK, SLOTS = 5;
@@ -566,64 +573,83 @@ gemm_w8a8_big_kernel(const Args a) {
             __builtin_amdgcn_global_load_lds((const void *)(xsrc[g] + ks * BK), (lds_ptr_t)(base + g * 1024), 16, 0, 0);
     };
 
-    const int frow = lane & 31;
+    // lane reads row (lane % 16) of a 16-row MFMA tile; for k half h its 16 bytes are k chunk 4h + lane / 16
+    const int frow = lane & 15;
     const int fsw = (frow >> 1) & 7;
-    int foff[4];
+    int foff[2];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) foff[q] = frow * BK + ((2 * q + (lane >> 5)) ^ fsw) * 16;
-    struct Frag {
-        v4i32 w[TN], x[TM];
+    for (int h = 0; h < 2; ++h) foff[h] = frow * BK + ((4 * h + (lane >> 4)) ^ fsw) * 16;
+    struct WFrag {  // two weight tiles, both row halves, one k half
+        v4i32 v[2][2];
     };
-    auto read_q = [&](int ks, int q, Frag &f) {
-        const int8_t *wt = lds + slot_of(2 * ks) + wn * 32 * TN * BK + foff[q];
-        const int8_t *xt = lds + slot_of(2 * ks + 1) + wm * 32 * TM * BK + foff[q];
+    struct XFrag {  // the activation tiles, both row halves, one k half
+        v4i32 v[TM][2];
+    };
+    // Quarter q of a step: weight tiles 2 (q % 2) and 2 (q % 2) + 1 in k half q / 2.
+    auto read_w = [&](int ks, int q, WFrag &f) {
+        const int8_t *wt = lds + slot_of(2 * ks) + (wn * 32 * TN + (q & 1) * 64) * BK + foff[q >> 1];
 #pragma unroll
-        for (int t = 0; t < TN; ++t) f.w[t] = *reinterpret_cast<const v4i32 *>(wt + t * 32 * BK);
+        for (int t = 0; t < 4; ++t) f.v[t >> 1][t & 1] = *reinterpret_cast<const v4i32 *>(wt + t * 16 * BK);
+    };
+    auto read_x = [&](int ks, int h, XFrag &f) {
+        const int8_t *xt = lds + slot_of(2 * ks + 1) + wm * 32 * TM * BK + foff[h];
 #pragma unroll
-        for (int t = 0; t < TM; ++t) f.x[t] = *reinterpret_cast<const v4i32 *>(xt + t * 32 * BK);
+        for (int t = 0; t < 2 * TM; ++t) f.v[t >> 1][t & 1] = *reinterpret_cast<const v4i32 *>(xt + t * 16 * BK);
     };
 
-    Acc32 acc[TN][TM];
+    Acc16 acc[TN][TM];
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
         for (int j = 0; j < TM; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j].v[v] = 0;
-    auto mma_q = [&](const Frag &f) {
+            for (int q = 0; q < 4; ++q) acc[i][j].v[q] = v4i32{0, 0, 0, 0};
+    auto mma_q = [&](auto pair_tag, const WFrag &w, const XFrag &x) {
+        constexpr int P = decltype(pair_tag)::value;
 #pragma unroll
-        for (int i = 0; i < TN; ++i)
+        for (int t = 0; t < 4; ++t)
 #pragma unroll
             for (int j = 0; j < TM; ++j)
-                acc[i][j].v = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.w[i], f.x[j], acc[i][j].v, 0, 0, 0);
+#pragma unroll
+                for (int mh = 0; mh < 2; ++mh) {
+                    v4i32 &c = acc[2 * P + (t >> 1)][j].v[2 * (t & 1) + mh];
+                    c = __builtin_amdgcn_mfma_i32_16x16x64_i8(w.v[t >> 1][t & 1], x.v[j][mh], c, 0, 0, 0);
+                }
     };
-    // 8 MFMAs with the 6 fragment reads of the next quarter spread between them
-    auto pace_quarter = [&]() {
+    using even_t = std::integral_constant<int, 0>;
+    using odd_t = std::integral_constant<int, 1>;
+    // 16 MFMAs with the next quarter's fragment reads (4, or 8 with activations) spread between them
+    auto pace_quarter = [&](auto reads_tag) {
+        constexpr int PER = decltype(reads_tag)::value / 4;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (i < 6) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            if (i < 4) __builtin_amdgcn_sched_group_barrier(0x100, PER, 0);
         }
     };
+    using w_only_t = std::integral_constant<int, 4>;
+    using w_and_x_t = std::integral_constant<int, 8>;
 
     const int ksteps = a.K / BK;
-    Frag f0, f1;
-    // Step ks computes from units 2ks, 2ks+1 (first-quarter fragments in f0).
+    WFrag w0, w1;
+    XFrag x0, x1;
+    // Step ks computes from units 2ks, 2ks+1 (first-quarter fragments in w0, x0).
     // PHASE 2: steady state, two more units are requested (W of step ks+3 goes to
     // the slot of this step's X... no slot arithmetic is needed: unit u always
     // lives in slot u % 5, and units 2ks+5, 2ks+6 map onto the slots of 2ks, 2ks+1).
     // PHASE 1: only unit 2ks+5 exists (X of step ks+2).  PHASE 0: nothing left.
     auto step = [&](auto phase_tag, int ks) {
         constexpr int PHASE = decltype(phase_tag)::value;
-        read_q(ks, 1, f1);
-        mma_q(f0);
-        pace_quarter();
-        read_q(ks, 2, f0);
-        mma_q(f1);
-        pace_quarter();
-        read_q(ks, 3, f1);
-        mma_q(f0);
-        pace_quarter();
+        read_w(ks, 1, w1);
+        mma_q(even_t{}, w0, x0);
+        pace_quarter(w_only_t{});
+        read_w(ks, 2, w0);
+        read_x(ks, 1, x1);
+        mma_q(odd_t{}, w1, x0);
+        pace_quarter(w_and_x_t{});
+        read_w(ks, 3, w1);
+        mma_q(even_t{}, w0, x1);
+        pace_quarter(w_only_t{});
         // this wavefront's reads of the step's slots are done; units 2ks+2, 2ks+3 landed
         if constexpr (PHASE == 2) wait_vmcnt<LPU>();
         else wait_vmcnt<0>();
@@ -631,14 +657,15 @@ gemm_w8a8_big_kernel(const Args a) {
         asm volatile("" ::: "memory");
         if constexpr (PHASE >= 1) issue_x(ks + 2);
         if constexpr (PHASE == 2) issue_w(ks + 3);
-        read_q(ks + 1, 0, f0);  // past the last step: a stale slot nobody uses
-        mma_q(f1);
-        constexpr int VM_SLOTS = PHASE * 2;  // two loads per MFMA
+        read_w(ks + 1, 0, w0);  // past the last step: a stale slot nobody uses
+        read_x(ks + 1, 0, x0);
+        mma_q(odd_t{}, w1, x1);
+        constexpr int VM_SLOTS = PHASE * 2;  // two loads per pair of MFMAs
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
             if (i < VM_SLOTS) __builtin_amdgcn_sched_group_barrier(0x010, 2, 0);
-            else if (i - VM_SLOTS < 3) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            else if (i - VM_SLOTS < 3) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
         }
     };
     using steady_t = std::integral_constant<int, 2>;
@@ -662,7 +689,8 @@ gemm_w8a8_big_kernel(const Args a) {
     }
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    read_q(0, 0, f0);
+    read_w(0, 0, w0);
+    read_x(0, 0, x0);
     // Step ks requests X of step ks+2 and W of step ks+3.
     int ks = 0;
     for (; ks + 3 < ksteps; ++ks) step(steady_t{}, ks);
