@@ -330,6 +330,7 @@ gemv_w8a16_kernel(const GemvArgs a) {
         auto consume = [&](const WStage<R, CHT> &w, int t) {
 #pragma unroll
             for (int mh = 0; mh < MH; ++mh) {
+                if (M == 16 && mh * MT >= a.M) break;  // 9..12 rows: three tiles of four do
                 // keep one activation tile in registers: no LDS reads of the next
                 // tile hoisted above this one's arithmetic (other wavefronts fill in)
                 load_x(x0, u, t, mh);
@@ -573,6 +574,14 @@ Plan make_plan(int M, int N, int K) {
     // reads of the activation fragments (154 -> 133 us at 2560 -> 151936); on the layer shapes, and
     // at 16 rows (registers), two rows stay faster.
     if (p.mt == 8 && N >= 65536) p.r = 4;
+    // The same at three and four rows, one segment of K at a time (registers: the next one's weights are in
+    // flight), where K is one unit: 2560 -> 151936 75.4 -> 72.1 / 85.3 -> 75.2 us at three / four rows; 2560 -> 19456 12.9 -> 14.0,
+    // 2560 -> 6144 6.0 -> 6.4 stay with two rows.
+    if (p.mt == 4 && N >= 65536 && units == 1 && unit >= 2) p.r = 4, p.cht = 1, p.mode = 2;
+    // 9..16 rows put 16 wavefronts in a workgroup: with two weight rows each, up to 4096 outputs would be at most 128
+    // workgroups.  4096 -> 2560 at 16 rows 16.6 -> 11.0 us; with more outputs the shared fragments win
+    // (2560 -> 6144 14.4 against 15.8).
+    if (p.mt == 16 && N <= 4096) p.r = 1;
     return p;
 }
 
@@ -648,8 +657,9 @@ int dispatch_ch(GemvArgs &a, const Plan &p, hipStream_t st) {
 template <int M>
 int dispatch_r(GemvArgs &a, const Plan &p, hipStream_t st) {
     if (p.r == 2) return dispatch_ch<M, 2>(a, p, st);
-    if constexpr (M == 1) if (p.r == 1) return dispatch_ch<M, 1>(a, p, st);
+    if constexpr (M == 1 || M == 16) if (p.r == 1) return dispatch_ch<M, 1>(a, p, st);
     if constexpr (M == 8) if (p.r == 4) return dispatch_ch<M, 4>(a, p, st);
+    if constexpr (M == 4) if (p.r == 4) return dispatch_x<M, 4, 1>(a, p, st);  // make_plan: one segment at a time
     return fail(CMI_E_UNSUPPORTED, "cmi_gemv_w8a16: no kernel for %d rows per block", p.r);
 }
 

@@ -90,3 +90,24 @@ def test_w4a8_tiles_with_a_step_count_that_is_no_whole_chunk(orc, k):
         G.set_option("gemm_tile", tile)
         _, y = G.w4a8(w4, ws, G.dev(xq), G.dev(xs), k, gemm=True, want_acc=False)
         assert (G.bits(y) == y_ref).all(), tile
+
+
+@pytest.mark.parametrize("n,k", [(65535, 2064), (65536, 1040), (65537, 3072), (70001, 4096), (65536, 1024), (65600, 4112), (300, 2560),
+                                 (4096, 4096), (4097, 4096), (33, 9728)])
+def test_weight_only_rows_keep_the_single_row_s_bits_at_the_edges_of_the_row_blocks(n, k):
+    """Four weight rows per wavefront for very tall weights at 3..4 rows, one at 9..16 rows and few outputs, three
+    tiles of activation rows at 9..12: integers of both signs, every row against the call with that row alone."""
+    gen = torch.Generator(device=G.DEV).manual_seed(n + k)
+    wq = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=G.DEV, generator=gen)
+    ws = torch.rand(n, device=G.DEV, generator=gen) * 0.01
+    x = torch.randn((16, k), device=G.DEV, generator=gen).to(torch.bfloat16)
+    lib = _native.load()
+
+    def call(rows):
+        y = torch.full((rows.shape[0], n), float("nan"), dtype=torch.bfloat16, device=G.DEV)
+        _native.check(lib.cmi_gemv_w8a16(G.ptr(wq), G.ptr(ws), G.ptr(rows), G.ptr(y), rows.shape[0], n, k, G.stream()), "gemv")
+        return y
+
+    ref = torch.cat([call(x[r:r + 1].contiguous()) for r in range(16)])
+    for m in (3, 4, 8, 9, 12, 13, 16):
+        assert torch.equal(call(x[:m].contiguous()).view(torch.int16), ref[:m].view(torch.int16)), m
