@@ -29,7 +29,7 @@
 //   gemm_w8a8_pipe_kernel: 128 x 128 block tile, 4 wavefronts of 64 x 64, two
 //     LDS stages, whole-step fragment double buffering in registers, two
 //     workgroups per CU (one's prologue/epilogue hides under the other's MFMAs).
-//   gemm_w8a8_big_kernel: 256 x 256 block tile, 8 wavefronts of 128 x 64, a ring
+//   gemm_w8a8_big_kernel: 256 x 256 (and 192 x 256) block tile, 8 wavefronts, a ring
 //     of five single-operand LDS slots.  Half the L2 -> LDS bytes per MFMA.
 //   gemm_w8a8_wide_kernel: 256 x 320 block tile, 8 wavefronts of 64 x 160, two LDS
 //     stages; for shapes whose n extent tiles better by 320 (9728 = 30.4 x 320).
@@ -94,9 +94,11 @@ __device__ __forceinline__ void wait_vmcnt() {
     else if constexpr (N == 3) asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)" ::: "memory");
     else if constexpr (N == 4) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
     else if constexpr (N == 6) asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
+    else if constexpr (N == 7) asm volatile("s_waitcnt vmcnt(7) lgkmcnt(0)" ::: "memory");
     else if constexpr (N == 8) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
     else if constexpr (N == 9) asm volatile("s_waitcnt vmcnt(9) lgkmcnt(0)" ::: "memory");
     else if constexpr (N == 10) asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)" ::: "memory");
+    else if constexpr (N == 11) asm volatile("s_waitcnt vmcnt(11) lgkmcnt(0)" ::: "memory");
     else if constexpr (N == 12) asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)" ::: "memory");
     else if constexpr (N == 16) asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
     else if constexpr (N == 18) asm volatile("s_waitcnt vmcnt(18) lgkmcnt(0)" ::: "memory");
@@ -512,7 +514,8 @@ int launch_split(Args &a, hipStream_t st) {
 
 // ---------------------------------------------------------------------------
 // 256 x 256 block tile, 8 wavefronts (2 along n x 4 along m, two per SIMD), each
-// 128(n) x 64(m) = 4 x 2 MFMA tiles.  The operand bytes a CU must pull from L2
+// 128(n) x 64(m) = 4 x 2 pieces of 32 x 32, or 192(m) x 256(n), 4 x 2 wavefronts of
+// 64(n) x 96(m) = 2 x 3 (whole-tile counts: see the tile choice).  The operand bytes a CU must pull from L2
 // per MFMA cycle halve against the 128 x 128 tile, which is what bounds that
 // kernel.  LDS is a ring of five 32 KiB slots; the ring units alternate W tile,
 // X tile of successive k steps (unit 2s = W of step s, unit 2s+1 = X of step s),
@@ -523,53 +526,66 @@ int launch_split(Args &a, hipStream_t st) {
 // when the last quarter's fragments have been read the step's two slots are
 // free and take units 2s+5, 2s+6, while units 2s+2, 2s+3 must have landed (only
 // unit 2s+4 may still be in flight); those loads and the first fragments of
-// step s+1 are issued under the last quarter's MFMAs.  A quarter is two weight tiles
-// against both activation tiles in one k half (16x16x64 MFMAs want 64 k at a time).
+// step s+1 are issued under the last quarter's MFMAs.  A quarter is half of the weight
+// tiles against all activation tiles in one k half (16x16x64 MFMAs want 64 k at a time).
 // With 32x32x32 MFMAs and quarters of 32 k: 8192 x 6144 x 2560 125.6 -> 115.0 us,
 // 8192 x 19456 404 -> 379, 2048 x 6144 37.7 -> 36.3, 500 x 19456 36.5 -> 36.6.
 namespace big {
-constexpr int BM = 256, BN = 256, TN = 4, TM = 2;
+constexpr int BN = 256;
 constexpr int SLOT_BYTES = 256 * BK, SLOTS = 5;
-constexpr int PARK_BYTES = 8 * 32 * TM * (64 * TN + 16);
-constexpr int LDS_BYTES = SLOTS * SLOT_BYTES > PARK_BYTES ? SLOTS * SLOT_BYTES : PARK_BYTES;
-constexpr int LPU = 4;  // loads per wavefront and unit
+constexpr int WL = 4;  // loads per wavefront and weight unit
+// TN x TM pieces of 32 x 32 per wavefront, 8 / TN wavefronts along n: 4 x 2 is the 256(m) tile, 2 x 3 the 192(m) one.
+template <int TN, int TM>
+struct Cfg {
+    static constexpr int WAVES_N = 8 / TN, BM = 32 * TM * (8 / WAVES_N);
+    static constexpr int XL = BM / 64;  // loads per wavefront and activation unit
+    static constexpr int PARK_BYTES = 8 * 32 * TM * (64 * TN + 16);
+    static constexpr int LDS_BYTES = SLOTS * SLOT_BYTES > PARK_BYTES ? SLOTS * SLOT_BYTES : PARK_BYTES;
+    static_assert(BM <= 256, "an activation unit is one slot");
+};
 }  // namespace big
 
+template <int TN, int TM>
 __global__ void __launch_bounds__(512, 2)
 gemm_w8a8_big_kernel(const Args a) {
     using namespace big;
+    using C = big::Cfg<TN, TM>;
+    constexpr int BM = C::BM, XL = C::XL, WT = TN / 2;
     extern __shared__ __align__(16) int8_t lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wn = wave & 1, wm = wave >> 1;
+    const int wn = wave % C::WAVES_N, wm = wave / C::WAVES_N;
 
     int tm, tn;
     tile_coords(a, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
 
-    // Wavefront w fills rows 32w .. 32w+31 of an operand tile: 4 loads of
+    // Wavefront w fills a contiguous run of an operand tile's rows, BM / 8 (256 / 8) of them: loads of
     // 8 rows x 128 B each; slot and swizzle as in the 4-wavefront kernel.
     const int lrow = lane >> 3;
-    const int8_t *wsrc[4], *xsrc[4];
+    const int8_t *wsrc[WL], *xsrc[XL];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        const int row = (4 * wave + g) * 8 + lrow;
-        const int kc = (lane & 7) ^ ((row >> 1) & 7);
-        wsrc[g] = a.wq + (size_t)min(n0 + row, a.N - 1) * a.K + kc * 16;
-        xsrc[g] = a.xq + (size_t)min(m0 + row, a.M - 1) * a.K + kc * 16;
+    for (int g = 0; g < WL; ++g) {
+        const int row = (WL * wave + g) * 8 + lrow;
+        wsrc[g] = a.wq + (size_t)min(n0 + row, a.N - 1) * a.K + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+    }
+#pragma unroll
+    for (int g = 0; g < XL; ++g) {
+        const int row = (XL * wave + g) * 8 + lrow;
+        xsrc[g] = a.xq + (size_t)min(m0 + row, a.M - 1) * a.K + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
     }
     // ring slot of a unit, as a byte offset
     auto slot_of = [](int unit) { return (unit % SLOTS) * SLOT_BYTES; };
     auto issue_w = [&](int ks) {
-        int8_t *base = lds + slot_of(2 * ks) + (4 * wave) * 1024;
+        int8_t *base = lds + slot_of(2 * ks) + (WL * wave) * 1024;
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
+        for (int g = 0; g < WL; ++g)
             __builtin_amdgcn_global_load_lds((const void *)(wsrc[g] + ks * BK), (lds_ptr_t)(base + g * 1024), 16, 0, 0);
     };
     auto issue_x = [&](int ks) {
-        int8_t *base = lds + slot_of(2 * ks + 1) + (4 * wave) * 1024;
+        int8_t *base = lds + slot_of(2 * ks + 1) + (XL * wave) * 1024;
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
+        for (int g = 0; g < XL; ++g)
             __builtin_amdgcn_global_load_lds((const void *)(xsrc[g] + ks * BK), (lds_ptr_t)(base + g * 1024), 16, 0, 0);
     };
 
@@ -579,17 +595,17 @@ gemm_w8a8_big_kernel(const Args a) {
     int foff[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) foff[h] = frow * BK + ((4 * h + (lane >> 4)) ^ fsw) * 16;
-    struct WFrag {  // two weight tiles, both row halves, one k half
-        v4i32 v[2][2];
+    struct WFrag {  // half of the weight tiles, both row halves, one k half
+        v4i32 v[WT][2];
     };
     struct XFrag {  // the activation tiles, both row halves, one k half
         v4i32 v[TM][2];
     };
-    // Quarter q of a step: weight tiles 2 (q % 2) and 2 (q % 2) + 1 in k half q / 2.
+    // Quarter q of a step: weight tiles WT (q % 2) .. in k half q / 2.
     auto read_w = [&](int ks, int q, WFrag &f) {
-        const int8_t *wt = lds + slot_of(2 * ks) + (wn * 32 * TN + (q & 1) * 64) * BK + foff[q >> 1];
+        const int8_t *wt = lds + slot_of(2 * ks) + (wn * 32 * TN + (q & 1) * WT * 32) * BK + foff[q >> 1];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) f.v[t >> 1][t & 1] = *reinterpret_cast<const v4i32 *>(wt + t * 16 * BK);
+        for (int t = 0; t < 2 * WT; ++t) f.v[t >> 1][t & 1] = *reinterpret_cast<const v4i32 *>(wt + t * 16 * BK);
     };
     auto read_x = [&](int ks, int h, XFrag &f) {
         const int8_t *xt = lds + slot_of(2 * ks + 1) + wm * 32 * TM * BK + foff[h];
@@ -607,28 +623,29 @@ gemm_w8a8_big_kernel(const Args a) {
     auto mma_q = [&](auto pair_tag, const WFrag &w, const XFrag &x) {
         constexpr int P = decltype(pair_tag)::value;
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < 2 * WT; ++t)
 #pragma unroll
             for (int j = 0; j < TM; ++j)
 #pragma unroll
                 for (int mh = 0; mh < 2; ++mh) {
-                    v4i32 &c = acc[2 * P + (t >> 1)][j].v[2 * (t & 1) + mh];
+                    v4i32 &c = acc[WT * P + (t >> 1)][j].v[2 * (t & 1) + mh];
                     c = __builtin_amdgcn_mfma_i32_16x16x64_i8(w.v[t >> 1][t & 1], x.v[j][mh], c, 0, 0, 0);
                 }
     };
     using even_t = std::integral_constant<int, 0>;
     using odd_t = std::integral_constant<int, 1>;
-    // 16 MFMAs with the next quarter's fragment reads (4, or 8 with activations) spread between them
+    // a quarter's MFMAs, in pairs, with the next one's fragment reads spread between the first of them
+    constexpr int PAIRS = 2 * WT * TM;
     auto pace_quarter = [&](auto reads_tag) {
-        constexpr int PER = decltype(reads_tag)::value / 4;
+        constexpr int READS = decltype(reads_tag)::value, PER = READS > PAIRS - 2 ? 2 : 1;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < PAIRS; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-            if (i < 4) __builtin_amdgcn_sched_group_barrier(0x100, PER, 0);
+            if (i * PER < READS) __builtin_amdgcn_sched_group_barrier(0x100, PER, 0);
         }
     };
-    using w_only_t = std::integral_constant<int, 4>;
-    using w_and_x_t = std::integral_constant<int, 8>;
+    using w_only_t = std::integral_constant<int, 2 * WT>;
+    using w_and_x_t = std::integral_constant<int, 2 * WT + 2 * TM>;
 
     const int ksteps = a.K / BK;
     WFrag w0, w1;
@@ -651,7 +668,7 @@ gemm_w8a8_big_kernel(const Args a) {
         mma_q(even_t{}, w0, x1);
         pace_quarter(w_only_t{});
         // this wavefront's reads of the step's slots are done; units 2ks+2, 2ks+3 landed
-        if constexpr (PHASE == 2) wait_vmcnt<LPU>();
+        if constexpr (PHASE == 2) wait_vmcnt<WL>();
         else wait_vmcnt<0>();
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -660,12 +677,14 @@ gemm_w8a8_big_kernel(const Args a) {
         read_w(ks + 1, 0, w0);  // past the last step: a stale slot nobody uses
         read_x(ks + 1, 0, x0);
         mma_q(odd_t{}, w1, x1);
-        constexpr int VM_SLOTS = PHASE * 2;  // two loads per pair of MFMAs
+        constexpr int N_VM = PHASE == 2 ? XL + WL : PHASE == 1 ? XL : 0;
+        constexpr int VM_SLOTS = (N_VM + 1) / 2;  // two loads per pair of MFMAs
+        constexpr int READS = 2 * WT + 2 * TM, DS_PER = (READS + PAIRS - VM_SLOTS - 2) / (PAIRS - VM_SLOTS - 1);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < PAIRS; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
             if (i < VM_SLOTS) __builtin_amdgcn_sched_group_barrier(0x010, 2, 0);
-            else if (i - VM_SLOTS < 3) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+            else if ((i - VM_SLOTS) * DS_PER < READS) __builtin_amdgcn_sched_group_barrier(0x100, DS_PER, 0);
         }
     };
     using steady_t = std::integral_constant<int, 2>;
@@ -681,9 +700,9 @@ gemm_w8a8_big_kernel(const Args a) {
     }
     if (ksteps > 2) {
         issue_w(2);
-        wait_vmcnt<3 * LPU>();
+        wait_vmcnt<2 * WL + XL>();
     } else if (ksteps > 1) {
-        wait_vmcnt<2 * LPU>();
+        wait_vmcnt<WL + XL>();
     } else {
         wait_vmcnt<0>();
     }
@@ -700,14 +719,16 @@ gemm_w8a8_big_kernel(const Args a) {
     epilogue<TN, TM>(a, acc, lds, wave, lane, n0 + wn * 32 * TN, m0 + wm * 32 * TM);
 }
 
+template <int TN, int TM>
 int launch_big(Args &a, hipStream_t st) {
-    a.tiles_m = (a.M + big::BM - 1) / big::BM;
+    using C = big::Cfg<TN, TM>;
+    a.tiles_m = (a.M + C::BM - 1) / C::BM;
     a.tiles_n = (a.N + big::BN - 1) / big::BN;
     static std::atomic<uint64_t> devices{0};
-    if (const int rc = reserve_lds(reinterpret_cast<const void *>(gemm_w8a8_big_kernel),
-                                   big::LDS_BYTES, devices, "cmi_gemm_w8a8"))
+    if (const int rc = reserve_lds(reinterpret_cast<const void *>(gemm_w8a8_big_kernel<TN, TM>), C::LDS_BYTES, devices,
+                                   "cmi_gemm_w8a8"))
         return rc;
-    gemm_w8a8_big_kernel<<<dim3(a.tiles_m * a.tiles_n), dim3(512), big::LDS_BYTES, st>>>(a);
+    gemm_w8a8_big_kernel<TN, TM><<<dim3(a.tiles_m * a.tiles_n), dim3(512), C::LDS_BYTES, st>>>(a);
     return check_launch("cmi_gemm_w8a8");
 }
 
@@ -1302,10 +1323,14 @@ int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, co
     // same form as for 17..256 rows, fitted to cold-weight measurements of every kernel on
     // sixteen layer shapes x eleven batch sizes (272..8192 rows): their choice is 0.3 % above the
     // best measured in total, the fill-and-area rule this replaces 2.4 % (and up to 40 % on
-    // single shapes, e.g. 2048 x 9728 -> 2560: 84 -> 63 us).
+    // single shapes, e.g. 2048 x 9728 -> 2560: 84 -> 63 us).  The 192(m) x 256(n) tile fills the gap between
+    // 4-wavefront tiles that need two rounds and 256-row ones that leave CUs idle: 500 x 19456 x 2560
+    // 38.0 -> 34.9 us (228 tiles instead of 152), 1152 x 19456 76.5 -> 65.2, 768 x 11008 x 4096 50.9 -> 44.9,
+    // 2048 x 11008 x 4096 103 -> 92; it and 256 x 320 are fitted to a sweep of eight shapes x twelve
+    // batch sizes, where the choice is 0.2 % above the best (1.9 % without it).
     // CMI_GEMM_TILE=64|128|192|256|320 overrides the tile along n (tests, tuning); 128192 forces
-    // 128(n) x 192(m), 6464 the 64 x 64 tile of the mid-batch route.
-    int pick;  // 64, 128, 192, 256 or 320: block tile along n; 128192; 6464
+    // 128(n) x 192(m), 256192 256(n) x 192(m), 6464 the 64 x 64 tile of the mid-batch route.
+    int pick;  // 64, 128, 192, 256 or 320: block tile along n; 128192; 256192; 6464
     if (force || mid) {
         pick = force ? force : mid;
     } else {
@@ -1313,7 +1338,7 @@ int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, co
         auto cost = [&](int bm, int bn, double a0, double b0, double c0) {
             const double tiles = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
             // the 4-wavefront tiles on up to 192 CUs: the idle CUs warm the caches (see above)
-            const double warmed = bm <= 192 && tiles <= 192 && (double)N * K <= 64.0 * 1048576.0 ? 0.8 : 1.0;
+            const double warmed = bm <= 192 && bn <= 192 && tiles <= 192 && (double)N * K <= 64.0 * 1048576.0 ? 0.8 : 1.0;
             return 2.5 + steps * (a0 + b0 * N) * warmed * (1.0 + c0 * (ceil(tiles / 256.0) - 1.0));
         };
         const struct { int pick; double us; } candidates[] = {
@@ -1322,7 +1347,8 @@ int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, co
             {192, cost(128, 192, 0.723, 1.89e-5, 1.03)},
             {128192, cost(192, 128, 0.709, 1.19e-5, 1.12)},
             {256, cost(256, 256, 1.29, 2.33e-5, 1.28)},
-            {320, cost(256, 320, 1.60, 3.39e-5, 1.13)},
+            {320, cost(256, 320, 1.634, 1.73e-5, 1.19)},
+            {256192, cost(192, 256, 1.175, 1.32e-5, 1.07)},
         };
         pick = 128;
         double best = 1e30;
@@ -1350,7 +1376,8 @@ int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, co
     // 7 % faster at 2048 x 4096 x 2560); a forced 320 still names the two-stage kernel
     if (pick == 321 || pick == 322 || (pick == 320 && !force)) return launch_wide_tilewise(a, st);
     if (pick == 320) return launch_wide(a, st);
-    if (pick == 256) return launch_big(a, st);
+    if (pick == 256) return launch_big<4, 2>(a, st);
+    if (pick == 256192) return launch_big<2, 3>(a, st);
     if (pick == 192) return launch<3, 2, 3>(a, st);
     if (pick == 128192) return launch<2, 3, 3>(a, st);
     // 64 x 64 tiles, four LDS stages (more stages measured the same): half the bytes per step and

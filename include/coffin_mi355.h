@@ -38,7 +38,7 @@ int cmi_abi_version(void);
 
 /* Kernel-selection override for tests and tuning; no counterpart in the reference.
  *   "gemm_tile"     0 (the library chooses) | 64 | 128 | 192 | 256 | 320 (tile along n) | 6464 (64 x 64)
- *                   | 128192 (128 n x 192 m) | 321 (the 256 x 320 tile walked weight tile by weight
+ *                   | 128192 (128 n x 192 m) | 256192 (256 n x 192 m) | 321 (the 256 x 320 tile walked weight tile by weight
  *                   tile: what the library runs where it chooses that tile; 320 names the older
  *                   two-stage kernel; 322 is taken as 321):
  *                   block tile of cmi_gemm_w8a8 (non-zero also bypasses its few-row routes).

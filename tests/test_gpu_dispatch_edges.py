@@ -111,3 +111,17 @@ def test_weight_only_rows_keep_the_single_row_s_bits_at_the_edges_of_the_row_blo
     ref = torch.cat([call(x[r:r + 1].contiguous()) for r in range(16)])
     for m in (3, 4, 8, 9, 12, 13, 16):
         assert torch.equal(call(x[:m].contiguous()).view(torch.int16), ref[:m].view(torch.int16)), m
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 24, 128), (192, 256, 256), (193, 257, 384), (500, 300, 512), (385, 1000, 640), (576, 520, 2560),
+                                   (31, 513, 4096)])
+def test_192_row_tile_of_the_w8a8_gemm(orc, m, n, k):
+    """Ragged in both directions, one to many K steps."""
+    gen = synth.generator(m + n + k)
+    q = synth.int8_weight(n, k, gen)
+    x = synth.activations(m, k, gen, outliers=True)
+    xq, xs = orc.quant_act_i8(G.bits(x))
+    acc_ref, y_ref = orc.gemm_w8a8(xq, q.wq.numpy(), xs, q.scale.numpy())
+    G.set_option("gemm_tile", 256192)  # (conftest resets it)
+    acc, y = G.gemm_w8a8(G.dev(xq), q.wq.to(G.DEV), G.dev(xs), q.scale.to(G.DEV))
+    assert (acc.cpu().numpy() == acc_ref).all() and (G.bits(y) == y_ref).all()
