@@ -261,10 +261,11 @@ struct NormArgs {
 
 // The mean is the correctly rounded quotient: one Newton correction of ss * (1 / N) leaves an error near
 // 2^-104, and a quotient of a 53-bit number by an N below 2^31 stays further than that from every
-// rounding boundary.
+// rounding boundary.  A row with an infinity has an infinite mean and so the scale 0 (the correction would be
+// inf - inf); a NaN stays one.
 __device__ __forceinline__ float inv_rms(double ss, const NormArgs &a) {
     const double q = ss * a.rcp_n;
-    const double mean = fma(fma(-q, (double)a.N, ss), a.rcp_n, q);
+    const double mean = q < __builtin_inf() ? fma(fma(-q, (double)a.N, ss), a.rcp_n, q) : q;
     return __fdiv_rn(1.0f, __fsqrt_rn((float)mean + a.eps));
 }
 

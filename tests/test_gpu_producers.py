@@ -186,6 +186,41 @@ def test_rms_norm_i8_adapter_and_special_rows(orc):
         backend.rms_norm_i8(x.float(), w, out_q, out_s)
 
 
+def _same_or_both_nan(orc, got_bits, want_bits):
+    got, want = orc.bf16_to_f32(got_bits), orc.bf16_to_f32(want_bits)
+    nan = np.isnan(want)
+    return (np.isnan(got) == nan).all() and (got_bits[~nan] == want_bits[~nan]).all()
+
+
+@pytest.mark.parametrize("m,n", [(6, 512), (300, 512), (6, 2560), (257, 1032), (6, 16384), (6, 1001), (6, 33000)])
+@pytest.mark.parametrize("with_add", [False, True])
+def test_rms_norm_of_rows_that_hold_infinities_or_nan(orc, m, n, with_add):
+    """An infinity makes the mean infinite and the scale 0: the row's finite elements become 0 and the infinite
+    ones NaN, as in the oracle and in torch; a NaN makes the whole row NaN.  Every layout of the kernel, with
+    and without the quantised rows, whose scale and codes are those of the quantiser on the rows as written."""
+    g = synth.generator(m + n)
+    x = torch.randn((m, n), generator=g).to(torch.bfloat16)
+    x[1, 3], x[2, n - 1], x[3, 7] = float("inf"), float("-inf"), float("nan")
+    x[4, 0], x[4, n // 2] = float("inf"), float("-inf")
+    add = torch.randn((m, n), generator=g).to(torch.bfloat16) if with_add else None
+    w = (1.0 + 0.1 * torch.randn(n, generator=g)).to(torch.bfloat16)
+    y_ref, _ = orc.rms_norm(G.bits(x), G.bits(w), 1e-6, None if add is None else G.bits(add))
+    wd, ad = w.to(G.DEV), None if add is None else add.to(G.DEV)
+    y, q, s = _rms_norm_i8(x.to(G.DEV), wd, ad)
+    assert _same_or_both_nan(orc, G.bits(y), y_ref)
+    assert (y[1, :3].float() == 0).all() and (y[2, :-1].float() == 0).all()
+    q2, s2 = G.quant(y)
+    assert (s.view(torch.int32) == s2.view(torch.int32)).all()
+    finite = ~torch.isnan(y.float())                               # the code of a NaN element is nobody's promise
+    assert (q[finite] == q2[finite]).all()
+    if with_add:
+        out = torch.empty_like(y)
+        backend.add_rms_norm(x.to(G.DEV), ad, wd, out)
+    else:
+        out = backend.rms_norm(x.to(G.DEV), wd)
+    assert _same_or_both_nan(orc, G.bits(out), y_ref)
+
+
 def test_rms_norm_table_entries_share_the_fused_arithmetic(orc):
     """rms_norm / add_rms_norm of the table followed by kv_quant give what rms_norm_i8 gives."""
     g = synth.generator(11, G.DEV)
