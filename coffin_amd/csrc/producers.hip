@@ -70,6 +70,14 @@ __device__ __forceinline__ double block_sum(double v, double *smem) {
     return r;
 }
 
+// A launch holds fewer than 2^32 threads: more rows than that allows run in slices of whole rows.
+// launch(first row, rows) is called for each.
+template <typename LAUNCH>
+void in_row_slices(int M, long threads_per_row, LAUNCH launch) {
+    const long step = std::max(1L, INT32_MAX / threads_per_row);
+    for (long lo = 0; lo < M; lo += step) launch(lo, (int)std::min(step, M - lo));
+}
+
 // ----------------------------------------------------------------- silu
 
 // silu(g) for a bf16 g as the fp32 value whose narrowing is the result: g / (1 + exp(-g))
@@ -163,6 +171,11 @@ struct SiluArgs {
     float *s;
     int K;
     long ldg, ldu, ldo;
+
+    SiluArgs from_row(long r) const {
+        return {gate + r * ldg, up + r * ldu, out ? out + r * ldo : nullptr, q ? q + r * K : nullptr, s ? s + r : nullptr,
+                K, ldg, ldu, ldo};
+    }
 };
 
 // K % 8 == 0, every row 16-byte aligned; the row fits VPT vectors per thread.  A workgroup per row, all
@@ -257,6 +270,11 @@ struct NormArgs {
     long ldx, lda, ldy;
     float eps;
     double rcp_n;         // 1 / N, rounded
+
+    NormArgs from_row(long r) const {
+        return {x + r * ldx, add ? add + r * lda : nullptr, w, y ? y + r * ldy : nullptr, q ? q + r * N : nullptr,
+                s ? s + r : nullptr, N, ldx, lda, ldy, eps, rcp_n};
+    }
 };
 
 // The mean is the correctly rounded quotient: one Newton correction of ss * (1 / N) leaves an error near
@@ -432,24 +450,25 @@ int norm_entry(const char *who, uint16_t *x, const uint16_t *add, const void *w,
     const bool vec = N % 8 == 0 && nvec <= 4 * MAX_THREADS && aligned(x, 16) && ldx % 8 == 0 && aligned(w, 16) &&
                      (!add || (aligned(add, 16) && lda % 8 == 0)) && (!y || (aligned(y, 16) && ldy % 8 == 0)) &&
                      (!q || aligned(q, 8));
-    if (vec) {
-        const int waves = norm_waves(M, nvec);
-        add ? launch_norm<true>(a, M, waves, st) : launch_norm<false>(a, M, waves, st);
-    }
-    else
-        rms_norm_i8_scalar<<<dim3(M), dim3(THREADS), 0, st>>>(a);
+    const int waves = vec ? norm_waves(M, nvec) : THREADS / 64;
+    in_row_slices(M, 64 * waves, [&](long lo, int rows) {
+        const NormArgs part = a.from_row(lo);
+        if (!vec) rms_norm_i8_scalar<<<dim3(rows), dim3(THREADS), 0, st>>>(part);
+        else if (add) launch_norm<true>(part, rows, waves, st);
+        else launch_norm<false>(part, rows, waves, st);
+    });
     return check_launch(who);
 }
 
 // Threads per row: one per 16-byte vector for a few rows, one per two of them otherwise (2048 x 4096: 17.2
 // us with one each, 15.7 with two), more vectors where the row would need over 1024 threads; a power of two of
 // wavefronts, so that the workgroup loads the four SIMDs alike (2048 x 14336: 45 us on 14, 41 on 16).
-void launch_silu(const SiluArgs &a, int M, hipStream_t st) {
+void launch_silu(const SiluArgs &a, int rows, int M, hipStream_t st) {
     const int nvec = a.K / 8;
     const int vpt = std::max(M <= FEW_ROWS ? 1 : 2, (nvec + MAX_THREADS - 1) / MAX_THREADS);
     int threads = 64;
     while (threads * vpt < nvec) threads *= 2;
-    const dim3 grid(M), block(threads);
+    const dim3 grid(rows), block(threads);
     if (vpt == 1) silu_mul_quant_vec<1><<<grid, block, 0, st>>>(a);
     else if (vpt == 2) silu_mul_quant_vec<2><<<grid, block, 0, st>>>(a);
     else if (vpt == 3) silu_mul_quant_vec<3><<<grid, block, 0, st>>>(a);
@@ -474,10 +493,13 @@ extern "C" int cmi_silu_mul_quant(const void *gate, const void *up, void *out, i
     const bool vec = K % 8 == 0 && aligned(gate, 16) && aligned(up, 16) && ld_gate % 8 == 0 &&
                      ld_up % 8 == 0 && (!out || (aligned(out, 16) && ld_out % 8 == 0)) && (!out_q || aligned(out_q, 8));
     const int chunks = (nvec + THREADS - 1) / THREADS;
-    if (vec && !out_q && (long)M * chunks <= INT32_MAX) silu_mul_vec<<<dim3(M * chunks), dim3(THREADS), 0, st>>>(a, chunks);
-    else if (vec && out_q && nvec <= 4 * MAX_THREADS) launch_silu(a, M, st);
-    else
-        silu_mul_quant_scalar<<<dim3(M), dim3(THREADS), 0, st>>>(a);
+    const bool plain = vec && !out_q, whole_rows = vec && out_q && nvec <= 4 * MAX_THREADS;
+    in_row_slices(M, plain ? (long)chunks * THREADS : whole_rows ? MAX_THREADS : THREADS, [&](long lo, int rows) {
+        const SiluArgs part = a.from_row(lo);
+        if (plain) silu_mul_vec<<<dim3(rows * chunks), dim3(THREADS), 0, st>>>(part, chunks);
+        else if (whole_rows) launch_silu(part, rows, M, st);
+        else silu_mul_quant_scalar<<<dim3(rows), dim3(THREADS), 0, st>>>(part);
+    });
     return check_launch("cmi_silu_mul_quant");
 }
 

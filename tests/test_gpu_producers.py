@@ -186,6 +186,28 @@ def test_rms_norm_i8_adapter_and_special_rows(orc):
         backend.rms_norm_i8(x.float(), w, out_q, out_s)
 
 
+@pytest.mark.parametrize("op,m,n", [("rms_norm", (1 << 24) + 5, 1032), ("silu_mul", (1 << 23) + 3, 2056)])
+def test_more_rows_than_one_launch_holds(op, m, n):
+    """2^32 threads or more would be one launch too large: the rows run in slices.  In place on one block of 35 GB;
+    rows at the edges of the slices against the same rows in a call of their own."""
+    if torch.cuda.mem_get_info()[0] < 3 * m * n:
+        pytest.skip("needs 50 GB of device memory")
+    x = torch.zeros((m, n), dtype=torch.bfloat16, device=G.DEV)
+    edges = [0, 1] + [e for at in range(1, 9) for e in ((1 << 21) * at - 1, (1 << 21) * at, (1 << 21) * at - at) if e < m] + [m - 2, m - 1]
+    rows = torch.tensor(sorted(set(edges)), device=G.DEV)
+    few = torch.randn((len(rows), n), generator=synth.generator(m, G.DEV), device=G.DEV).to(torch.bfloat16)
+    x[rows] = few
+    w = torch.ones(n, dtype=torch.bfloat16, device=G.DEV)
+    lib = _native.load()
+    for t in (x, few):
+        if op == "rms_norm":
+            rc = lib.cmi_rms_norm_i8(G.ptr(t), G.ptr(w), G.ptr(t), None, None, t.shape[0], n, n, n, 1e-6, G.stream())
+        else:
+            rc = lib.cmi_silu_mul_quant(G.ptr(t), G.ptr(t), G.ptr(t), None, None, t.shape[0], n, n, n, n, G.stream())
+        _native.check(rc, op)
+    assert (x[rows].view(torch.int16) == few.view(torch.int16)).all()
+
+
 def _same_or_both_nan(orc, got_bits, want_bits):
     got, want = orc.bf16_to_f32(got_bits), orc.bf16_to_f32(want_bits)
     nan = np.isnan(want)
