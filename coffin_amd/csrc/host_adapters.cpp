@@ -91,21 +91,37 @@ bool holds(PyObject *w, const Weight &e) {
     return same;
 }
 
-// The entry of `w`, or null: a plain tensor, or a weight the adapter has not resolved yet.
-const Weight *find_weight(PyObject *w) {
+void drop(const Weight &e) {
+    Py_DECREF(e.src);
+    Py_DECREF(e.src2);
+}
+
+// The entry of `w` in `out`; false: a plain tensor, or a weight the adapter has not resolved yet.  Reading an attribute of
+// a weight may run Python code (a property), and with it other calls and threads that change the table, so
+// nothing points into the table across such a read.
+bool find_weight(PyObject *w, Weight *out) {
     auto it = g_weights.find(w);
     if (it != g_weights.end()) {
-        if (holds(w, it->second)) return &it->second;
-        Py_DECREF(it->second.src);
-        Py_DECREF(it->second.src2);
-        g_weights.erase(it);
+        const Weight e = it->second;
+        Py_INCREF(e.src);
+        Py_INCREF(e.src2);
+        const bool same = holds(w, e);
+        if (!same && (it = g_weights.find(w)) != g_weights.end() && it->second.src == e.src && it->second.src2 == e.src2) {
+            g_weights.erase(it);
+            drop(e);  // the table's references
+        }
+        drop(e);
+        if (same) {
+            *out = e;
+            return true;
+        }
     }
-    if (THPVariable_CheckExact(w)) return nullptr;
+    if (THPVariable_CheckExact(w)) return false;
     PyObject *fn = var(N.lookup);
     PyObject *rec = fn ? PyObject_CallOneArg(fn, w) : nullptr;
     if (!rec) {
         PyErr_Clear();
-        return nullptr;
+        return false;
     }
     Weight e{};
     long long kind, n, k, kd, gs, index = -1;
@@ -132,15 +148,20 @@ const Weight *find_weight(PyObject *w) {
     Py_XDECREF(family);
     Py_DECREF(rec);
     if (PyErr_Occurred()) PyErr_Clear();
-    if (!ok) return nullptr;
+    if (!ok) return false;
     if (g_weights.size() >= WEIGHTS_MAX) {
-        for (auto &w_e : g_weights) {
-            Py_DECREF(w_e.second.src);
-            Py_DECREF(w_e.second.src2);
-        }
-        g_weights.clear();
+        std::unordered_map<PyObject *, Weight> all;
+        all.swap(g_weights);
+        for (auto &w_e : all) drop(w_e.second);
     }
-    return &(g_weights[w] = e);
+    const auto [at, fresh] = g_weights.try_emplace(w, e);
+    if (!fresh) {  // the lookup's Python code, or another thread during it, has entered the weight
+        const Weight before = at->second;
+        at->second = e;
+        drop(before);
+    }
+    *out = e;
+    return true;
 }
 
 // ------------------------------------------------------------------------------- tensors
@@ -344,17 +365,16 @@ PyObject *project(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     const at::Tensor &x = *xp;
     const int64_t nd = x.dim();
     if ((nd != 1 && nd != 2) || !x.is_contiguous()) Py_RETURN_NONE;
-    const Weight *w = find_weight(args[0]);
-    if (!w || w->dev != here || x.size(-1) != w->k) Py_RETURN_NONE;
+    Weight e;
+    if (!find_weight(args[0], &e) || e.dev != here || x.size(-1) != e.k) Py_RETURN_NONE;
     const int64_t rows = nd == 1 ? 1 : x.size(0);
     if (rows < 1 || rows > INT32_MAX) Py_RETURN_NONE;
     const long flags = PyLong_AsLong(args[2]);
-    const bool quantised = w->kind == 4 || ((flags & PREFILL) && rows >= PREFILL_MIN_ROWS);
-    if (w->kind == 4 ? truth(N.w4a16) : ((flags & MFMA) && !(flags & PREFILL) && truth(N.w8a8_verify))) Py_RETURN_NONE;
+    const bool quantised = e.kind == 4 || ((flags & PREFILL) && rows >= PREFILL_MIN_ROWS);
+    if (e.kind == 4 ? truth(N.w4a16) : ((flags & MFMA) && !(flags & PREFILL) && truth(N.w8a8_verify))) Py_RETURN_NONE;
 
     void *stream = c10::hip::getCurrentHIPStream(here).stream();
-    const int M = (int)rows, Nn = w->n, K = w->k;
-    const Weight e = *w;  // the entry may go while the lock is released
+    const int M = (int)rows, Nn = e.n, K = e.k;
     const int8_t *xq = nullptr;
     const float *xs = nullptr;
     size_t need = 0;
@@ -562,9 +582,8 @@ PyObject *embed_rows(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     const c10::DeviceIndex here = c10::hip::current_device();
     const at::Tensor *ids = plain(args[1], here);
     if (!ids || ids->scalar_type() != at::kLong || !ids->is_contiguous() || ids->numel() < 1 || ids->numel() > INT32_MAX) Py_RETURN_NONE;
-    const Weight *w = find_weight(args[0]);
-    if (!w || w->dev != here) Py_RETURN_NONE;
-    const Weight e = *w;
+    Weight e;
+    if (!find_weight(args[0], &e) || e.dev != here) Py_RETURN_NONE;
     void *stream = c10::hip::getCurrentHIPStream(here).stream();
     const int64_t size[2] = {ids->numel(), e.k};
     at::Tensor y = new_bf16(size, here);

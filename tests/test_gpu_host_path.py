@@ -1,0 +1,84 @@
+"""The compiled host path of the table entries (``csrc/host_adapters.cpp``) against the Python adapters it stands in for."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from coffin_amd import backend, synth
+from coffin_amd.weights import QWeight, W4A8Weight
+from tests import gpu_util as G
+
+pytestmark = pytest.mark.gpu
+
+K, N = 2560, 1536
+
+
+def _q8(n=N, k=K, seed=1):
+    q = synth.int8_weight(n, k, synth.generator(seed))
+    return QWeight(q.wq.to(G.DEV), q.scale.to(G.DEV))
+
+
+def _w4(n=N, k=K, seed=1):
+    w = synth.int4_weight(n, k, synth.generator(seed))
+    return W4A8Weight(w.packed.to(G.DEV), w.scale.to(G.DEV), k=k)
+
+
+def _x(rows, k=K, seed=7):
+    return synth.activations(rows, k, synth.generator(seed)).to(G.DEV)
+
+
+def _same(a, b):
+    return a.shape == b.shape and bool((a.view(torch.int16) == b.view(torch.int16)).all())
+
+
+def test_tensors_replaced_under_the_same_weight_object():
+    """An entry is good while the weight object holds the tensors it was made from."""
+    x = _x(4)
+    w, other = _q8(seed=1), _q8(seed=2)
+    want, want_other = backend.linear(_q8(seed=1), x), backend.linear(_q8(seed=2), x)
+    for _ in range(3):
+        assert _same(backend.linear(w, x), want)
+    w.wq, w.scale = other.wq, other.scale
+    for _ in range(3):
+        assert _same(backend.linear(w, x), want_other)
+    w.scale = torch.ones_like(w.scale)                             # one of the two
+    ones = QWeight(other.wq, torch.ones_like(w.scale))
+    for _ in range(2):
+        assert _same(backend.linear(w, x), backend.linear(ones, x))
+
+
+class _Swaps:
+    """A weight whose ``wq`` is a property that, when told to, replaces the tensors and projects with itself: the
+    outer call's table entry goes while its attributes are being read."""
+
+    def __init__(self, q):
+        self._wq, self.scale, self.k, self.n = q.wq, q.scale, q.k, q.n
+        self.swap = None
+
+    @property
+    def wq(self):
+        if self.swap is not None:
+            swap, self.swap = self.swap, None
+            self._wq, self.scale = swap.wq, swap.scale
+            for _ in range(3):
+                self.inner = backend.linear(self, _x(1)[0])
+            others = [_q8(64, 256, seed) for seed in range(40)]    # and the table grows
+            for o in others:
+                for _ in range(2):
+                    backend.linear(o, _x(1, 256)[0])
+        return self._wq
+
+
+def test_an_entry_that_goes_while_the_weight_is_being_read():
+    first, second = _q8(seed=3), _q8(seed=4)
+    x = _x(1)[0]
+    want = backend.linear(second, x)
+    w = _Swaps(first)
+    for _ in range(3):
+        assert _same(backend.linear(w, x), backend.linear(first, x))
+    for _ in range(4):
+        w.swap = second
+        assert _same(backend.linear(w, x), want) and _same(w.inner, want)
+        first, second = second, first
+        want = backend.linear(second, x)
