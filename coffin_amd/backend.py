@@ -587,8 +587,10 @@ def _dense(w, x: torch.Tensor) -> torch.Tensor:
     return F.linear(x.to(compute), dense).to(x.dtype)
 
 
-def _project(w, x: torch.Tensor, prefill: bool, min_rows: int = PREFILL_MIN_ROWS,
+def _project(w, x: torch.Tensor, prefill: bool, min_rows: int | None = None,
              mfma: bool = False) -> torch.Tensor:
+    if min_rows is None:
+        min_rows = PREFILL_MIN_ROWS
     rec = _lookup(w)
     if rec is None and not (_is_w4(w) or _is_q8(w)):
         return _dense(w, x)

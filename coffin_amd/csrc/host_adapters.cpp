@@ -35,7 +35,7 @@ PyObject *g_rows_quantised = nullptr;  // backend._rows_quantised as defined; a 
 
 struct Names {
     PyObject *wq, *packed, *scale, *lookup, *kind, *src, *src2, *a, *b, *n, *k, *kd, *gs, *dev, *family, *index, *device;
-    PyObject *batch_mfma, *w8a8_verify, *w4a16, *handover, *handover_min, *handover_max, *seen, *handed, *rows_quantised;
+    PyObject *prefill_min, *mfma_min, *batch_mfma, *w8a8_verify, *w4a16, *handover, *handover_min, *handover_max, *seen, *handed, *rows_quantised;
     PyObject *workspace, *handover_arena, *take;
 } N;
 
@@ -313,7 +313,6 @@ bool handed_matches(const Handed *h, const at::Tensor &x, int64_t rows, int64_t 
 
 // --------------------------------------------------------------------------------- entries
 constexpr int PREFILL = 1, MFMA = 2;
-constexpr int64_t PREFILL_MIN_ROWS = 64, MFMA_MIN_ROWS = 3;  // backend.PREFILL_MIN_ROWS, backend.MFMA_MIN_ROWS
 
 // Column ranges of a projection's output as views that share its memory and version counter.
 PyObject *parts_of(const at::Tensor &y, PyObject *sizes) {
@@ -370,7 +369,7 @@ PyObject *project(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     const int64_t rows = nd == 1 ? 1 : x.size(0);
     if (rows < 1 || rows > INT32_MAX) Py_RETURN_NONE;
     const long flags = PyLong_AsLong(args[2]);
-    const bool quantised = e.kind == 4 || ((flags & PREFILL) && rows >= PREFILL_MIN_ROWS);
+    const bool quantised = e.kind == 4 || ((flags & PREFILL) && rows >= number(N.prefill_min));
     if (e.kind == 4 ? truth(N.w4a16) : ((flags & MFMA) && !(flags & PREFILL) && truth(N.w8a8_verify))) Py_RETURN_NONE;
 
     void *stream = c10::hip::getCurrentHIPStream(here).stream();
@@ -403,7 +402,7 @@ PyObject *project(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     void *yp = y.mutable_data_ptr();
     const void *xd = x.const_data_ptr();
     const bool fast = !quantised && K % 128 == 0 &&
-                      ((e.family >= 0 ? e.family == 1 : truth(N.batch_mfma)) || ((flags & MFMA) && rows >= MFMA_MIN_ROWS));
+                      ((e.family >= 0 ? e.family == 1 : truth(N.batch_mfma)) || ((flags & MFMA) && rows >= number(N.mfma_min)));
     int rc;
     const char *what;
     {
@@ -642,7 +641,7 @@ PyMODINIT_FUNC PyInit__host(void) {
     } const all[] = {{&N.wq, "wq"}, {&N.packed, "packed"}, {&N.scale, "scale"}, {&N.lookup, "_lookup"}, {&N.kind, "kind"},
                      {&N.src, "src"}, {&N.src2, "src2"}, {&N.a, "a"}, {&N.b, "b"}, {&N.n, "n"}, {&N.k, "k"}, {&N.kd, "kd"},
                      {&N.gs, "gs"}, {&N.dev, "dev"}, {&N.family, "family"}, {&N.index, "index"}, {&N.device, "device"},
-                     {&N.batch_mfma, "BATCH_MFMA"}, {&N.w8a8_verify, "W8A8_VERIFY"}, {&N.w4a16, "W4A16"},
+                     {&N.prefill_min, "PREFILL_MIN_ROWS"}, {&N.mfma_min, "MFMA_MIN_ROWS"}, {&N.batch_mfma, "BATCH_MFMA"}, {&N.w8a8_verify, "W8A8_VERIFY"}, {&N.w4a16, "W4A16"},
                      {&N.handover, "HANDOVER"}, {&N.handover_min, "HANDOVER_MIN_ROWS"}, {&N.handover_max, "HANDOVER_MAX_BYTES"},
                      {&N.seen, "_QUANT_CONSUMER_SEEN"}, {&N.handed, "_HANDED"}, {&N.rows_quantised, "_rows_quantised"},
                      {&N.workspace, "_WORKSPACE"}, {&N.handover_arena, "_HANDOVER_ARENA"}, {&N.take, "take"}};

@@ -28,6 +28,12 @@ def _x(rows, k=K, seed=7):
     return synth.activations(rows, k, synth.generator(seed)).to(G.DEV)
 
 
+def _adapters(monkeypatch):
+    """From here on the Python adapters answer every call."""
+    for name in backend._HOST_CALLS:
+        monkeypatch.setattr(backend, "_host_" + name, lambda *args: None)
+
+
 def _same(a, b):
     return a.shape == b.shape and bool((a.view(torch.int16) == b.view(torch.int16)).all())
 
@@ -82,3 +88,17 @@ def test_an_entry_that_goes_while_the_weight_is_being_read():
         assert _same(backend.linear(w, x), want) and _same(w.inner, want)
         first, second = second, first
         want = backend.linear(second, x)
+
+
+def test_row_thresholds_are_read_on_every_call(monkeypatch):
+    """A changed threshold moves the compiled calls and the adapters alike, to the bits of the other route."""
+    w, x = _q8(), _x(70)
+    weight_only, quantised = backend.linear_prefill(w, x[:63]), backend.linear_prefill(w, x)
+    dot, mfma = backend.linear(w, x[:4]), backend.linear_m_verify(w, x[:4])
+    assert not _same(weight_only, quantised[:63]) and not _same(dot, mfma)
+    monkeypatch.setattr(backend, "PREFILL_MIN_ROWS", 63)
+    monkeypatch.setattr(backend, "MFMA_MIN_ROWS", 5)
+    for _ in range(2):
+        assert _same(backend.linear_prefill(w, x[:63]), quantised[:63])
+        assert _same(backend.linear_m_verify(w, x[:4]), dot)
+        _adapters(monkeypatch)
