@@ -34,7 +34,7 @@ PyObject *g_check = nullptr;  // coffin_amd._native.check
 PyObject *g_rows_quantised = nullptr;  // backend._rows_quantised as defined; a replaced one is called by the Python adapter
 
 struct Names {
-    PyObject *wq, *packed, *scale, *lookup, *kind, *src, *src2, *a, *b, *n, *k, *kd, *gs, *dev, *family, *index, *device;
+    PyObject *wq, *packed, *scale, *records, *kind, *src, *src2, *a, *b, *n, *k, *kd, *gs, *dev, *family, *index, *device;
     PyObject *prefill_min, *mfma_min, *batch_mfma, *w8a8_verify, *w4a16, *handover, *handover_min, *handover_max, *seen, *handed, *rows_quantised;
     PyObject *workspace, *handover_arena, *take;
 } N;
@@ -117,17 +117,17 @@ bool find_weight(PyObject *w, Weight *out) {
         }
     }
     if (THPVariable_CheckExact(w)) return false;
-    PyObject *fn = var(N.lookup);
-    PyObject *rec = fn ? PyObject_CallOneArg(fn, w) : nullptr;
-    if (!rec) {
-        PyErr_Clear();
-        return false;
-    }
+    // The adapter's record, by the weight's id; a new weight has none, and its first call pays only this look.
+    PyObject *records = var(N.records), *id = PyLong_FromVoidPtr(w);
+    PyObject *rec = records && PyDict_Check(records) && id ? PyDict_GetItem(records, id) : nullptr;
+    Py_XINCREF(rec);
+    Py_XDECREF(id);
+    if (!rec) return false;
     Weight e{};
     long long kind, n, k, kd, gs, index = -1;
     const void *b = nullptr;
     PyObject *dev = nullptr, *family = nullptr;
-    bool ok = rec != Py_None && get_ll(rec, N.kind, &kind) && get_ll(rec, N.n, &n) && get_ll(rec, N.k, &k) &&
+    bool ok = get_ll(rec, N.kind, &kind) && get_ll(rec, N.n, &n) && get_ll(rec, N.k, &k) &&
               get_ll(rec, N.kd, &kd) && get_ll(rec, N.gs, &gs) && get_ptr(rec, N.a, &e.a) && get_ptr(rec, N.b, &b) &&
               (dev = PyObject_GetAttr(rec, N.dev)) && get_ll(dev, N.index, &index) &&
               (family = PyObject_GetAttr(rec, N.family));
@@ -138,7 +138,7 @@ bool find_weight(PyObject *w, Weight *out) {
         e.family = family == Py_None ? -1 : PyUnicode_CompareWithASCIIString(family, "mfma") == 0;
         e.src = PyObject_GetAttr(rec, N.src);
         e.src2 = e.src ? PyObject_GetAttr(rec, N.src2) : nullptr;
-        ok = e.src2 && PyWeakref_Check(e.src) && PyWeakref_Check(e.src2);
+        ok = e.src2 && PyWeakref_Check(e.src) && PyWeakref_Check(e.src2) && holds(w, e);
         if (!ok) {
             Py_XDECREF(e.src);
             Py_XDECREF(e.src2);
@@ -155,7 +155,7 @@ bool find_weight(PyObject *w, Weight *out) {
         for (auto &w_e : all) drop(w_e.second);
     }
     const auto [at, fresh] = g_weights.try_emplace(w, e);
-    if (!fresh) {  // the lookup's Python code, or another thread during it, has entered the weight
+    if (!fresh) {  // a property's Python code, or another thread during it, has entered the weight
         const Weight before = at->second;
         at->second = e;
         drop(before);
@@ -638,7 +638,7 @@ PyMODINIT_FUNC PyInit__host(void) {
     struct {
         PyObject **slot;
         const char *text;
-    } const all[] = {{&N.wq, "wq"}, {&N.packed, "packed"}, {&N.scale, "scale"}, {&N.lookup, "_lookup"}, {&N.kind, "kind"},
+    } const all[] = {{&N.wq, "wq"}, {&N.packed, "packed"}, {&N.scale, "scale"}, {&N.records, "_RECORDS"}, {&N.kind, "kind"},
                      {&N.src, "src"}, {&N.src2, "src2"}, {&N.a, "a"}, {&N.b, "b"}, {&N.n, "n"}, {&N.k, "k"}, {&N.kd, "kd"},
                      {&N.gs, "gs"}, {&N.dev, "dev"}, {&N.family, "family"}, {&N.index, "index"}, {&N.device, "device"},
                      {&N.prefill_min, "PREFILL_MIN_ROWS"}, {&N.mfma_min, "MFMA_MIN_ROWS"}, {&N.batch_mfma, "BATCH_MFMA"}, {&N.w8a8_verify, "W8A8_VERIFY"}, {&N.w4a16, "W4A16"},

@@ -102,3 +102,20 @@ def test_row_thresholds_are_read_on_every_call(monkeypatch):
         assert _same(backend.linear_prefill(w, x[:63]), quantised[:63])
         assert _same(backend.linear_m_verify(w, x[:4]), dot)
         _adapters(monkeypatch)
+
+
+@pytest.mark.parametrize("make", [_q8, _w4])
+def test_a_new_weight_costs_one_lookup_and_is_known_from_its_second_call(monkeypatch, make):
+    x = _x(3)
+    backend.linear(make(seed=11), x)                               # the host path is bound
+    lookups, real = [], backend._lookup
+    monkeypatch.setattr(backend, "_lookup", lambda w: lookups.append(w) or real(w))
+    w = make(seed=12)
+    first = backend.linear(w, x)
+    assert len(lookups) == 1
+
+    def unexpected(*args, **kwargs):
+        raise AssertionError("a known weight went to the Python adapter")
+
+    monkeypatch.setattr(backend, "_project", unexpected)
+    assert _same(backend.linear(w, x), first) and len(lookups) == 1
