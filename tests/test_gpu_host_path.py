@@ -119,3 +119,42 @@ def test_a_new_weight_costs_one_lookup_and_is_known_from_its_second_call(monkeyp
 
     monkeypatch.setattr(backend, "_project", unexpected)
     assert _same(backend.linear(w, x), first) and len(lookups) == 1
+
+
+@pytest.mark.parametrize("mode", ["grad", "no_grad", "inference"])
+@pytest.mark.parametrize("rows", [0, 1, 5, 70])                    # 0: a [K] activation
+def test_parts_of_a_fused_projection_are_those_of_split(monkeypatch, mode, rows):
+    """Values, sizes, pitch, offset, shared version counter, view relation and what autograd allows on them."""
+    x = _x(rows) if rows else _x(1)[0]
+    sizes = [1024, 128, 384]
+    switch = {"grad": torch.enable_grad, "no_grad": torch.no_grad, "inference": torch.inference_mode}[mode]
+    for make in (_q8, _w4):
+        w = make()
+        for entry in ("linear", "linear_m", "linear_m_verify", "linear_prefill") if rows else ("linear",):
+            with switch():
+                backend.linear_parts(entry, w, x, sizes)           # the weight is known
+                got = backend.linear_parts(entry, w, x, sizes)
+                whole = getattr(backend, entry)(w, x)
+                want = whole.split(sizes, dim=-1)
+            assert type(got) is tuple and len(got) == 3
+            base = None
+            for a, b in zip(got, want):
+                assert _same(a, b) and a.stride() == b.stride() and a.storage_offset() == b.storage_offset()
+                assert a._is_view() == b._is_view() and a.is_inference() == b.is_inference()
+                assert a.untyped_storage().data_ptr() == got[0].untyped_storage().data_ptr()
+                if mode != "inference":
+                    base = a._base
+                    assert base is got[0]._base and _same(base, whole)
+            if mode == "inference":
+                continue
+            got[1].add_(1)
+            assert got[0]._version == got[2]._version == base._version == 1
+            assert torch.equal(base[..., 1024:1152], got[1]) and torch.equal(base[..., 1152:], want[2])
+            leaf = torch.ones(1024, dtype=torch.bfloat16, device=G.DEV, requires_grad=True)
+            for part in (got[0], want[0]):                         # a write that would need the other parts' history
+                with pytest.raises(RuntimeError):
+                    part.mul_(leaf)
+    with pytest.raises(RuntimeError):
+        backend.linear_parts("linear", w, x, [1024, 128])
+    with pytest.raises(RuntimeError):
+        backend.linear_parts("linear", w, x, [1024, 128, 385])
