@@ -112,9 +112,10 @@ def load_host():
 
 
 def available() -> bool:
-    """True when the shared library loads (says nothing about a GPU being present)."""
+    """True when the shared library and the compiled host path load, i.e. when a call would find what it needs (says
+    nothing about a GPU being present)."""
     try:
-        load()
+        load_host()
     except RuntimeError:
         return False
     return True

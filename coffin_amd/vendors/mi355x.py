@@ -41,7 +41,7 @@ def build_ops() -> "Ops":
         if not _device_is_gfx950():
             return Ops()
         from coffin_amd import _native, backend
-        _native.load()
+        _native.load_host()
         return Ops.from_mapping(backend.native_table())
     except Exception:
         return Ops()

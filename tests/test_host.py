@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import ctypes
 import re
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -53,6 +54,21 @@ def test_vendor_spec_validation_and_declaration():
         # no card: claim is "not mine" and build_ops degrades to an empty table
         assert contract.detect(spec.detection) == contract.CLAIM_NONE
         assert mi355x.build_ops().implemented() == ()
+
+
+def test_without_the_compiled_host_path_nothing_is_claimed(monkeypatch):
+    """Every entry's first GPU call loads ``_host``: where it is missing (or was built for another torch) the backend
+    says so up front and its table is empty."""
+    import coffin_amd
+    from coffin_amd.vendors import mi355x
+    monkeypatch.setattr(mi355x, "_device_is_gfx950", lambda: True)
+    assert _native.available() and mi355x.build_ops().implemented() != ()
+    monkeypatch.delattr(coffin_amd, "_host", raising=False)
+    monkeypatch.setitem(sys.modules, "coffin_amd._host", None)
+    assert not _native.available()
+    with pytest.raises(RuntimeError, match="host extension unusable"):
+        _native.load_host()
+    assert mi355x.build_ops().implemented() == ()
 
 
 # ------------------------------------------------------------------- weights
