@@ -547,7 +547,7 @@ _HOST_CALLS = ("project", "rms_norm", "add_rms_norm", "silu_mul", "kv_quant", "e
 
 def _bind_host() -> None:
     host = _native.load_host()
-    host.bind(globals(), _native.check, _rows_quantised)
+    host.bind(globals(), _native.check)
     for name in _HOST_CALLS:
         globals()["_host_" + name] = getattr(host, name)
 

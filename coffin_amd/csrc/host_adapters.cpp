@@ -32,11 +32,11 @@ namespace {
 // ------------------------------------------------------------------- the Python module's state
 PyObject *g_vars = nullptr;   // coffin_amd.backend.__dict__ (borrowed: the module outlives every call)
 PyObject *g_check = nullptr;  // coffin_amd._native.check
-PyObject *g_rows_quantised = nullptr;  // backend._rows_quantised as defined; a replaced one is called by the Python adapter
+long long g_handed_uses[2];   // projections that took handed rows: int4 weights, int8 weights
 
 struct Names {
     PyObject *wq, *packed, *scale, *records, *kind, *src, *src2, *a, *b, *n, *k, *kd, *gs, *dev, *family, *index, *device;
-    PyObject *prefill_min, *mfma_min, *batch_mfma, *w8a8_verify, *w4a16, *handover, *handover_min, *handover_max, *seen, *handed, *rows_quantised;
+    PyObject *prefill_min, *mfma_min, *batch_mfma, *w8a8_verify, *w4a16, *handover, *handover_min, *handover_max, *seen, *handed;
     PyObject *workspace, *handover_arena, *take;
 } N;
 
@@ -385,12 +385,13 @@ PyObject *project(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         if (e.kind == 8) need = cmi_linear_w8a8_workspace_bytes(M, Nn, K);
         PyObject *handed = var(N.handed);
         if (handed && handed != Py_None && e.kd == K) {
-            if (Py_TYPE(handed) != &HandedType || var(N.rows_quantised) != g_rows_quantised) Py_RETURN_NONE;
+            if (Py_TYPE(handed) != &HandedType) Py_RETURN_NONE;  // left by the Python adapter, which can read it
             const Handed *h = reinterpret_cast<Handed *>(handed);
             // a W8A8 shape that may split K needs the quantiser's launch, which clears its counters
             if ((e.kind == 4 || need == cmi_linear_workspace_bytes(M, K)) && handed_matches(h, x, rows, K, stream)) {
                 xq = reinterpret_cast<const int8_t *>(static_cast<intptr_t>(h->xq));
                 xs = reinterpret_cast<const float *>(static_cast<intptr_t>(h->xs));
+                ++g_handed_uses[e.kind == 8];
             }
         }
         if (!xq) {
@@ -603,21 +604,26 @@ PyObject *embed_rows(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
-// bind(vars, check, rows_quantised): the module whose state this is (once).
+// handed_uses(): how many projections took rows a producer had quantised, (int4 weights, int8 weights).
+PyObject *handed_uses(PyObject *, PyObject *const *, Py_ssize_t) {
+    return Py_BuildValue("LL", g_handed_uses[0], g_handed_uses[1]);
+}
+
+// bind(vars, check): the module whose state this is (once).
 PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
-    if (nargs != 3 || !PyDict_Check(args[0])) {
-        PyErr_SetString(PyExc_TypeError, "bind(module dict, check, rows_quantised)");
+    if (nargs != 2 || !PyDict_Check(args[0])) {
+        PyErr_SetString(PyExc_TypeError, "bind(module dict, check)");
         return nullptr;
     }
-    for (int i = 0; i < 3; ++i) Py_INCREF(args[i]);
+    for (int i = 0; i < 2; ++i) Py_INCREF(args[i]);
     g_vars = args[0];
     g_check = args[1];
-    g_rows_quantised = args[2];
     Py_RETURN_NONE;
 }
 
 PyMethodDef methods[] = {
     {"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, nullptr},
+    {"handed_uses", (PyCFunction)(void (*)(void))handed_uses, METH_FASTCALL, nullptr},
     {"project", (PyCFunction)(void (*)(void))project, METH_FASTCALL, nullptr},
     {"rms_norm", (PyCFunction)(void (*)(void))rms_norm, METH_FASTCALL, nullptr},
     {"add_rms_norm", (PyCFunction)(void (*)(void))add_rms_norm, METH_FASTCALL, nullptr},
@@ -646,7 +652,7 @@ PyMODINIT_FUNC PyInit__host(void) {
                      {&N.gs, "gs"}, {&N.dev, "dev"}, {&N.family, "family"}, {&N.index, "index"}, {&N.device, "device"},
                      {&N.prefill_min, "PREFILL_MIN_ROWS"}, {&N.mfma_min, "MFMA_MIN_ROWS"}, {&N.batch_mfma, "BATCH_MFMA"}, {&N.w8a8_verify, "W8A8_VERIFY"}, {&N.w4a16, "W4A16"},
                      {&N.handover, "HANDOVER"}, {&N.handover_min, "HANDOVER_MIN_ROWS"}, {&N.handover_max, "HANDOVER_MAX_BYTES"},
-                     {&N.seen, "_QUANT_CONSUMER_SEEN"}, {&N.handed, "_HANDED"}, {&N.rows_quantised, "_rows_quantised"},
+                     {&N.seen, "_QUANT_CONSUMER_SEEN"}, {&N.handed, "_HANDED"},
                      {&N.workspace, "_WORKSPACE"}, {&N.handover_arena, "_HANDOVER_ARENA"}, {&N.take, "take"}};
     for (const auto &e : all)
         if (!(*e.slot = PyUnicode_InternFromString(e.text))) return nullptr;

@@ -450,20 +450,46 @@ def test_pre_quantised_directory_feeds_the_kernels(tmp_path, orc):
 
 # ------------------------------------------------ quantised rows handed forward by the producers
 
-def _count_quantised_routes(monkeypatch):
-    calls = []
-    real = backend._rows_quantised
+class _QuantisedRoutes:
+    """The projections that took handed rows since it was made."""
 
-    def spy(rec, xq, xs, rows, out, stream):
-        calls.append((rec.kind, rows))
-        return real(rec, xq, xs, rows, out, stream)
+    def __init__(self, monkeypatch, path):
+        self.path, self.host = path, backend._native.load_host()
+        self.by_adapters, real = [], backend._rows_quantised
 
-    monkeypatch.setattr(backend, "_rows_quantised", spy)
-    return calls
+        def spy(rec, xq, xs, rows, out, stream):
+            self.by_adapters.append(rec.kind)
+            return real(rec, xq, xs, rows, out, stream)
+
+        monkeypatch.setattr(backend, "_rows_quantised", spy)
+        if path == "adapters":
+            for name in backend._HOST_CALLS:
+                monkeypatch.setattr(backend, "_host_" + name, lambda *args: None)
+        self.start = self.host.handed_uses()
+
+    def kinds(self, by_adapters=0):
+        """How many on int4 weights, how many on int8 weights, all by the path under test (compiled calls leave
+        ``by_adapters`` of them, on rows with a pitch, to the adapters)."""
+        now = self.host.handed_uses()
+        compiled = (now[0] - self.start[0], now[1] - self.start[1])
+        if self.path == "adapters":
+            assert compiled == (0, 0)
+        else:
+            assert len(self.by_adapters) == by_adapters
+        return compiled[0] + self.by_adapters.count(4), compiled[1] + self.by_adapters.count(8)
+
+    def __len__(self):
+        return sum(self.kinds())
 
 
+#: The compiled calls, which answer known weights, and the Python adapters, which answer the rest, each check handed rows
+#: with code of their own.
+both_paths = pytest.mark.parametrize("path", ["compiled", "adapters"])
+
+
+@both_paths
 @pytest.mark.parametrize("rows", [1, 2, 16, 70, 300, 1100])
-def test_table_entry_sequence_hands_quantised_rows_to_the_projection(monkeypatch, rows):
+def test_table_entry_sequence_hands_quantised_rows_to_the_projection(monkeypatch, rows, path):
     """The reference's own call sequence -- ``rms_norm`` then ``linear``, ``add_rms_norm`` then
     ``linear``, ``silu_mul`` then ``linear`` (ops/norm.py:87,135, models/qwen35/blocks.py:69) -- runs
     the integer kernels on the rows the producer quantised, with the bits of the route that
@@ -498,24 +524,25 @@ def test_table_entry_sequence_hands_quantised_rows_to_the_projection(monkeypatch
     monkeypatch.setattr(backend, "HANDOVER", False)
     want = sequence()
     monkeypatch.setattr(backend, "HANDOVER", True)
-    calls = _count_quantised_routes(monkeypatch)
+    calls = _QuantisedRoutes(monkeypatch, path)
     gu.copy_(gu0)
     got = sequence()
     for i, (a, b) in enumerate(zip(got, want)):
         assert (a.view(torch.int16) == b.view(torch.int16)).all(), i
-    kinds = [c[0] for c in calls]
-    assert kinds.count(4) == 4                                     # every int4 projection took the handed rows
-    assert kinds.count(8) == (1 if rows >= 64 and not backend._splits_k(rows, n, k, x.device) else 0)
+    int4, int8 = calls.kinds(by_adapters=int(rows > 1))             # silu_mul's rows have the fused output's pitch
+    assert int4 == 4                                               # every int4 projection took the handed rows
+    assert int8 == (1 if rows >= 64 and not backend._splits_k(rows, n, k, x.device) else 0)
 
 
-def test_handed_rows_are_not_trusted_after_the_tensor_changed(monkeypatch):
+@both_paths
+def test_handed_rows_are_not_trusted_after_the_tensor_changed(monkeypatch, path):
     g = synth.generator(6)
     k, n = 2560, 1024
     w4 = _w4(n, k, g)
     x = synth.activations(4, k, g).to(G.DEV)
     gain = synth.activations(1, k, g)[0].to(G.DEV).contiguous()
     backend.linear(w4, x)                                          # a quantising consumer has been seen
-    calls = _count_quantised_routes(monkeypatch)
+    calls = _QuantisedRoutes(monkeypatch, path)
 
     def fresh(t):                                                  # the same values in memory of their own
         return backend.linear_m(w4, t.clone())
@@ -556,7 +583,8 @@ def test_handed_rows_are_not_trusted_after_the_tensor_changed(monkeypatch):
         backend.configure(handover=True)
 
 
-def test_handed_rows_inside_a_captured_graph_and_not_across_its_edge(monkeypatch):
+@both_paths
+def test_handed_rows_inside_a_captured_graph_and_not_across_its_edge(monkeypatch, path):
     """Producer and consumer recorded into one capture replay together (fresh inputs, same bits as
     eager); a consumer recorded into a capture does not read rows an eager producer left."""
     g = synth.generator(8)
@@ -574,7 +602,7 @@ def test_handed_rows_inside_a_captured_graph_and_not_across_its_edge(monkeypatch
 
     step()
     torch.cuda.synchronize()
-    calls = _count_quantised_routes(monkeypatch)
+    calls = _QuantisedRoutes(monkeypatch, path)
     eager_h = backend.rms_norm(x, gain)                            # handed eagerly, consumed under capture: refused
     graph = torch.cuda.CUDAGraph()
     side = torch.cuda.Stream()
