@@ -22,8 +22,10 @@
 //     matrix and steps past K read zeros), NST steps in flight, one barrier per step;
 //   - a wavefront reads packed rows in the MFMA arrangement and widens them itself, three vector instructions
 //     per eight codes: 16 (code - 8) is the code with its top bit flipped in the high nibble of a byte.  The
-//     sums are 16 times too large, exactly, and the flush multiplies by scale / 16 (exact for scales from
-//     2^-122 up; the encoder's are above 1e-9);
+//     sums are 16 times too large, exactly, and the flush multiplies by scale / 16, which is exact for scales from
+//     2^-122 up.  The encoder's are above 1e-9; a wavefront that meets a smaller one (a running minimum, 0..2 % of
+//     the launch: 1024 x 51200 x 5120 344 -> 348 us; a compare and branch per flush took 5 % and made 128 x 160
+//     spill) forms its results anew at the end, element by element;
 //   - the output is walked column tile by column tile: while column j multiplies, the sums of column j - 1 are
 //     flushed and column j + 1 is widened, in slots of one MFMA and the vector instructions beside it (left to
 //     itself the compiler clumps them, 6 % slower);
@@ -71,6 +73,24 @@ template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
     static_assert(N >= 0 && N < 64, "vmcnt range");
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// One element's sum over the groups, from memory: the statement at the head of this file as it stands.  A word of the
+// packed weight holds k 0..3 in its low nibbles and k 4..7 in its high ones.
+template <int LG>
+__device__ __forceinline__ float total_of(const Args &a, int m, int n) {
+    const int8_t *x = a.xq + (size_t)m * a.K;
+    const uint8_t *w = a.w4 + (size_t)n * (a.K / 2);
+    float total = 0.f;
+    for (int g = 0; g < a.G; ++g) {
+        int sum = 0;
+        for (int k = g * (32 << LG); k < (g + 1) * (32 << LG); ++k) {
+            const int b = k % 8;
+            sum += x[k] * (((w[k / 8 * 4 + b % 4] >> (b / 4 * 4)) & 15) - 8);
+        }
+        total = fmaf((float)sum, a.ws[(size_t)n * a.G + g], total);
+    }
+    return total;
 }
 
 // LG: log2(group size / 32).  2: a step is a group.  3: a group is two steps, the first one's sums are kept.  1: a
@@ -158,6 +178,10 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_tile_kernel(const A
     constexpr int PG = LG == 1 ? 2 : 1;  // groups a step closes in a column
     v4i32 pend[PG][TM];                  // the latest closed column's sums, flushed under the next column's MFMAs
     float pend_scale[PG];
+    // The smallest magnitude of a scale so far but zero, as 2 * bits - 1, and the lanes where it was below 2^-122.
+    constexpr uint32_t TINY = 2 * (5u << 23) - 1;
+    uint32_t least = ~0u;
+    uint64_t inexact = 0;
     v4i32 part[LG == 3 ? TN : 1][TM];    // LG 3: sums of the first half of a group
 #pragma unroll
     for (int g = 0; g < PG; ++g) {
@@ -258,6 +282,14 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_tile_kernel(const A
         slot = next;
     };
     for (int c = 0; 4 * c < ksteps; ++c) {
+        if constexpr (LG == 3) least = ~0u;
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < SV; ++v)
+#pragma unroll
+                for (int i = 0; i < (LG == 3 ? 2 : 4); ++i) least = min(least, 2 * __float_as_uint(sc[j][v][i]) - 1);
+        if constexpr (LG == 3) inexact |= __builtin_amdgcn_ballot_w64(least < TINY);  // no vector register to spare
         step(std::integral_constant<int, 0>{}, 4 * c);
         if (4 * c + 1 < ksteps) step(std::integral_constant<int, 1>{}, 4 * c + 1);
         if (4 * c + 2 < ksteps) step(std::integral_constant<int, 2>{}, 4 * c + 2);
@@ -274,6 +306,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_tile_kernel(const A
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 total[i][TN - 1][r] = fmaf((float)pend[g][i][r], pend_scale[g], total[i][TN - 1][r]);
+    if constexpr (LG != 3) inexact = __builtin_amdgcn_ballot_w64(least < TINY);
     wait_vmcnt<0>();  // requests past the last step (they read zeros or the next rows)
 
     // y[m,n] = bf16(total * xs[m]), parked in LDS so that whole 16-byte pieces of rows leave
@@ -288,6 +321,12 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_tile_kernel(const A
 #pragma unroll
             for (int j = 0; j < TN; ++j)
                 park[ml * (C::YPITCH / 2) + wn * 16 * TN + j * 16 + fr] = (uint16_t)f32_to_bf16_bits(total[i][j][r] * xm);
+        }
+    if (inexact)
+        for (int e = lane; e < 16 * TM * 16 * TN; e += 64) {
+            const int ml = wm * 16 * TM + e / (16 * TN), nl = wn * 16 * TN + e % (16 * TN);
+            if (m0 + ml < a.M && n0 + nl < a.N)
+                park[ml * (C::YPITCH / 2) + nl] = (uint16_t)f32_to_bf16_bits(total_of<LG>(a, m0 + ml, n0 + nl) * a.xs[m0 + ml]);
         }
     __syncthreads();
     const int rows = min(a.M - m0, C::BM), cols = min(a.N - n0, C::BN);

@@ -77,6 +77,32 @@ def test_w4a8_tiles_at_their_edges(orc, tile, m, n, k, gs):
     assert (G.bits(y) == y_ref).all()
 
 
+@pytest.mark.parametrize("gs", [128, 64, 256])
+def test_w4a8_tiles_with_scales_near_the_end_of_the_range(orc, gs):
+    """Scales whose sixteenth is not exact (below 2^-122, down to the last denormal), beside ordinary ones, zero and the
+    largest: the tiles carry 16 times the sums and a sixteenth of the scale where they can."""
+    g = synth.generator(gs)
+    m, n, k = 70, 200, 1024
+    w = synth.int4_weight(n, k, g, group_size=gs)
+    exponent = torch.randint(-149, -118, w.scale.shape, generator=g)
+    scale = torch.ldexp(1 + torch.rand(w.scale.shape, generator=g, dtype=torch.float64), exponent.double()).float()
+    scale[:, ::3] = w.scale[:, ::3]                                # columns without a tiny scale
+    scale[1, 3::5] = 0.0
+    scale[0, 6::12] = 1e30
+    x = (synth.activations(m, k, g).float() * 1e4).to(torch.bfloat16)
+    xq, xs = orc.quant_act_i8(G.bits(x))
+    _, y_ref = orc.linear_w4a8(xq, xs, w.packed.numpy(), scale.numpy(), k, gs)
+    w4, ws = G.w4_repack(w.packed.to(G.DEV), scale.to(G.DEV), k, gs)
+    assert (ws.cpu().view(torch.int32) == scale.t().contiguous().view(torch.int32)).all()
+    for tile in (64, 128, 192, 128192, 256, 320, 321, 6464):
+        G.set_option("gemm_tile", tile)
+        _, y = G.w4a8(w4, ws, G.dev(xq), G.dev(xs), k, gemm=True, want_acc=False, gs=gs)
+        assert (G.bits(y) == y_ref).all(), tile
+    G.set_option("gemm_tile", 0)
+    _, y = G.w4a8(w4, ws, G.dev(xq[:5]), G.dev(xs[:5]), k, gemm=False, want_acc=False, gs=gs)
+    assert (G.bits(y) == y_ref[:5]).all()
+
+
 @pytest.mark.parametrize("k", [128, 384, 640])
 def test_w4a8_tiles_with_a_step_count_that_is_no_whole_chunk(orc, k):
     g = synth.generator(k)
