@@ -330,7 +330,9 @@ gemv_w8a16_kernel(const GemvArgs a) {
         auto consume = [&](const WStage<R, CHT> &w, int t) {
 #pragma unroll
             for (int mh = 0; mh < MH; ++mh) {
-                if (M == 16 && mh * MT >= a.M) break;  // 9..12 rows: three tiles of four do
+                // 9..12 rows: three tiles of four do.  (Where a unit is one trip, K <= 1024, the test between the tiles
+                // costs more than the tile: 16 rows of 1024 -> 151936 80 -> 93 us, 9 rows 78 -> 81.)
+                if (M == 16 && MODE == 2 && mh * MT >= a.M) break;
                 // keep one activation tile in registers: no LDS reads of the next
                 // tile hoisted above this one's arithmetic (other wavefronts fill in)
                 load_x(x0, u, t, mh);
