@@ -577,9 +577,12 @@ Plan make_plan(int M, int N, int K) {
     // at 16 rows (registers), two rows stay faster.
     if (p.mt == 8 && N >= 65536) p.r = 4;
     // The same at three and four rows, one segment of K at a time (registers: the next one's weights are in
-    // flight), where K is one unit: 2560 -> 151936 75.4 -> 72.1 / 85.3 -> 75.2 us at three / four rows; 2560 -> 19456 12.9 -> 14.0,
-    // 2560 -> 6144 6.0 -> 6.4 stay with two rows.
-    if (p.mt == 4 && N >= 65536 && units == 1 && unit >= 2) p.r = 4, p.cht = 1, p.mode = 2;
+    // flight), where K is one unit: 2560 -> 151936 75.4 -> 72.1 / 85.3 -> 75.2 us at three / four rows, 4096 -> 151936 18 % less;
+    // 2560 -> 19456 12.9 -> 14.0, 2560 -> 6144 6.0 -> 6.4 stay with two rows.  Two or three segments all full stay
+    // too, in one trip (three rows of 2048 -> 65536 24.9 -> 27.6 with four, 3072 -> 128256 6 % more): segment by segment
+    // wins where the last one is at most five eighths full, so that a trip over all of them has idle lanes.
+    if (p.mt == 4 && N >= 65536 && units == 1 && unit >= 2 && (unit == 4 || K / 16 - (nseg - 1) * 64 <= 40))
+        p.r = 4, p.cht = 1, p.mode = 2;
     // 9..16 rows put 16 wavefronts in a workgroup: with two weight rows each, up to 4096 outputs would be at most 128
     // workgroups.  4096 -> 2560 at 16 rows 16.6 -> 11.0 us; with more outputs the shared fragments win
     // (2560 -> 6144 14.4 against 15.8).

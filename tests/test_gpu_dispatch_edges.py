@@ -118,7 +118,7 @@ def test_w4a8_tiles_with_a_step_count_that_is_no_whole_chunk(orc, k):
         assert (G.bits(y) == y_ref).all(), tile
 
 
-@pytest.mark.parametrize("n,k", [(65535, 2064), (65536, 1040), (65537, 3072), (70001, 4096), (65536, 1024), (65600, 4112), (300, 2560),
+@pytest.mark.parametrize("n,k", [(65535, 2064), (65536, 1040), (65537, 3072), (70001, 4096), (65536, 1024), (65600, 4112), (65537, 1664), (65539, 2560), (300, 2560),
                                  (4096, 4096), (4097, 4096), (33, 9728)])
 def test_weight_only_rows_keep_the_single_row_s_bits_at_the_edges_of_the_row_blocks(n, k):
     """Four weight rows per wavefront for very tall weights at 3..4 rows, one at 9..16 rows and few outputs, three
