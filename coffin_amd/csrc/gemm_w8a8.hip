@@ -1339,7 +1339,7 @@ int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, co
             const double tiles = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
             // the 4-wavefront tiles on up to 192 CUs: the idle CUs warm the caches (see above)
             const double warmed = bm <= 192 && bn <= 192 && tiles <= 192 && (double)N * K <= 64.0 * 1048576.0 ? 0.8 : 1.0;
-            return 2.5 + steps * (a0 + b0 * N) * warmed * (1.0 + c0 * (ceil(tiles / 256.0) - 1.0));
+            return 2.5 + steps * (a0 + b0 * fmin(N, 32768)) * warmed * (1.0 + c0 * (ceil(tiles / 256.0) - 1.0));
         };
         const struct { int pick; double us; } candidates[] = {
             {64, N > 64 ? cost(128, 64, 0.407, 5.54e-6, 0.796) : 1e30},
