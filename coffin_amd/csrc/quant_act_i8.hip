@@ -171,12 +171,14 @@ int cmi::quant_act_i8_and_clear(const void *x, int8_t *q, float *s, int M, int K
         // Up to 1024 elements a wavefront or less owns a row.  Two rows per lane group once one each would
         // be more than two workgroups per CU: twice the bytes in flight per wavefront (65536 x 128: 9.8 ->
         // 7.8 us; below that the second row only lengthens the launch, 2048 x 576: 3.3 -> 3.9 us).
+        // Two vectors a lane pay from 257 rows on; below, a workgroup per row is shorter (1 x 576 1.99 us against 2.16,
+        // 256 x 576 2.40 against 2.55, 512 x 576 5 % the other way).
         const auto many = [&](int rows_per_block) { return M > 512 * rows_per_block; };
         if (nvec <= 8) many(32) ? rows_launch(quant_act_i8_rows<8, 1, 2>, 64) : rows_launch(quant_act_i8_rows<8, 1, 1>, 32);
         else if (nvec <= 16) many(16) ? rows_launch(quant_act_i8_rows<16, 1, 2>, 32) : rows_launch(quant_act_i8_rows<16, 1, 1>, 16);
         else if (nvec <= 32) many(8) ? rows_launch(quant_act_i8_rows<32, 1, 2>, 16) : rows_launch(quant_act_i8_rows<32, 1, 1>, 8);
         else if (nvec <= 64) many(4) ? rows_launch(quant_act_i8_rows<64, 1, 2>, 8) : rows_launch(quant_act_i8_rows<64, 1, 1>, 4);
-        else if (nvec <= 128) rows_launch(quant_act_i8_rows<64, 2, 1>, 4);
+        else if (nvec <= 128 && M > QUANT_THREADS) rows_launch(quant_act_i8_rows<64, 2, 1>, 4);
         else if (vpt <= 1) quant_act_i8_vec<1><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);
         else if (vpt <= 2) quant_act_i8_vec<2><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);
         else if (vpt <= 4) quant_act_i8_vec<4><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);

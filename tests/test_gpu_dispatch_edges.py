@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("m,k", [(1, 8), (513, 64), (16385, 64), (31, 72), (8193, 128), (8192, 136), (4097, 256), (17, 264),
-                                 (2049, 512), (2048, 520), (5, 1024), (3, 1032)])
+                                 (2049, 512), (2048, 520), (5, 1024), (3, 1032), (256, 520), (257, 1024)])
 def test_quantiser_of_short_rows(orc, m, k):
     """Lane groups of 8 .. 64 per row, one or two rows each; rows that do not fill a workgroup."""
     x = synth.activations(m, k, synth.generator(m + k), outliers=True)
