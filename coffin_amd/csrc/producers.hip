@@ -416,7 +416,9 @@ void launch_norm(const NormArgs &a, int M, int waves, hipStream_t st) {
     if (waves == 1) {
         const dim3 grid((M + THREADS / 64 - 1) / (THREADS / 64)), block(THREADS);
         if (nvec <= 64) rms_norm_i8_vec<1, ADD, true><<<grid, block, 0, st>>>(a, M);
-        else rms_norm_i8_vec<2, ADD, true><<<grid, block, 0, st>>>(a, M);
+        else if (nvec <= 128) rms_norm_i8_vec<2, ADD, true><<<grid, block, 0, st>>>(a, M);
+        else if (nvec <= 192) rms_norm_i8_vec<3, ADD, true><<<grid, block, 0, st>>>(a, M);
+        else rms_norm_i8_vec<4, ADD, true><<<grid, block, 0, st>>>(a, M);
         return;
     }
     const dim3 grid(M), block(64 * waves);
@@ -428,12 +430,16 @@ void launch_norm(const NormArgs &a, int M, int waves, hipStream_t st) {
 }
 
 // Wavefronts per row: four up to 8192 elements (add + norm + quantiser on cold operands, 2560 elements: 500 rows
-// 10.3 -> 6.0 us against a wavefront per row as before, 8192 rows 41.6 -> 36.5; two and eight are slower at
-// most sizes), one per 256 vectors beyond, a single one -- four rows per workgroup -- for many rows of at
-// most 1024 elements, where a workgroup per row is mostly its own start.
-int norm_waves(int M, int nvec) {
+// 10.3 -> 6.0 us against a wavefront per row, 8192 rows 41.6 -> 36.5; two and eight are slower at
+// most sizes), four per 8192 beyond, a single one -- four rows per workgroup -- for many rows of at
+// most 1024 elements, where a workgroup per row is mostly its own start.  With the quantised row, whose second
+// reduction is a second barrier, the single one also wins for many rows of up to 2048 elements (4096 x 1032 8.7 us
+// against 12.2 with four, 8192 x 2048 22.5 against 24.4; 1024 rows lose), with the add up to 1536 or, from 4096 rows
+// on, 1280 (2048 x 1536 9.1 against 9.9, 8192 x 1536 5 % the other way).
+int norm_waves(int M, int nvec, bool add, bool quantised) {
     if (nvec <= 128) return M <= FEW_ROWS ? (nvec + 63) / 64 : 1;
-    return nvec <= 1024 ? 4 : (nvec + 255) / 256;
+    if (quantised && M > 1280 && nvec <= (!add ? 256 : M <= 4096 ? 192 : 160)) return 1;
+    return nvec <= 1024 ? 4 : (nvec + 1023) / 1024 * 4;
 }
 
 int norm_entry(const char *who, uint16_t *x, const uint16_t *add, const void *w, void *y, int8_t *q, float *s,
@@ -450,7 +456,7 @@ int norm_entry(const char *who, uint16_t *x, const uint16_t *add, const void *w,
     const bool vec = N % 8 == 0 && nvec <= 4 * MAX_THREADS && aligned(x, 16) && ldx % 8 == 0 && aligned(w, 16) &&
                      (!add || (aligned(add, 16) && lda % 8 == 0)) && (!y || (aligned(y, 16) && ldy % 8 == 0)) &&
                      (!q || aligned(q, 8));
-    const int waves = vec ? norm_waves(M, nvec) : THREADS / 64;
+    const int waves = vec ? norm_waves(M, nvec, add, q) : THREADS / 64;
     in_row_slices(M, 64 * waves, [&](long lo, int rows) {
         const NormArgs part = a.from_row(lo);
         if (!vec) rms_norm_i8_scalar<<<dim3(rows), dim3(THREADS), 0, st>>>(part);

@@ -41,8 +41,10 @@ def test_silu_mul_quant_at_the_edges_of_a_thread_s_share(orc, m, k):
 
 
 @pytest.mark.parametrize("m,n", [(256, 1024), (257, 512), (259, 520), (257, 1024), (2, 1032), (300, 8192), (3, 8200), (2, 16392),
-                                 (257, 32768), (2, 32776)])
-def test_add_rms_norm_i8_at_the_edges_of_a_row_s_wavefronts(orc, m, n):
+                                 (257, 32768), (2, 32776), (1281, 1032), (1280, 1280), (2049, 1536), (1283, 1544), (4097, 1280),
+                                 (4098, 1288), (3, 12288), (258, 8200), (1281, 2048), (1300, 2056)])
+@pytest.mark.parametrize("with_add", [True, False])
+def test_rms_norm_i8_at_the_edges_of_a_row_s_wavefronts(orc, m, n, with_add):
     g = synth.generator(m + n)
     x, add = synth.activations(m, n, g), synth.activations(m, n, g)
     gain = (1 + 0.1 * torch.randn(n, generator=g)).to(torch.bfloat16)
@@ -50,10 +52,14 @@ def test_add_rms_norm_i8_at_the_edges_of_a_row_s_wavefronts(orc, m, n):
     q = torch.empty((m, n), dtype=torch.int8, device=G.DEV)
     s = torch.empty(m, dtype=torch.float32, device=G.DEV)
     ad, gd = add.to(G.DEV), gain.to(G.DEV)
-    _native.check(_native.load().cmi_add_rms_norm_i8(G.ptr(xd), G.ptr(ad), G.ptr(gd), G.ptr(y), G.ptr(q), G.ptr(s), m, n,
-                                                     n, n, n, 1e-6, G.stream()), "add_rms_norm_i8")
+    lib = _native.load()
+    if with_add:
+        rc = lib.cmi_add_rms_norm_i8(G.ptr(xd), G.ptr(ad), G.ptr(gd), G.ptr(y), G.ptr(q), G.ptr(s), m, n, n, n, n, 1e-6, G.stream())
+    else:
+        rc = lib.cmi_rms_norm_i8(G.ptr(xd), G.ptr(gd), G.ptr(y), G.ptr(q), G.ptr(s), m, n, n, n, 1e-6, G.stream())
+    _native.check(rc, "rms_norm_i8")
     rows = [0, 1, m - 1]
-    total = (x.float() + add.float()).to(torch.bfloat16)[rows].contiguous()
+    total = ((x.float() + add.float()).to(torch.bfloat16) if with_add else x)[rows].contiguous()
     y_ref, _ = orc.rms_norm(G.bits(total), G.bits(gain))
     q_ref, s_ref = orc.quant_act_i8(y_ref)
     assert (G.bits(xd[rows]) == G.bits(total)).all() and (G.bits(y[rows]) == y_ref).all()
