@@ -466,12 +466,12 @@ int norm_entry(const char *who, uint16_t *x, const uint16_t *add, const void *w,
     return check_launch(who);
 }
 
-// Threads per row: one per 16-byte vector for a few rows, one per two of them otherwise (2048 x 4096: 17.2
-// us with one each, 15.7 with two), more vectors where the row would need over 1024 threads; a power of two of
+// Threads per row: one per 16-byte vector for a few rows (up to 512 of at most 2048 elements: 512 x 2048 5.1 us, 5.5 with
+// two vectors each), one per two of them otherwise (2048 x 4096: 17.2 us with one each, 15.7 with two), more vectors where the row would need over 1024 threads; a power of two of
 // wavefronts, so that the workgroup loads the four SIMDs alike (2048 x 14336: 45 us on 14, 41 on 16).
 void launch_silu(const SiluArgs &a, int rows, int M, hipStream_t st) {
     const int nvec = a.K / 8;
-    const int vpt = std::max(M <= FEW_ROWS ? 1 : 2, (nvec + MAX_THREADS - 1) / MAX_THREADS);
+    const int vpt = std::max(M <= (nvec <= 256 ? 2 : 1) * FEW_ROWS ? 1 : 2, (nvec + MAX_THREADS - 1) / MAX_THREADS);
     int threads = 64;
     while (threads * vpt < nvec) threads *= 2;
     const dim3 grid(rows), block(threads);
