@@ -1327,7 +1327,10 @@ int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, co
     // 4-wavefront tiles that need two rounds and 256-row ones that leave CUs idle: 500 x 19456 x 2560
     // 38.0 -> 34.9 us (228 tiles instead of 152), 1152 x 19456 76.5 -> 65.2, 768 x 11008 x 4096 50.9 -> 44.9,
     // 2048 x 11008 x 4096 103 -> 92; it and 256 x 320 are fitted to a sweep of eight shapes x twelve
-    // batch sizes, where the choice is 0.2 % above the best (1.9 % without it).
+    // batch sizes, where the choice is 0.2 % above the best (1.9 % without it).  A step's growth with N is fitted up to
+    // 32768 outputs and stays there beyond: carried on it preferred 256 x 320 to 256 x 256 for 385..512 rows of 51200
+    // outputs (400 x 51200 x 4096 122 against 107 us; eight shapes of 19456..51200 outputs x fifteen batch sizes:
+    // the choice 0.8 -> 0.1 % above the best).
     // CMI_GEMM_TILE=64|128|192|256|320 overrides the tile along n (tests, tuning); 128192 forces
     // 128(n) x 192(m), 256192 256(n) x 192(m), 6464 the 64 x 64 tile of the mid-batch route.
     int pick;  // 64, 128, 192, 256 or 320: block tile along n; 128192; 256192; 6464

@@ -21,7 +21,8 @@ def test_quantiser_of_short_rows(orc, m, k):
     assert (q.cpu().numpy() == q_ref).all() and (s.cpu().numpy() == s_ref).all()
 
 
-@pytest.mark.parametrize("m,k", [(256, 8192), (257, 8192), (2, 8200), (257, 1032), (258, 16392), (3, 24584), (257, 32768), (2, 32776)])
+@pytest.mark.parametrize("m,k", [(256, 8192), (257, 8192), (2, 8200), (257, 1032), (258, 16392), (3, 24584), (257, 32768), (2, 32776),
+                                 (512, 2048), (513, 2048), (300, 2056), (3, 520), (7, 1544), (5, 2560), (9, 3072)])
 def test_silu_mul_quant_at_the_edges_of_a_thread_s_share(orc, m, k):
     g = synth.generator(m + k)
     gate, up = (torch.randn((m, 2 * k), generator=g) * 3).to(torch.bfloat16).split(k, dim=1)
