@@ -1,4 +1,4 @@
-// cmi_gemm_w4a8: the choice of route, and the kernel for calls that ask for the integer group sums.
+// cmi_gemm_w4a8: the choice of route, and the two-stage kernel.
 //
 //   sum_g  = sum_{k in group g} xq[m,k] * (code(n,k) - 8)     int32, exact
 //   total  = fma((float)sum_g, ws[n,g], total)                 g = 0,1,.. from 0.f
@@ -7,14 +7,15 @@
 // Same bits from every route: the integer part is exact and the fp32 part is the one chain over the groups in
 // ascending order.  The product alone runs the tile kernels of gemm_w4a8_tile.hip or, for a few rows, the GEMV.
 //
-// With group sums (parity checks): block tile 128(m) x 128(n), 4 wavefronts (2 x 2) of 64 x 64,
+// Two-stage kernel, for calls that ask for the group sums and for many rows of groups of 64: block tile 128(m) x 128(n), 4 wavefronts (2 x 2) of 64 x 64,
 // v_mfma_i32_32x32x32_i8, K walked 128 per step, two LDS stages, two workgroups per CU.
 //   - activations go global -> LDS directly (global_load_lds_dwordx4, chunk index XOR-swizzled on the global side);
 //   - the packed weight (64 B per row and step) is fetched into registers one step ahead, widened there to int8
 //     code-8 (no cross-byte borrow), and written to LDS once per workgroup;
 //   - the activation is the MFMA row operand and the weight the column operand: a lane owns ONE n per MFMA tile (and
 //     16 m), so the flush needs one scale per tile and lane, fetched from memory a step ahead;
-//   - the integer accumulators restart every group (first MFMA takes C = 0) and are written out before the flush.
+//   - the integer accumulators restart every group (first MFMA takes C = 0) and, where asked for, are written out
+//     before the flush.
 #include "common.hpp"
 #include "gemm_tiles.hpp"
 
@@ -36,7 +37,7 @@ struct Args {
     const float *xs;
     const float *ws;  // [N, G]
     uint16_t *y;
-    int32_t *group_acc;  // [M, G, N]
+    int32_t *group_acc;  // [M, G, N], null without DUMP
     int M, N, K, G;
     int tiles_m, tiles_n;
 };
@@ -45,9 +46,11 @@ typedef __attribute__((address_space(3))) void *lds_ptr_t;
 
 // LG: log2(group size / 32).  2: a K step is a group.  3: a group is two steps, the integer accumulators run on over
 // the odd step and flush behind it.  1: a step holds two groups, flushed behind the second and the fourth k quarter.
-template <int LG>
+// DUMP: also write the int32 group sums (parity checks); a separate instantiation, the 64 extra store addresses per
+// lane would otherwise be carried through the hot loop.
+template <int LG, bool DUMP>
 __global__ void __launch_bounds__(THREADS, 2)
-gemm_w4a8_group_sums_kernel(const Args a) {
+gemm_w4a8_two_stage_kernel(const Args a) {
     static_assert(LG >= 1 && LG <= 3, "group sizes 64, 128, 256");
     extern __shared__ __align__(16) int8_t lds[];
     const int lane = threadIdx.x & 63;
@@ -200,7 +203,7 @@ gemm_w4a8_group_sums_kernel(const Args a) {
         mma_q(f1, false);
         pace_quarter();
         if constexpr (LG == 1) {  // the step's first group is complete
-            dump(2 * ks);
+            if constexpr (DUMP) dump(2 * ks);
             flush(sc);
         }
         read_q(cur, 3, f1);
@@ -235,7 +238,7 @@ gemm_w4a8_group_sums_kernel(const Args a) {
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
         if (closes) {
-            dump(LG == 3 ? ks >> 1 : LG == 1 ? 2 * ks + 1 : ks);
+            if constexpr (DUMP) dump(LG == 3 ? ks >> 1 : LG == 1 ? 2 * ks + 1 : ks);
             if constexpr (LG == 1) flush(sc_b);
             else flush(sc);
         }
@@ -288,6 +291,15 @@ gemm_w4a8_group_sums_kernel(const Args a) {
         }
 }
 
+// Time of the two-stage kernel's launch with groups of 64, in us: rounds of two tiles per CU, the last one cheaper if it is
+// at most one per CU.  Within 12 % of eleven layer shapes x fourteen batch sizes (64..8192 rows).
+double two_stage_us(int M, int N, int K) {
+    const double steps = K / 128.0;
+    const long tiles = (long)((M + BM - 1) / BM) * ((N + BN - 1) / BN), rest = tiles % 512;
+    const double round = 9.0 + 1.74 * steps;
+    return 3.0 + tiles / 512 * round + (rest == 0 ? 0.0 : rest <= 256 ? 6.0 + 1.35 * steps : round);
+}
+
 }  // namespace
 
 extern "C" int cmi_gemm_w4a8(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs,
@@ -328,7 +340,13 @@ extern "C" int cmi_gemm_w4a8(const uint8_t *w4, const float *ws, const int8_t *x
             return CMI_OK;
         }
     }
-    if (!group_acc)
+    // Groups of 64 flush twice a step, which costs the 64-row tiles 1.2 .. 1.4 times the time their model (fitted to
+    // groups of 128) gives; there is no 128 x 128 one of that kind (two groups' sums do not fit the registers).
+    // From about 1024 rows on the two-stage kernel's is the better: 2048 x 51200 x 5120 1000 against 1110 us, 3000 x
+    // 2560 x 9728 138 against 165; 2048 x 6144 x 2560 81 against 72.  Chosen with the factor 1.45 the 151 sizes of its
+    // fit take 2.0 % more than the best tile of each, 4.8 % without it.
+    const bool two_stage = gs == 64 && (forced ? forced == 128 : two_stage_us(M, N, K) < 1.45 * t_tile);
+    if (!group_acc && !two_stage)
         return gemm_w4a8_tile(w4, ws, xq, xs, y, M, N, K, gs, forced ? gemm_w4a8_forced_tile(forced, gs) : tile, stream);
     Args a;
     a.xq = xq;
@@ -343,13 +361,14 @@ extern "C" int cmi_gemm_w4a8(const uint8_t *w4, const float *ws, const int8_t *x
     a.G = K / gs;
     a.tiles_m = (M + BM - 1) / BM;
     a.tiles_n = (N + BN - 1) / BN;
-    static std::atomic<uint64_t> devices[3];
+    static std::atomic<uint64_t> devices[4];
     auto run = [&](auto kernel, int slot) {
         if (const int rc = reserve_lds(reinterpret_cast<const void *>(kernel), LDS_BYTES, devices[slot], "cmi_gemm_w4a8"))
             return rc;
         kernel<<<dim3(a.tiles_m * a.tiles_n), dim3(THREADS), LDS_BYTES, static_cast<hipStream_t>(stream)>>>(a);
         return check_launch("cmi_gemm_w4a8");
     };
-    if (gs == 64) return run(gemm_w4a8_group_sums_kernel<1>, 0);
-    return gs == 256 ? run(gemm_w4a8_group_sums_kernel<3>, 1) : run(gemm_w4a8_group_sums_kernel<2>, 2);
+    if (!group_acc) return run(gemm_w4a8_two_stage_kernel<1, false>, 0);
+    if (gs == 64) return run(gemm_w4a8_two_stage_kernel<1, true>, 1);
+    return gs == 256 ? run(gemm_w4a8_two_stage_kernel<3, true>, 2) : run(gemm_w4a8_two_stage_kernel<2, true>, 3);
 }

@@ -44,7 +44,8 @@ int cmi_abi_version(void);
  *                   block tile of cmi_gemm_w8a8 (non-zero also bypasses its few-row routes).
  *                   cmi_gemm_w4a8 has tiles of its own under the same values (m x n): 64 32 x 64,
  *                   128 128 x 128, 192 64 x 96, 128192 64 x 128, 256 32 x 128, 320 128 x 160, 321
- *                   16 x 32, 322 and 6464 64 x 64 (groups of 64 and 256: the nearest it is built for);
+ *                   16 x 32, 322 and 6464 64 x 64 (groups of 64: 128 the two-stage kernel; otherwise groups of
+ *                   64 and 256 the nearest it is built for);
  *   "gemv_wholerow" -1 (the library chooses) | 0 (never) | 1: the one-wavefront-per-weight-row
  *                   kernel of cmi_gemv_w8a16;
  *   "w4_decode_waves" 0 (the library chooses) | 4 | 16: wavefronts per workgroup of the W4A8
