@@ -378,6 +378,8 @@ def _hand_target(rows: int, k: int, device: torch.device):
 
 def _hand_over(t: torch.Tensor, rows: int, k: int, ld: int, target, stream: int) -> None:
     global _HANDED
+    if t.is_inference():
+        return                           # no version counter: writes to it would go unseen
     h = _Handed()
     h.tensor, h.version, h.ptr, h.rows, h.k, h.ld, h.dev = t, t._version, t.data_ptr(), rows, k, ld, t.device
     h.xq, h.xs = target
@@ -390,8 +392,8 @@ def _hand_over(t: torch.Tensor, rows: int, k: int, ld: int, target, stream: int)
 def _handed_rows(x: torch.Tensor, rows: int, k: int, stream: int):
     """The quantised copy of ``x`` left by the producer that wrote it, or ``None``."""
     h = _HANDED
-    if h is None or x.data_ptr() != h.ptr or rows != h.rows or k != h.k or x._version != h.version \
-            or x.device != h.dev:
+    if h is None or x.data_ptr() != h.ptr or rows != h.rows or k != h.k or x.device != h.dev or x.is_inference() \
+            or x._version != h.version:
         return None
     if x.stride(-1) != 1 or (x.dim() == 2 and rows > 1 and x.stride(0) != h.ld):
         return None

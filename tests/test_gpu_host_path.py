@@ -158,3 +158,103 @@ def test_parts_of_a_fused_projection_are_those_of_split(monkeypatch, mode, rows)
         backend.linear_parts("linear", w, x, [1024, 128])
     with pytest.raises(RuntimeError):
         backend.linear_parts("linear", w, x, [1024, 128, 385])
+
+
+class _Rows(torch.Tensor):
+    """A tensor subclass: the compiled calls leave it to the adapters."""
+
+
+def _odd_rows(kind, rows, k):
+    x = _x(rows, k)
+    if kind == "cpu":
+        return x.cpu()
+    if kind in ("float32", "float16"):
+        return x.to(getattr(torch, kind))
+    if kind == "columns":
+        return x.t().contiguous().t()
+    if kind == "pitch":
+        return torch.cat([x, x], dim=1)[:, :k]
+    if kind == "offset":                                           # rows that start 2 bytes past a 16-byte boundary
+        flat = torch.empty(rows * k + 1, dtype=x.dtype, device=x.device)
+        flat[1:] = x.reshape(-1)
+        return flat[1:].view(rows, k)
+    if kind == "subclass":
+        return x.as_subclass(_Rows)
+    if kind == "empty":
+        return x[:0]
+    if kind == "3-D":
+        return x.view(1, rows, k)
+    if kind == "narrow":
+        return x[:, :k - 16].contiguous()
+    assert kind == "plain"
+    return x
+
+
+def _outcome(call):
+    try:
+        return None, call()
+    except Exception as exc:                                       # noqa: BLE001 - the two paths must raise alike
+        return type(exc), None
+
+
+@pytest.mark.parametrize("mode", ["grad", "inference"])
+@pytest.mark.parametrize("kind", ["plain", "cpu", "float32", "float16", "columns", "pitch", "offset", "subclass", "empty", "3-D",
+                                  "narrow"])
+def test_calls_that_are_not_the_common_case_end_as_the_adapters_end_them(monkeypatch, kind, mode):
+    """Other devices, types, layouts, subclasses, shapes and inference tensors: values, shape, type and kind of error of
+    every entry with the compiled calls and without them."""
+    rows = 5
+    weights = {"int8": _q8(), "int4": _w4()}
+    gain = _x(1, seed=9)[0].contiguous()
+    calls = {}
+    for name, w in weights.items():
+        for entry in ("linear", "linear_m", "linear_m_verify", "linear_prefill"):
+            calls[name, entry] = lambda x, w=w, entry=entry: getattr(backend, entry)(w, x)
+            calls[name, entry, "parts"] = lambda x, w=w, entry=entry: backend.linear_parts(entry, w, x, [1024, 512])
+
+    def zeros(x, shape, dtype):
+        return torch.zeros(shape, dtype=dtype, device=x.device)
+
+    def gain_for(x):
+        return gain.to(x.device, x.dtype)[:x.shape[-1]]
+
+    def silu_mul(x):
+        out = zeros(x, x.shape, x.dtype)
+        return backend.silu_mul(x, x, out), out
+
+    def kv_quant(x):
+        q, s = zeros(x, x.shape, torch.int8), zeros(x, x.shape[:-1], torch.float32)
+        return backend.kv_quant(x, q, s), q, s
+
+    def add_rms_norm(x):
+        total, out = x.clone(), zeros(x, x.shape, x.dtype)
+        return backend.add_rms_norm(total, x, gain_for(x), out), total, out
+
+    calls["rms_norm"] = lambda x: backend.rms_norm(x, gain_for(x))
+    calls["silu_mul"], calls["kv_quant"], calls["add_rms_norm"] = silu_mul, kv_quant, add_rms_norm
+    calls["embed_rows"] = lambda x: backend.embed_rows(weights["int8"], torch.arange(3, device=x.device))
+    calls["embed_rows", "int32"] = lambda x: backend.embed_rows(weights["int4"], torch.arange(3, dtype=torch.int32, device=x.device))
+    switch = {"grad": torch.enable_grad, "inference": torch.inference_mode}[mode]
+
+    def outcomes():
+        with switch():
+            x = _odd_rows(kind, rows, K)
+            return {name: _outcome(lambda: call(x)) for name, call in calls.items()}
+
+    for call in calls.values():                                    # the weights are known
+        _outcome(lambda: call(_x(rows)))
+    got = outcomes()
+    _adapters(monkeypatch)
+    want = outcomes()
+
+    def flat(v):
+        return [t for e in v for t in flat(e)] if isinstance(v, (tuple, list)) else [v]
+
+    for name in calls:
+        assert got[name][0] == want[name][0], (name, got[name][0], want[name][0])
+        for a, b in zip(flat(got[name][1]), flat(want[name][1]), strict=True):
+            if b is None:
+                continue
+            assert type(a) is type(b) and a.dtype == b.dtype and a.device == b.device and a.shape == b.shape, name
+            assert a.is_inference() == b.is_inference() and a.requires_grad == b.requires_grad, name
+            assert torch.equal(a.float().cpu(), b.float().cpu()), name
