@@ -44,17 +44,6 @@ int reserve_lds(const void *kernel, int bytes, std::atomic<uint64_t> &devices, c
     return CMI_OK;
 }
 
-int compute_units() {
-    static std::atomic<int> count[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 0;
-    int n = count[dev & 63].load(std::memory_order_relaxed);
-    if (n > 0) return n;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
-    count[dev & 63].store(n, std::memory_order_relaxed);
-    return n;
-}
-
 // ------------------------------------------------------------------ options
 // Kernel-selection overrides for tests and tuning.  Each is read from its environment variable
 // once, when first asked for, and validated there; afterwards only cmi_set_option changes it, so
