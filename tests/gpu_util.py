@@ -78,14 +78,27 @@ def w4_repack(packed, scale, k, gs=128):
 
 
 def w4a8(w4, ws, xq, xs, k, gemm: bool, want_acc=True, gs=128):
+    """(group sums or None, y).  The GEMM's tile kernels do not write the group sums: a call that asks for them runs
+    another kernel.  ``y`` is that of the call without them, the product's, and the other kernel's must equal it."""
     m = xq.shape[0]
     n = w4.shape[0]
-    y = torch.empty((m, n), dtype=torch.bfloat16, device=DEV)
-    gacc = torch.empty((m, k // gs, n), dtype=torch.int32, device=DEV) if want_acc else None
     lib = _native.load()
     fn = lib.cmi_gemm_w4a8 if gemm else lib.cmi_gemv_w4a8
-    _native.check(fn(ptr(w4), ptr(ws), ptr(xq), ptr(xs), ptr(y), ptr(gacc), m, n, k, gs, stream()),
-                  "gemm_w4a8" if gemm else "gemv_w4a8")
+
+    def call(gacc):
+        y = torch.empty((m, n), dtype=torch.bfloat16, device=DEV)
+        _native.check(fn(ptr(w4), ptr(ws), ptr(xq), ptr(xs), ptr(y), ptr(gacc), m, n, k, gs, stream()),
+                      "gemm_w4a8" if gemm else "gemv_w4a8")
+        return y
+
+    if not want_acc:
+        return None, call(None)
+    gacc = torch.empty((m, k // gs, n), dtype=torch.int32, device=DEV)
+    y_acc = call(gacc)
+    if not gemm:
+        return gacc, y_acc
+    y = call(None)
+    assert torch.equal(y.view(torch.int16), y_acc.view(torch.int16))
     return gacc, y
 
 
