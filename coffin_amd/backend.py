@@ -469,6 +469,16 @@ def _make_record(w) -> _Record:
     return rec
 
 
+def _resolve(w, k: int, device: int) -> _Record | None:
+    """For the compiled calls: the record of a weight at its first use, on bf16 activations of width ``k`` on the current
+    ``device``; ``None`` where :func:`_project` would answer otherwise or raise."""
+    int4 = _is_w4(w)
+    if not (int4 or _is_q8(w)) or not _kernels_take(w) or int(w.k) != k:
+        return None
+    wdev = (w.packed if int4 else w.wq).device
+    return _make_record(w) if wdev.type == "cuda" and wdev.index == device else None
+
+
 def _gemv_q8(rec: _Record, act: torch.Tensor, rows: int, out: torch.Tensor, mfma: bool = False) -> None:
     """Weight-only projection, one native call for any number of rows.  ``mfma``: the call site may
     use the matrix-pipe family (verify, short prefill chunks: from ``MFMA_MIN_ROWS`` rows); a weight
@@ -541,8 +551,8 @@ def _rows_w4a16(rec: _Record, act: torch.Tensor, rows: int, out: torch.Tensor) -
 # What an entry does on every call is compiled (csrc/host_adapters.cpp): at one row the Python adapters
 # below cost 7 us per call in front of kernels of 2.5 .. 10 us.  A compiled call reads the switches, records and
 # scratch of this module, does the whole entry for plain bf16 tensors on the current device and a weight
-# that has been seen before, and answers ``None`` for anything else, which the adapters below then do
-# (first uses, other dtypes and layouts, errors).  Loaded by the first call that holds a GPU tensor.
+# that the kernels take, and answers ``None`` for anything else, which the adapters below then do
+# (other dtypes and layouts, errors).  Loaded by the first call that holds a GPU tensor.
 
 _HOST_CALLS = ("project", "rms_norm", "add_rms_norm", "silu_mul", "kv_quant", "embed_rows")
 

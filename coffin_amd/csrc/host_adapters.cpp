@@ -3,9 +3,9 @@
 // At one row a projection kernel takes 2.5 .. 10 us and the Python adapter in front of it (argument
 // checks, weight lookup, output allocation, foreign-function call) took 7.3 us, so eager decode was
 // bound by the host.  Each function here does one entry's whole call for the common case -- exact bf16
-// torch tensors on the current device, a weight that has been seen before -- in about 3 us, most of it
+// torch tensors on the current device, a weight that the kernels take -- in about 3 us, most of it
 // the runtime's own launch, and answers `None` for everything else: the caller then takes the Python
-// adapter, which resolves first uses, converts, and raises the errors.  Nothing is decided differently
+// adapter, which converts and raises the errors.  A weight's first use resolves it through the module.  Nothing is decided differently
 // here; the switches and the scratch blocks are the Python module's, read on every call.
 //
 //   2560 -> 1024, one row, through GEMV.__call__: 7.4 us per call with the Python adapter (kernel 2.6).
@@ -37,7 +37,7 @@ long long g_handed_uses[2];   // projections that took handed rows: int4 weights
 struct Names {
     PyObject *wq, *packed, *scale, *records, *kind, *src, *src2, *a, *b, *n, *k, *kd, *gs, *dev, *family, *index, *device;
     PyObject *prefill_min, *mfma_min, *batch_mfma, *w8a8_verify, *w4a16, *handover, *handover_min, *handover_max, *seen, *handed;
-    PyObject *workspace, *handover_arena, *take;
+    PyObject *workspace, *handover_arena, *take, *resolve;
 } N;
 
 PyObject *var(PyObject *name) { return PyDict_GetItem(g_vars, name); }  // borrowed
@@ -97,10 +97,40 @@ void drop(const Weight &e) {
     Py_DECREF(e.src2);
 }
 
-// The entry of `w` in `out`; false: a plain tensor, or a weight the adapter has not resolved yet.  Reading an attribute of
-// a weight may run Python code (a property), and with it other calls and threads that change the table, so
-// nothing points into the table across such a read.
-bool find_weight(PyObject *w, Weight *out) {
+// Makes `e` from an adapter's record; false: the record is about other tensors than `w` holds (a dead weight's under the
+// same id; not asked of one just made), or an error was set.  The tensors are looked at first: a stale record costs no
+// more than that.
+bool from_record(PyObject *rec, PyObject *w, bool made, Weight *e) {
+    long long kind, n, k, kd, gs, index = -1;
+    const void *b = nullptr;
+    PyObject *dev = nullptr, *family = nullptr;
+    if (!get_ll(rec, N.kind, &kind)) return false;
+    e->kind = (int)kind;
+    e->src = PyObject_GetAttr(rec, N.src);
+    e->src2 = e->src ? PyObject_GetAttr(rec, N.src2) : nullptr;
+    bool ok = e->src2 && PyWeakref_Check(e->src) && PyWeakref_Check(e->src2) && (made || holds(w, *e));
+    ok = ok && get_ll(rec, N.n, &n) && get_ll(rec, N.k, &k) && get_ll(rec, N.kd, &kd) && get_ll(rec, N.gs, &gs) &&
+         get_ptr(rec, N.a, &e->a) && get_ptr(rec, N.b, &b) && (dev = PyObject_GetAttr(rec, N.dev)) &&
+         get_ll(dev, N.index, &index) && (family = PyObject_GetAttr(rec, N.family));
+    if (ok) {
+        e->b = static_cast<const float *>(b);
+        e->n = (int)n, e->k = (int)k, e->kd = (int)kd, e->gs = (int)gs;
+        e->dev = (c10::DeviceIndex)index;
+        e->family = family == Py_None ? -1 : PyUnicode_CompareWithASCIIString(family, "mfma") == 0;
+    } else {
+        Py_XDECREF(e->src);
+        Py_XDECREF(e->src2);
+    }
+    Py_XDECREF(dev);
+    Py_XDECREF(family);
+    return ok;
+}
+
+// The entry of `w` in `out`: 1, or 0 where the adapter has to answer (a plain tensor, a weight that the kernels do not
+// take), or -1 with the Python error set.  Reading an attribute of a weight may run Python code (a property), and with it
+// other calls and threads that change the table, so nothing points into the table across such a read.
+// resolve_k >= 0: a weight of that width that nobody has used yet is resolved here, by the module's own function.
+int find_weight(PyObject *w, Weight *out, int64_t resolve_k, c10::DeviceIndex here) {
     auto it = g_weights.find(w);
     if (it != g_weights.end()) {
         const Weight e = it->second;
@@ -114,42 +144,30 @@ bool find_weight(PyObject *w, Weight *out) {
         drop(e);
         if (same) {
             *out = e;
-            return true;
+            return 1;
         }
     }
-    if (THPVariable_CheckExact(w)) return false;
-    // The adapter's record, by the weight's id; a new weight has none, and its first call pays only this look.
+    if (THPVariable_CheckExact(w)) return 0;
+    // The adapter's record, by the weight's id.
     PyObject *records = var(N.records), *id = PyLong_FromVoidPtr(w);
     PyObject *rec = records && PyDict_Check(records) && id ? PyDict_GetItem(records, id) : nullptr;
     Py_XINCREF(rec);
     Py_XDECREF(id);
-    if (!rec) return false;
     Weight e{};
-    long long kind, n, k, kd, gs, index = -1;
-    const void *b = nullptr;
-    PyObject *dev = nullptr, *family = nullptr;
-    bool ok = get_ll(rec, N.kind, &kind) && get_ll(rec, N.n, &n) && get_ll(rec, N.k, &k) &&
-              get_ll(rec, N.kd, &kd) && get_ll(rec, N.gs, &gs) && get_ptr(rec, N.a, &e.a) && get_ptr(rec, N.b, &b) &&
-              (dev = PyObject_GetAttr(rec, N.dev)) && get_ll(dev, N.index, &index) &&
-              (family = PyObject_GetAttr(rec, N.family));
-    if (ok) {
-        e.b = static_cast<const float *>(b);
-        e.kind = (int)kind, e.n = (int)n, e.k = (int)k, e.kd = (int)kd, e.gs = (int)gs;
-        e.dev = (c10::DeviceIndex)index;
-        e.family = family == Py_None ? -1 : PyUnicode_CompareWithASCIIString(family, "mfma") == 0;
-        e.src = PyObject_GetAttr(rec, N.src);
-        e.src2 = e.src ? PyObject_GetAttr(rec, N.src2) : nullptr;
-        ok = e.src2 && PyWeakref_Check(e.src) && PyWeakref_Check(e.src2) && holds(w, e);
-        if (!ok) {
-            Py_XDECREF(e.src);
-            Py_XDECREF(e.src2);
-        }
-    }
-    Py_XDECREF(dev);
-    Py_XDECREF(family);
-    Py_DECREF(rec);
+    bool ok = rec && from_record(rec, w, false, &e);
     if (PyErr_Occurred()) PyErr_Clear();
-    if (!ok) return false;
+    if (!ok && resolve_k >= 0) {
+        Py_XDECREF(rec);
+        PyObject *width = PyLong_FromLongLong(resolve_k), *device = PyLong_FromLong(here), *resolve = var(N.resolve);
+        rec = width && device && resolve ? PyObject_CallFunctionObjArgs(resolve, w, width, device, nullptr) : nullptr;
+        Py_XDECREF(width);
+        Py_XDECREF(device);
+        if (!rec) return -1;
+        ok = rec != Py_None && from_record(rec, w, true, &e);
+        if (PyErr_Occurred()) PyErr_Clear();
+    }
+    Py_XDECREF(rec);
+    if (!ok) return 0;
     if (g_weights.size() >= WEIGHTS_MAX) {
         std::unordered_map<PyObject *, Weight> all;
         all.swap(g_weights);
@@ -162,7 +180,7 @@ bool find_weight(PyObject *w, Weight *out) {
         drop(before);
     }
     *out = e;
-    return true;
+    return 1;
 }
 
 // ------------------------------------------------------------------------------- tensors
@@ -367,10 +385,12 @@ PyObject *project(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     const at::Tensor &x = *xp;
     const int64_t nd = x.dim();
     if ((nd != 1 && nd != 2) || !x.is_contiguous()) Py_RETURN_NONE;
-    Weight e;
-    if (!find_weight(args[0], &e) || e.dev != here || x.size(-1) != e.k) Py_RETURN_NONE;
     const int64_t rows = nd == 1 ? 1 : x.size(0);
     if (rows < 1 || rows > INT32_MAX) Py_RETURN_NONE;
+    Weight e;
+    const int found = find_weight(args[0], &e, x.size(-1), here);
+    if (found < 0) return nullptr;
+    if (!found || e.dev != here || x.size(-1) != e.k) Py_RETURN_NONE;
     const long flags = PyLong_AsLong(args[2]);
     const bool quantised = e.kind == 4 || ((flags & PREFILL) && rows >= number(N.prefill_min));
     if (e.kind == 4 ? truth(N.w4a16) : ((flags & MFMA) && !(flags & PREFILL) && truth(N.w8a8_verify))) Py_RETURN_NONE;
@@ -586,7 +606,7 @@ PyObject *embed_rows(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     const at::Tensor *ids = plain(args[1], here);
     if (!ids || ids->scalar_type() != at::kLong || !ids->is_contiguous() || ids->numel() < 1 || ids->numel() > INT32_MAX) Py_RETURN_NONE;
     Weight e;
-    if (!find_weight(args[0], &e) || e.dev != here) Py_RETURN_NONE;
+    if (find_weight(args[0], &e, -1, here) != 1 || e.dev != here) Py_RETURN_NONE;
     void *stream = c10::hip::getCurrentHIPStream(here).stream();
     const int64_t size[2] = {ids->numel(), e.k};
     at::Tensor y = new_bf16(size, here);
@@ -653,7 +673,7 @@ PyMODINIT_FUNC PyInit__host(void) {
                      {&N.prefill_min, "PREFILL_MIN_ROWS"}, {&N.mfma_min, "MFMA_MIN_ROWS"}, {&N.batch_mfma, "BATCH_MFMA"}, {&N.w8a8_verify, "W8A8_VERIFY"}, {&N.w4a16, "W4A16"},
                      {&N.handover, "HANDOVER"}, {&N.handover_min, "HANDOVER_MIN_ROWS"}, {&N.handover_max, "HANDOVER_MAX_BYTES"},
                      {&N.seen, "_QUANT_CONSUMER_SEEN"}, {&N.handed, "_HANDED"},
-                     {&N.workspace, "_WORKSPACE"}, {&N.handover_arena, "_HANDOVER_ARENA"}, {&N.take, "take"}};
+                     {&N.workspace, "_WORKSPACE"}, {&N.handover_arena, "_HANDOVER_ARENA"}, {&N.take, "take"}, {&N.resolve, "_resolve"}};
     for (const auto &e : all)
         if (!(*e.slot = PyUnicode_InternFromString(e.text))) return nullptr;
     return PyModule_Create(&module);

@@ -105,20 +105,54 @@ def test_row_thresholds_are_read_on_every_call(monkeypatch):
 
 
 @pytest.mark.parametrize("make", [_q8, _w4])
-def test_a_new_weight_costs_one_lookup_and_is_known_from_its_second_call(monkeypatch, make):
+def test_a_new_weight_is_resolved_once_and_by_the_compiled_call(monkeypatch, make):
+    """Also one that lives where a dead one did, whose record is still under the same id."""
     x = _x(3)
-    backend.linear(make(seed=11), x)                               # the host path is bound
-    lookups, real = [], backend._lookup
-    monkeypatch.setattr(backend, "_lookup", lambda w: lookups.append(w) or real(w))
-    w = make(seed=12)
-    first = backend.linear(w, x)
-    assert len(lookups) == 1
+    want = backend.linear(make(seed=12), x)                        # the host path is bound
+    made, real = [], backend._make_record
+    monkeypatch.setattr(backend, "_make_record", lambda w: made.append(id(w)) or real(w))
 
     def unexpected(*args, **kwargs):
-        raise AssertionError("a known weight went to the Python adapter")
+        raise AssertionError("a weight that the kernels take went to the Python adapter")
 
     monkeypatch.setattr(backend, "_project", unexpected)
-    assert _same(backend.linear(w, x), first) and len(lookups) == 1
+    for n in range(1, 9):
+        w = make(seed=12 if n % 2 else 13)
+        for _ in range(2):
+            assert _same(backend.linear(w, x), want) == bool(n % 2) and len(made) == n
+        del w
+
+
+class _Views:
+    """An int8 weight that hands out new tensor objects each time it is read."""
+
+    def __init__(self, q):
+        self.q, self.k, self.n = q, q.k, q.n
+
+    wq = property(lambda self: self.q.wq[:])
+    scale = property(lambda self: self.q.scale[:])
+
+
+def test_weights_that_cannot_be_remembered_or_taken_end_as_before(monkeypatch):
+    q, x = _q8(seed=21), _x(3)
+    want = backend.linear(q, x)
+    views = _Views(q)
+    for _ in range(3):
+        assert _same(backend.linear(views, x), want)
+    with pytest.raises(ValueError):                                # the width is looked at before the weight is resolved
+        backend.linear(_q8(seed=22), _x(3, K - 128))
+    with pytest.raises(ValueError):
+        backend.linear(QWeight(q.wq.cpu(), q.scale.cpu()), x)
+    wide = _w4(seed=23)
+    wide.scale = wide.scale[:-1]                                   # buffers that do not hold the weight
+    with pytest.raises(ValueError):
+        backend.linear(wide, x)
+    fresh, graph = _q8(seed=24), torch.cuda.CUDAGraph()
+    with pytest.raises(RuntimeError, match="first use"):
+        with torch.cuda.graph(graph):
+            backend.linear(fresh, x)
+    torch.cuda.synchronize()
+    assert _same(backend.linear(fresh, x), backend.linear(_q8(seed=24), x))
 
 
 @pytest.mark.parametrize("mode", ["grad", "no_grad", "inference"])
