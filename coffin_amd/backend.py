@@ -429,8 +429,9 @@ def _lookup(w) -> _Record | None:
     if rec is None:
         return None
     try:
-        first = w.wq if rec.kind == 8 else w.packed
-        if rec.src() is first and rec.src2() is w.scale:
+        first, second = w.wq if rec.kind == 8 else w.packed, w.scale
+        # (a dead reference reads as None, which is also what a released weight may hold)
+        if first is not None and second is not None and rec.src() is first and rec.src2() is second:
             _RECORDS.move_to_end(key)
             return rec
     except AttributeError:

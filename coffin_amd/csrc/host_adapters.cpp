@@ -86,7 +86,9 @@ bool holds(PyObject *w, const Weight &e) {
     PyObject *first = PyObject_GetAttr(w, e.kind == 8 ? N.wq : N.packed);
     PyObject *second = first ? PyObject_GetAttr(w, N.scale) : nullptr;
     if (!second) PyErr_Clear();
-    const bool same = second && PyWeakref_GetObject(e.src) == first && PyWeakref_GetObject(e.src2) == second;
+    // (a dead reference reads as None, which is also what a released weight may hold)
+    const bool same = second && first != Py_None && second != Py_None && PyWeakref_GetObject(e.src) == first &&
+                      PyWeakref_GetObject(e.src2) == second;
     Py_XDECREF(first);
     Py_XDECREF(second);
     return same;

@@ -54,6 +54,20 @@ def test_tensors_replaced_under_the_same_weight_object():
         assert _same(backend.linear(w, x), backend.linear(ones, x))
 
 
+@pytest.mark.parametrize("make", [_q8, _w4])
+def test_a_released_weight_is_refused(make):
+    """One whose tensors are gone, which both its entry's dead references and its attributes then say as None."""
+    w, x = make(), _x(4)
+    for _ in range(2):
+        backend.linear(w, x)
+    torch.cuda.synchronize()
+    for name in ("wq", "packed", "scale"):
+        if hasattr(w, name):
+            setattr(w, name, None)
+    with pytest.raises(AttributeError):
+        backend.linear(w, x)
+
+
 class _Swaps:
     """A weight whose ``wq`` is a property that, when told to, replaces the tensors and projects with itself: the
     outer call's table entry goes while its attributes are being read."""

@@ -337,6 +337,10 @@ def test_weight_records_are_cached_weakly_and_revalidated():
     gc.collect()
     assert alive() is None                   # the cache holds weak references only
     assert backend._lookup(torch.zeros(2, 2)) is None
+    q = synth.int8_weight(6, 32, g)
+    backend._make_record(q)
+    q.wq = q.scale = None                                  # released: its references are as dead as None
+    assert backend._lookup(q) is None
 
 
 def test_kv_quant_torch_branch_matches_oracle(orc):
