@@ -2,7 +2,7 @@
 
 When this package runs inside a coffin checkout the vendor file binds to coffin's
 own ``backends.protocol`` / ``backends.vendor`` classes; everywhere else (this
-repository's tests, the benchmark, a GPU box without the reference tree) these
+repository's tests, the benchmark, a machine without the reference tree) these
 stand-ins carry the same names, fields and error behaviour for the nine table
 entries on the path:
 
