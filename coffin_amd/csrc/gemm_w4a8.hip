@@ -340,12 +340,15 @@ extern "C" int cmi_gemm_w4a8(const uint8_t *w4, const float *ws, const int8_t *x
             return CMI_OK;
         }
     }
-    // Groups of 64 flush twice a step, which costs the 64-row tiles 1.2 .. 1.4 times the time their model (fitted to
-    // groups of 128) gives; there is no 128 x 128 one of that kind (two groups' sums do not fit the registers).
-    // From about 1024 rows on the two-stage kernel's is the better: 2048 x 51200 x 5120 1000 against 1110 us, 3000 x
-    // 2560 x 9728 138 against 165; 2048 x 6144 x 2560 81 against 72.  Chosen with the factor 1.45 the 151 sizes of its
-    // fit take 2.0 % more than the best tile of each, 4.8 % without it.
-    const bool two_stage = gs == 64 && (forced ? forced == 128 : two_stage_us(M, N, K) < 1.45 * t_tile);
+    // Groups of 64 flush twice a step, which costs the 64-row tiles up to 1.4 times the time their model (fitted to
+    // groups of 128) gives, the more the longer the launch: 1.05 .. 1.3 up to 128 rows, where a chain of a few rounds waits for
+    // memory (128 x 34816 x 5120 67 us, modelled 57; the two-stage kernel 83), 1.35 .. 1.4 beyond (3000 x 22016 x 4096 617,
+    // modelled 400; 544).  There is no 128 x 128 tile of that kind (two groups' sums do not fit the registers), so for
+    // many rows the two-stage kernel is the better: 2048 x 51200 x 5120 1000 against 1110 us; 2048 x 6144 x 2560 81 against 72.
+    // Of 431 sizes (25 layer shapes, 64..8192 rows) the choice is 0.05 % above the better of the two, at most 7 % (0.5 and
+    // 34 % with 1.45 throughout).
+    const double longer = M <= 128 ? 1.33 : M <= 512 ? 1.4 : 1.45;
+    const bool two_stage = gs == 64 && (forced ? forced == 128 : two_stage_us(M, N, K) < longer * t_tile);
     if (!group_acc && !two_stage)
         return gemm_w4a8_tile(w4, ws, xq, xs, y, M, N, K, gs, forced ? gemm_w4a8_forced_tile(forced, gs) : tile, stream);
     Args a;
