@@ -499,10 +499,15 @@ extern "C" int cmi_silu_mul_quant(const void *gate, const void *up, void *out, i
     const bool vec = K % 8 == 0 && aligned(gate, 16) && aligned(up, 16) && ld_gate % 8 == 0 &&
                      ld_up % 8 == 0 && (!out || (aligned(out, 16) && ld_out % 8 == 0)) && (!out_q || aligned(out_q, 8));
     // Vectors per workgroup of the plain product: the width from 256 down that leaves the fewest threads idle (320 and
-    // 384 vectors a row: 8192 x 2560 27.2 us at 256, 24.9 at 64; 8192 x 3072 30.9 at 256, 29.6 at 192).
+    // 384 vectors a row: 8192 x 2560 29.6 us at 256, 25.2 at 64; 8192 x 3072 32.7 and 29.5).  Of equal ones the narrower where a row
+    // is more than 256 vectors and not a whole number of them (4096 x 5120 26.4 us at 128, 25.1 at 64, 25.4 at 256), else the wider
+    // (512 x 576 3.05 us at 128, 3.46 at 64; 600 x 6144 6.5 at 256, 6.7 at 64).
     int width = THREADS;
-    for (int t = THREADS - 64; t >= 64; t -= 64)
-        if ((nvec + t - 1) / t * t < (nvec + width - 1) / width * width) width = t;
+    const bool narrow = nvec > THREADS && nvec % THREADS;
+    for (int t = THREADS - 64; t >= 64; t -= 64) {
+        const int held = (nvec + t - 1) / t * t, best = (nvec + width - 1) / width * width;
+        if (held < best || (narrow && held == best)) width = t;
+    }
     const int chunks = (nvec + width - 1) / width;
     const bool plain = vec && !out_q, whole_rows = vec && out_q && nvec <= 4 * MAX_THREADS;
     in_row_slices(M, plain ? (long)chunks * width : whole_rows ? MAX_THREADS : THREADS, [&](long lo, int rows) {
