@@ -25,28 +25,56 @@ __device__ __forceinline__ float block_max(float v, float *smem) {
     return r;
 }
 
-// K % 8 == 0, rows 16-byte aligned.  VPT > 0: the row fits in VPT vectors per
-// thread and stays in registers; VPT == 0: generic, second pass re-reads.
+// How a row of K elements is read, eight at a time.  Whole: K % 8 == 0, rows 16-byte aligned.  Ragged: any K, any
+// alignment of two bytes (a vector load needs no more on gfx950); the elements past K of the last vector are zeros and
+// are not read.
+struct Whole {
+    const uint4 *x;
+    int nvec;
+    __device__ __forceinline__ uint4 load(int row, int idx) const {
+        return idx < nvec ? x[(size_t)row * nvec + idx] : make_uint4(0, 0, 0, 0);
+    }
+    __device__ __forceinline__ int vecs() const { return nvec; }
+};
+struct Ragged {
+    const uint16_t *x;
+    int K;
+    __device__ __forceinline__ uint4 load(int row, int idx) const {
+        const uint16_t *p = x + (size_t)row * K + 8 * idx;
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (8 * idx + 8 <= K) {
+            __builtin_memcpy(&v, p, 16);
+        } else if (8 * idx < K) {
+            uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < 7; ++e)
+                if (8 * idx + e < K) w[e / 2] |= (uint32_t)p[e] << (16 * (e & 1));
+            v = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+        return v;
+    }
+    __device__ __forceinline__ int vecs() const { return (K + 7) / 8; }
+};
+
+// VPT > 0: the row fits in VPT vectors per thread and stays in registers; VPT == 0: generic, second pass re-reads.
+// Rows of q have pvec vectors; past the row's own they are zeros, as quant8 makes of zeros under every scale (rows
+// padded to whole groups of an int4 weight).
 // zero / n_zero: a few ints of the caller's that the first workgroup clears on the way (the
 // arrival counters of a split-K GEMM that follows in the stream), or null / 0.
-template <int VPT>
+template <int VPT, typename SRC>
 __global__ void __launch_bounds__(QUANT_THREADS)
-quant_act_i8_vec(const uint4 *__restrict__ x, uint2 *__restrict__ q, float *__restrict__ s,
-                 int nvec, int *__restrict__ zero, int n_zero) {
+quant_act_i8_vec(const SRC x, uint2 *__restrict__ q, float *__restrict__ s, int pvec, int *__restrict__ zero, int n_zero) {
     __shared__ float smem[QUANT_THREADS / 64];
     const int row = blockIdx.x;
     if (row == 0)
         for (int i = threadIdx.x; i < n_zero; i += QUANT_THREADS) zero[i] = 0;
-    const uint4 *xr = x + (size_t)row * nvec;
-    uint2 *qr = q + (size_t)row * nvec;
+    const int nvec = x.vecs();
+    uint2 *qr = q + (size_t)row * pvec;
     float amax = 0.f;
     if constexpr (VPT > 0) {
         uint4 v[VPT];
 #pragma unroll
-        for (int i = 0; i < VPT; ++i) {
-            const int idx = threadIdx.x + i * QUANT_THREADS;
-            v[i] = idx < nvec ? xr[idx] : make_uint4(0, 0, 0, 0);
-        }
+        for (int i = 0; i < VPT; ++i) v[i] = x.load(row, threadIdx.x + i * QUANT_THREADS);
 #pragma unroll
         for (int i = 0; i < VPT; ++i) amax = absmax8(v[i], amax);
         amax = block_max(amax, smem);
@@ -56,15 +84,15 @@ quant_act_i8_vec(const uint4 *__restrict__ x, uint2 *__restrict__ q, float *__re
 #pragma unroll
         for (int i = 0; i < VPT; ++i) {
             const int idx = threadIdx.x + i * QUANT_THREADS;
-            if (idx < nvec) qr[idx] = quant8(v[i], rs);
+            if (idx < pvec) qr[idx] = quant8(v[i], rs);
         }
     } else {
-        for (int idx = threadIdx.x; idx < nvec; idx += QUANT_THREADS) amax = absmax8(xr[idx], amax);
+        for (int idx = threadIdx.x; idx < nvec; idx += QUANT_THREADS) amax = absmax8(x.load(row, idx), amax);
         amax = block_max(amax, smem);
         const RowScale rs = row_scale(amax);
         const float sc = rs.sc;
         if (threadIdx.x == 0) s[row] = sc;
-        for (int idx = threadIdx.x; idx < nvec; idx += QUANT_THREADS) qr[idx] = quant8(xr[idx], rs);
+        for (int idx = threadIdx.x; idx < pvec; idx += QUANT_THREADS) qr[idx] = quant8(x.load(row, idx), rs);
     }
 }
 
@@ -93,9 +121,9 @@ __device__ __forceinline__ float group_max(float v) {
 // row left 15 of 16 lanes idle at 128 elements and was bound by the rate at which workgroups are started.
 // Cold operands in a graph: 16384 x 128 13.1 -> 3.6 us (1.7 TB/s; 1.6 us of it are the launch), 65536 x 128
 // 45.9 -> 7.8 us (3.2 TB/s), 8192 x 512 9.0 -> 5.6 us, 3000 x 1024 6.1 -> 4.5 us.  Same arithmetic, same bits.
-template <int LANES, int VPT, int R>
+template <int LANES, int VPT, int R, typename SRC>
 __global__ void __launch_bounds__(QUANT_THREADS)
-quant_act_i8_rows(const uint4 *__restrict__ x, uint2 *__restrict__ q, float *__restrict__ s, int nvec, int rows,
+quant_act_i8_rows(const SRC x, uint2 *__restrict__ q, float *__restrict__ s, int pvec, int rows,
                   int *__restrict__ zero, int n_zero) {
     constexpr int STEP = QUANT_THREADS / LANES;
     if (blockIdx.x == 0)
@@ -105,12 +133,9 @@ quant_act_i8_rows(const uint4 *__restrict__ x, uint2 *__restrict__ q, float *__r
     uint4 v[R][VPT];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const size_t at = (size_t)min(row0 + r * STEP, rows - 1) * nvec;
+        const int row = min(row0 + r * STEP, rows - 1);
 #pragma unroll
-        for (int i = 0; i < VPT; ++i) {
-            const int idx = l + i * LANES;
-            v[r][i] = idx < nvec ? x[at + idx] : make_uint4(0, 0, 0, 0);
-        }
+        for (int i = 0; i < VPT; ++i) v[r][i] = x.load(row, l + i * LANES);
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -124,22 +149,21 @@ quant_act_i8_rows(const uint4 *__restrict__ x, uint2 *__restrict__ q, float *__r
 #pragma unroll
         for (int i = 0; i < VPT; ++i) {
             const int idx = l + i * LANES;
-            if (idx < nvec) q[(size_t)row * nvec + idx] = quant8(v[r][i], rs);
+            if (idx < pvec) q[(size_t)row * pvec + idx] = quant8(v[r][i], rs);
         }
     }
 }
 
-// Any K, any alignment; q rows have pitch ldq >= K and the tail K .. ldq-1 is cleared.
+// Any K, any alignment of x and q.
 __global__ void __launch_bounds__(QUANT_THREADS)
 quant_act_i8_scalar(const uint16_t *__restrict__ x, int8_t *__restrict__ q,
-                    float *__restrict__ s, int K, int ldq, int *__restrict__ zero, int n_zero) {
+                    float *__restrict__ s, int K, int *__restrict__ zero, int n_zero) {
     __shared__ float smem[QUANT_THREADS / 64];
     const int row = blockIdx.x;
     if (row == 0)
         for (int i = threadIdx.x; i < n_zero; i += QUANT_THREADS) zero[i] = 0;
     const uint16_t *xr = x + (size_t)row * K;
-    int8_t *qr = q + (size_t)row * ldq;
-    for (int k = K + threadIdx.x; k < ldq; k += QUANT_THREADS) qr[k] = 0;
+    int8_t *qr = q + (size_t)row * K;
     float amax = 0.f;
     for (int k = threadIdx.x; k < K; k += QUANT_THREADS)
         amax = fmaxf(amax, fabsf(bf16_bits_to_f32(xr[k])));
@@ -151,6 +175,35 @@ quant_act_i8_scalar(const uint16_t *__restrict__ x, int8_t *__restrict__ q,
         qr[k] = (int8_t)quant1(bf16_bits_to_f32(xr[k]), rs);
 }
 
+// The vector kernels' launch: rows of pvec vectors in q.
+template <typename SRC>
+void launch_vectors(const SRC &x, int8_t *q, float *s, int M, int pvec, int *zero, int n_zero, hipStream_t st) {
+    const dim3 grid(M), block(QUANT_THREADS);
+    uint2 *qv = reinterpret_cast<uint2 *>(q);
+    const int vpt = (pvec + QUANT_THREADS - 1) / QUANT_THREADS;
+    const auto rows_launch = [&](auto kernel, int rows_per_block) {
+        kernel<<<dim3((M + rows_per_block - 1) / rows_per_block), block, 0, st>>>(x, qv, s, pvec, M, zero, n_zero);
+    };
+    const auto row_launch = [&](auto kernel) { kernel<<<grid, block, 0, st>>>(x, qv, s, pvec, zero, n_zero); };
+    // Up to 1024 elements a wavefront or less owns a row.  Two rows per lane group once one each would
+    // be more than two workgroups per CU: twice the bytes in flight per wavefront (65536 x 128: 9.8 ->
+    // 7.8 us; below that the second row only lengthens the launch, 2048 x 576: 3.3 -> 3.9 us).
+    // Two vectors a lane pay from 257 rows on; below, a workgroup per row is shorter (1 x 576 1.99 us against 2.16,
+    // 256 x 576 2.40 against 2.55, 512 x 576 5 % the other way).
+    const auto many = [&](int rows_per_block) { return M > 512 * rows_per_block; };
+    if (pvec <= 8) many(32) ? rows_launch(quant_act_i8_rows<8, 1, 2, SRC>, 64) : rows_launch(quant_act_i8_rows<8, 1, 1, SRC>, 32);
+    else if (pvec <= 16) many(16) ? rows_launch(quant_act_i8_rows<16, 1, 2, SRC>, 32) : rows_launch(quant_act_i8_rows<16, 1, 1, SRC>, 16);
+    else if (pvec <= 32) many(8) ? rows_launch(quant_act_i8_rows<32, 1, 2, SRC>, 16) : rows_launch(quant_act_i8_rows<32, 1, 1, SRC>, 8);
+    else if (pvec <= 64) many(4) ? rows_launch(quant_act_i8_rows<64, 1, 2, SRC>, 8) : rows_launch(quant_act_i8_rows<64, 1, 1, SRC>, 4);
+    else if (pvec <= 128 && M > QUANT_THREADS) rows_launch(quant_act_i8_rows<64, 2, 1, SRC>, 4);
+    else if (vpt <= 1) row_launch(quant_act_i8_vec<1, SRC>);
+    else if (vpt <= 2) row_launch(quant_act_i8_vec<2, SRC>);
+    else if (vpt <= 4) row_launch(quant_act_i8_vec<4, SRC>);
+    else if (vpt <= 8) row_launch(quant_act_i8_vec<8, SRC>);
+    else if (vpt <= 16) row_launch(quant_act_i8_vec<16, SRC>);
+    else row_launch(quant_act_i8_vec<0, SRC>);
+}
+
 }  // namespace
 
 int cmi::quant_act_i8_and_clear(const void *x, int8_t *q, float *s, int M, int K, int *zero, int n_zero,
@@ -159,45 +212,25 @@ int cmi::quant_act_i8_and_clear(const void *x, int8_t *q, float *s, int M, int K
     if (M == 0) return CMI_OK;  // an empty batch has no storage to point at
     CMI_REQUIRE(x && q && s, CMI_E_ARG, "cmi_quant_act_i8: null pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const dim3 grid(M), block(QUANT_THREADS);
-    if (K % 8 == 0 && aligned(x, 16) && aligned(q, 8)) {
-        const int nvec = K / 8;
-        const uint4 *xv = static_cast<const uint4 *>(x);
-        uint2 *qv = reinterpret_cast<uint2 *>(q);
-        const int vpt = (nvec + QUANT_THREADS - 1) / QUANT_THREADS;
-        const auto rows_launch = [&](auto kernel, int rows_per_block) {
-            kernel<<<dim3((M + rows_per_block - 1) / rows_per_block), block, 0, st>>>(xv, qv, s, nvec, M, zero, n_zero);
-        };
-        // Up to 1024 elements a wavefront or less owns a row.  Two rows per lane group once one each would
-        // be more than two workgroups per CU: twice the bytes in flight per wavefront (65536 x 128: 9.8 ->
-        // 7.8 us; below that the second row only lengthens the launch, 2048 x 576: 3.3 -> 3.9 us).
-        // Two vectors a lane pay from 257 rows on; below, a workgroup per row is shorter (1 x 576 1.99 us against 2.16,
-        // 256 x 576 2.40 against 2.55, 512 x 576 5 % the other way).
-        const auto many = [&](int rows_per_block) { return M > 512 * rows_per_block; };
-        if (nvec <= 8) many(32) ? rows_launch(quant_act_i8_rows<8, 1, 2>, 64) : rows_launch(quant_act_i8_rows<8, 1, 1>, 32);
-        else if (nvec <= 16) many(16) ? rows_launch(quant_act_i8_rows<16, 1, 2>, 32) : rows_launch(quant_act_i8_rows<16, 1, 1>, 16);
-        else if (nvec <= 32) many(8) ? rows_launch(quant_act_i8_rows<32, 1, 2>, 16) : rows_launch(quant_act_i8_rows<32, 1, 1>, 8);
-        else if (nvec <= 64) many(4) ? rows_launch(quant_act_i8_rows<64, 1, 2>, 8) : rows_launch(quant_act_i8_rows<64, 1, 1>, 4);
-        else if (nvec <= 128 && M > QUANT_THREADS) rows_launch(quant_act_i8_rows<64, 2, 1>, 4);
-        else if (vpt <= 1) quant_act_i8_vec<1><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);
-        else if (vpt <= 2) quant_act_i8_vec<2><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);
-        else if (vpt <= 4) quant_act_i8_vec<4><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);
-        else if (vpt <= 8) quant_act_i8_vec<8><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);
-        else if (vpt <= 16) quant_act_i8_vec<16><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);
-        else quant_act_i8_vec<0><<<grid, block, 0, st>>>(xv, qv, s, nvec, zero, n_zero);
-    } else {
-        quant_act_i8_scalar<<<grid, block, 0, st>>>(static_cast<const uint16_t *>(x), q, s, K, K, zero, n_zero);
-    }
+    if (K % 8 == 0 && aligned(x, 16) && aligned(q, 8))
+        launch_vectors(Whole{static_cast<const uint4 *>(x), K / 8}, q, s, M, K / 8, zero, n_zero, st);
+    else
+        quant_act_i8_scalar<<<dim3(M), dim3(QUANT_THREADS), 0, st>>>(static_cast<const uint16_t *>(x), q, s, K, zero, n_zero);
     return check_launch("cmi_quant_act_i8");
 }
 
+// Rows of an int4 weight whose K is not whole groups: the vector kernels as well, whatever K is, since the padded rows
+// of q are whole vectors.  Element by element, each read twice, the projection behind it included: 9664 -> 2560, one
+// row 15.7 -> 9.0 us, 16 rows 24.6 -> 12.9, 8000 rows 395 -> 308; 100 rows of 2497 -> 9000 21.7 -> 17.5.
 int cmi::quant_act_i8_padded(const void *x, int8_t *q, float *s, int M, int K, int ldq, void *stream) {
     if (ldq == K) return quant_act_i8_and_clear(x, q, s, M, K, nullptr, 0, stream);
-    CMI_REQUIRE(M >= 0 && K > 0 && ldq > K, CMI_E_ARG, "cmi_quant_act_i8: bad shape M=%d K=%d pitch=%d", M, K, ldq);
+    CMI_REQUIRE(M >= 0 && K > 0 && ldq > K && ldq % 8 == 0, CMI_E_ARG, "cmi_quant_act_i8: bad shape M=%d K=%d pitch=%d", M, K, ldq);
     if (M == 0) return CMI_OK;
     CMI_REQUIRE(x && q && s, CMI_E_ARG, "cmi_quant_act_i8: null pointer");
-    quant_act_i8_scalar<<<dim3(M), dim3(QUANT_THREADS), 0, static_cast<hipStream_t>(stream)>>>(
-        static_cast<const uint16_t *>(x), q, s, K, ldq, nullptr, 0);
+    CMI_REQUIRE(aligned(q, 8), CMI_E_ARG, "cmi_quant_act_i8: rows must be 8-byte aligned");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (K % 8 == 0 && aligned(x, 16)) launch_vectors(Whole{static_cast<const uint4 *>(x), K / 8}, q, s, M, ldq / 8, nullptr, 0, st);
+    else launch_vectors(Ragged{static_cast<const uint16_t *>(x), K}, q, s, M, ldq / 8, nullptr, 0, st);
     return check_launch("cmi_quant_act_i8");
 }
 

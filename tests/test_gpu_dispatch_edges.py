@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from coffin_amd import _native, synth
+from coffin_amd.weights import W4A8Weight
 from tests import gpu_util as G
 
 pytestmark = pytest.mark.gpu
@@ -19,6 +20,33 @@ def test_quantiser_of_short_rows(orc, m, k):
     q_ref, s_ref = orc.quant_act_i8(G.bits(x))
     q, s = G.quant(x.to(G.DEV))
     assert (q.cpu().numpy() == q_ref).all() and (s.cpu().numpy() == s_ref).all()
+
+
+@pytest.mark.parametrize("m,k,skip", [(3, 1, 0), (2, 57, 0), (600, 100, 0), (5, 130, 0), (9000, 200, 1), (3, 504, 1), (300, 999, 0),
+                                      (2, 1016, 0), (5, 1500, 0), (4, 3000, 3), (3, 9664, 0), (2, 16383, 0), (2, 32776, 0),
+                                      (3, 33001, 0)])
+def test_quantiser_of_rows_padded_to_whole_groups(orc, m, k, skip):
+    """Every share of a row a lane can have, whole vectors and not, rows that start ``skip`` elements off a 16-byte boundary,
+    and one whose scale is infinite: the rows that the entry leaves in its workspace, cleared past K."""
+    g = synth.generator(m + k)
+    x = synth.activations(m, k, g, outliers=True)
+    x[m // 2, k // 2] = float("inf")
+    q_ref, s_ref = orc.quant_act_i8(G.bits(x))
+    xd = torch.empty(m * k + skip, dtype=torch.bfloat16, device=G.DEV)[skip:].view(m, k)
+    xd.copy_(x)
+    w = W4A8Weight.quantize(synth.dense_weight(16, k, g), group_size=128)
+    w4, ws = G.w4_repack(w.packed.to(G.DEV), w.scale.to(G.DEV), k)
+    lib = _native.load()
+    kd = int(lib.cmi_w4_device_k(k, 128))
+    nbytes = int(lib.cmi_linear_workspace_bytes(m, kd))
+    work = torch.full((nbytes,), 0xA5, dtype=torch.uint8, device=G.DEV)
+    y = torch.empty((m, 16), dtype=torch.bfloat16, device=G.DEV)
+    _native.check(lib.cmi_linear_w4a8_bf16(G.ptr(w4), G.ptr(ws), G.ptr(xd), G.ptr(y), m, 16, k, 128, G.ptr(work), nbytes,
+                                           G.stream()), "linear_w4a8_bf16")
+    rows = work[:m * kd].view(torch.int8).view(m, kd).cpu()
+    at = (m * kd + 255) // 256 * 256
+    assert (rows[:, :k].numpy() == q_ref).all() and not rows[:, k:].any()
+    assert (work[at:at + 4 * m].view(torch.float32).cpu().numpy() == s_ref).all()
 
 
 @pytest.mark.parametrize("m,k", [(256, 8192), (257, 8192), (2, 8200), (257, 1032), (258, 16392), (3, 24584), (257, 32768), (2, 32776),
