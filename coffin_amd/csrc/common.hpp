@@ -29,11 +29,11 @@ int option_w4_decode_chain();  // 0 = the library chooses, 1 = never, else a var
         if (!(cond)) return cmi::fail(code, __VA_ARGS__); \
     } while (0)
 
-// gemm_mfma.hip: register-staged W8A8 GEMM for K % 64 != 0 (see gemm_w8a8.hip for the fast path).
+// gemm_mfma.hip: register-staged W8A8 GEMM for rows under 128 elements or over 4 Mi, and for under 8 outputs (see gemm_w8a8.hip for the fast path).
 int gemm_w8a8_generic(const int8_t *xq, const int8_t *wq, const float *xs, const float *ws, void *y,
                       int32_t *acc_out, int M, int N, int K, int ldy, void *stream);
-// gemm_w8a8_rows16.hip: W8A8 for up to 16 rows with the weight read once (K % 128 == 0,
-// K <= 10240); CMI_E_UNSUPPORTED (no error text) outside that range.
+// gemm_w8a8_rows16.hip: W8A8 for up to 128 rows with the weight read once (K % 16 == 0,
+// 128 <= K <= 10240); CMI_E_UNSUPPORTED (no error text) outside that range.
 int gemm_w8a8_rows16(const int8_t *xq, const int8_t *wq, const float *xs, const float *ws, void *y,
                      int32_t *acc_out, int M, int N, int K, int ldy, void *stream);
 // gemm_w8a8.hip: cmi_gemm_w8a8 with room for split-K (arrival counters, 256 ints, zero; partial

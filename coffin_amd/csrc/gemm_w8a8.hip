@@ -1,4 +1,4 @@
-// W8A8 prefill GEMM for CDNA4 int8 MFMA (K a multiple of 128).
+// W8A8 prefill GEMM for CDNA4 int8 MFMA (K a multiple of 16, from 128 up).
 //
 //   acc[m,n] = sum_k xq[m,k] * wq[n,k]           int32, exact
 //   y[m,n]   = bf16((float)acc * xs[m] * ws[n])   left to right, one narrowing
@@ -47,6 +47,7 @@ namespace {
 using namespace cmi;
 
 constexpr int BK = 128;        // one 128-byte cache line per row and step
+constexpr int MAX_K = 1 << 22; // a tile's operand offsets are 30 bits (Operand); longer rows take the generic kernel
 constexpr double SPLIT128_HANDOVER_US = 11.0;  // split-K on 128 x 128 tiles: partials out, arrival, partials in (measured 10..11.5)
 constexpr int THREADS = 256;   // 2 x 2 wavefronts
 
@@ -123,6 +124,41 @@ __device__ __forceinline__ void stage_scales(const Args &a, float *dst, int n0, 
     for (int i = threadIdx.x; i < BN + BM; i += blockDim.x)
         dst[i] = i < BN ? a.ws[min(n0 + i, a.N - 1)] : a.xs[min(m0 + i - BN, a.M - 1)];
 }
+
+// The rows of one operand that a block tile multiplies, as direct global -> LDS loads (buffer_load_dwordx4 ... lds) of 8
+// rows x 128 B: lane i lands in slot i of the 1 KiB, row i / 8, stored chunk i % 8, which holds k chunk
+// (i % 8) ^ ((row / 2) % 8).  Rows past the matrix read as zeros (a buffer access is checked against the resource's size
+// with the scalar offset included, measured on gfx950).
+//
+// K need not be whole steps of 128: in the last one the chunks past K belong to the next row.  Those of the activations
+// are asked for past the resource's end and read as zeros, so what the weight's hold does not matter.  Two vector
+// instructions a step; on the register-staged kernel such rows took, 9664 -> 2560, 100 rows 98.8 us against 19.8 now,
+// 1000 rows 100.7 / 51.5, 8000 rows 377 / 187, 200 rows of 2496 -> 9000 34.2 / 20.6.
+struct Operand {
+    static constexpr uint32_t PAST = 1u << 30;  // beyond any tile: launches keep rows x K below it
+    __amdgpu_buffer_rsrc_t res;
+    uint32_t off[2];   // lane offsets of even and odd loads
+    uint32_t mask[2];  // PAST where the lane's chunk of the last step is past K
+    int K, last, first;
+    // Rows row0 .. row0 + tile - 1 of `rows`; this wavefront's loads start at row 8 first_load of them.
+    __device__ __forceinline__ Operand(const int8_t *base, int row0, int rows, int tile, int k, int lane, int first_load)
+        : K(k), last((k - 1) / BK), first(first_load) {
+        res = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(base) + (size_t)row0 * k, 0, min(rows - row0, tile) * k, 0x00020000);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const int chunk = ((lane & 7) ^ (lane >> 4) ^ (4 * ((first + p) & 1))) * 16;
+            off[p] = (uint32_t)((lane >> 3) * k + chunk);
+            mask[p] = last * BK + chunk >= k ? PAST : 0;
+        }
+    }
+    // Selector of `load`: all ones in the last step.
+    __device__ __forceinline__ uint32_t past_end(int ks) const { return ks == last ? ~0u : 0u; }
+    // The wavefront's load g (a constant) of step ks into its 1 KiB behind `base`.
+    __device__ __forceinline__ void load(int8_t *base, int g, int ks, uint32_t past) const {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(res, (lds_ptr_t)(base + (first + g) * 1024), 16, off[g & 1] | (mask[g & 1] & past),
+                                                 ks * BK + (first + g) * 8 * K, 0, 0);
+    }
+};
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
@@ -282,39 +318,22 @@ gemm_w8a8_pipe_kernel(const Args a) {
     float *scales = reinterpret_cast<float *>(lds + NST * C::STAGE_BYTES);
     stage_scales<C::BN, C::BM>(a, scales, n0, m0);
     // this workgroup's K steps: all of them, or part `split` of a.splits nearly equal parts
-    const int ksteps_all = a.K / BK;
+    const int ksteps_all = (a.K + BK - 1) / BK;
     const int k_first = SPLIT ? (int)((long long)ksteps_all * split / a.splits) : 0;
     const int ksteps = SPLIT ? (int)((long long)ksteps_all * (split + 1) / a.splits) - k_first : ksteps_all;
 
     // Global side of the direct loads.  One load instruction moves 8 rows x 128 B
     // (whole cache lines) into 1 KiB of LDS; each wavefront fills a contiguous run
     // of rows (consecutive loads on consecutive rows measured 30 % faster than
-    // wavefronts interleaved row group by row group).  Lane i lands in slot i of the group: row = i/8, stored chunk
-    // = i%8, which holds k chunk (i%8) ^ ((row/2) % 8).
-    const int lrow = lane >> 3;
-    const int8_t *wsrc[C::WL], *xsrc[C::XL];
-#pragma unroll
-    for (int g = 0; g < C::WL; ++g) {
-        const int row = (C::WL * wave + g) * 8 + lrow;
-        const int kc = (lane & 7) ^ ((row >> 1) & 7);
-        wsrc[g] = a.wq + (size_t)min(n0 + row, a.N - 1) * a.K + kc * 16 + k_first * BK;
-    }
-#pragma unroll
-    for (int g = 0; g < C::XL; ++g) {
-        const int row = (C::XL * wave + g) * 8 + lrow;
-        const int kc = (lane & 7) ^ ((row >> 1) & 7);
-        xsrc[g] = a.xq + (size_t)min(m0 + row, a.M - 1) * a.K + kc * 16 + k_first * BK;
-    }
+    // wavefronts interleaved row group by row group).
+    const Operand w(a.wq, n0, a.N, C::BN, a.K, lane, C::WL * wave), x(a.xq, m0, a.M, C::BM, a.K, lane, C::XL * wave);
     auto issue = [&](int stage, int ks) {
         int8_t *base = lds + stage * C::STAGE_BYTES;
-        const int k = ks * BK;
+        const uint32_t past = x.past_end(k_first + ks);
 #pragma unroll
-        for (int g = 0; g < C::WL; ++g)
-            __builtin_amdgcn_global_load_lds((const void *)(wsrc[g] + k), (lds_ptr_t)(base + (C::WL * wave + g) * 1024), 16, 0, 0);
+        for (int g = 0; g < C::WL; ++g) w.load(base, g, k_first + ks, 0);
 #pragma unroll
-        for (int g = 0; g < C::XL; ++g)
-            __builtin_amdgcn_global_load_lds((const void *)(xsrc[g] + k),
-                                             (lds_ptr_t)(base + C::W_BYTES + (C::XL * wave + g) * 1024), 16, 0, 0);
+        for (int g = 0; g < C::XL; ++g) x.load(base + C::W_BYTES, g, k_first + ks, past);
     };
 
     // LDS side: lane reads row (lane%32) of a 32-row MFMA tile; for k quarter q
@@ -560,33 +579,18 @@ gemm_w8a8_big_kernel(const Args a) {
     tile_coords(a, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
 
-    // Wavefront w fills a contiguous run of an operand tile's rows, BM / 8 (256 / 8) of them: loads of
-    // 8 rows x 128 B each; slot and swizzle as in the 4-wavefront kernel.
-    const int lrow = lane >> 3;
-    const int8_t *wsrc[WL], *xsrc[XL];
-#pragma unroll
-    for (int g = 0; g < WL; ++g) {
-        const int row = (WL * wave + g) * 8 + lrow;
-        wsrc[g] = a.wq + (size_t)min(n0 + row, a.N - 1) * a.K + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
-    }
-#pragma unroll
-    for (int g = 0; g < XL; ++g) {
-        const int row = (XL * wave + g) * 8 + lrow;
-        xsrc[g] = a.xq + (size_t)min(m0 + row, a.M - 1) * a.K + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
-    }
+    // Wavefront w fills a contiguous run of an operand tile's rows, BM / 8 (256 / 8) of them.
+    const Operand w(a.wq, n0, a.N, BN, a.K, lane, WL * wave), x(a.xq, m0, a.M, BM, a.K, lane, XL * wave);
     // ring slot of a unit, as a byte offset
     auto slot_of = [](int unit) { return (unit % SLOTS) * SLOT_BYTES; };
     auto issue_w = [&](int ks) {
-        int8_t *base = lds + slot_of(2 * ks) + (WL * wave) * 1024;
 #pragma unroll
-        for (int g = 0; g < WL; ++g)
-            __builtin_amdgcn_global_load_lds((const void *)(wsrc[g] + ks * BK), (lds_ptr_t)(base + g * 1024), 16, 0, 0);
+        for (int g = 0; g < WL; ++g) w.load(lds + slot_of(2 * ks), g, ks, 0);
     };
     auto issue_x = [&](int ks) {
-        int8_t *base = lds + slot_of(2 * ks + 1) + (XL * wave) * 1024;
+        const uint32_t past = x.past_end(ks);
 #pragma unroll
-        for (int g = 0; g < XL; ++g)
-            __builtin_amdgcn_global_load_lds((const void *)(xsrc[g] + ks * BK), (lds_ptr_t)(base + g * 1024), 16, 0, 0);
+        for (int g = 0; g < XL; ++g) x.load(lds + slot_of(2 * ks + 1), g, ks, past);
     };
 
     // lane reads row (lane % 16) of a 16-row MFMA tile; for k half h its 16 bytes are k chunk 4h + lane / 16
@@ -647,7 +651,7 @@ gemm_w8a8_big_kernel(const Args a) {
     using w_only_t = std::integral_constant<int, 2 * WT>;
     using w_and_x_t = std::integral_constant<int, 2 * WT + 2 * TM>;
 
-    const int ksteps = a.K / BK;
+    const int ksteps = (a.K + BK - 1) / BK;
     WFrag w0, w1;
     XFrag x0, x1;
     // Step ks computes from units 2ks, 2ks+1 (first-quarter fragments in w0, x0).
@@ -887,7 +891,9 @@ gemm_w8a8_wide_kernel(const Args a) {
                         scales + BN + wm * 32 * TM);
 }
 
+// Whole steps only: the clamped loads of this kernel stay inside a row.
 int launch_wide(Args &a, hipStream_t st) {
+    if (a.K % BK != 0) return launch_big<4, 2>(a, st);
     a.tiles_m = (a.M + wide::BM - 1) / wide::BM;
     a.tiles_n = (a.N + wide::BN - 1) / wide::BN;
     static std::atomic<uint64_t> devices{0};
@@ -955,6 +961,8 @@ __device__ __forceinline__ void lds_wait(v4i32 &f0, v4i32 &f1, v4i32 &x0, v4i32 
 }
 }  // namespace tilewise
 
+// TAIL: K is not whole steps (its own instance: beside the others' two instructions a step cost this kernel 1..2 %).
+template <bool TAIL>
 __global__ void __launch_bounds__(512, 2)
 gemm_w8a8_wide_tilewise_kernel(const Args a) {
     using namespace wide;
@@ -985,10 +993,14 @@ gemm_w8a8_wide_tilewise_kernel(const Args a) {
     const int wrow = wn * 160 + wm * 8 + lrow;  // + 32 i: the swizzle does not depend on i
     const uint32_t wvoff = (uint32_t)wrow * (uint32_t)a.K + (((lane & 7) ^ ((wrow >> 1) & 7)) * 16);
     const int xrow = XL * wave * 8 + lrow;      // + 8 g: odd g flip bit 2 of the swizzle
-    uint32_t xvoff[2];
+    uint32_t xvoff[2], xmask[2];
+    const int last = (a.K - 1) / BK;
 #pragma unroll
-    for (int g = 0; g < 2; ++g)
-        xvoff[g] = (uint32_t)xrow * (uint32_t)a.K + (((lane & 7) ^ (((xrow + 8 * g) >> 1) & 7)) * 16);
+    for (int g = 0; g < 2; ++g) {
+        const int chunk = ((lane & 7) ^ (((xrow + 8 * g) >> 1) & 7)) * 16;
+        xvoff[g] = (uint32_t)xrow * (uint32_t)a.K + chunk;
+        xmask[g] = TAIL && last * BK + chunk >= a.K ? 1u << 31 : 0;  // chunks past K: past the resource's end (see Operand)
+    }
     const __amdgpu_buffer_rsrc_t wres =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(a.wq), 0, (int)((size_t)a.N * a.K), 0x00020000);
     const __amdgpu_buffer_rsrc_t xres =
@@ -1002,10 +1014,11 @@ gemm_w8a8_wide_tilewise_kernel(const Args a) {
                                                  wtile + i * k32 + ks * BK, 0, 0);
     };
     auto issue_a = [&](int stage, int ks) {
+        const uint32_t past = TAIL && ks == last ? ~0u : 0u;
 #pragma unroll
         for (int g = 0; g < XL; ++g)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (lds_ptr_t)(xslot + stage * X_QUARTER + g * 1024), 16,
-                                                     xvoff[g & 1], xtile + g * k8 + ks * BK, 0, 0);
+                                                     xvoff[g & 1] | (xmask[g & 1] & past), xtile + g * k8 + ks * BK, 0, 0);
         issue_w(stage, ks, 0);
         issue_w(stage, ks, 1);
     };
@@ -1074,7 +1087,7 @@ gemm_w8a8_wide_tilewise_kernel(const Args a) {
         lds_wait<N>(wf[BUF[P][K]][0], wf[BUF[P][K]][1], xf[0][2 * H], xf[1][2 * H], xf[0][2 * H + 1], xf[1][2 * H + 1]);
     };
     auto fence = [&]() { __builtin_amdgcn_sched_barrier(0); };
-    const int ksteps = a.K / BK;
+    const int ksteps = (a.K + BK - 1) / BK;
     // One K step from stage P.  On entry the fragments of half groups 0 and 1 are on their way (12
     // reads, issued in that order).  It requests step `rks`, two steps ahead; past the end the last
     // step's operands once more instead of nothing (into rows that are free, nobody reads them), so
@@ -1171,6 +1184,7 @@ gemm_w8a8_wide_tilewise_kernel(const Args a) {
 
 int launch_wide(Args &a, hipStream_t st);
 
+template <bool TAIL>
 int launch_wide_tilewise(Args &a, hipStream_t st) {
     // buffer offsets are 32 bits: matrices (and the tile rows past their end) must stay below 2 GiB
     if ((size_t)(a.N + wide::BN) * a.K >= ((size_t)1 << 31) || (size_t)(a.M + wide::BM) * a.K >= ((size_t)1 << 31))
@@ -1178,10 +1192,10 @@ int launch_wide_tilewise(Args &a, hipStream_t st) {
     a.tiles_m = (a.M + wide::BM - 1) / wide::BM;
     a.tiles_n = (a.N + wide::BN - 1) / wide::BN;
     static std::atomic<uint64_t> devices{0};
-    if (const int rc = reserve_lds(reinterpret_cast<const void *>(gemm_w8a8_wide_tilewise_kernel),
+    if (const int rc = reserve_lds(reinterpret_cast<const void *>(gemm_w8a8_wide_tilewise_kernel<TAIL>),
                                    wide::LDS_BYTES, devices, "cmi_gemm_w8a8"))
         return rc;
-    gemm_w8a8_wide_tilewise_kernel<<<dim3(a.tiles_m * a.tiles_n), dim3(512), wide::LDS_BYTES, st>>>(a);
+    gemm_w8a8_wide_tilewise_kernel<TAIL><<<dim3(a.tiles_m * a.tiles_n), dim3(512), wide::LDS_BYTES, st>>>(a);
     return check_launch("cmi_gemm_w8a8");
 }
 
@@ -1194,7 +1208,7 @@ extern "C" int cmi_gemm_w8a8(const int8_t *xq, const int8_t *wq, const float *xs
 }
 
 size_t cmi::gemm_w8a8_split_bytes(int M, int N, int K) {
-    if (M <= 16 || K % BK != 0 || N < 8) return 0;
+    if (M <= 16 || K < BK || K > MAX_K || N < 8) return 0;
     // up to 256 workgroups of 64 x 64 or 128 x 64 int32 each, whatever the split
     if (M <= 256) return (size_t)256 * 128 * 64 * 4;
     // up to 1024 rows of a narrow, long projection (at most 128 tiles of 128 x 128, 16 K steps and
@@ -1220,7 +1234,7 @@ int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, co
         if (rc != CMI_E_UNSUPPORTED) return rc;
     }
     int mid = 0;  // 17..256 rows: the tile kernel the cost models below chose (64 x 64: 6464), if any
-    if (M > 16 && M <= 256 && K % BK == 0 && N >= 8 && !force) {
+    if (M > 16 && M <= 256 && K >= BK && K <= MAX_K && N >= 8 && !force) {
         // Between the GEMV-like batch and the full tile pipeline every kernel is bound by what its
         // workgroups pull through L2 per dependent step, and which one is fastest changes with the
         // shape: the read-once kernel pays per 16-row chunk, a tile kernel K / 128 steps whose
@@ -1228,7 +1242,7 @@ int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, co
         // Cost models (us) fitted to cold-weight measurements of all five kernels on eleven layer
         // shapes x ten batch sizes; their choice is within 1 % of the best measured in total
         // (the two-candidate rule this replaces: 19 % above).
-        const double steps = K / 128.0, wbytes = (double)N * K;
+        const double steps = (K + BK - 1) / BK, wbytes = (double)N * K;
         auto rounds = [](double tiles) { return ceil(tiles / 256.0); };
         const double tiles_h = (double)((M + 63) / 64) * ((N + 63) / 64);
         const double tiles_g = (double)((M + 127) / 128) * ((N + 63) / 64);
@@ -1300,7 +1314,7 @@ int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, co
         }
         mid = t_h <= t_g && t_h <= t_t ? 6464 : t_g <= t_t ? 64 : 128;
     }
-    if (K % BK != 0 || N < 8) return gemm_w8a8_generic(xq, wq, xs, ws, y, acc_out, M, N, K, ldy, stream);
+    if (K < BK || K > MAX_K || N < 8) return gemm_w8a8_generic(xq, wq, xs, ws, y, acc_out, M, N, K, ldy, stream);
     Args a;
     a.xq = xq;
     a.wq = wq;
@@ -1337,7 +1351,7 @@ int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, co
     if (force || mid) {
         pick = force ? force : mid;
     } else {
-        const double steps = K / 128.0;
+        const double steps = (K + BK - 1) / BK;
         auto cost = [&](int bm, int bn, double a0, double b0, double c0) {
             const double tiles = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
             // the 4-wavefront tiles on up to 192 CUs: the idle CUs warm the caches (see above)
@@ -1377,7 +1391,7 @@ int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, co
     }
     // the 256 x 320 tile: the tile-wise kernel (within 1 % of the two-stage one on the large shapes,
     // 7 % faster at 2048 x 4096 x 2560); a forced 320 still names the two-stage kernel
-    if (pick == 321 || pick == 322 || (pick == 320 && !force)) return launch_wide_tilewise(a, st);
+    if (pick == 321 || pick == 322 || (pick == 320 && !force)) return K % BK == 0 ? launch_wide_tilewise<false>(a, st) : launch_wide_tilewise<true>(a, st);
     if (pick == 320) return launch_wide(a, st);
     if (pick == 256) return launch_big<4, 2>(a, st);
     if (pick == 256192) return launch_big<2, 3>(a, st);

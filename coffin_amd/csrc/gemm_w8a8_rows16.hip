@@ -31,8 +31,17 @@ struct Args {
     int M, N, K, ldy;
 };
 
+// One of this lane's 16-byte pieces of a line of activation rows (tile_src).  TAIL: rows end inside their last line; the
+// pieces past K are zeros, so it does not matter that the weight's repeat the row's last piece.
+template <bool TAIL>
+__device__ __forceinline__ v4i32 load_x(const Args &a, int lane, int half, int first_row, int line) {
+    const v4i32 v = *reinterpret_cast<const v4i32 *>(a.xq + tile_src<TAIL>(lane, half, first_row, a.M - 1, a.K, line * LINE));
+    if constexpr (TAIL) return line * LINE + (lane & 7) * 16 < a.K ? v : v4i32{0, 0, 0, 0};
+    return v;
+}
+
 // NLP: lines per wavefront (upper bound; surplus slots are skipped).  WAVES: 4 or 8.
-template <int NLP, int WAVES>
+template <int NLP, int WAVES, bool TAIL>
 __global__ void __launch_bounds__(WAVES * 64)
 gemm_w8a8_rows16_kernel(const Args a) {
     __shared__ __align__(16) int32_t partial[WAVES][64][4];
@@ -42,7 +51,7 @@ gemm_w8a8_rows16_kernel(const Args a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kq = lane >> 4;
     const int n0 = blockIdx.x * ROWS;
-    const int lines = a.K / LINE;
+    const int lines = (a.K + LINE - 1) / LINE;
     uint8_t *patch = patches[wave];
 
     // activations first (L2 resident; memory answers in request order), then every weight byte
@@ -53,7 +62,7 @@ gemm_w8a8_rows16_kernel(const Args a) {
         if (line >= lines) break;  // uniform per wavefront
 #pragma unroll
         for (int h = 0; h < 2; ++h)  // rows past M repeat the last one; their sums are dropped
-            xr[i][h] = *reinterpret_cast<const v4i32 *>(a.xq + tile_src(lane, h, 0, a.M - 1, a.K, line * LINE));
+            xr[i][h] = load_x<TAIL>(a, lane, h, 0, line);
     }
 #pragma unroll
     for (int i = 0; i < NLP; ++i) {
@@ -62,7 +71,7 @@ gemm_w8a8_rows16_kernel(const Args a) {
 #pragma unroll
         for (int h = 0; h < 2; ++h)
             wr[i][h] = __builtin_nontemporal_load(
-                reinterpret_cast<const v4i32 *>(a.wq + tile_src(lane, h, n0, a.N - 1, a.K, line * LINE)));
+                reinterpret_cast<const v4i32 *>(a.wq + tile_src<TAIL>(lane, h, n0, a.N - 1, a.K, line * LINE)));
     }
 
     // the scales of the output this thread will finish, requested behind the operands: asked for at
@@ -109,7 +118,8 @@ gemm_w8a8_rows16_kernel(const Args a) {
 template <int NLP, int WAVES>
 int launch(const Args &a, hipStream_t st) {
     const dim3 grid((a.N + ROWS - 1) / ROWS);
-    gemm_w8a8_rows16_kernel<NLP, WAVES><<<grid, dim3(WAVES * 64), 0, st>>>(a);
+    if (a.K % LINE == 0) gemm_w8a8_rows16_kernel<NLP, WAVES, false><<<grid, dim3(WAVES * 64), 0, st>>>(a);
+    else gemm_w8a8_rows16_kernel<NLP, WAVES, true><<<grid, dim3(WAVES * 64), 0, st>>>(a);
     return check_launch("cmi_gemm_w8a8");
 }
 
@@ -122,7 +132,7 @@ int launch(const Args &a, hipStream_t st) {
 // chunk with ds_add and the bits are those of the 16-row kernel by construction.
 constexpr int MAX_CHUNKS = 8;
 
-template <int NLP, int WAVES, int T>
+template <int NLP, int WAVES, int T, bool TAIL>
 __global__ void __launch_bounds__(WAVES * 64)
 gemm_w8a8_rows128_kernel(const Args a) {
     __shared__ __align__(16) int32_t sums[MAX_CHUNKS * T][64][4];
@@ -133,7 +143,7 @@ gemm_w8a8_rows128_kernel(const Args a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kq = lane >> 4;
     const int n0 = blockIdx.x * (ROWS * T);
-    const int lines = a.K / LINE;
+    const int lines = (a.K + LINE - 1) / LINE;
     const int chunks = (a.M + ROWS - 1) / ROWS;
     uint8_t *patch = patches[wave];
     auto line_of = [&](int i) { return min(wave + i * WAVES, lines - 1); };  // surplus slots repeat the last line
@@ -142,8 +152,7 @@ gemm_w8a8_rows128_kernel(const Args a) {
     auto request_x = [&](int c, int i) {
 #pragma unroll
         for (int h = 0; h < 2; ++h)  // rows past M repeat the last one; their sums are dropped
-            xr[i][h] = *reinterpret_cast<const v4i32 *>(
-                a.xq + tile_src(lane, h, c * ROWS, a.M - 1, a.K, line_of(i) * LINE));
+            xr[i][h] = load_x<TAIL>(a, lane, h, c * ROWS, line_of(i));
     };
 #pragma unroll
     for (int i = 0; i < NLP; ++i) request_x(0, i);
@@ -154,7 +163,7 @@ gemm_w8a8_rows128_kernel(const Args a) {
 #pragma unroll
             for (int h = 0; h < 2; ++h)
                 wr[t][i][h] = __builtin_nontemporal_load(reinterpret_cast<const v4i32 *>(
-                    a.wq + tile_src(lane, h, n0 + t * ROWS, a.N - 1, a.K, line_of(i) * LINE)));
+                    a.wq + tile_src<TAIL>(lane, h, n0 + t * ROWS, a.N - 1, a.K, line_of(i) * LINE)));
     // the scales of the tile, requested behind the operands instead of cold at the end
     if (threadIdx.x < T * ROWS) ws_tile[threadIdx.x] = a.ws[min(n0 + (int)threadIdx.x, a.N - 1)];
     else if (threadIdx.x < T * ROWS + MAX_CHUNKS * ROWS)
@@ -213,7 +222,8 @@ gemm_w8a8_rows128_kernel(const Args a) {
 template <int NLP, int WAVES, int T>
 int launch128(const Args &a, hipStream_t st) {
     const dim3 grid((a.N + ROWS * T - 1) / (ROWS * T));
-    gemm_w8a8_rows128_kernel<NLP, WAVES, T><<<grid, dim3(WAVES * 64), 0, st>>>(a);
+    if (a.K % LINE == 0) gemm_w8a8_rows128_kernel<NLP, WAVES, T, false><<<grid, dim3(WAVES * 64), 0, st>>>(a);
+    else gemm_w8a8_rows128_kernel<NLP, WAVES, T, true><<<grid, dim3(WAVES * 64), 0, st>>>(a);
     return check_launch("cmi_gemm_w8a8");
 }
 
@@ -232,7 +242,7 @@ int gemm_w8a8_rows_tiles(int N) {
 // outside this kernel's range (the caller then uses a tiled kernel).
 int gemm_w8a8_rows16(const int8_t *xq, const int8_t *wq, const float *xs, const float *ws, void *y,
                      int32_t *acc_out, int M, int N, int K, int ldy, void *stream) {
-    if (M < 1 || M > MAX_CHUNKS * ROWS || N < 1 || K < LINE || K % LINE != 0 || K > 80 * LINE)
+    if (M < 1 || M > MAX_CHUNKS * ROWS || N < 1 || K < LINE || K % 16 != 0 || K > 80 * LINE)
         return CMI_E_UNSUPPORTED;
     if (!aligned(xq, 16) || !aligned(wq, 16)) return CMI_E_UNSUPPORTED;
     Args a;
@@ -247,7 +257,7 @@ int gemm_w8a8_rows16(const int8_t *xq, const int8_t *wq, const float *xs, const 
     a.K = K;
     a.ldy = ldy;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const int lines = K / LINE;
+    const int lines = (K + LINE - 1) / LINE;
     // eight wavefronts (shorter chains of dependent steps) measured 0.3-0.7 us faster up to
     // N = 19456; no difference at N = 151936
     const bool eight = (N + ROWS - 1) / ROWS <= 2048;

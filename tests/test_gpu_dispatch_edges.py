@@ -186,3 +186,35 @@ def test_192_row_tile_of_the_w8a8_gemm(orc, m, n, k):
     G.set_option("gemm_tile", 256192)  # (conftest resets it)
     acc, y = G.gemm_w8a8(G.dev(xq), q.wq.to(G.DEV), G.dev(xs), q.scale.to(G.DEV))
     assert (acc.cpu().numpy() == acc_ref).all() and (G.bits(y) == y_ref).all()
+
+
+def _with_neighbours(a: torch.Tensor) -> torch.Tensor:
+    """``a`` on the device, the bytes behind its last row 127."""
+    home = torch.full((a.numel() + 512,), 127, dtype=a.dtype, device=G.DEV)
+    home[:a.numel()] = a.reshape(-1).to(G.DEV)
+    return home[:a.numel()].view(a.shape)
+
+
+@pytest.mark.parametrize("m,n,k", [(3, 40, 144), (16, 33, 2064), (17, 8, 240), (31, 530, 1232), (70, 200, 9664), (100, 300, 10256), (129, 161, 208),
+                                   (200, 520, 192), (260, 264, 1040), (300, 2560, 2496), (577, 650, 320)])
+def test_w8a8_rows_that_end_inside_a_step(orc, m, n, k):
+    """K of 16 .. 112 more than whole steps of 128: the library's choice (up to 16 rows, 17..256, beyond), then every tile,
+    with and without room to split K; beyond a row's end lie other rows' values."""
+    g = synth.generator(m + n + k)
+    q = synth.int8_weight(n, k, g)
+    x = synth.activations(m, k, g, outliers=True)
+    xq, xs = orc.quant_act_i8(G.bits(x))
+    acc_ref, y_ref = orc.gemm_w8a8(xq, q.wq.numpy(), xs, q.scale.numpy())
+    xd, wd = _with_neighbours(torch.from_numpy(xq)), _with_neighbours(q.wq)
+    xsd, wsd = G.dev(xs), q.scale.to(G.DEV)
+    for tile in (0, 6464, 64, 128, 192, 128192, 256, 256192, 320, 321):
+        G.set_option("gemm_tile", tile)
+        acc, y = G.gemm_w8a8(xd, wd, xsd, wsd)
+        assert (acc.cpu().numpy() == acc_ref).all() and (G.bits(y) == y_ref).all(), tile
+    G.set_option("gemm_tile", 0)
+    lib = _native.load()
+    nbytes = int(lib.cmi_linear_w8a8_workspace_bytes(m, n, k))
+    work = torch.full((nbytes,), 0xA5, dtype=torch.uint8, device=G.DEV)
+    xb, y = x.to(G.DEV), torch.empty((m, n), dtype=torch.bfloat16, device=G.DEV)
+    _native.check(lib.cmi_linear_w8a8_bf16(G.ptr(xb), G.ptr(wd), G.ptr(wsd), G.ptr(y), m, n, k, n, G.ptr(work), nbytes, G.stream()), "linear")
+    assert (G.bits(y) == y_ref).all()
