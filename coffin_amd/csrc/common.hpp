@@ -22,6 +22,7 @@ int reserve_lds(const void *kernel, int bytes, std::atomic<uint64_t> &devices, c
 int option_gemm_tile();      // 0 = the library chooses, else a tile code of cmi_set_option
 int option_gemv_wholerow();  // -1 = the library chooses, 0 = never, 1 = where it can
 int option_w4_decode_waves();  // 0 = the library chooses, else 4 or 16 wavefronts per workgroup
+int option_w4_gemm_deep();     // 0 = the library chooses, 1 = never, else a tile code (gemm_w4a8_deep_code)
 int option_w4_decode_chain();  // 0 = the library chooses, 1 = never, else a variant code of gemv_w4a8_chain
 
 #define CMI_REQUIRE(cond, code, ...)                 \
@@ -66,10 +67,13 @@ int gemv_w4a8_chain(const uint8_t *w4, const float *ws, const void *x, const int
 int gemv_w4a8_rows16(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs, const void *x,
                      void *y, int32_t *group_acc, int8_t *xq_out, float *xs_out, int M, int N, int K,
                      void *stream);
-// gemm_w4a8_tile.hip: W4A8 tile GEMM, arguments already checked by cmi_gemm_w4a8.  The cheapest tile for a shape
-// and its modelled time (us); the tile a gemm_tile option names; the launch.
+// gemm_w4a8_tile.hip: W4A8 tile GEMM, arguments already checked by cmi_gemm_w4a8 / cmi_gemv_w4a8.  The cheapest tile for a
+// shape and its modelled time (us), of all tiles and of those of four groups a step (groups of 128); the tile a gemm_tile
+// option names; whether a w4_gemm_deep option names one; the launch.
 double gemm_w4a8_tile_us(int M, int N, int K, int gs, int *tile);
+double gemm_w4a8_deep_us(int M, int N, int K, int *tile);
 int gemm_w4a8_forced_tile(int option, int gs);
+bool gemm_w4a8_deep_code(int code);
 int gemm_w4a8_tile(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs, void *y, int M, int N,
                    int K, int gs, int tile, void *stream);
 // linear_bf16.hip: quantiser + W4A8 GEMV / GEMM (or the GEMV that quantises by itself where that

@@ -93,6 +93,56 @@ __device__ __forceinline__ float total_of(const Args &a, int m, int n) {
     return total;
 }
 
+// y[m,n] = bf16(total * xs[m]) of a wavefront's TM x TN tiles of 16 x 16 at (mw, nw) of its workgroup's, into LDS.
+// inexact: lanes that met a scale below 2^-122; the wavefront's results are formed anew.
+template <int TM, int TN, int YPITCH, int LG>
+__device__ __forceinline__ void park_results(const Args &a, const float (&total)[TM][TN][4], uint64_t inexact, uint16_t *park, int m0,
+                                             int n0, int mw, int nw, int lane) {
+    const int fr = lane & 15, fc = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int ml = mw + i * 16 + fc * 4 + r;
+            const float xm = a.xs[min(m0 + ml, a.M - 1)];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) park[ml * (YPITCH / 2) + nw + j * 16 + fr] = (uint16_t)f32_to_bf16_bits(total[i][j][r] * xm);
+        }
+    if (inexact)
+        for (int e = lane; e < 16 * TM * 16 * TN; e += 64) {
+            const int ml = mw + e / (16 * TN), nl = nw + e % (16 * TN);
+            if (m0 + ml < a.M && n0 + nl < a.N)
+                park[ml * (YPITCH / 2) + nl] = (uint16_t)f32_to_bf16_bits(total_of<LG>(a, m0 + ml, n0 + nl) * a.xs[m0 + ml]);
+        }
+}
+
+// The results of a BM x BN tile, parked in LDS in rows of YPITCH bytes, leave as whole 16-byte pieces of rows.
+template <int BM, int BN, int YPITCH, int THREADS>
+__device__ __forceinline__ void store_parked(const Args &a, const uint16_t *park, int m0, int n0) {
+    const int rows = min(a.M - m0, BM), cols = min(a.N - n0, BN);
+    if (a.N % 8 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0) {
+        constexpr int CH = BN / 8;
+        for (int t = threadIdx.x; t < rows * CH; t += THREADS) {
+            const int m = t / CH, c = t - m * CH;
+            const uint4 v = *reinterpret_cast<const uint4 *>(reinterpret_cast<const int8_t *>(park) + m * YPITCH + c * 16);
+            uint16_t *dst = a.y + (size_t)(m0 + m) * a.N + n0 + c * 8;
+            if (c * 8 + 8 <= cols) {
+                *reinterpret_cast<uint4 *>(dst) = v;
+            } else {
+                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    if (c * 8 + k < cols) dst[k] = (uint16_t)(w[k / 2] >> (16 * (k & 1)));
+            }
+        }
+    } else {  // rows that are not 16-byte aligned: element by element, a wavefront's stores side by side
+        for (int t = threadIdx.x; t < rows * BN; t += THREADS) {
+            const int m = t / BN, c = t - m * BN;
+            if (c < cols) a.y[(size_t)(m0 + m) * a.N + n0 + c] = park[m * (YPITCH / 2) + c];
+        }
+    }
+}
+
 // LG: log2(group size / 32).  2: a step is a group.  3: a group is two steps, the first one's sums are kept.  1: a
 // step holds two groups, one MFMA each.
 template <int WM, int WN, int TM, int TN, int NST, int LG>
@@ -312,45 +362,198 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_tile_kernel(const A
     // y[m,n] = bf16(total * xs[m]), parked in LDS so that whole 16-byte pieces of rows leave
     __syncthreads();
     uint16_t *park = reinterpret_cast<uint16_t *>(lds);
+    park_results<TM, TN, C::YPITCH, LG>(a, total, inexact, park, m0, n0, wm * 16 * TM, wn * 16 * TN, lane);
+    __syncthreads();
+    store_parked<C::BM, C::BN, C::YPITCH, C::THREADS>(a, park, m0, n0);
+}
+
+// ---------------------------------------------------------------------------
+// Few tiles, or few rows (2 .. several hundred): a step of four groups.
+//
+// What bounds it.  With a tile or two per CU the kernel above is a chain of K / 128 steps of 0.27 us whatever is in them:
+// the barrier, the trip to LDS for the next fragments and one wavefront per SIMD with 40 vector instructions to issue.
+// Here a barrier buys four groups: 0.6 .. 0.9 us per step of 512 k, of which, taken apart for 100 rows of 9728 -> 2560 (32
+// x 64 tiles, 20.6 us in all with the quantiser), the operands' way from L2 to LDS takes 10 us (62 B/ns per CU of the 75 that
+// such loads reach) and fragments and arithmetic 10, half of it hidden under the other.
+//
+// A row's 512 (activations) or 256 (packed weight) bytes of a step are requested together and lie together in LDS, 16-byte
+// piece index XOR row % 16; the step's scales come the same way.  A wavefront reads its fragments of all four groups behind
+// the barrier and has no others in flight (reading them a step ahead measured 2..5 % slower: registers and the same
+// LDS time).  NST = 2 stages leave room for two or three workgroups per CU, which hide each other's trips; 3 or 4 are
+// for launches of one per CU.  A wavefront on 16 rows at a time widens every code again for the next 16: the 32- and 48-row
+// tiles of wavefronts side by side do it once.  Sharing K among wavefronts that hand their sums over through LDS was built
+// first and took 32 us for that shape: operands straight into registers in the MFMA arrangement come at 16 bytes a clock.
+//
+// ONCE: a single tile of rows, so that every weight byte is read by one workgroup and need not stay in the caches.
+//
+// Cold weights, with the quantiser: 100 rows of 9728 -> 2560 29.2 -> 20.6 us, 40 rows 23.8 -> 16.7, 200 rows 34.6 ->
+// 27.1; 100 rows of 4096 -> 2560 14.3 -> 10.8; 40 rows of 25600 -> 5120 60.7 -> 39.6; 16 rows of 2560 -> 151936 54.3 -> 48.7,
+// of 4096 -> 12288 12.1 -> 9.2 (both against the matrix-pipe GEMV).
+constexpr int NT = 2;  // cache policy of a load: nontemporal
+constexpr int U = 4, X_ROW = U * BK, P_ROW = U * BK / 2;  // groups of a stage; bytes of a row in it: 512 and 256
+
+template <int WM, int WN, int TM, int TN, int NST>
+struct DeepCfg {
+    static constexpr int WAVES = WM * WN, THREADS = 64 * WAVES;
+    static constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
+    static constexpr int X_BYTES = BM * X_ROW, P_BYTES = BN * P_ROW;
+    static constexpr int S_BYTES = BN * U * 4, STAGE = X_BYTES + P_BYTES + S_BYTES;
+    static constexpr int XL = X_BYTES / 1024 / WAVES, PL = P_BYTES / 1024 / WAVES;  // requests per wavefront and stage
+    static constexpr int SL = (BN * U / 64 + WAVES - 1) / WAVES;
+    static constexpr int LOADS = XL + PL + SL;
+    static constexpr int YPITCH = 2 * BN + 16;
+    static constexpr int LDS_BYTES = NST * STAGE;
+    static_assert(BM % (2 * WAVES) == 0 && BN % (4 * WAVES) == 0, "whole requests per wavefront");
+    static_assert(BM * YPITCH <= LDS_BYTES, "result does not fit");
+};
+
+template <int WM, int WN, int TM, int TN, int NST, bool ONCE>
+__global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_deep_kernel(const Args a) {
+    using C = DeepCfg<WM, WN, TM, TN, NST>;
+    extern __shared__ __align__(16) int8_t lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wn = wave % WN, wm = wave / WN;
+    int tm, tn;
+    banded_tile(a.tiles_m, a.tiles_n, blockIdx.x, tm, tn);
+    const int m0 = tm * C::BM, n0 = tn * C::BN;
+
+    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t *>(a.xq) + (size_t)m0 * a.K, 0, min(a.M - m0, C::BM) * a.K, 0x00020000);
+    const __amdgpu_buffer_rsrc_t pres = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(a.w4) + (size_t)n0 * (a.K / 2), 0, min(a.N - n0, C::BN) * (a.K / 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t sres = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(a.ws) + (size_t)n0 * a.G, 0, min(a.N - n0, C::BN) * a.G * 4, 0x00020000);
+
+    // Requests of a stage: two rows x 512 B of activations, four rows x 256 B of packed weight each, 16-byte piece index
+    // XOR row % 16; then the scales, [column][U].
+    int xoff[C::XL], poff[C::PL];
+#pragma unroll
+    for (int h = 0; h < C::XL; ++h) xoff[h] = (lane >> 5) * a.K + ((lane & 31) ^ ((2 * (C::XL * wave + h) + (lane >> 5)) & 15)) * 16;
+#pragma unroll
+    for (int h = 0; h < C::PL; ++h) poff[h] = (lane >> 4) * (a.K / 2) + ((lane & 15) ^ ((4 * (C::PL * wave + h) + (lane >> 4)) & 15)) * 16;
+    const int soff = (lane / U) * a.G * 4 + (lane % U) * 4;
+    auto issue = [&](int slot, int stage) {
+        int8_t *base = lds + slot * C::STAGE;
+#pragma unroll
+        for (int h = 0; h < C::PL; ++h) {
+            const int q = C::PL * wave + h, off = poff[h];
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(pres, (lds_ptr_t)(base + C::X_BYTES + q * 1024), 16, off,
+                                                     stage * P_ROW + q * 4 * (a.K / 2), 0, ONCE ? NT : 0);
+        }
+#pragma unroll
+        for (int h = 0; h < C::XL; ++h) {
+            const int q = C::XL * wave + h, off = xoff[h];
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (lds_ptr_t)(base + q * 1024), 16, off, stage * X_ROW + q * 2 * a.K, 0, 0);
+        }
+#pragma unroll
+        for (int h = 0; h < C::SL; ++h) {
+            const int r = min(C::SL * wave + h, C::BN * U / 64 - 1);  // past the last: the last again, same bytes
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(sres, (lds_ptr_t)(base + C::X_BYTES + C::P_BYTES + r * 256), 4, soff,
+                                                     stage * U * 4 + r * (64 / U) * a.G * 4, 0, 0);
+        }
+    };
+    // a lane's pieces: row fr of a tile, piece u * 4 + fc of the packed row and pieces u * 8 + 2 fc + e of the activations
+    const int fr = lane & 15, fc = lane >> 4;
+    int xf[2][2], pf[U];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) xf[h][e] = (wm * 16 * TM + fr) * X_ROW + ((8 * h + 2 * fc + e) ^ fr) * 16;  // u = h, h + 2: 256 B on
+#pragma unroll
+    for (int u = 0; u < U; ++u) pf[u] = C::X_BYTES + (wn * 16 * TN + fr) * P_ROW + ((4 * u + fc) ^ fr) * 16;
+    const int sf = C::X_BYTES + C::P_BYTES + (wn * 16 * TN + fr) * (U * 4);
+    auto nibbles = [](int word, int high) {
+        return (int)(((high ? (uint32_t)word : (uint32_t)word << 4) & 0xF0F0F0F0u) ^ 0x80808080u);
+    };
+
+    float total[TM][TN][4];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int ml = wm * 16 * TM + i * 16 + fc * 4 + r;
-            const float xm = a.xs[min(m0 + ml, a.M - 1)];
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
-                park[ml * (C::YPITCH / 2) + wn * 16 * TN + j * 16 + fr] = (uint16_t)f32_to_bf16_bits(total[i][j][r] * xm);
-        }
-    if (inexact)
-        for (int e = lane; e < 16 * TM * 16 * TN; e += 64) {
-            const int ml = wm * 16 * TM + e / (16 * TN), nl = wn * 16 * TN + e % (16 * TN);
-            if (m0 + ml < a.M && n0 + nl < a.N)
-                park[ml * (C::YPITCH / 2) + nl] = (uint16_t)f32_to_bf16_bits(total_of<LG>(a, m0 + ml, n0 + nl) * a.xs[m0 + ml]);
-        }
-    __syncthreads();
-    const int rows = min(a.M - m0, C::BM), cols = min(a.N - n0, C::BN);
-    if (a.N % 8 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0) {
-        constexpr int CH = C::BN / 8;
-        for (int t = threadIdx.x; t < rows * CH; t += C::THREADS) {
-            const int m = t / CH, c = t - m * CH;
-            const uint4 v = *reinterpret_cast<const uint4 *>(lds + m * C::YPITCH + c * 16);
-            uint16_t *dst = a.y + (size_t)(m0 + m) * a.N + n0 + c * 8;
-            if (c * 8 + 8 <= cols) {
-                *reinterpret_cast<uint4 *>(dst) = v;
-            } else {
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+            for (int r = 0; r < 4; ++r) total[i][j][r] = 0.f;
+    constexpr uint32_t TINY = 2 * (5u << 23) - 1;  // as above
+    uint32_t least = ~0u;
+
 #pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    if (c * 8 + k < cols) dst[k] = (uint16_t)(w[k / 2] >> (16 * (k & 1)));
+    for (int s = 0; s < NST - 1; ++s) issue(s, s);
+    int slot = 0;
+    auto stage = [&](auto whole_tag, int s) {
+        constexpr bool WHOLE = decltype(whole_tag)::value;
+        wait_vmcnt<(NST - 2) * C::LOADS>();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        // the slot that the stage before was read from
+        issue(slot == 0 ? NST - 1 : slot - 1, s + NST - 1);
+        const int8_t *base = lds + slot * C::STAGE;
+        f32x4 sc[TN];
+        v4i32 x[U][TM][2], p[U][TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) sc[j] = *reinterpret_cast<const f32x4 *>(base + sf + j * 16 * U * 4);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) p[u][j] = *reinterpret_cast<const v4i32 *>(base + pf[u] + j * 16 * P_ROW);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    x[u][i][e] = *reinterpret_cast<const v4i32 *>(base + xf[u & 1][e] + (u >> 1) * 256 + i * 16 * X_ROW);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (!WHOLE && s * U + u >= a.G) break;  // uniform
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                v4i32 w[2];
+#pragma unroll
+                for (int h = 0; h < 8; ++h) w[h / 4][h % 4] = nibbles(p[u][j][h / 2], h & 1);
+                least = min(least, 2 * __float_as_uint(sc[j][u]) - 1);
+                const float scale = sc[j][u] * 0.0625f;
+#pragma unroll
+                for (int i = 0; i < TM; ++i) {
+                    v4i32 acc = {0, 0, 0, 0};
+                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[u][i][0], w[0], acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[u][i][1], w[1], acc, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) total[i][j][r] = fmaf((float)acc[r], scale, total[i][j][r]);
+                }
             }
         }
-    } else {  // rows that are not 16-byte aligned: element by element, a wavefront's stores side by side
-        for (int t = threadIdx.x; t < rows * C::BN; t += C::THREADS) {
-            const int m = t / C::BN, c = t - m * C::BN;
-            if (c < cols) a.y[(size_t)(m0 + m) * a.N + n0 + c] = park[m * (C::YPITCH / 2) + c];
-        }
-    }
+        slot = slot + 1 == NST ? 0 : slot + 1;
+    };
+    const int whole = a.G / U;
+    for (int s = 0; s < whole; ++s) stage(std::true_type{}, s);
+    if (whole * U < a.G) stage(std::false_type{}, whole);
+    const uint64_t inexact = __builtin_amdgcn_ballot_w64(least < TINY);
+    wait_vmcnt<0>();
+    __syncthreads();
+    uint16_t *park = reinterpret_cast<uint16_t *>(lds);
+    park_results<TM, TN, C::YPITCH, 2>(a, total, inexact, park, m0, n0, wm * 16 * TM, wn * 16 * TN, lane);
+    __syncthreads();
+    store_parked<C::BM, C::BN, C::YPITCH, C::THREADS>(a, park, m0, n0);
+}
+
+template <int WM, int WN, int TM, int TN, int NST>
+int launch_deep(Args &a, hipStream_t st) {
+    using C = DeepCfg<WM, WN, TM, TN, NST>;
+    a.tiles_m = (a.M + C::BM - 1) / C::BM;
+    a.tiles_n = (a.N + C::BN - 1) / C::BN;
+    // the tile's operand offsets are 32-bit
+    CMI_REQUIRE((size_t)(C::BM > C::BN ? C::BM : C::BN) * (a.K + NST * X_ROW) < ((size_t)1 << 31), CMI_E_UNSUPPORTED,
+                "cmi_gemm_w4a8: K=%d too long", a.K);
+    static std::atomic<uint64_t> devices[2];
+    const auto run = [&](auto kernel, std::atomic<uint64_t> &done) {
+        if (const int rc = reserve_lds(reinterpret_cast<const void *>(kernel), C::LDS_BYTES, done, "cmi_gemm_w4a8")) return rc;
+        kernel<<<dim3(a.tiles_m * a.tiles_n), dim3(C::THREADS), C::LDS_BYTES, st>>>(a);
+        return check_launch("cmi_gemm_w4a8");
+    };
+    return a.tiles_m == 1 ? run(gemm_w4a8_deep_kernel<WM, WN, TM, TN, NST, true>, devices[1])
+                          : run(gemm_w4a8_deep_kernel<WM, WN, TM, TN, NST, false>, devices[0]);
 }
 
 template <int WM, int WN, int TM, int TN, int NST, int LG>
@@ -371,7 +574,8 @@ int launch(Args &a, hipStream_t st) {
 
 // The tiles (rows x columns).  Two workgroups of four wavefronts share a CU; 128 x 160 exists for the tile count
 // (1024 x 5120: 256 tiles, one per CU).
-enum Tile { T128x160, T128x128, T64x128, T64x96, T64x64, T32x64, T32x128, T16x32, TILES };
+// (D: of four groups a step, L with more stages)
+enum Tile { T128x160, T128x128, T64x128, T64x96, T64x64, T32x64, T32x128, T16x32, D16x64, D16x64L, D32x32, D32x32L, D32x64, D32x64L, D48x64, TILES };
 
 template <int LG>
 int launch_tile(Args &a, Tile tile, hipStream_t st) {
@@ -381,6 +585,13 @@ int launch_tile(Args &a, Tile tile, hipStream_t st) {
             case T128x128: return launch<2, 2, 4, 4, 3, 2>(a, st);
             case T64x96: return launch<2, 2, 2, 3, 3, 2>(a, st);
             case T32x128: return launch<1, 4, 2, 2, 4, 2>(a, st);
+            case D16x64: return launch_deep<1, 4, 1, 1, 2>(a, st);
+            case D16x64L: return launch_deep<1, 4, 1, 1, 4>(a, st);
+            case D32x32: return launch_deep<2, 2, 1, 1, 2>(a, st);
+            case D32x32L: return launch_deep<2, 2, 1, 1, 4>(a, st);
+            case D32x64: return launch_deep<1, 4, 2, 1, 2>(a, st);
+            case D32x64L: return launch_deep<2, 4, 1, 1, 3>(a, st);
+            case D48x64: return launch_deep<1, 4, 3, 1, 2>(a, st);
             default: break;
         }
     }
@@ -401,7 +612,7 @@ struct Cost {
     double fixed, step, tile, odd, n;
     bool any_group;  // built for groups of 64 and 256 too
 };
-const Cost COSTS[TILES] = {
+const Cost COSTS[D16x64] = {
     {128, 160, 6.82, 0.0000, 0.7856, 0.0163, 0.0024, false},
     {128, 128, 5.36, 0.0000, 0.6325, 0.0240, 0.0059, false},
     {64, 128, 4.18, 0.0071, 0.3823, 0.0521, 0.0376, true},
@@ -411,6 +622,32 @@ const Cost COSTS[TILES] = {
     {32, 128, 3.44, 0.0000, 0.2513, 0.0209, 0.0682, false},
     {16, 32, 2.76, 0.0342, 0.0615, 0.0152, 0.0926, true},
 };
+
+// The same for the tiles of four groups a step: fixed part, per step a share of every tile the CU holds, of every round
+// of the workgroups it can hold at a time and of the cold weight, and what a tile and a round cost beside their steps.  Fitted to
+// cold-weight sweeps on fifteen layer shapes x 21 batch sizes (17..1024 rows) and twenty x five (2..16).
+struct DeepCost {
+    int bm, bn, per_cu, code;  // code: cmi_set_option("w4_gemm_deep"), rows x 100 + columns, one more for more stages
+    double fixed, tile, round, n, tiles, rounds;
+};
+const DeepCost DEEP_COSTS[TILES - D16x64] = {
+    {16, 64, 3, 1664, 1.84, 0.196, 0.297, 0.289, 0.41, 0.28}, {16, 64, 1, 1665, 1.40, 0.463, 0.0, 0.219, 0.0, 1.57},
+    {32, 32, 3, 3232, 1.84, 0.198, 0.273, 0.222, 0.28, 0.52}, {32, 32, 1, 3233, 1.47, 0.452, 0.0, 0.121, 0.0, 1.53},
+    {32, 64, 2, 3264, 1.64, 0.266, 0.412, 0.203, 0.31, 0.93}, {32, 64, 1, 3265, 1.41, 0.420, 0.188, 0.165, 0.0, 1.65},
+    {48, 64, 1, 4864, 1.37, 0.865, 0.0, 0.180, 0.0, 1.88},
+};
+
+Tile deep_tile(int code) {
+    int t = 0;
+    while (t < TILES - D16x64 && DEEP_COSTS[t].code != code) ++t;
+    return static_cast<Tile>(D16x64 + t);
+}
+
+double cost(const DeepCost &c, int M, int N, int K) {
+    const double steps = (K + U * BK - 1) / (U * BK), r = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) / 256.0;
+    const double held = r <= 6 ? ceil(r) : r + 0.5, rounds = ceil(r / c.per_cu);
+    return c.fixed + steps * (c.tile * held + c.round * rounds + c.n * N * 1e-4) + c.tiles * held + c.rounds * rounds;
+}
 
 double cost(const Cost &c, int M, int N, int K) {
     const double steps = K / 128.0, r = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) / 256.0;
@@ -423,13 +660,32 @@ double cost(const Cost &c, int M, int N, int K) {
 
 namespace cmi {
 
+double gemm_w4a8_deep_us(int M, int N, int K, int *tile) {
+    const int option = option_w4_gemm_deep();
+    if (option > 1) {
+        *tile = deep_tile(option);
+        return 0.0;
+    }
+    double best = 1e30;
+    for (int t = 0; option == 0 && K <= 1 << 24 && t < TILES - D16x64; ++t) {  // (longer rows: the tile's offsets are 32-bit)
+        const double us = cost(DEEP_COSTS[t], M, N, K);
+        if (us < best) best = us, *tile = D16x64 + t;
+    }
+    return best;
+}
+
 double gemm_w4a8_tile_us(int M, int N, int K, int gs, int *tile) {
     double best = 1e30;
-    for (int t = 0; t < TILES; ++t) {
+    for (int t = 0; t < D16x64; ++t) {
         if (gs != BK && !COSTS[t].any_group) continue;
         const double us = cost(COSTS[t], M, N, K);
         if (us < best) best = us, *tile = t;
     }
+    // Four groups a step where they are modelled to gain at least 3 %: 315 sizes of 17..1024 rows 6678 -> 5997 us in all (5908
+    // with the best of every size; the worst loss 9 %, 40 rows of 8960 -> 1536 6.0 -> 6.6 us).
+    int deep = 0;
+    const double us = gs == BK ? gemm_w4a8_deep_us(M, N, K, &deep) : 1e30;
+    if (us < 0.97 * best) best = us, *tile = deep;
     return best;
 }
 
@@ -441,6 +697,8 @@ int gemm_w4a8_forced_tile(int option, int gs) {
         if (e.option == option && (gs == BK || COSTS[e.tile].any_group)) return e.tile;
     return T64x64;
 }
+
+bool gemm_w4a8_deep_code(int code) { return deep_tile(code) < TILES; }
 
 int gemm_w4a8_tile(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs, void *y, int M, int N, int K,
                    int gs, int tile, void *stream) {

@@ -53,6 +53,7 @@ constexpr int UNREAD = INT32_MIN;
 std::atomic<int> g_gemm_tile{UNREAD};      // 0 = the library chooses
 std::atomic<int> g_gemv_wholerow{UNREAD};  // -1 = the library chooses, 0 = never, 1 = where it can
 std::atomic<int> g_w4_decode_waves{0};     // 0 = the library chooses, 4 or 16 wavefronts per workgroup
+std::atomic<int> g_w4_gemm_deep{0};        // 0 = the library chooses, 1 = never, else a tile code
 std::atomic<int> g_w4_decode_chain{0};     // 0 = the library chooses, 1 = never, else a variant code
 
 bool valid_gemm_tile(int v) { return v == 0 || v == 64 || v == 128 || v == 256 || v == 192 || v == 320 || v == 321 || v == 322 || v == 6464 || v == 128192 || v == 256192; }
@@ -90,6 +91,7 @@ int option_gemv_wholerow() {
 }
 
 int option_w4_decode_waves() { return g_w4_decode_waves.load(std::memory_order_relaxed); }
+int option_w4_gemm_deep() { return g_w4_gemm_deep.load(std::memory_order_relaxed); }
 int option_w4_decode_chain() { return g_w4_decode_chain.load(std::memory_order_relaxed); }
 
 }  // namespace cmi
@@ -113,6 +115,12 @@ extern "C" int cmi_set_option(const char *name, int value) {
         CMI_REQUIRE(value == 0 || value == 4 || value == 16, CMI_E_ARG,
                     "cmi_set_option: w4_decode_waves=%d, expected 0 (library's choice), 4 or 16", value);
         g_w4_decode_waves.store(value, std::memory_order_relaxed);
+        return CMI_OK;
+    }
+    if (!strcmp(name, "w4_gemm_deep")) {
+        CMI_REQUIRE(value == 0 || value == 1 || gemm_w4a8_deep_code(value), CMI_E_ARG,
+                    "cmi_set_option: w4_gemm_deep=%d, expected 0 (library's choice), 1 (never), 1664, 1665, 3232, 3233, 3264, 3265 or 4864", value);
+        g_w4_gemm_deep.store(value, std::memory_order_relaxed);
         return CMI_OK;
     }
     if (!strcmp(name, "w4_decode_chain")) {

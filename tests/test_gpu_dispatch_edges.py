@@ -153,6 +153,46 @@ def test_w4a8_tiles_with_a_step_count_that_is_no_whole_chunk(orc, k):
         assert (G.bits(y) == y_ref).all(), tile
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 24, 128), (3, 40, 512), (17, 33, 640), (16, 64, 1024), (33, 65, 384), (47, 130, 1152), (49, 129, 2560), (97, 200, 3712),
+                                   (65, 96, 4608)])
+def test_w4a8_tiles_of_four_groups_a_step(orc, m, n, k):
+    """One to many steps and one to four groups in the last, ragged in both directions, odd and 16-byte rows of results; then
+    with scales below 2^-122 in some columns."""
+    g = synth.generator(m + n + k)
+    w = synth.int4_weight(n, k, g)
+    x = synth.activations(m, k, g, outliers=True)
+    xq, xs = orc.quant_act_i8(G.bits(x))
+    tiny = w.scale.clone()
+    tiny[:, ::3] = torch.ldexp(torch.ones(1), torch.tensor(-126)).item()
+    tiny[k // 128 - 1, 1::3] = 2.0 ** -140
+    tiny[0, 2::3] = 0.0
+    for scale in (w.scale, tiny):
+        _, y_ref = orc.linear_w4a8(xq, xs, w.packed.numpy(), scale.numpy(), k, 128)
+        w4, ws = G.w4_repack(w.packed.to(G.DEV), scale.to(G.DEV), k)
+        for code in (1664, 1665, 3232, 3233, 3264, 3265, 4864):
+            G.set_option("w4_gemm_deep", code)
+            _, y = G.w4a8(w4, ws, G.dev(xq), G.dev(xs), k, gemm=True, want_acc=False)
+            assert (G.bits(y) == y_ref).all(), code
+            if 3 <= m <= 16:
+                _, y = G.w4a8(w4, ws, G.dev(xq), G.dev(xs), k, gemm=False, want_acc=False)
+                assert (G.bits(y) == y_ref).all(), code
+        G.set_option("w4_gemm_deep", 0)
+
+
+@pytest.mark.parametrize("m,n,k", [(16, 12288, 4096), (4, 24000, 768), (9, 5120, 25600), (40, 2560, 9728), (70, 6144, 2560), (200, 2560, 9728)])
+def test_w4a8_rows_through_the_chosen_tile(m, n, k):
+    """Sizes where the choice is a tile of four groups a step: the results of the kernels without them."""
+    gen = torch.Generator(device=G.DEV).manual_seed(m + n + k)
+    w4 = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=G.DEV, generator=gen)
+    ws = torch.rand((n, k // 128), device=G.DEV, generator=gen) * 0.01 + 1e-4
+    xq = torch.randint(-127, 128, (m, k), dtype=torch.int8, device=G.DEV, generator=gen)
+    xs = torch.rand(m, device=G.DEV, generator=gen) + 0.5
+    _, y = G.w4a8(w4, ws, xq, xs, k, gemm=m > 16, want_acc=False)
+    G.set_option("w4_gemm_deep", 1)
+    _, ref = G.w4a8(w4, ws, xq, xs, k, gemm=m > 16, want_acc=False)
+    assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
+
+
 @pytest.mark.parametrize("n,k", [(65535, 2064), (65536, 1040), (65537, 3072), (70001, 4096), (65536, 1024), (65600, 4112), (65537, 1664), (65539, 2560), (300, 2560),
                                  (4096, 4096), (4097, 4096), (33, 9728)])
 def test_weight_only_rows_keep_the_single_row_s_bits_at_the_edges_of_the_row_blocks(n, k):

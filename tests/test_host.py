@@ -377,6 +377,7 @@ def test_set_option_validates_names_and_values():
     for name, good, bad in ((b"gemm_tile", (64, 128, 192, 256, 320, 6464, 128192, 0), (1, 100, -1)),
                             (b"gemv_wholerow", (0, 1, -1), (2, -2)),
                             (b"w4_decode_waves", (4, 16, 0), (1, 8, -1)),
+                            (b"w4_gemm_deep", (1, 1664, 1665, 3232, 3233, 3264, 3265, 4864, 0), (2, 64, 4865, -1)),
                             (b"w4_decode_chain", (1, 40108, 40116, 80216, 160416, 0), (2, 8, 16, 40132, 40316, 20116, -1))):
         for v in bad:
             assert lib.cmi_set_option(name, v) == _native.E_ARG
