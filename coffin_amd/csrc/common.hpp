@@ -52,23 +52,24 @@ int quant_act_i8_padded(const void *x, int8_t *q, float *s, int M, int K, int ld
 int gemm_w8a8_rows_tiles(int N);
 
 // gemv_w4a8_decode.hip: W4A8 GEMV for 1..4 rows, K <= 10240, from bf16 activations (x) or
-// quantised ones (xq, xs); returns CMI_E_UNSUPPORTED (no error text) for other shapes.
+// quantised ones (xq, xs), groups of 64 and 256 for one row; returns CMI_E_UNSUPPORTED (no error text) for other shapes.
 int gemv_w4a8_decode(const uint8_t *w4, const float *ws, const void *x, const int8_t *xq, const float *xs,
-                     void *y, int32_t *group_acc, int8_t *xq_out, float *xs_out, int M, int N, int K,
+                     void *y, int32_t *group_acc, int8_t *xq_out, float *xs_out, int M, int N, int K, int gs,
                      void *stream);
 // gemv_w4a8_chain.hip: the same for 1..2 rows with the fp32 chain in registers; `variant` = lanes per
 // weight row (8, 16) + 100 * wavefronts sharing a row (1, 2, 4, 8) + 10000 * wavefronts per workgroup
-// (4, 8, 16); CMI_E_UNSUPPORTED (no error text) outside the variant's range.
+// (4, 8, 16); groups of 64 and 256: one row, 16 lanes; CMI_E_UNSUPPORTED (no error text) outside the variant's range.
 int gemv_w4a8_chain(const uint8_t *w4, const float *ws, const void *x, const int8_t *xq, const float *xs,
                     void *y, int32_t *group_acc, int8_t *xq_out, float *xs_out, int M, int N, int K,
-                    int variant, void *stream);
+                    int gs, int variant, void *stream);
 // gemv_w4a8_rows16.hip: W4A8 GEMV for up to 16 quantised rows (xq, xs) or up to 4 bf16 rows (x,
-// quantised in the kernel), K <= 10240, integer sums on the matrix pipe; CMI_E_UNSUPPORTED (no error text) outside that range.
+// quantised in the kernel), K <= 10240, integer sums on the matrix pipe; groups of 64 and 256 up to 16 quantised rows;
+// CMI_E_UNSUPPORTED (no error text) outside that range.
 int gemv_w4a8_rows16(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs, const void *x,
-                     void *y, int32_t *group_acc, int8_t *xq_out, float *xs_out, int M, int N, int K,
+                     void *y, int32_t *group_acc, int8_t *xq_out, float *xs_out, int M, int N, int K, int gs,
                      void *stream);
 // gemm_w4a8_tile.hip: W4A8 tile GEMM, arguments already checked by cmi_gemm_w4a8 / cmi_gemv_w4a8.  The cheapest tile for a
-// shape and its modelled time (us), of all tiles and of those of four groups a step (groups of 128); the tile a gemm_tile
+// shape and its modelled time (us), of all tiles and of those of four groups a step; the tile a gemm_tile
 // option names; whether a w4_gemm_deep option names one; the launch.
 double gemm_w4a8_tile_us(int M, int N, int K, int gs, int *tile);
 double gemm_w4a8_deep_us(int M, int N, int K, int *tile);

@@ -334,7 +334,7 @@ extern "C" int cmi_gemm_w4a8(const uint8_t *w4, const float *ws, const int8_t *x
                 const int rc = gemv_w4a8_rows16(w4, ws, xq + (size_t)lo * K, xs + lo, nullptr,
                                                 static_cast<uint16_t *>(y) + (size_t)lo * N,
                                                 group_acc ? group_acc + (size_t)lo * G * N : nullptr, nullptr,
-                                                nullptr, m, N, K, stream);
+                                                nullptr, m, N, K, gs, stream);
                 if (rc != CMI_OK) return rc == CMI_E_UNSUPPORTED ? fail(rc, "cmi_gemm_w4a8: internal dispatch") : rc;
             }
             return CMI_OK;

@@ -384,22 +384,26 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_tile_kernel(const A
 // tiles of wavefronts side by side do it once.  Sharing K among wavefronts that hand their sums over through LDS was built
 // first and took 32 us for that shape: operands straight into registers in the MFMA arrangement come at 16 bytes a clock.
 //
+// Groups of 64 and 256: a stage is eight or two groups; 64 close one after each MFMA (operand pieces as above), 256 after
+// every second 128.
+//
 // ONCE: a single tile of rows, so that every weight byte is read by one workgroup and need not stay in the caches.
 //
 // Cold weights, with the quantiser: 100 rows of 9728 -> 2560 29.2 -> 20.6 us, 40 rows 23.8 -> 16.7, 200 rows 34.6 ->
 // 27.1; 100 rows of 4096 -> 2560 14.3 -> 10.8; 40 rows of 25600 -> 5120 60.7 -> 39.6; 16 rows of 2560 -> 151936 54.3 -> 48.7,
 // of 4096 -> 12288 12.1 -> 9.2 (both against the matrix-pipe GEMV).
 constexpr int NT = 2;  // cache policy of a load: nontemporal
-constexpr int U = 4, X_ROW = U * BK, P_ROW = U * BK / 2;  // groups of a stage; bytes of a row in it: 512 and 256
+constexpr int U = 4, X_ROW = U * BK, P_ROW = U * BK / 2;  // 128s of a stage; bytes of a row in it: 512 and 256
 
-template <int WM, int WN, int TM, int TN, int NST>
+template <int WM, int WN, int TM, int TN, int NST, int LG>
 struct DeepCfg {
     static constexpr int WAVES = WM * WN, THREADS = 64 * WAVES;
     static constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
     static constexpr int X_BYTES = BM * X_ROW, P_BYTES = BN * P_ROW;
-    static constexpr int S_BYTES = BN * U * 4, STAGE = X_BYTES + P_BYTES + S_BYTES;
+    static constexpr int SU = (U * 4) >> LG;  // groups of a stage: 8, 4, 2
+    static constexpr int S_BYTES = BN * SU * 4, STAGE = X_BYTES + P_BYTES + S_BYTES;
     static constexpr int XL = X_BYTES / 1024 / WAVES, PL = P_BYTES / 1024 / WAVES;  // requests per wavefront and stage
-    static constexpr int SL = (BN * U / 64 + WAVES - 1) / WAVES;
+    static constexpr int SL = (BN * SU / 64 + WAVES - 1) / WAVES;
     static constexpr int LOADS = XL + PL + SL;
     static constexpr int YPITCH = 2 * BN + 16;
     static constexpr int LDS_BYTES = NST * STAGE;
@@ -407,9 +411,9 @@ struct DeepCfg {
     static_assert(BM * YPITCH <= LDS_BYTES, "result does not fit");
 };
 
-template <int WM, int WN, int TM, int TN, int NST, bool ONCE>
+template <int WM, int WN, int TM, int TN, int NST, int LG, bool ONCE>
 __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_deep_kernel(const Args a) {
-    using C = DeepCfg<WM, WN, TM, TN, NST>;
+    using C = DeepCfg<WM, WN, TM, TN, NST, LG>;
     extern __shared__ __align__(16) int8_t lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -426,13 +430,13 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_deep_kernel(const A
         const_cast<float *>(a.ws) + (size_t)n0 * a.G, 0, min(a.N - n0, C::BN) * a.G * 4, 0x00020000);
 
     // Requests of a stage: two rows x 512 B of activations, four rows x 256 B of packed weight each, 16-byte piece index
-    // XOR row % 16; then the scales, [column][U].
+    // XOR row % 16; then the scales, [column][SU].
     int xoff[C::XL], poff[C::PL];
 #pragma unroll
     for (int h = 0; h < C::XL; ++h) xoff[h] = (lane >> 5) * a.K + ((lane & 31) ^ ((2 * (C::XL * wave + h) + (lane >> 5)) & 15)) * 16;
 #pragma unroll
     for (int h = 0; h < C::PL; ++h) poff[h] = (lane >> 4) * (a.K / 2) + ((lane & 15) ^ ((4 * (C::PL * wave + h) + (lane >> 4)) & 15)) * 16;
-    const int soff = (lane / U) * a.G * 4 + (lane % U) * 4;
+    const int soff = (lane / C::SU) * a.G * 4 + (lane % C::SU) * 4;
     auto issue = [&](int slot, int stage) {
         int8_t *base = lds + slot * C::STAGE;
 #pragma unroll
@@ -448,21 +452,39 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_deep_kernel(const A
         }
 #pragma unroll
         for (int h = 0; h < C::SL; ++h) {
-            const int r = min(C::SL * wave + h, C::BN * U / 64 - 1);  // past the last: the last again, same bytes
+            const int r = min(C::SL * wave + h, C::BN * C::SU / 64 - 1);  // past the last: the last again, same bytes
             __builtin_amdgcn_raw_ptr_buffer_load_lds(sres, (lds_ptr_t)(base + C::X_BYTES + C::P_BYTES + r * 256), 4, soff,
-                                                     stage * U * 4 + r * (64 / U) * a.G * 4, 0, 0);
+                                                     stage * C::SU * 4 + r * (64 / C::SU) * a.G * 4, 0, 0);
         }
     };
-    // a lane's pieces: row fr of a tile, piece u * 4 + fc of the packed row and pieces u * 8 + 2 fc + e of the activations
+    // a lane's pieces: row fr of a tile, piece u * 4 + fc of the packed row and pieces u * 8 + 2 fc + e of the activations;
+    // with groups of 64, half fc % 2 of piece u * 4 + 2 e + fc / 2 and piece u * 8 + 4 e + fc (as above)
     const int fr = lane & 15, fc = lane >> 4;
-    int xf[2][2], pf[U];
+    int xf[2][2], pf[U][LG == 1 ? 2 : 1];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int e = 0; e < 2; ++e) xf[h][e] = (wm * 16 * TM + fr) * X_ROW + ((8 * h + 2 * fc + e) ^ fr) * 16;  // u = h, h + 2: 256 B on
+        for (int e = 0; e < 2; ++e) xf[h][e] = (wm * 16 * TM + fr) * X_ROW + ((8 * h + (LG == 1 ? 4 * e + fc : 2 * fc + e)) ^ fr) * 16;  // u = h, h + 2: 256 B on
 #pragma unroll
-    for (int u = 0; u < U; ++u) pf[u] = C::X_BYTES + (wn * 16 * TN + fr) * P_ROW + ((4 * u + fc) ^ fr) * 16;
-    const int sf = C::X_BYTES + C::P_BYTES + (wn * 16 * TN + fr) * (U * 4);
+    for (int u = 0; u < U; ++u) {
+        const int row = C::X_BYTES + (wn * 16 * TN + fr) * P_ROW;
+        if constexpr (LG != 1) {
+            pf[u][0] = row + ((4 * u + fc) ^ fr) * 16;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) pf[u][e] = row + ((4 * u + 2 * e + (fc >> 1)) ^ fr) * 16 + (fc & 1) * 8;
+        }
+    }
+    const int sf = C::X_BYTES + C::P_BYTES + (wn * 16 * TN + fr) * (C::SU * 4);
+    auto read_p = [&](const int8_t *base, int u, int j) {
+        const int8_t *row = base + j * 16 * P_ROW;
+        if constexpr (LG != 1) {
+            return *reinterpret_cast<const v4i32 *>(row + pf[u][0]);
+        } else {
+            const v2i32 p0 = *reinterpret_cast<const v2i32 *>(row + pf[u][0]), p1 = *reinterpret_cast<const v2i32 *>(row + pf[u][1]);
+            return v4i32{p0.x, p0.y, p1.x, p1.y};
+        }
+    };
     auto nibbles = [](int word, int high) {
         return (int)(((high ? (uint32_t)word : (uint32_t)word << 4) & 0xF0F0F0F0u) ^ 0x80808080u);
     };
@@ -479,6 +501,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_deep_kernel(const A
 
 #pragma unroll
     for (int s = 0; s < NST - 1; ++s) issue(s, s);
+    const int ksteps = a.K / BK;
     int slot = 0;
     auto stage = [&](auto whole_tag, int s) {
         constexpr bool WHOLE = decltype(whole_tag)::value;
@@ -489,14 +512,15 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_deep_kernel(const A
         // the slot that the stage before was read from
         issue(slot == 0 ? NST - 1 : slot - 1, s + NST - 1);
         const int8_t *base = lds + slot * C::STAGE;
-        f32x4 sc[TN];
+        typedef float scales_t __attribute__((ext_vector_type(C::SU)));
+        scales_t sc[TN];
         v4i32 x[U][TM][2], p[U][TN];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) sc[j] = *reinterpret_cast<const f32x4 *>(base + sf + j * 16 * U * 4);
+        for (int j = 0; j < TN; ++j) sc[j] = *reinterpret_cast<const scales_t *>(base + sf + j * 16 * C::SU * 4);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
 #pragma unroll
-            for (int j = 0; j < TN; ++j) p[u][j] = *reinterpret_cast<const v4i32 *>(base + pf[u] + j * 16 * P_ROW);
+            for (int j = 0; j < TN; ++j) p[u][j] = read_p(base, u, j);
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -504,43 +528,52 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_deep_kernel(const A
                     x[u][i][e] = *reinterpret_cast<const v4i32 *>(base + xf[u & 1][e] + (u >> 1) * 256 + i * 16 * X_ROW);
             __builtin_amdgcn_sched_barrier(0);
         }
+        v4i32 acc[TN][TM];  // (groups of 256: kept over two u)
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (!WHOLE && s * U + u >= a.G) break;  // uniform
+            if (!WHOLE && s * U + u >= ksteps) break;  // uniform
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 v4i32 w[2];
 #pragma unroll
                 for (int h = 0; h < 8; ++h) w[h / 4][h % 4] = nibbles(p[u][j][h / 2], h & 1);
-                least = min(least, 2 * __float_as_uint(sc[j][u]) - 1);
-                const float scale = sc[j][u] * 0.0625f;
+                const auto flush = [&](int g) {
+                    least = min(least, 2 * __float_as_uint(sc[j][g]) - 1);
+                    const float scale = sc[j][g] * 0.0625f;
 #pragma unroll
-                for (int i = 0; i < TM; ++i) {
-                    v4i32 acc = {0, 0, 0, 0};
-                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[u][i][0], w[0], acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[u][i][1], w[1], acc, 0, 0, 0);
+                    for (int i = 0; i < TM; ++i)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) total[i][j][r] = fmaf((float)acc[r], scale, total[i][j][r]);
+                        for (int r = 0; r < 4; ++r) total[i][j][r] = fmaf((float)acc[j][i][r], scale, total[i][j][r]);
+                };
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const bool opens = LG == 1 || (e == 0 && (LG == 2 || u % 2 == 0)), closes = LG == 1 || (e == 1 && (LG == 2 || u % 2 == 1));
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) {
+                        const v4i32 from = opens ? v4i32{0, 0, 0, 0} : acc[j][i];
+                        acc[j][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[u][i][e], w[e], from, 0, 0, 0);
+                    }
+                    if (closes) flush(LG == 1 ? 2 * u + e : LG == 2 ? u : u / 2);
                 }
             }
         }
         slot = slot + 1 == NST ? 0 : slot + 1;
     };
-    const int whole = a.G / U;
+    const int whole = ksteps / U;
     for (int s = 0; s < whole; ++s) stage(std::true_type{}, s);
-    if (whole * U < a.G) stage(std::false_type{}, whole);
+    if (whole * U < ksteps) stage(std::false_type{}, whole);
     const uint64_t inexact = __builtin_amdgcn_ballot_w64(least < TINY);
     wait_vmcnt<0>();
     __syncthreads();
     uint16_t *park = reinterpret_cast<uint16_t *>(lds);
-    park_results<TM, TN, C::YPITCH, 2>(a, total, inexact, park, m0, n0, wm * 16 * TM, wn * 16 * TN, lane);
+    park_results<TM, TN, C::YPITCH, LG>(a, total, inexact, park, m0, n0, wm * 16 * TM, wn * 16 * TN, lane);
     __syncthreads();
     store_parked<C::BM, C::BN, C::YPITCH, C::THREADS>(a, park, m0, n0);
 }
 
-template <int WM, int WN, int TM, int TN, int NST>
+template <int WM, int WN, int TM, int TN, int NST, int LG>
 int launch_deep(Args &a, hipStream_t st) {
-    using C = DeepCfg<WM, WN, TM, TN, NST>;
+    using C = DeepCfg<WM, WN, TM, TN, NST, LG>;
     a.tiles_m = (a.M + C::BM - 1) / C::BM;
     a.tiles_n = (a.N + C::BN - 1) / C::BN;
     // the tile's operand offsets are 32-bit
@@ -552,8 +585,8 @@ int launch_deep(Args &a, hipStream_t st) {
         kernel<<<dim3(a.tiles_m * a.tiles_n), dim3(C::THREADS), C::LDS_BYTES, st>>>(a);
         return check_launch("cmi_gemm_w4a8");
     };
-    return a.tiles_m == 1 ? run(gemm_w4a8_deep_kernel<WM, WN, TM, TN, NST, true>, devices[1])
-                          : run(gemm_w4a8_deep_kernel<WM, WN, TM, TN, NST, false>, devices[0]);
+    return a.tiles_m == 1 ? run(gemm_w4a8_deep_kernel<WM, WN, TM, TN, NST, LG, true>, devices[1])
+                          : run(gemm_w4a8_deep_kernel<WM, WN, TM, TN, NST, LG, false>, devices[0]);
 }
 
 template <int WM, int WN, int TM, int TN, int NST, int LG>
@@ -585,13 +618,6 @@ int launch_tile(Args &a, Tile tile, hipStream_t st) {
             case T128x128: return launch<2, 2, 4, 4, 3, 2>(a, st);
             case T64x96: return launch<2, 2, 2, 3, 3, 2>(a, st);
             case T32x128: return launch<1, 4, 2, 2, 4, 2>(a, st);
-            case D16x64: return launch_deep<1, 4, 1, 1, 2>(a, st);
-            case D16x64L: return launch_deep<1, 4, 1, 1, 4>(a, st);
-            case D32x32: return launch_deep<2, 2, 1, 1, 2>(a, st);
-            case D32x32L: return launch_deep<2, 2, 1, 1, 4>(a, st);
-            case D32x64: return launch_deep<1, 4, 2, 1, 2>(a, st);
-            case D32x64L: return launch_deep<2, 4, 1, 1, 3>(a, st);
-            case D48x64: return launch_deep<1, 4, 3, 1, 2>(a, st);
             default: break;
         }
     }
@@ -600,6 +626,13 @@ int launch_tile(Args &a, Tile tile, hipStream_t st) {
         case T64x64: return launch<2, 2, 2, 2, 4, LG>(a, st);
         case T32x64: return launch<2, 2, 1, 2, 4, LG>(a, st);
         case T16x32: return launch<1, 2, 1, 1, 4, LG>(a, st);
+        case D16x64: return launch_deep<1, 4, 1, 1, 2, LG>(a, st);
+        case D16x64L: return launch_deep<1, 4, 1, 1, 4, LG>(a, st);
+        case D32x32: return launch_deep<2, 2, 1, 1, 2, LG>(a, st);
+        case D32x32L: return launch_deep<2, 2, 1, 1, 4, LG>(a, st);
+        case D32x64: return launch_deep<1, 4, 2, 1, 2, LG>(a, st);
+        case D32x64L: return launch_deep<2, 4, 1, 1, 3, LG>(a, st);
+        case D48x64: return launch_deep<1, 4, 3, 1, 2, LG>(a, st);
         default: return CMI_E_UNSUPPORTED;
     }
 }
@@ -682,10 +715,14 @@ double gemm_w4a8_tile_us(int M, int N, int K, int gs, int *tile) {
         if (us < best) best = us, *tile = t;
     }
     // Four groups a step where they are modelled to gain at least 3 %: 315 sizes of 17..1024 rows 6678 -> 5997 us in all (5908
-    // with the best of every size; the worst loss 9 %, 40 rows of 8960 -> 1536 6.0 -> 6.6 us).
+    // with the best of every size; the worst loss 9 %, 40 rows of 8960 -> 1536 6.0 -> 6.6 us).  The same with groups of 256 (twelve
+    // shapes x fourteen batch sizes; 24 rows of 14336 -> 4096 28.0 -> 16.5 us, 100 rows of 9728 -> 2560 21.6 -> 15.0).  Groups of 64
+    // flush twice as often, which costs these tiles 1.35 times their model and the others 1.17: up to 16 rows, where they
+    // are modelled to gain more than that (1106 us in all, 1095 with the best of every size, 1230 without them; 16 rows of
+    // 5120 -> 32768 28.3 -> 21.1); beyond, the gain is 2 % in all and the model does not find it.
     int deep = 0;
-    const double us = gs == BK ? gemm_w4a8_deep_us(M, N, K, &deep) : 1e30;
-    if (us < 0.97 * best) best = us, *tile = deep;
+    const double us = gs == 64 && M > 16 && option_w4_gemm_deep() == 0 ? 1e30 : gemm_w4a8_deep_us(M, N, K, &deep);
+    if (us < (gs == 64 ? 0.82 : 0.97) * best) best = us, *tile = deep;
     return best;
 }
 

@@ -368,6 +368,22 @@ int run_gemv_w4a8(const char *who, const uint8_t *w4, const float *ws, const int
 
 }  // namespace
 
+namespace {
+
+// Time in us of the matrix-pipe GEMV for up to 16 rows of groups of 64 and 256, fitted to cold-weight sweeps of 14 layer
+// shapes x 1..16 rows (within 10 % of four in five).  Groups of 64: a workgroup's LDS (K / 64 KiB of sums) is what bounds how
+// many a CU holds.
+double rows16_us(int M, int N, int K, int gs) {
+    const double mb = N * 0.5e-6 * K, k = K * 1e-3, share = M / 16.0, wgs = (N + 15) / 16;
+    if (gs == 256) return K > 10240 ? mb * (0.395 + 0.033 * share) : 2.81 + 0.28 * k + mb * (0.185 + 0.056 * share);
+    if (K > 8192) return 2.1 + 4.06 * ceil(wgs / 256) * ceil(K / 6144.0) + mb * 0.03 * share;
+    const int lines = (K / 128 + 1) / 2, waves = lines > 20 || (wgs <= 640 && lines >= 8) ? 8 : 4;
+    const int by_lds = 163840 / (K / 64 * 1088 + waves * 2304), per_cu = by_lds < 32 / waves ? by_lds : 32 / waves;
+    return 2.69 + fmax(1.0, wgs / (256.0 * per_cu)) * (0.344 + 0.628 * k) + mb * (0.174 + 0.0735 * share);
+}
+
+}  // namespace
+
 extern "C" int cmi_gemv_w4a8(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs,
                              void *y, int32_t *group_acc, int M, int N, int K, int gs,
                              void *stream) {
@@ -399,12 +415,28 @@ extern "C" int cmi_gemv_w4a8(const uint8_t *w4, const float *ws, const int8_t *x
         }
         if ((M == 1 && (whole_rows || shared_rows || (chain_on && K <= 20480))) ||
             (M == 2 && whole_rows && N >= 12288) || forced)
-            rc = gemv_w4a8_decode(w4, ws, nullptr, xq, xs, y, group_acc, nullptr, nullptr, M, N, K, stream);
+            rc = gemv_w4a8_decode(w4, ws, nullptr, xq, xs, y, group_acc, nullptr, nullptr, M, N, K, gs, stream);
         if (rc == CMI_E_UNSUPPORTED)
-            rc = gemv_w4a8_rows16(w4, ws, xq, xs, nullptr, y, group_acc, nullptr, nullptr, M, N, K, stream);
+            rc = gemv_w4a8_rows16(w4, ws, xq, xs, nullptr, y, group_acc, nullptr, nullptr, M, N, K, gs, stream);
         if (rc == CMI_E_UNSUPPORTED && M <= 2)
-            rc = gemv_w4a8_decode(w4, ws, nullptr, xq, xs, y, group_acc, nullptr, nullptr, M, N, K, stream);
+            rc = gemv_w4a8_decode(w4, ws, nullptr, xq, xs, y, group_acc, nullptr, nullptr, M, N, K, gs, stream);
         if (rc != CMI_E_UNSUPPORTED) return rc;
+    }
+    // Groups of 64 and 256.  One row: the dot-product kernel with the chain in registers.  Up to 16: the matrix-pipe GEMV or the tile
+    // GEMM, whichever is modelled to be faster (groups of 64: 0.9 for the tiles' model, which is fitted to groups of 128; of
+    // 180 sizes the choice is 7 and 1 % above the best).  The general kernel below keeps calls that ask for
+    // the group sums of several rows and rows that are not whole steps of 128; cold weights, the projection with its quantiser: one
+    // row of 2560 -> 19456 17.2 -> 8.4 us (64), 12.9 -> 7.4 (256); 4 rows 27.2 -> 14.3, 23.3 -> 11.4; 16 rows 62.9 -> 14.7, 62.1 ->
+    // 13.3; 16 rows of 2560 -> 151936 451 -> 60, 432 -> 51; of 9728 -> 2560 37.6 -> 14.7, 31.9 -> 12.2.
+    if ((gs == 64 || gs == 256) && K >= gs && K % GS == 0 && K % gs == 0 && N >= 1 && M >= 1 && M <= 16) {
+        int rc = CMI_E_UNSUPPORTED, tile = 0;
+        if (M == 1) rc = gemv_w4a8_decode(w4, ws, nullptr, xq, xs, y, group_acc, nullptr, nullptr, M, N, K, gs, stream);
+        if (rc != CMI_E_UNSUPPORTED) return rc;
+        if (!group_acc) {
+            if (rows16_us(M, N, K, gs) * (gs == 64 ? 0.9 : 1.0) <= gemm_w4a8_tile_us(M, N, K, gs, &tile))
+                return gemv_w4a8_rows16(w4, ws, xq, xs, nullptr, y, nullptr, nullptr, nullptr, M, N, K, gs, stream);
+            return gemm_w4a8_tile(w4, ws, xq, xs, y, M, N, K, gs, tile, stream);
+        }
     }
     return run_gemv_w4a8("cmi_gemv_w4a8", w4, ws, xq, xs, nullptr, nullptr, nullptr, y, group_acc, M, N, K, gs,
                          stream);
@@ -433,12 +465,12 @@ extern "C" int cmi_gemv_w4a8_bf16(const uint8_t *w4, const float *ws, const void
     const bool one_shared_row = M == 1 && (N + 15) / 16 < 256;
     const int whole_row_k = option_w4_decode_chain() == 1 ? 4096 : 5120;
     if (K > whole_row_k && !one_shared_row && !(option_w4_decode_chain() > 1))
-        rc = gemv_w4a8_rows16(w4, ws, nullptr, nullptr, x, y, group_acc, xq_out, xs_out, M, N, K, stream);
+        rc = gemv_w4a8_rows16(w4, ws, nullptr, nullptr, x, y, group_acc, xq_out, xs_out, M, N, K, gs, stream);
     if (rc != CMI_E_UNSUPPORTED) return rc;
-    rc = gemv_w4a8_decode(w4, ws, x, nullptr, nullptr, y, group_acc, xq_out, xs_out, M, N, K, stream);
+    rc = gemv_w4a8_decode(w4, ws, x, nullptr, nullptr, y, group_acc, xq_out, xs_out, M, N, K, gs, stream);
     if (rc != CMI_E_UNSUPPORTED) return rc;
     if (K > 4096 && one_shared_row)  // beyond the decode kernel's K
-        rc = gemv_w4a8_rows16(w4, ws, nullptr, nullptr, x, y, group_acc, xq_out, xs_out, M, N, K, stream);
+        rc = gemv_w4a8_rows16(w4, ws, nullptr, nullptr, x, y, group_acc, xq_out, xs_out, M, N, K, gs, stream);
     if (rc != CMI_E_UNSUPPORTED) return rc;
     return run_gemv_w4a8("cmi_gemv_w4a8_bf16", w4, ws, nullptr, nullptr, x, xq_out, xs_out, y, group_acc, M, N, K,
                          gs, stream);

@@ -24,6 +24,10 @@
 //   in order: no parking of partial sums in LDS, no serial walk at the end, no second barrier.
 //   Groups past K meet a scale of 0.f: fma(finite, 0, total) is total (the chain starts at +0
 //   and cannot reach -0).
+// * Groups of 64 and 256 (one row): a group is two or eight lanes, so one or three DPP steps form its sum and a load
+//   instruction covers LPR/2 or LPR/8 groups.  Against the kernel that kept a row's sums in LDS and walked them serially,
+//   cold weights, quantised here instead of in a launch before: 2560 -> 19456 17.2 -> 8.4 us (64), 12.9 -> 7.4 (256); 2560 -> 151936 97 -> 39,
+//   67 -> 35; 9728 -> 2560 21.3 -> 9.8, 11.4 -> 7.4; 4096 -> 2560 8.8 -> 4.6, 6.8 -> 3.7.
 // * Longer rows are shared by S wavefronts of a workgroup, each a contiguous run of loads: every
 //   wavefront forms and converts its integer sums as its bytes arrive, then the chain passes
 //   through the S wavefronts in k order, its running value handed over in LDS (S - 1 barriers).
@@ -73,12 +77,13 @@ struct Lds {
 // each covering LPR * 32 elements of every row.  PREQ: activations arrive quantised.
 // EXACT: K == S * NL * LPR * 32 and the integer sums are not asked for -- no clamped addresses, no
 // scale selects, no early exit from the loads.  S: wavefronts that share the same rows, each taking
-// NL consecutive loads.  WAVES: wavefronts per workgroup (WAVES / S teams).
-template <int M, int LPR, int NL, bool PREQ, bool EXACT, int S, int WAVES>
+// NL consecutive loads.  WAVES: wavefronts per workgroup (WAVES / S teams).  LG: log2(group size / 32).
+template <int M, int LPR, int NL, bool PREQ, bool EXACT, int S, int WAVES, int LG>
 __global__ void __launch_bounds__(64 * WAVES)
 gemv_w4a8_chain_kernel(const Args a) {
+    static_assert(LG >= 1 && LG <= 3 && LPR >= 1 << LG, "groups of 64, 128, 256");
     constexpr int THREADS = 64 * WAVES;
-    constexpr int RPW = 64 / LPR, Q = LPR / 4, CP = S * NL * LPR;
+    constexpr int RPW = 64 / LPR, LPG = 1 << LG, Q = LPR / LPG, CP = S * NL * LPR;
     using L = Lds<M, CP, WAVES>;
     extern __shared__ __align__(16) uint8_t lds[];
     uint4 *planes = reinterpret_cast<uint4 *>(lds + L::planes);
@@ -215,9 +220,18 @@ gemv_w4a8_chain_kernel(const Args a) {
     for (int m = 0; m < M; ++m) total[m] = 0.f;
     auto extend = [&](int m, int j, float f) {
         total[m] = fmaf(f, wsr[j][0], total[m]);
-        if constexpr (Q >= 2) total[m] = fmaf(dpp_f32<0x104, 0xf>(f), wsr[j][1], total[m]);  // row_shl:4
-        if constexpr (Q >= 3) total[m] = fmaf(dpp_f32<0x108, 0xf>(f), wsr[j][2], total[m]);  // row_shl:8
-        if constexpr (Q >= 4) total[m] = fmaf(dpp_f32<0x10C, 0xf>(f), wsr[j][3], total[m]);  // row_shl:12
+        // the sums of the row's other groups, LPG lanes on each (row_shl)
+        if constexpr (Q >= 2) total[m] = fmaf(dpp_f32<0x100 + LPG % 16, 0xf>(f), wsr[j][1 % Q], total[m]);
+        if constexpr (Q >= 4) {
+            total[m] = fmaf(dpp_f32<0x100 + 2 * LPG % 16, 0xf>(f), wsr[j][2 % Q], total[m]);
+            total[m] = fmaf(dpp_f32<0x100 + 3 * LPG % 16, 0xf>(f), wsr[j][3 % Q], total[m]);
+        }
+        if constexpr (Q >= 8) {
+            total[m] = fmaf(dpp_f32<0x108, 0xf>(f), wsr[j][4 % Q], total[m]);
+            total[m] = fmaf(dpp_f32<0x10A, 0xf>(f), wsr[j][5 % Q], total[m]);
+            total[m] = fmaf(dpp_f32<0x10C, 0xf>(f), wsr[j][6 % Q], total[m]);
+            total[m] = fmaf(dpp_f32<0x10E, 0xf>(f), wsr[j][7 % Q], total[m]);
+        }
     };
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
@@ -244,11 +258,12 @@ gemv_w4a8_chain_kernel(const Args a) {
             }
             int s = (int)(((hi - c8) << 4) + lo);
             s += dpp_i32<0xB1, 0xf>(s);
-            s += dpp_i32<0x4E, 0xf>(s);
+            if constexpr (LG >= 2) s += dpp_i32<0x4E, 0xf>(s);
+            if constexpr (LG >= 3) s += dpp_i32<0x141, 0xf>(s);  // row_half_mirror: the other quad of eight lanes
             if constexpr (!EXACT) {
                 if (a.group_acc) {  // uniform
-                    const int g = (j0 + j) * Q + (c >> 2);
-                    if ((c & 3) == 0 && g < a.G && n_raw < a.N && m < a.M)
+                    const int g = (j0 + j) * Q + (c >> LG);
+                    if ((c & (LPG - 1)) == 0 && g < a.G && n_raw < a.N && m < a.M)
                         a.group_acc[((size_t)m * a.G + g) * a.N + n] = s;
                 }
             }
@@ -287,30 +302,30 @@ gemv_w4a8_chain_kernel(const Args a) {
     }
 }
 
-template <int M, int LPR, int NL, bool PREQ, int S, int WAVES>
+template <int M, int LPR, int NL, bool PREQ, int S, int WAVES, int LG = 2>
 int launch(const Args &a, hipStream_t st) {
     constexpr int RPB = (WAVES / S) * (64 / LPR);
     constexpr int LDS_BYTES = Lds<M, S * NL * LPR, WAVES>::total;
     const dim3 grid((a.N + RPB - 1) / RPB), block(64 * WAVES);
     if (a.K == S * NL * LPR * 32 && !a.group_acc)
-        gemv_w4a8_chain_kernel<M, LPR, NL, PREQ, true, S, WAVES><<<grid, block, LDS_BYTES, st>>>(a);
+        gemv_w4a8_chain_kernel<M, LPR, NL, PREQ, true, S, WAVES, LG><<<grid, block, LDS_BYTES, st>>>(a);
     else
-        gemv_w4a8_chain_kernel<M, LPR, NL, PREQ, false, S, WAVES><<<grid, block, LDS_BYTES, st>>>(a);
+        gemv_w4a8_chain_kernel<M, LPR, NL, PREQ, false, S, WAVES, LG><<<grid, block, LDS_BYTES, st>>>(a);
     return check_launch("cmi_gemv_w4a8");
 }
 
 // Loads per wavefront: the instantiations cover up to 20 (80 registers of weights).
-template <int M, int LPR, bool PREQ, int S, int WAVES>
+template <int M, int LPR, bool PREQ, int S, int WAVES, int LG = 2>
 int dispatch_nl(const Args &a, hipStream_t st) {
     const int loads = ((a.K + LPR * 32 - 1) / (LPR * 32) + S - 1) / S;
-    if (loads <= 2) return launch<M, LPR, 2, PREQ, S, WAVES>(a, st);
-    if (loads <= 4) return launch<M, LPR, 4, PREQ, S, WAVES>(a, st);
-    if (loads <= 5) return launch<M, LPR, 5, PREQ, S, WAVES>(a, st);
-    if (loads <= 8) return launch<M, LPR, 8, PREQ, S, WAVES>(a, st);
-    if (loads <= 10) return launch<M, LPR, 10, PREQ, S, WAVES>(a, st);
+    if (loads <= 2) return launch<M, LPR, 2, PREQ, S, WAVES, LG>(a, st);
+    if (loads <= 4) return launch<M, LPR, 4, PREQ, S, WAVES, LG>(a, st);
+    if (loads <= 5) return launch<M, LPR, 5, PREQ, S, WAVES, LG>(a, st);
+    if (loads <= 8) return launch<M, LPR, 8, PREQ, S, WAVES, LG>(a, st);
+    if (loads <= 10) return launch<M, LPR, 10, PREQ, S, WAVES, LG>(a, st);
     if constexpr (LPR == 8 && S == 1) {
-        if (loads <= 16) return launch<M, LPR, 16, PREQ, S, WAVES>(a, st);
-        if (loads <= 20) return launch<M, LPR, 20, PREQ, S, WAVES>(a, st);
+        if (loads <= 16) return launch<M, LPR, 16, PREQ, S, WAVES, LG>(a, st);
+        if (loads <= 20) return launch<M, LPR, 20, PREQ, S, WAVES, LG>(a, st);
     }
 
     return CMI_E_UNSUPPORTED;
@@ -335,6 +350,19 @@ int dispatch(const Args &a, int lanes, int split, int waves, hipStream_t st) {
     return CMI_E_UNSUPPORTED;
 }
 
+// Groups of 64 and 256: one row, the variants that `chain_variant` names for it.
+template <bool PREQ, int LG>
+int dispatch_other_group(const Args &a, int lanes, int split, int waves, hipStream_t st) {
+    if (lanes != 16) return CMI_E_UNSUPPORTED;
+    if (split == 1 && waves == 4) return dispatch_nl<1, 16, PREQ, 1, 4, LG>(a, st);
+    if constexpr (PREQ) {
+        if (split == 4 && waves == 4) return dispatch_nl<1, 16, PREQ, 4, 4, LG>(a, st);
+    } else {
+        if (split == 2 && waves == 8) return dispatch_nl<1, 16, PREQ, 2, 8, LG>(a, st);
+    }
+    return CMI_E_UNSUPPORTED;
+}
+
 }  // namespace
 
 namespace cmi {
@@ -344,9 +372,9 @@ namespace cmi {
 // CMI_E_UNSUPPORTED (no error text) when the shape is outside the variant's range.
 int gemv_w4a8_chain(const uint8_t *w4, const float *ws, const void *x, const int8_t *xq, const float *xs,
                     void *y, int32_t *group_acc, int8_t *xq_out, float *xs_out, int M, int N, int K,
-                    int variant, void *stream) {
+                    int gs, int variant, void *stream) {
     const int lanes = variant % 100, split = variant / 100 % 100, waves = variant / 10000;
-    if (M < 1 || M > 2 || K < GS || K % GS != 0 || N < 1) return CMI_E_UNSUPPORTED;
+    if (M < 1 || M > 2 || K < gs || K % GS != 0 || K % gs != 0 || N < 1 || (gs != GS && M != 1)) return CMI_E_UNSUPPORTED;
     Args a;
     a.w4 = w4;
     a.ws = ws;
@@ -360,8 +388,10 @@ int gemv_w4a8_chain(const uint8_t *w4, const float *ws, const void *x, const int
     a.M = M;
     a.N = N;
     a.K = K;
-    a.G = K / GS;
+    a.G = K / gs;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (gs == 64) return x ? dispatch_other_group<false, 1>(a, lanes, split, waves, st) : dispatch_other_group<true, 1>(a, lanes, split, waves, st);
+    if (gs == 256) return x ? dispatch_other_group<false, 3>(a, lanes, split, waves, st) : dispatch_other_group<true, 3>(a, lanes, split, waves, st);
     if (x) return M <= 1 ? dispatch<1, false>(a, lanes, split, waves, st) : dispatch<2, false>(a, lanes, split, waves, st);
     return M <= 1 ? dispatch<1, true>(a, lanes, split, waves, st) : dispatch<2, true>(a, lanes, split, waves, st);
 }

@@ -26,6 +26,13 @@
 // -8s (the matrix pipe is idle here).  Each wavefront parks its int32 group sums
 // in LDS and, after one barrier, thread (n, m) walks the groups in ascending
 // order.
+//
+// Groups of 64 and 256 (up to 16 quantised rows).  256: the two halves of a line go into one sum.  64: an MFMA has to stay
+// inside a group, so lane l takes half l/16 % 2 of piece 2e + l/32 of the packed half line for group e of its two: eight
+// bytes, whose nibbles are 16 consecutive k, against 16 consecutive activation bytes.  The dot-product kernel that took
+// these rows forms 16 rows' products in the vector ALU: 16 rows of 9728 -> 2560 32.7 -> 10.9 us (64), 26.8 -> 8.5 (256), of 14336 ->
+// 4096 69.4 -> 15.5, 54.0 -> 12.4; 4 rows of 2560 -> 6144 9.4 -> 5.8, 7.9 -> 5.1.  The sums of 64s take twice the LDS, so K = 5120 leaves
+// room for one workgroup per CU (5120 -> 32768 51 us): the tile GEMM takes such sizes.
 #include "quant_math.hpp"
 #include "rows16_tile.hpp"
 
@@ -36,7 +43,7 @@ using namespace cmi::rows16;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int GS = 128;
+constexpr int GS = 128;        // k of half a line, the group of LG = 2
 constexpr int ROWS = 16;        // weight rows per workgroup = activation rows per MFMA
 constexpr int MAX_K = 10240;    // 40 lines: 8 wavefronts x 5
 
@@ -53,7 +60,9 @@ struct Args {
     float *xs_out;
     uint16_t *y;
     int32_t *group_acc;
-    int M, N, K, G;
+    int M, N, K;
+    int G;   // groups
+    int H;   // K / 128
 };
 
 // group sums [G][64 lanes][4], scales [16][G], one rearrangement patch per wavefront; FUSED adds
@@ -62,13 +71,49 @@ __host__ __device__ inline int lds_bytes(int G, int waves, bool fused = false) {
     return G * 1024 + ROWS * G * 4 + waves * PATCH_BYTES + (fused ? FUSED_ROWS * G * GS + 256 : 0);
 }
 
+// Groups of a row that fit the LDS beside the patches (64: K <= 8192).
+constexpr int max_groups(int lg) { return lg == 1 ? 128 : MAX_K >> (5 + lg); }
+
+// Integer sums of half line `half` (the h-th of its line, parked in `patch`): its group's, its two groups' (LG 1) or half its
+// group's (LG 3, completed by h = 1 in acc) into sums[group][lane]; lane holds (n = lane%16, m = 4*kq + v), v = 0..3.
+template <int LG>
+__device__ __forceinline__ void half_sums(const uint8_t *patch, int lane, int h, const v4i32 (&x)[2], v4i32 &acc, v4i32 *sums,
+                                          int half) {
+    const v4i32 minus8 = {(int)0xF8F8F8F8u, (int)0xF8F8F8F8u, (int)0xF8F8F8F8u, (int)0xF8F8F8F8u};
+    const int kq = lane >> 4;
+    if constexpr (LG == 1) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const uint2 ww = *reinterpret_cast<const uint2 *>(patch + (lane & 15) * TILE_PITCH + (4 * h + 2 * e + (kq >> 1)) * 16 + (kq & 1) * 8);
+            const u32x4 codes = {ww.x & 0x0F0F0F0Fu, (ww.x >> 4) & 0x0F0F0F0Fu, ww.y & 0x0F0F0F0Fu, (ww.y >> 4) & 0x0F0F0F0Fu};
+            v4i32 sum = {0, 0, 0, 0};
+            sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[e], minus8, sum, 0, 0, 0);
+            sums[(2 * half + e) * 64 + lane] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[e], __builtin_bit_cast(v4i32, codes), sum, 0, 0, 0);
+        }
+    } else {
+        const u32x4 ww = __builtin_bit_cast(u32x4, tile_take(patch, lane, 4 * h + kq));
+        const v4i32 x0 = {x[0].x, x[0].z, x[1].x, x[1].z};
+        const v4i32 x1 = {x[0].y, x[0].w, x[1].y, x[1].w};
+        const u32x4 lo = ww & 0x0F0F0F0Fu, hi = (ww >> 4) & 0x0F0F0F0Fu;
+        if (LG == 2 || h == 0) acc = v4i32{0, 0, 0, 0};
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x0, minus8, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x1, minus8, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x0, __builtin_bit_cast(v4i32, lo), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x1, __builtin_bit_cast(v4i32, hi), acc, 0, 0, 0);
+        if (LG == 2) sums[half * 64 + lane] = acc;
+        else if (h == 1) sums[(half >> 1) * 64 + lane] = acc;
+    }
+}
+
 // NLP: lines per wavefront.  WAVES: wavefronts per workgroup (4 or 8).
 // DUMP: also write the int32 group sums to a.group_acc.
+// LG: log2(group size / 32).
 // FUSED: activations arrive as bf16 (up to 4 rows) and every workgroup quantises them itself
 //        with the arithmetic of cmi_quant_act_i8 while its weights travel.
-template <int NLP, int WAVES, bool DUMP, bool FUSED>
+template <int NLP, int WAVES, bool DUMP, bool FUSED, int LG = 2>
 __global__ void __launch_bounds__(WAVES * 64)
 gemv_w4a8_rows16_kernel(const Args a) {
+    static_assert(LG == 2 || (!DUMP && !FUSED), "groups of 64 and 256: quantised rows, no group sums out");
     extern __shared__ __align__(16) uint8_t lds[];
     int32_t *sums = reinterpret_cast<int32_t *>(lds);             // [G][64 lanes][4]
     float *ws_lds = reinterpret_cast<float *>(lds + a.G * 1024);  // [16][G]
@@ -82,7 +127,7 @@ gemv_w4a8_rows16_kernel(const Args a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kq = lane >> 4;
     const int n0 = blockIdx.x * ROWS;
-    const int lines = (a.G + 1) / 2;
+    const int lines = (a.H + 1) / 2;
     uint8_t *patch = patches + wave * PATCH_BYTES;
 
     // 1. activations of this wavefront's groups (L2 resident; asked for first because
@@ -108,7 +153,7 @@ gemv_w4a8_rows16_kernel(const Args a) {
             if (line >= lines) break;  // uniform per wavefront
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int g = min(2 * line + h, a.G - 1);
+                const int g = min(2 * line + h, a.H - 1);
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
                     xa[i][h][j] =
@@ -122,7 +167,7 @@ gemv_w4a8_rows16_kernel(const Args a) {
     if constexpr (!FUSED) xs_out = a.xs[min((int)(4 * ((threadIdx.x >> 6) & 3) + (threadIdx.x & 3)), a.M - 1)];
     // 2. the scales of the 16 rows (contiguous), into registers until the weights are asked for
     const int ws_total = min(ROWS, a.N - n0) * a.G;
-    constexpr int WSN = (ROWS * (MAX_K / GS) + WAVES * 64 - 1) / (WAVES * 64);
+    constexpr int WSN = (ROWS * max_groups(LG) + WAVES * 64 - 1) / (WAVES * 64);
     float wsreg[WSN];
     {
         const float *src = a.ws + (size_t)n0 * a.G;
@@ -194,7 +239,7 @@ gemv_w4a8_rows16_kernel(const Args a) {
             if (line >= lines) break;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int g = min(2 * line + h, a.G - 1);
+                const int g = min(2 * line + h, a.H - 1);
                 xa[i][h][0] = *reinterpret_cast<const v4i32 *>(xrow + g * GS);
                 xa[i][h][1] = *reinterpret_cast<const v4i32 *>(xrow + g * GS + 16);
             }
@@ -207,32 +252,23 @@ gemv_w4a8_rows16_kernel(const Args a) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 tile_park(patch, lane, xa[i][h][0], xa[i][h][1]);
-                xa[i][h][0] = tile_take(patch, lane, 2 * kq);
-                xa[i][h][1] = tile_take(patch, lane, 2 * kq + 1);
+                xa[i][h][0] = tile_take(patch, lane, LG == 1 ? kq : 2 * kq);
+                xa[i][h][1] = tile_take(patch, lane, LG == 1 ? 4 + kq : 2 * kq + 1);
             }
         }
     }
     // 5. integer group sums: lane holds (n = lane%16, m = 4*kq + v), v = 0..3
-    const v4i32 minus8 = {(int)0xF8F8F8F8u, (int)0xF8F8F8F8u, (int)0xF8F8F8F8u, (int)0xF8F8F8F8u};
 #pragma unroll
     for (int i = 0; i < NLP; ++i) {
         const int line = wave + i * WAVES;
         if (line >= lines) break;
         tile_park(patch, lane, w[i][0], w[i][1]);
+        v4i32 acc = {0, 0, 0, 0};
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int g = 2 * line + h;
-            if (g >= a.G) break;  // uniform per wavefront
-            const u32x4 ww = __builtin_bit_cast(u32x4, tile_take(patch, lane, 4 * h + kq));
-            const v4i32 x0 = {xa[i][h][0].x, xa[i][h][0].z, xa[i][h][1].x, xa[i][h][1].z};
-            const v4i32 x1 = {xa[i][h][0].y, xa[i][h][0].w, xa[i][h][1].y, xa[i][h][1].w};
-            const u32x4 lo = ww & 0x0F0F0F0Fu, hi = (ww >> 4) & 0x0F0F0F0Fu;
-            v4i32 acc = {0, 0, 0, 0};
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x0, minus8, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x1, minus8, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x0, __builtin_bit_cast(v4i32, lo), acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x1, __builtin_bit_cast(v4i32, hi), acc, 0, 0, 0);
-            reinterpret_cast<v4i32 *>(sums)[g * 64 + lane] = acc;
+            const int half = 2 * line + h;
+            if (half >= a.H) break;  // uniform per wavefront
+            half_sums<LG>(patch, lane, h, xa[i][h], acc, reinterpret_cast<v4i32 *>(sums), half);
         }
     }
     __syncthreads();
@@ -273,20 +309,21 @@ gemv_w4a8_rows16_kernel(const Args a) {
     }
 }
 
-template <int NLP, int WAVES, bool DUMP, bool FUSED>
+template <int NLP, int WAVES, bool DUMP, bool FUSED, int LG = 2>
 int launch_one(const Args &a, hipStream_t st) {
     static std::atomic<uint64_t> devices{0};
-    if (const int rc = reserve_lds(reinterpret_cast<const void *>(gemv_w4a8_rows16_kernel<NLP, WAVES, DUMP, FUSED>),
-                                   lds_bytes(MAX_K / GS, WAVES, FUSED), devices, "cmi_gemv_w4a8"))
+    if (const int rc = reserve_lds(reinterpret_cast<const void *>(gemv_w4a8_rows16_kernel<NLP, WAVES, DUMP, FUSED, LG>),
+                                   lds_bytes(max_groups(LG), WAVES, FUSED), devices, "cmi_gemv_w4a8"))
         return rc;
     const dim3 grid((a.N + ROWS - 1) / ROWS);
-    gemv_w4a8_rows16_kernel<NLP, WAVES, DUMP, FUSED>
+    gemv_w4a8_rows16_kernel<NLP, WAVES, DUMP, FUSED, LG>
         <<<grid, dim3(WAVES * 64), lds_bytes(a.G, WAVES, FUSED), st>>>(a);
     return check_launch("cmi_gemv_w4a8");
 }
 
 template <int NLP, int WAVES>
-int launch(const Args &a, hipStream_t st) {
+int launch(const Args &a, int lg, hipStream_t st) {
+    if (lg != 2) return lg == 1 ? launch_one<NLP, WAVES, false, false, 1>(a, st) : launch_one<NLP, WAVES, false, false, 3>(a, st);
     if (a.x) {
         if (a.K > FUSED_XV * 8 * WAVES * 64) return CMI_E_UNSUPPORTED;
         return a.group_acc ? launch_one<NLP, WAVES, true, true>(a, st) : launch_one<NLP, WAVES, false, true>(a, st);
@@ -295,17 +332,18 @@ int launch(const Args &a, hipStream_t st) {
 }
 
 
-// Rows longer than MAX_K: the same work in passes of 80 groups (10240 k), the fp32 chain carried
+// Rows longer than MAX_K (groups of 64: than 8192): the same work in passes of 48 half lines (6144 k), the fp32 chain carried
 // from pass to pass in the register of its thread.  The next pass's bytes are requested as soon
 // as this pass's MFMAs have consumed their registers, so memory keeps working while the chain of
 // this pass runs.  Quantised activations only (a caller with bf16 rows quantises first).
-constexpr int LONG_NLP = 3, LONG_WAVES = 8, LONG_GP = 2 * LONG_NLP * LONG_WAVES;  // groups per pass
+constexpr int LONG_NLP = 3, LONG_WAVES = 8, LONG_HP = 2 * LONG_NLP * LONG_WAVES;  // half lines per pass
 constexpr int LONG_THREADS = LONG_WAVES * 64;
-constexpr int LONG_WSN = (ROWS * LONG_GP + LONG_THREADS - 1) / LONG_THREADS;
 
-template <bool DUMP>
+template <bool DUMP, int LG>
 __global__ void __launch_bounds__(LONG_THREADS)
 gemv_w4a8_rows16_long_kernel(const Args a) {
+    constexpr int LONG_GP = LONG_HP * 4 >> LG;  // groups per pass
+    constexpr int LONG_WSN = (ROWS * LONG_GP + LONG_THREADS - 1) / LONG_THREADS;
     extern __shared__ __align__(16) uint8_t lds[];
     int32_t *sums = reinterpret_cast<int32_t *>(lds);                 // [LONG_GP][64 lanes][4]
     float *ws_lds = reinterpret_cast<float *>(lds + LONG_GP * 1024);  // [16][LONG_GP]
@@ -315,7 +353,7 @@ gemv_w4a8_rows16_long_kernel(const Args a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kq = lane >> 4;
     const int n0 = blockIdx.x * ROWS;
-    const int lines = (a.G + 1) / 2;
+    const int lines = (a.H + 1) / 2;
     const int passes = (a.G + LONG_GP - 1) / LONG_GP;
     const int nrows = min(ROWS, a.N - n0);
     uint8_t *patch = patches + wave * PATCH_BYTES;
@@ -331,7 +369,7 @@ gemv_w4a8_rows16_long_kernel(const Args a) {
             if (line >= lines) break;  // uniform per wavefront
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int g = min(2 * line + h, a.G - 1);
+                const int g = min(2 * line + h, a.H - 1);
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
                     xa[i][h][j] =
@@ -361,7 +399,6 @@ gemv_w4a8_rows16_long_kernel(const Args a) {
     const int nn = l & 15, m = 4 * (l >> 4) + v, n = n0 + nn;
     const bool chain = p < 256 && n < a.N && m < a.M;
     float total = 0.f;
-    const v4i32 minus8 = {(int)0xF8F8F8F8u, (int)0xF8F8F8F8u, (int)0xF8F8F8F8u, (int)0xF8F8F8F8u};
 #pragma unroll 1
     for (int pass = 0; pass < passes; ++pass) {
         const int line0 = pass * (LONG_NLP * LONG_WAVES) + wave;
@@ -378,8 +415,8 @@ gemv_w4a8_rows16_long_kernel(const Args a) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 tile_park(patch, lane, xa[i][h][0], xa[i][h][1]);
-                xa[i][h][0] = tile_take(patch, lane, 2 * kq);
-                xa[i][h][1] = tile_take(patch, lane, 2 * kq + 1);
+                xa[i][h][0] = tile_take(patch, lane, LG == 1 ? kq : 2 * kq);
+                xa[i][h][1] = tile_take(patch, lane, LG == 1 ? 4 + kq : 2 * kq + 1);
             }
         }
         // integer group sums: lane holds (n = lane%16, m = 4*kq + v), v = 0..3
@@ -388,20 +425,12 @@ gemv_w4a8_rows16_long_kernel(const Args a) {
             const int line = line0 + i * LONG_WAVES;
             if (line >= lines) break;
             tile_park(patch, lane, w[i][0], w[i][1]);
+            v4i32 acc = {0, 0, 0, 0};
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int g = 2 * line + h;
-                if (g >= a.G) break;  // uniform per wavefront
-                const u32x4 ww = __builtin_bit_cast(u32x4, tile_take(patch, lane, 4 * h + kq));
-                const v4i32 x0 = {xa[i][h][0].x, xa[i][h][0].z, xa[i][h][1].x, xa[i][h][1].z};
-                const v4i32 x1 = {xa[i][h][0].y, xa[i][h][0].w, xa[i][h][1].y, xa[i][h][1].w};
-                const u32x4 lo = ww & 0x0F0F0F0Fu, hi = (ww >> 4) & 0x0F0F0F0Fu;
-                v4i32 acc = {0, 0, 0, 0};
-                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x0, minus8, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x1, minus8, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x0, __builtin_bit_cast(v4i32, lo), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x1, __builtin_bit_cast(v4i32, hi), acc, 0, 0, 0);
-                reinterpret_cast<v4i32 *>(sums)[(g - pass * LONG_GP) * 64 + lane] = acc;
+                const int half = 2 * line + h;
+                if (half >= a.H) break;  // uniform per wavefront
+                half_sums<LG>(patch, lane, h, xa[i][h], acc, reinterpret_cast<v4i32 *>(sums), half - pass * LONG_HP);
             }
         }
         if (pass + 1 < passes) request(pass + 1);
@@ -437,15 +466,15 @@ gemv_w4a8_rows16_long_kernel(const Args a) {
     if (chain) a.y[(size_t)m * a.N + n] = (uint16_t)f32_to_bf16_bits(total * a.xs[m]);
 }
 
-template <bool DUMP>
+template <bool DUMP, int LG>
 int launch_long(const Args &a, hipStream_t st) {
-    constexpr int LDS_BYTES = LONG_GP * 1024 + ROWS * LONG_GP * 4 + LONG_WAVES * PATCH_BYTES;
+    constexpr int GP = LONG_HP * 4 >> LG, LDS_BYTES = GP * 1024 + ROWS * GP * 4 + LONG_WAVES * PATCH_BYTES;
     static std::atomic<uint64_t> devices{0};
-    if (const int rc = reserve_lds(reinterpret_cast<const void *>(gemv_w4a8_rows16_long_kernel<DUMP>), LDS_BYTES,
+    if (const int rc = reserve_lds(reinterpret_cast<const void *>(gemv_w4a8_rows16_long_kernel<DUMP, LG>), LDS_BYTES,
                                    devices, "cmi_gemv_w4a8"))
         return rc;
     const dim3 grid((a.N + ROWS - 1) / ROWS);
-    gemv_w4a8_rows16_long_kernel<DUMP><<<grid, dim3(LONG_THREADS), LDS_BYTES, st>>>(a);
+    gemv_w4a8_rows16_long_kernel<DUMP, LG><<<grid, dim3(LONG_THREADS), LDS_BYTES, st>>>(a);
     return check_launch("cmi_gemv_w4a8");
 }
 
@@ -617,8 +646,10 @@ namespace cmi {
 // CMI_E_UNSUPPORTED without setting the error text when the shape is outside this kernel's range
 // (the caller then uses another kernel).
 int gemv_w4a8_rows16(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs, const void *x,
-                     void *y, int32_t *group_acc, int8_t *xq_out, float *xs_out, int M, int N, int K,
+                     void *y, int32_t *group_acc, int8_t *xq_out, float *xs_out, int M, int N, int K, int gs,
                      void *stream) {
+    const int lg = gs == 64 ? 1 : gs == 256 ? 3 : 2;
+    if (lg != 2 && (x || group_acc || M > ROWS || K % gs != 0)) return CMI_E_UNSUPPORTED;
     if (M < 1 || M > (x ? FUSED_ROWS : MAX_CHUNKS * ROWS) || K < GS || K % GS != 0 || N < 1) return CMI_E_UNSUPPORTED;
     if (K > MAX_K && (x || M > ROWS)) return CMI_E_UNSUPPORTED;
     Args a;
@@ -634,10 +665,13 @@ int gemv_w4a8_rows16(const uint8_t *w4, const float *ws, const int8_t *xq, const
     a.M = M;
     a.N = N;
     a.K = K;
-    a.G = K / GS;
+    a.G = K / gs;
+    a.H = K / GS;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (K > MAX_K) return group_acc ? launch_long<true>(a, st) : launch_long<false>(a, st);
-    const int lines = (a.G + 1) / 2;
+    if (lg == 1 && a.G > max_groups(1)) return launch_long<false, 1>(a, st);
+    if (K > MAX_K && lg == 3) return launch_long<false, 3>(a, st);
+    if (K > MAX_K) return group_acc ? launch_long<true, 2>(a, st) : launch_long<false, 2>(a, st);
+    const int lines = (a.H + 1) / 2;
     // Eight wavefronts per workgroup beyond 20 lines, and up to ~640 workgroups (2.5 per compute
     // unit) where a wavefront's chain of dependent steps is what is left to shorten (0.6-0.9 us
     // faster at N = 2560..9728); four on larger grids (7 % faster at N = 151936).
@@ -663,19 +697,19 @@ int gemv_w4a8_rows16(const uint8_t *w4, const float *ws, const int8_t *xq, const
     }
     if (!eight) {
         switch ((lines + 3) / 4) {
-            case 1: return launch<1, 4>(a, st);
-            case 2: return launch<2, 4>(a, st);
-            case 3: return launch<3, 4>(a, st);
-            case 4: return launch<4, 4>(a, st);
-            default: return launch<5, 4>(a, st);
+            case 1: return launch<1, 4>(a, lg, st);
+            case 2: return launch<2, 4>(a, lg, st);
+            case 3: return launch<3, 4>(a, lg, st);
+            case 4: return launch<4, 4>(a, lg, st);
+            default: return launch<5, 4>(a, lg, st);
         }
     }
     switch ((lines + 7) / 8) {
-        case 1: return launch<1, 8>(a, st);
-        case 2: return launch<2, 8>(a, st);
-        case 3: return launch<3, 8>(a, st);
-        case 4: return launch<4, 8>(a, st);
-        default: return launch<5, 8>(a, st);
+        case 1: return launch<1, 8>(a, lg, st);
+        case 2: return launch<2, 8>(a, lg, st);
+        case 3: return launch<3, 8>(a, lg, st);
+        case 4: return launch<4, 8>(a, lg, st);
+        default: return launch<5, 8>(a, lg, st);
     }
 }
 

@@ -37,6 +37,11 @@ int cmi::linear_w4a8_rows(const uint8_t *w4, const float *ws, const void *x, voi
         const int rc = cmi_gemv_w4a8_bf16(w4, ws, x, y, nullptr, nullptr, nullptr, M, N, K, gs, stream);
         if (rc != CMI_E_UNSUPPORTED) return rc;
     }
+    // groups of 64 and 256: one row, by the same rule (not through the entry above, which is for groups of 128)
+    if (gs != 128 && M == 1 && Kd == K && K <= 10240 && w4_fused_route(M, N, K) && aligned(x, 16) && aligned(w4, 16)) {
+        const int rc = gemv_w4a8_decode(w4, ws, x, nullptr, nullptr, y, nullptr, nullptr, nullptr, M, N, K, gs, stream);
+        if (rc != CMI_E_UNSUPPORTED) return rc;
+    }
     if (const int rc = quant_act_i8_padded(x, xq, xs, M, K, Kd, stream)) return rc;
     // up to 16 rows the GEMV entry; beyond, the GEMM entry (which itself goes through the
     // read-once kernels while they are cheaper than the tile pipeline)

@@ -179,6 +179,76 @@ def test_w4a8_tiles_of_four_groups_a_step(orc, m, n, k):
         G.set_option("w4_gemm_deep", 0)
 
 
+@pytest.mark.parametrize("gs,m,n,k", [(64, 1, 24, 128), (64, 3, 40, 512), (64, 17, 33, 640), (64, 16, 64, 1024), (64, 33, 65, 384), (64, 49, 129, 2560),
+                                      (64, 65, 96, 4608), (256, 1, 24, 256), (256, 5, 40, 512), (256, 17, 33, 768), (256, 16, 64, 1024),
+                                      (256, 47, 130, 1280), (256, 97, 200, 3840)])
+def test_w4a8_tiles_of_four_steps_of_other_groups(orc, gs, m, n, k):
+    """Groups of 64 and 256: part of a stage to many, ragged in both directions; then with scales below 2^-122 in some columns."""
+    g = synth.generator(gs + m + n + k)
+    w = synth.int4_weight(n, k, g, group_size=gs)
+    x = synth.activations(m, k, g, outliers=True)
+    xq, xs = orc.quant_act_i8(G.bits(x))
+    tiny = w.scale.clone()
+    tiny[:, ::3] = 2.0 ** -126
+    tiny[k // gs - 1, 1::3] = 2.0 ** -140
+    tiny[0, 2::3] = 0.0
+    for scale in (w.scale, tiny):
+        _, y_ref = orc.linear_w4a8(xq, xs, w.packed.numpy(), scale.numpy(), k, gs)
+        w4, ws = G.w4_repack(w.packed.to(G.DEV), scale.to(G.DEV), k, gs)
+        for code in (0, 1664, 1665, 3232, 3233, 3264, 3265, 4864):
+            G.set_option("w4_gemm_deep", code)
+            for gemm in (True, False) if m <= 16 else (True,):
+                _, y = G.w4a8(w4, ws, G.dev(xq), G.dev(xs), k, gemm=gemm, want_acc=False, gs=gs)
+                assert (G.bits(y) == y_ref).all(), (code, gemm)
+        G.set_option("w4_gemm_deep", 0)
+
+
+@pytest.mark.parametrize("gs,k", [(64, 128), (64, 384), (64, 640), (64, 1024), (64, 2560), (64, 2688), (64, 4096), (64, 5120), (64, 5248), (64, 8192),
+                                  (64, 8320), (64, 10240), (64, 12416), (64, 20480), (64, 20608), (256, 256), (256, 768), (256, 1024), (256, 2560),
+                                  (256, 2816), (256, 5120), (256, 5376), (256, 10240), (256, 10496), (256, 20480), (256, 20736)])
+def test_w4a8_rows_of_other_groups(orc, gs, k):
+    """One row (quantised by the kernel or before it; every number of loads per wavefront, whole and not) and 2..16 rows (one
+    line per wavefront to several passes, half lines)."""
+    g = synth.generator(gs + k)
+    n = 37
+    w = synth.int4_weight(n, k, g, group_size=gs)
+    x = synth.activations(16, k, g, outliers=True)
+    xq, xs = orc.quant_act_i8(G.bits(x))
+    sums_ref, y_ref = orc.linear_w4a8(xq, xs, w.packed.numpy(), w.scale.numpy(), k, gs, want_group_acc=True)
+    w4, ws = G.w4_repack(w.packed.to(G.DEV), w.scale.to(G.DEV), k, gs)
+    lib = _native.load()
+    work = torch.empty(int(lib.cmi_linear_workspace_bytes(16, k)), dtype=torch.uint8, device=G.DEV)
+    xd = x.to(G.DEV)
+    for m in (1, 2, 5, 16):
+        _, y = G.w4a8(w4, ws, G.dev(xq[:m]), G.dev(xs[:m]), k, gemm=False, want_acc=False, gs=gs)
+        assert (G.bits(y) == y_ref[:m]).all(), m
+        y = torch.empty((m, n), dtype=torch.bfloat16, device=G.DEV)
+        _native.check(lib.cmi_linear_w4a8_bf16(G.ptr(w4), G.ptr(ws), G.ptr(xd), G.ptr(y), m, n, k, gs, G.ptr(work), work.numel(),
+                                               G.stream()), "linear_w4a8_bf16")
+        assert (G.bits(y) == y_ref[:m]).all(), m
+    sums, y = G.w4a8(w4, ws, G.dev(xq[:1]), G.dev(xs[:1]), k, gemm=False, gs=gs)
+    assert (sums.cpu().numpy() == sums_ref[:1]).all() and (G.bits(y) == y_ref[:1]).all()
+
+
+@pytest.mark.parametrize("gs", [64, 256])
+def test_one_row_of_other_groups_off_a_16_byte_boundary(orc, gs):
+    g = synth.generator(gs)
+    k, n = 2560, 24
+    w = synth.int4_weight(n, k, g, group_size=gs)
+    x = synth.activations(1, k, g)
+    xq, xs = orc.quant_act_i8(G.bits(x))
+    _, y_ref = orc.linear_w4a8(xq, xs, w.packed.numpy(), w.scale.numpy(), k, gs)
+    w4, ws = G.w4_repack(w.packed.to(G.DEV), w.scale.to(G.DEV), k, gs)
+    xd = torch.empty(k + 1, dtype=torch.bfloat16, device=G.DEV)[1:].view(1, k)
+    xd.copy_(x)
+    lib = _native.load()
+    work = torch.empty(int(lib.cmi_linear_workspace_bytes(1, k)), dtype=torch.uint8, device=G.DEV)
+    y = torch.empty((1, n), dtype=torch.bfloat16, device=G.DEV)
+    _native.check(lib.cmi_linear_w4a8_bf16(G.ptr(w4), G.ptr(ws), G.ptr(xd), G.ptr(y), 1, n, k, gs, G.ptr(work), work.numel(),
+                                           G.stream()), "linear_w4a8_bf16")
+    assert (G.bits(y) == y_ref).all()
+
+
 @pytest.mark.parametrize("m,n,k", [(16, 12288, 4096), (4, 24000, 768), (9, 5120, 25600), (40, 2560, 9728), (70, 6144, 2560), (200, 2560, 9728)])
 def test_w4a8_rows_through_the_chosen_tile(m, n, k):
     """Sizes where the choice is a tile of four groups a step: the results of the kernels without them."""
