@@ -530,9 +530,10 @@ def _rows_quantised(rec: _Record, xq: int, xs: int, rows: int, out: torch.Tensor
 
 
 def _splits_k(rows: int, n: int, k: int, device: torch.device) -> bool:
-    """Whether the W8A8 entry would be given room to split K for this shape (it then needs the
-    quantiser's launch in front of it, which clears the arrival counters)."""
-    return _scratch(rows, k, device, n)[1] != _scratch(rows, k, device)[1]
+    """Whether the W8A8 entry splits K for this shape and gains by it what the quantiser's launch in front of it costs,
+    which clears the arrival counters (by the room it asks for alone, 500 rows of 2560 -> 19456 -> 2560 were quantised
+    twice on the way: 4 us a projection)."""
+    return bool(_native.load().cmi_linear_w8a8_splits(rows, n, k))
 
 
 def _rows_w4a16(rec: _Record, act: torch.Tensor, rows: int, out: torch.Tensor) -> None:

@@ -1199,6 +1199,125 @@ int launch_wide_tilewise(Args &a, hipStream_t st) {
     return check_launch("cmi_gemm_w8a8");
 }
 
+// Kernel of a launch and its modelled time (us).
+constexpr int READ_ONCE = -1;
+struct Choice {
+    int pick;         // READ_ONCE, or the block tile along n: 64, 128, 192, 256, 320; 128192; 256192; 6464 (64 x 64)
+    int splits;       // 1, or workgroups per tile of the split-K form of 6464, 64 and 128
+    double us;
+    double whole_us;  // of the best choice that does not split
+};
+
+Choice choose_few_rows(int M, int N, int K, size_t partial_bytes) {
+    // Between the GEMV-like batch and the full tile pipeline every kernel is bound by what its
+    // workgroups pull through L2 per dependent step, and which one is fastest changes with the
+    // shape: the read-once kernel pays per 16-row chunk, a tile kernel K / 128 steps whose
+    // length grows with N (bytes per step) and with the rounds of workgroups on the 256 CUs.
+    // Cost models (us) fitted to cold-weight measurements of all five kernels on eleven layer
+    // shapes x ten batch sizes; their choice is within 1 % of the best measured in total
+    // (the two-candidate rule this replaces: 19 % above).
+    const double steps = (K + BK - 1) / BK, wbytes = (double)N * K;
+    auto rounds = [](double tiles) { return ceil(tiles / 256.0); };
+    const double tiles_h = (double)((M + 63) / 64) * ((N + 63) / 64);
+    const double tiles_g = (double)((M + 127) / 128) * ((N + 63) / 64);
+    const double tiles_t = (double)((M + 127) / 128) * ((N + 127) / 128);
+    // up to 192 tiles the idle CUs read the weight through the caches meanwhile (warm_caches):
+    // steps measured 13 % (64 x 64) and 20-25 % (the larger tiles) shorter
+    auto warmed = [&](double tiles, double f) { return tiles <= 192 && wbytes <= 64.0 * 1048576.0 ? f : 1.0; };
+    const double t_h = 2.5 + steps * (0.22 + N * 1.6e-5) * warmed(tiles_h, 0.87) * (1.0 + 0.50 * (rounds(tiles_h) - 1));
+    const double t_g = 2.5 + steps * (0.36 + N * 1.2e-5) * warmed(tiles_g, 0.78) * (1.0 + 0.75 * (rounds(tiles_g) - 1));
+    const double t_t = 2.5 + steps * (0.50 + N * 1.5e-5) * warmed(tiles_t, 0.78) * (1.0 + 0.65 * (rounds(tiles_t) - 1));
+    double t_rows = 1e30;
+    if (K <= 10240) {
+        const double per_chunk = 0.5 + wbytes / (gemm_w8a8_rows_tiles(N) * 2.0e7);
+        t_rows = ((M + 127) / 128) * (3.2 + wbytes / 6.0e6) + ((M + 15) / 16) * per_chunk;
+    }
+    // Split-K on the 64 x 64 tile where the caller brought room for the partial tiles (the
+    // arrival counters cleared): few tiles and many steps, e.g. 64 rows of 9728 -> 2560 are
+    // 40 tiles x 76 steps on 40 of 256 CUs.  As many splits as keep one workgroup per CU and
+    // four steps per split.  With the whole chip pulling, the steps run into the weight stream
+    // (about 5 TB/s in so short a launch), and the hand-over -- partial tiles written through
+    // to memory, the arrival, the last workgroup's reads: three trips to memory, the L2s of
+    // the XCDs not being coherent with each other -- costs 5 us whatever the shape.
+    int splits = 1, splits_g = 1;
+    double t_s = 1e30, t_sg = 1e30;
+    auto split_count = [&](double tiles) {
+        int n = (int)(256.0 / tiles);
+        if (n > steps / 4) n = (int)(steps / 4);
+        return n > 8 ? 8 : n;
+    };
+    if (partial_bytes && tiles_h <= 128) {
+        splits = split_count(tiles_h);
+        if (splits >= 2 && (size_t)(splits * tiles_h) * 64 * 64 * 4 <= partial_bytes)
+            t_s = 2.5 + fmax(ceil(steps / splits) * 0.26, wbytes / 5.0e6) + 5.0;
+    }
+    // the same on the 128(m) x 64(n) tile (129..256 rows): a step is longer, the hand-over twice the bytes
+    if (partial_bytes && tiles_g <= 128 && M > 128) {
+        splits_g = split_count(tiles_g);
+        if (splits_g >= 2 && (size_t)(splits_g * tiles_g) * 128 * 64 * 4 <= partial_bytes)
+            t_sg = 2.5 + fmax(ceil(steps / splits_g) * 0.42, wbytes / 5.0e6) + 6.0;
+    }
+    const double whole = fmin(fmin(t_rows, t_h), fmin(t_g, t_t));
+    if (t_s < whole || t_sg < whole) return t_sg < t_s ? Choice{64, splits_g, t_sg, whole} : Choice{6464, splits, t_s, whole};
+    return {t_rows == whole ? READ_ONCE : t_h <= t_g && t_h <= t_t ? 6464 : t_g <= t_t ? 64 : 128, 1, whole, whole};
+}
+
+// Tile choice above 256 rows.  Every tile kernel is a chain of K / 128 dependent steps whose
+// length is set by the operand bytes a workgroup pulls per step (it grows with the tile and,
+// the weight being cold, with N) and by how many workgroups share a CU; larger tiles move
+// fewer bytes per MFMA, smaller ones fill the 256 CUs more evenly.  Cost models (us) of the
+// same form as for 17..256 rows, fitted to cold-weight measurements of every kernel on
+// sixteen layer shapes x eleven batch sizes (272..8192 rows): their choice is 0.3 % above the
+// best measured in total, the fill-and-area rule this replaces 2.4 % (and up to 40 % on
+// single shapes, e.g. 2048 x 9728 -> 2560: 84 -> 63 us).  The 192(m) x 256(n) tile fills the gap between
+// 4-wavefront tiles that need two rounds and 256-row ones that leave CUs idle: 500 x 19456 x 2560
+// 38.0 -> 34.9 us (228 tiles instead of 152), 1152 x 19456 76.5 -> 65.2, 768 x 11008 x 4096 50.9 -> 44.9,
+// 2048 x 11008 x 4096 103 -> 92; it and 256 x 320 are fitted to a sweep of eight shapes x twelve
+// batch sizes, where the choice is 0.2 % above the best (1.9 % without it).  A step's growth with N is fitted up to
+// 32768 outputs and stays there beyond: carried on it preferred 256 x 320 to 256 x 256 for 385..512 rows of 51200
+// outputs (400 x 51200 x 4096 122 against 107 us; eight shapes of 19456..51200 outputs x fifteen batch sizes:
+// the choice 0.8 -> 0.1 % above the best).
+Choice choose_many_rows(int M, int N, int K, size_t partial_bytes) {
+    const double steps = (K + BK - 1) / BK;
+    auto cost = [&](int bm, int bn, double a0, double b0, double c0) {
+        const double tiles = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        // the 4-wavefront tiles on up to 192 CUs: the idle CUs warm the caches (see above)
+        const double warmed = bm <= 192 && bn <= 192 && tiles <= 192 && (double)N * K <= 64.0 * 1048576.0 ? 0.8 : 1.0;
+        return 2.5 + steps * (a0 + b0 * fmin(N, 32768)) * warmed * (1.0 + c0 * (ceil(tiles / 256.0) - 1.0));
+    };
+    const struct { int pick; double us; } candidates[] = {
+        {64, N > 64 ? cost(128, 64, 0.407, 5.54e-6, 0.796) : 1e30},
+        {128, cost(128, 128, 0.555, 9.82e-6, 0.91)},
+        {192, cost(128, 192, 0.723, 1.89e-5, 1.03)},
+        {128192, cost(192, 128, 0.709, 1.19e-5, 1.12)},
+        {256, cost(256, 256, 1.29, 2.33e-5, 1.28)},
+        {320, cost(256, 320, 1.634, 1.73e-5, 1.19)},
+        {256192, cost(192, 256, 1.175, 1.32e-5, 1.07)},
+    };
+    int pick = 128;
+    double best = 1e30;
+    for (const auto &c : candidates)
+        if (c.us < best) best = c.us, pick = c.pick;
+    // Split-K on the 128 x 128 tile where the caller brought room for the partial tiles: a long,
+    // narrow projection (9728 -> 2560 at 257..512 rows: 60..80 tiles x 76 steps) leaves most
+    // of the CUs idle for a long chain of steps (quantiser + GEMM 38..42 -> 30..34.5 us).  Model
+    // as for the smaller tiles; the hand-over moves 64 KiB per workgroup.
+    const int tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
+    if (partial_bytes && tiles128 <= 128 && steps >= 16) {
+        int splits = 256 / tiles128;
+        if (splits > steps / 4) splits = (int)(steps / 4);
+        if (splits > 8) splits = 8;
+        const double t_split = 2.5 + fmax(ceil(steps / splits) * (0.554 + 1.11e-5 * N), (double)N * K / 5.0e6) + SPLIT128_HANDOVER_US;
+        if (splits >= 2 && (size_t)splits * tiles128 * 128 * 128 * 4 <= partial_bytes && t_split < best) return {128, splits, t_split, best};
+    }
+    return {pick, 1, best, best};
+}
+
+// (16 rows and fewer come here where the read-once kernel does not take them.)
+Choice choose(int M, int N, int K, size_t partial_bytes) {
+    return M > 16 && M <= 256 ? choose_few_rows(M, N, K, partial_bytes) : choose_many_rows(M, N, K, partial_bytes);
+}
+
 }  // namespace
 
 extern "C" int cmi_gemm_w8a8(const int8_t *xq, const int8_t *wq, const float *xs, const float *ws,
@@ -1217,6 +1336,15 @@ size_t cmi::gemm_w8a8_split_bytes(int M, int N, int K) {
     return M <= 1024 && tiles128 <= 128 && K / BK >= 16 ? (size_t)256 * 128 * 128 * 4 : 0;
 }
 
+// Where rows arrive quantised the split has to gain more than the launch that clears its counters, the quantiser's, costs:
+// 2 us and 0.55 ps an element (500 x 9728 4.7 us).
+extern "C" int cmi_linear_w8a8_splits(int M, int N, int K) {
+    const size_t bytes = cmi::gemm_w8a8_split_bytes(M, N, K);
+    if (bytes == 0 || cmi::option_gemm_tile()) return 0;
+    const Choice c = choose(M, N, K, bytes);
+    return c.splits > 1 && c.us + 2.0 + 5.5e-7 * M * K < c.whole_us;
+}
+
 int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, const float *ws, void *y,
                          int32_t *acc_out, int M, int N, int K, int ldy, int *arrivals, void *partials,
                          size_t partial_bytes, void *stream) {
@@ -1233,88 +1361,20 @@ int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, co
         const int rc = gemm_w8a8_rows16(xq, wq, xs, ws, y, acc_out, M, N, K, ldy, stream);
         if (rc != CMI_E_UNSUPPORTED) return rc;
     }
-    int mid = 0;  // 17..256 rows: the tile kernel the cost models below chose (64 x 64: 6464), if any
-    if (M > 16 && M <= 256 && K >= BK && K <= MAX_K && N >= 8 && !force) {
-        // Between the GEMV-like batch and the full tile pipeline every kernel is bound by what its
-        // workgroups pull through L2 per dependent step, and which one is fastest changes with the
-        // shape: the read-once kernel pays per 16-row chunk, a tile kernel K / 128 steps whose
-        // length grows with N (bytes per step) and with the rounds of workgroups on the 256 CUs.
-        // Cost models (us) fitted to cold-weight measurements of all five kernels on eleven layer
-        // shapes x ten batch sizes; their choice is within 1 % of the best measured in total
-        // (the two-candidate rule this replaces: 19 % above).
-        const double steps = (K + BK - 1) / BK, wbytes = (double)N * K;
-        auto rounds = [](double tiles) { return ceil(tiles / 256.0); };
-        const double tiles_h = (double)((M + 63) / 64) * ((N + 63) / 64);
-        const double tiles_g = (double)((M + 127) / 128) * ((N + 63) / 64);
-        const double tiles_t = (double)((M + 127) / 128) * ((N + 127) / 128);
-        // up to 192 tiles the idle CUs read the weight through the caches meanwhile (warm_caches):
-        // steps measured 13 % (64 x 64) and 20-25 % (the larger tiles) shorter
-        auto warmed = [&](double tiles, double f) { return tiles <= 192 && wbytes <= 64.0 * 1048576.0 ? f : 1.0; };
-        const double t_h = 2.5 + steps * (0.22 + N * 1.6e-5) * warmed(tiles_h, 0.87) * (1.0 + 0.50 * (rounds(tiles_h) - 1));
-        const double t_g = 2.5 + steps * (0.36 + N * 1.2e-5) * warmed(tiles_g, 0.78) * (1.0 + 0.75 * (rounds(tiles_g) - 1));
-        const double t_t = 2.5 + steps * (0.50 + N * 1.5e-5) * warmed(tiles_t, 0.78) * (1.0 + 0.65 * (rounds(tiles_t) - 1));
-        double t_rows = 1e30;
-        if (K <= 10240) {
-            const double per_chunk = 0.5 + wbytes / (gemm_w8a8_rows_tiles(N) * 2.0e7);
-            t_rows = ((M + 127) / 128) * (3.2 + wbytes / 6.0e6) + ((M + 15) / 16) * per_chunk;
-        }
-        // Split-K on the 64 x 64 tile where the caller brought room for the partial tiles (the
-        // arrival counters cleared): few tiles and many steps, e.g. 64 rows of 9728 -> 2560 are
-        // 40 tiles x 76 steps on 40 of 256 CUs.  As many splits as keep one workgroup per CU and
-        // four steps per split.  With the whole chip pulling, the steps run into the weight stream
-        // (about 5 TB/s in so short a launch), and the hand-over -- partial tiles written through
-        // to memory, the arrival, the last workgroup's reads: three trips to memory, the L2s of
-        // the XCDs not being coherent with each other -- costs 5 us whatever the shape.
-        int splits = 1, splits_g = 1;
-        double t_s = 1e30, t_sg = 1e30;
-        auto split_count = [&](double tiles) {
-            int n = (int)(256.0 / tiles);
-            if (n > steps / 4) n = (int)(steps / 4);
-            return n > 8 ? 8 : n;
-        };
-        if (arrivals && partials && tiles_h <= 128) {
-            splits = split_count(tiles_h);
-            if (splits >= 2 && (size_t)(splits * tiles_h) * 64 * 64 * 4 <= partial_bytes)
-                t_s = 2.5 + fmax(ceil(steps / splits) * 0.26, wbytes / 5.0e6) + 5.0;
-        }
-        // the same on the 128(m) x 64(n) tile (129..256 rows): a step is longer, the hand-over twice the bytes
-        if (arrivals && partials && tiles_g <= 128 && M > 128) {
-            splits_g = split_count(tiles_g);
-            if (splits_g >= 2 && (size_t)(splits_g * tiles_g) * 128 * 64 * 4 <= partial_bytes)
-                t_sg = 2.5 + fmax(ceil(steps / splits_g) * 0.42, wbytes / 5.0e6) + 6.0;
-        }
-        if ((t_s < t_rows && t_s < t_h && t_s < t_g && t_s < t_t) || (t_sg < t_rows && t_sg < t_h && t_sg < t_g && t_sg < t_t)) {
-            const bool wide_m = t_sg < t_s;
-            Args a;
-            a.xq = xq;
-            a.wq = wq;
-            a.xs = xs;
-            a.ws = ws;
-            a.y = static_cast<uint16_t *>(y);
-            a.acc_out = acc_out;
-            a.M = M;
-            a.N = N;
-            a.K = K;
-            a.ldy = ldy;
-            a.splits = wide_m ? splits_g : splits;
-            a.partials = static_cast<int32_t *>(partials);
-            a.arrivals = arrivals;
-            return wide_m ? launch_split<1, 2, 3>(a, static_cast<hipStream_t>(stream))
-                          : launch_split<1, 1, 4>(a, static_cast<hipStream_t>(stream));
-        }
-        if (t_rows <= t_h && t_rows <= t_g && t_rows <= t_t) {
-            for (int lo = 0; lo < M; lo += 128) {
-                const int m = M - lo < 128 ? M - lo : 128;
-                const int rc = gemm_w8a8_rows16(xq + (size_t)lo * K, wq, xs + lo, ws,
-                                                static_cast<uint16_t *>(y) + (size_t)lo * ldy,
-                                                acc_out ? acc_out + (size_t)lo * N : nullptr, m, N, K, ldy, stream);
-                if (rc != CMI_OK) return rc == CMI_E_UNSUPPORTED ? fail(rc, "cmi_gemm_w8a8: internal dispatch") : rc;
-            }
-            return CMI_OK;
-        }
-        mid = t_h <= t_g && t_h <= t_t ? 6464 : t_g <= t_t ? 64 : 128;
-    }
     if (K < BK || K > MAX_K || N < 8) return gemm_w8a8_generic(xq, wq, xs, ws, y, acc_out, M, N, K, ldy, stream);
+    // CMI_GEMM_TILE=64|128|192|256|320 overrides the tile along n (tests, tuning); 128192 forces
+    // 128(n) x 192(m), 256192 256(n) x 192(m), 6464 the 64 x 64 tile of the mid-batch route.
+    const Choice c = force ? Choice{force, 1, 0.0, 0.0} : choose(M, N, K, arrivals && partials ? partial_bytes : 0);
+    if (c.pick == READ_ONCE) {
+        for (int lo = 0; lo < M; lo += 128) {
+            const int m = M - lo < 128 ? M - lo : 128;
+            const int rc = gemm_w8a8_rows16(xq + (size_t)lo * K, wq, xs + lo, ws,
+                                            static_cast<uint16_t *>(y) + (size_t)lo * ldy,
+                                            acc_out ? acc_out + (size_t)lo * N : nullptr, m, N, K, ldy, stream);
+            if (rc != CMI_OK) return rc == CMI_E_UNSUPPORTED ? fail(rc, "cmi_gemm_w8a8: internal dispatch") : rc;
+        }
+        return CMI_OK;
+    }
     Args a;
     a.xq = xq;
     a.wq = wq;
@@ -1330,64 +1390,12 @@ int cmi::gemm_w8a8_split(const int8_t *xq, const int8_t *wq, const float *xs, co
     a.partials = nullptr;
     a.arrivals = nullptr;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // Tile choice above 256 rows.  Every tile kernel is a chain of K / 128 dependent steps whose
-    // length is set by the operand bytes a workgroup pulls per step (it grows with the tile and,
-    // the weight being cold, with N) and by how many workgroups share a CU; larger tiles move
-    // fewer bytes per MFMA, smaller ones fill the 256 CUs more evenly.  Cost models (us) of the
-    // same form as for 17..256 rows, fitted to cold-weight measurements of every kernel on
-    // sixteen layer shapes x eleven batch sizes (272..8192 rows): their choice is 0.3 % above the
-    // best measured in total, the fill-and-area rule this replaces 2.4 % (and up to 40 % on
-    // single shapes, e.g. 2048 x 9728 -> 2560: 84 -> 63 us).  The 192(m) x 256(n) tile fills the gap between
-    // 4-wavefront tiles that need two rounds and 256-row ones that leave CUs idle: 500 x 19456 x 2560
-    // 38.0 -> 34.9 us (228 tiles instead of 152), 1152 x 19456 76.5 -> 65.2, 768 x 11008 x 4096 50.9 -> 44.9,
-    // 2048 x 11008 x 4096 103 -> 92; it and 256 x 320 are fitted to a sweep of eight shapes x twelve
-    // batch sizes, where the choice is 0.2 % above the best (1.9 % without it).  A step's growth with N is fitted up to
-    // 32768 outputs and stays there beyond: carried on it preferred 256 x 320 to 256 x 256 for 385..512 rows of 51200
-    // outputs (400 x 51200 x 4096 122 against 107 us; eight shapes of 19456..51200 outputs x fifteen batch sizes:
-    // the choice 0.8 -> 0.1 % above the best).
-    // CMI_GEMM_TILE=64|128|192|256|320 overrides the tile along n (tests, tuning); 128192 forces
-    // 128(n) x 192(m), 256192 256(n) x 192(m), 6464 the 64 x 64 tile of the mid-batch route.
-    int pick;  // 64, 128, 192, 256 or 320: block tile along n; 128192; 256192; 6464
-    if (force || mid) {
-        pick = force ? force : mid;
-    } else {
-        const double steps = (K + BK - 1) / BK;
-        auto cost = [&](int bm, int bn, double a0, double b0, double c0) {
-            const double tiles = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-            // the 4-wavefront tiles on up to 192 CUs: the idle CUs warm the caches (see above)
-            const double warmed = bm <= 192 && bn <= 192 && tiles <= 192 && (double)N * K <= 64.0 * 1048576.0 ? 0.8 : 1.0;
-            return 2.5 + steps * (a0 + b0 * fmin(N, 32768)) * warmed * (1.0 + c0 * (ceil(tiles / 256.0) - 1.0));
-        };
-        const struct { int pick; double us; } candidates[] = {
-            {64, N > 64 ? cost(128, 64, 0.407, 5.54e-6, 0.796) : 1e30},
-            {128, cost(128, 128, 0.555, 9.82e-6, 0.91)},
-            {192, cost(128, 192, 0.723, 1.89e-5, 1.03)},
-            {128192, cost(192, 128, 0.709, 1.19e-5, 1.12)},
-            {256, cost(256, 256, 1.29, 2.33e-5, 1.28)},
-            {320, cost(256, 320, 1.634, 1.73e-5, 1.19)},
-            {256192, cost(192, 256, 1.175, 1.32e-5, 1.07)},
-        };
-        pick = 128;
-        double best = 1e30;
-        for (const auto &c : candidates)
-            if (c.us < best) best = c.us, pick = c.pick;
-        // Split-K on the 128 x 128 tile where the caller brought room for the partial tiles: a long,
-        // narrow projection (9728 -> 2560 at 257..512 rows: 60..80 tiles x 76 steps) leaves most
-        // of the CUs idle for a long chain of steps (quantiser + GEMM 38..42 -> 30..34.5 us).  Model
-        // as for the smaller tiles; the hand-over moves 64 KiB per workgroup.
-        const int tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
-        if (arrivals && partials && tiles128 <= 128 && steps >= 16) {
-            int splits = 256 / tiles128;
-            if (splits > steps / 4) splits = (int)(steps / 4);
-            if (splits > 8) splits = 8;
-            const double t_split = 2.5 + fmax(ceil(steps / splits) * (0.554 + 1.11e-5 * N), (double)N * K / 5.0e6) + SPLIT128_HANDOVER_US;
-            if (splits >= 2 && (size_t)splits * tiles128 * 128 * 128 * 4 <= partial_bytes && t_split < best) {
-                a.splits = splits;
-                a.partials = static_cast<int32_t *>(partials);
-                a.arrivals = arrivals;
-                return launch_split<2, 2, 3>(a, st);
-            }
-        }
+    const int pick = c.pick;
+    if (c.splits > 1) {
+        a.splits = c.splits;
+        a.partials = static_cast<int32_t *>(partials);
+        a.arrivals = arrivals;
+        return pick == 64 ? launch_split<1, 2, 3>(a, st) : pick == 6464 ? launch_split<1, 1, 4>(a, st) : launch_split<2, 2, 3>(a, st);
     }
     // the 256 x 320 tile: the tile-wise kernel (within 1 % of the two-stage one on the large shapes,
     // 7 % faster at 2048 x 4096 x 2560); a forced 320 still names the two-stage kernel

@@ -404,20 +404,19 @@ PyObject *project(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     size_t need = 0;
     unsigned char *work = nullptr;
     if (quantised) {
-        if (e.kind == 8) need = cmi_linear_w8a8_workspace_bytes(M, Nn, K);
         PyObject *handed = var(N.handed);
         if (handed && handed != Py_None && e.kd == K) {
             if (Py_TYPE(handed) != &HandedType) Py_RETURN_NONE;  // left by the Python adapter, which can read it
             const Handed *h = reinterpret_cast<Handed *>(handed);
-            // a W8A8 shape that may split K needs the quantiser's launch, which clears its counters
-            if ((e.kind == 4 || need == cmi_linear_workspace_bytes(M, K)) && handed_matches(h, x, rows, K, stream)) {
+            // a W8A8 shape that splits K needs the quantiser's launch, which clears its counters
+            if (handed_matches(h, x, rows, K, stream) && (e.kind == 4 || !cmi_linear_w8a8_splits(M, Nn, K))) {
                 xq = reinterpret_cast<const int8_t *>(static_cast<intptr_t>(h->xq));
                 xs = reinterpret_cast<const float *>(static_cast<intptr_t>(h->xs));
                 ++g_handed_uses[e.kind == 8];
             }
         }
         if (!xq) {
-            if (e.kind == 4) need = cmi_linear_workspace_bytes(M, e.kd);
+            need = e.kind == 4 ? cmi_linear_workspace_bytes(M, e.kd) : cmi_linear_w8a8_workspace_bytes(M, Nn, K);
             work = g_workspace.take(need, args[1], here);
             if (!work) return nullptr;
             if (!truth(N.seen)) PyDict_SetItem(g_vars, N.seen, Py_True);

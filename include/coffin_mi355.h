@@ -214,6 +214,9 @@ size_t cmi_linear_workspace_bytes(int M, int K);
  * CUs where a projection is few tiles and many K steps (same bits: the partial sums are
  * integers); with the smaller workspace it does not split.  No counterpart in the reference. */
 size_t cmi_linear_w8a8_workspace_bytes(int M, int N, int K);
+/* 1 where that entry splits K with such a workspace and gains more by it than the quantiser's launch costs, else 0: what a
+ * caller with quantised rows in hand asks before it takes them to cmi_gemm_w8a8, which never splits. */
+int cmi_linear_w8a8_splits(int M, int N, int K);
 int cmi_linear_w8a8_bf16(const void *x, const int8_t *wq, const float *ws, void *y, int M, int N,
                          int K, int ldy, void *workspace, size_t workspace_bytes, void *stream);
 int cmi_linear_w4a8_bf16(const uint8_t *w4, const float *ws, const void *x, void *y, int M, int N,

@@ -5,8 +5,8 @@ from __future__ import annotations
 import pytest
 import torch
 
-from coffin_amd import _native, synth
-from coffin_amd.weights import W4A8Weight
+from coffin_amd import _native, backend, synth
+from coffin_amd.weights import QWeight, W4A8Weight
 from tests import gpu_util as G
 
 pytestmark = pytest.mark.gpu
@@ -328,3 +328,27 @@ def test_w8a8_rows_that_end_inside_a_step(orc, m, n, k):
     xb, y = x.to(G.DEV), torch.empty((m, n), dtype=torch.bfloat16, device=G.DEV)
     _native.check(lib.cmi_linear_w8a8_bf16(G.ptr(xb), G.ptr(wd), G.ptr(wsd), G.ptr(y), m, n, k, n, G.ptr(work), nbytes, G.stream()), "linear")
     assert (G.bits(y) == y_ref).all()
+
+
+@pytest.mark.parametrize("path", ["compiled", "adapters"])
+@pytest.mark.parametrize("rows,k,n", [(64, 2560, 512), (65, 9728, 512), (100, 9728, 2560), (256, 4096, 512), (257, 9728, 2560), (500, 9728, 2560), (500, 2560, 6144),
+                                      (1024, 2048, 256), (1025, 2048, 256)])
+def test_w8a8_rows_are_handed_over_where_k_is_not_split(monkeypatch, rows, k, n, path):
+    """Both sides of the rule at its edges: the bits of the call that quantises the bf16 rows."""
+    g = synth.generator(rows + k)
+    if path == "adapters":
+        for name in backend._HOST_CALLS:
+            monkeypatch.setattr(backend, "_host_" + name, lambda *args: None)
+    used, real = [], backend._rows_quantised
+    monkeypatch.setattr(backend, "_rows_quantised", lambda *args: (used.append(1), real(*args)))
+    q = synth.int8_weight(n, k, g)
+    w = QWeight(q.wq.to(G.DEV), q.scale.to(G.DEV))
+    x = synth.activations(rows, k, g).to(G.DEV)
+    gain = synth.activations(1, k, g)[0].to(G.DEV).contiguous()
+    backend.linear_prefill(w, x)                                   # a quantising consumer has been seen
+    before = _native.load_host().handed_uses()[1]
+    h = backend.rms_norm(x, gain)
+    y = backend.linear_prefill(w, h)
+    taken = len(used) + _native.load_host().handed_uses()[1] - before
+    assert taken == (0 if backend._splits_k(rows, n, k, x.device) else 1)
+    assert torch.equal(y.view(torch.int16), backend.linear_prefill(w, h.clone()).view(torch.int16))
