@@ -28,6 +28,7 @@ SIGNATURES: dict[str, list] = {
     "cmi_gemv_w8a16": [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _vp],
     "cmi_gemv_w8a16_mfma": [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _vp],
     "cmi_linear_w8a16": [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp],
+    "cmi_linear_w8a16_rows": [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _vp],
     "cmi_w4_repack": [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _vp],
     "cmi_gemv_w4a8": [_vp, _vp, _vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp],
     "cmi_gemv_w4a16": [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _vp],

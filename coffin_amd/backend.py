@@ -83,6 +83,10 @@ W4A16_MAX_ROWS = 4
 W4A16_MAX_K = 32768
 #: Rows from which the matrix-pipe GEMV beats the dot-product one (measured on every layer shape).
 MFMA_MIN_ROWS = 3
+#: The same for K that is not whole lines of 128 (2624 -> 9728: the dot-product kernel takes four rows in 8.7 us, the
+#: matrix-pipe one five in 11.4; five take the former 12.0, nine 20.2 against 11.5).  A weight whose family is "mfma" keeps such
+#: rows on the dot-product kernel, single rows included.
+RAGGED_MFMA_MIN_ROWS = 5
 #: ``rms_norm`` / ``add_rms_norm`` / ``silu_mul`` also leave their output rows quantised (int8 +
 #: scale) in private scratch, and a ``linear*`` call on that very output -- W4A8 at any row count,
 #: W8A8 prefill -- takes them from there instead of quantising the bf16 rows again: the
@@ -486,9 +490,12 @@ def _gemv_q8(rec: _Record, act: torch.Tensor, rows: int, out: torch.Tensor, mfma
     or a process whose family is "mfma" uses it for every call, single rows included."""
     n, k = rec.n, rec.k
     whole = rec.family == "mfma" if rec.family is not None else BATCH_MFMA
-    fast = (whole or (mfma and rows >= MFMA_MIN_ROWS)) and k % 128 == 0
-    rc = _native.load().cmi_linear_w8a16(rec.a, rec.b, act.data_ptr(), out.data_ptr(), rows, n, k,
-                                         1 if fast else 0, _stream())
+    if mfma and not whole and k % 128 and k % 16 == 0 and k >= 128 and rows >= RAGGED_MFMA_MIN_ROWS:
+        rc = _native.load().cmi_linear_w8a16_rows(rec.a, rec.b, act.data_ptr(), out.data_ptr(), rows, n, k, _stream())
+    else:
+        fast = (whole or (mfma and rows >= MFMA_MIN_ROWS)) and k % 128 == 0
+        rc = _native.load().cmi_linear_w8a16(rec.a, rec.b, act.data_ptr(), out.data_ptr(), rows, n, k,
+                                             1 if fast else 0, _stream())
     if rc:
         _native.check(rc, "linear_w8a16")
 

@@ -23,6 +23,11 @@
 // summation order), which is why this kernel has an entry point of its own:
 // callers that owe their users "a batched row equals the single-row call"
 // (static-batch decode) stay on cmi_gemv_w8a16.
+//
+// TAIL: rows that end inside a line.  Of the last line the activations past K are zeros that are not read, so what
+// the weight's pieces hold there (bytes of the row again) does not matter.  Against the dot-product kernel, which such rows
+// took at every count, cold weights: 9 rows of 2624 -> 9728 20.9 -> 11.6 us, 63 rows 98 -> 21.5; 16 rows of 9792 -> 2560 36.2 -> 13.9; 50
+// rows of 1344 -> 1000 22.7 -> 9.9; 63 rows of 13888 -> 5120 710 -> 74.
 #include "rows16_tile.hpp"
 
 namespace {
@@ -57,13 +62,21 @@ __device__ __forceinline__ void widen4(uint32_t w, uint32_t &lo, uint32_t &hi) {
     hi = __builtin_amdgcn_perm(__float_as_uint(f3), __float_as_uint(f2), 0x07060302u);
 }
 
+// Sixteen bytes of an activation row: zeros past the row's end (TAIL).
+template <bool TAIL>
+__device__ __forceinline__ v4i32 load_x(const uint8_t *x, int lane, int half, int first_row, int last_row, size_t row_bytes, int byte) {
+    const v4i32 v = *reinterpret_cast<const v4i32 *>(x + tile_src<TAIL>(lane, half, first_row, last_row, row_bytes, byte));
+    const v4i32 zero = {0, 0, 0, 0};
+    return TAIL && byte + (lane & 7) * 16 >= (int)row_bytes ? zero : v;
+}
+
 // NLP: lines per wavefront and round.  WAVES: wavefronts per workgroup.  ROUNDS: 1, or 2 for
 // K above 128*NLP*WAVES (the second round's bytes are requested line by line as the first
 // round frees their registers; asking for all weight bytes at the start took 179 registers
 // and measured slower), or 0: as many rounds as K takes, counted at run time (K above 10240).
 // T: 16-row tiles of weight rows per workgroup (the activation tiles a wavefront fetched and
 // rearranged serve all of them: at 16 rows they are two thirds of the bytes a wavefront asks for).
-template <int NLP, int WAVES, int ROUNDS, int T = 1>
+template <int NLP, int WAVES, int ROUNDS, int T, bool TAIL>
 __global__ void __launch_bounds__(WAVES * 64)
 gemv_w8a16_rows16_kernel(const Args a) {
     static_assert(T == 1 || ROUNDS == 1, "several tiles only in the single-round arrangement");
@@ -75,7 +88,7 @@ gemv_w8a16_rows16_kernel(const Args a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kq = lane >> 4;
     const int n0 = blockIdx.x * (T * ROWS);
-    const int lines = a.K / LINE;
+    const int lines = (a.K + LINE - 1) / LINE;
     uint8_t *wpatch = patches + wave * (PATCH_BYTES + XPATCH_BYTES), *xpatch = wpatch + PATCH_BYTES;
     const uint8_t *xbytes = reinterpret_cast<const uint8_t *>(a.x);
     auto line_of = [&](int r, int i) { return (r * NLP + i) * WAVES + wave; };
@@ -87,7 +100,7 @@ gemv_w8a16_rows16_kernel(const Args a) {
     // One or two activation rows: every lane's row is one of two, so the MFMA arrangement (row
     // lane%16, bytes 64*kq .. +63 of the line) can be loaded as it is -- the requests collapse
     // onto a few cache lines -- and the LDS rearrangement is skipped.
-    const bool direct_x = a.M <= 2;
+    const bool direct_x = !TAIL && a.M <= 2;
     const uint8_t *xdirect = xbytes + (size_t)min(lane & 15, a.M - 1) * a.K * 2 + kq * 64;
     auto request_x = [&](int r, int i) {
         const int line = line_of(r, i);
@@ -100,8 +113,7 @@ gemv_w8a16_rows16_kernel(const Args a) {
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-            xr[i][q] = *reinterpret_cast<const v4i32 *>(
-                xbytes + tile_src(lane, q & 1, 0, a.M - 1, (size_t)a.K * 2, line * 256 + (q >> 1) * 128));
+            xr[i][q] = load_x<TAIL>(xbytes, lane, q & 1, 0, a.M - 1, (size_t)a.K * 2, line * 256 + (q >> 1) * 128);
     };
     auto request_w = [&](int r, int i) {
         const int line = line_of(r, i);
@@ -111,7 +123,7 @@ gemv_w8a16_rows16_kernel(const Args a) {
 #pragma unroll
             for (int h = 0; h < 2; ++h)
                 wr[t][i][h] = __builtin_nontemporal_load(reinterpret_cast<const v4i32 *>(
-                    a.wq + tile_src(lane, h, n0 + t * ROWS, a.N - 1, a.K, line * LINE)));
+                    a.wq + tile_src<TAIL>(lane, h, n0 + t * ROWS, a.N - 1, a.K, line * LINE)));
     };
 #pragma unroll
     for (int i = 0; i < NLP; ++i) request_x(0, i);
@@ -193,13 +205,14 @@ gemv_w8a16_rows16_kernel(const Args a) {
 template <int NLP, int WAVES, int ROUNDS = 1, int T = 1>
 int launch(const Args &a, hipStream_t st) {
     constexpr int LDS_BYTES = WAVES * (T * 1024 + PATCH_BYTES + XPATCH_BYTES);
-    static std::atomic<uint64_t> devices{0};
-    if (const int rc = reserve_lds(reinterpret_cast<const void *>(gemv_w8a16_rows16_kernel<NLP, WAVES, ROUNDS, T>),
-                                   LDS_BYTES, devices, "cmi_gemv_w8a16_mfma"))
-        return rc;
-    const dim3 grid((a.N + T * ROWS - 1) / (T * ROWS));
-    gemv_w8a16_rows16_kernel<NLP, WAVES, ROUNDS, T><<<grid, dim3(WAVES * 64), LDS_BYTES, st>>>(a);
-    return check_launch("cmi_gemv_w8a16_mfma");
+    static std::atomic<uint64_t> devices[2];
+    const auto run = [&](auto kernel, std::atomic<uint64_t> &done) {
+        if (const int rc = reserve_lds(reinterpret_cast<const void *>(kernel), LDS_BYTES, done, "cmi_gemv_w8a16_mfma")) return rc;
+        kernel<<<dim3((a.N + T * ROWS - 1) / (T * ROWS)), dim3(WAVES * 64), LDS_BYTES, st>>>(a);
+        return check_launch("cmi_gemv_w8a16_mfma");
+    };
+    return a.K % LINE == 0 ? run(gemv_w8a16_rows16_kernel<NLP, WAVES, ROUNDS, T, false>, devices[0])
+                           : run(gemv_w8a16_rows16_kernel<NLP, WAVES, ROUNDS, T, true>, devices[1]);
 }
 
 
@@ -215,7 +228,7 @@ constexpr int MAX_CHUNKS = 4;
 // T: 16-row tiles of weight rows per workgroup (single-round arrangements only): every workgroup
 // pulls all activation rows through L2 once per chunk, M * K * 2 bytes times N / (16 T) workgroups,
 // which from three chunks up is what the launch waits for.
-template <int NLP, int WAVES, int ROUNDS, int T = 1>
+template <int NLP, int WAVES, int ROUNDS, int T, bool TAIL>
 __global__ void __launch_bounds__(WAVES * 64)
 gemv_w8a16_rows64_kernel(const Args a) {
     static_assert(T == 1 || ROUNDS == 1, "several tiles only in the single-round arrangement");
@@ -228,7 +241,7 @@ gemv_w8a16_rows64_kernel(const Args a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kq = lane >> 4;
     const int n0 = blockIdx.x * (T * ROWS);
-    const int lines = a.K / LINE;
+    const int lines = (a.K + LINE - 1) / LINE;
     uint8_t *wpatch = patches + wave * (PATCH_BYTES + XPATCH_BYTES), *xpatch = wpatch + PATCH_BYTES;
     const uint8_t *xbytes = reinterpret_cast<const uint8_t *>(a.x);
     auto line_of = [&](int r, int i) { return (r * NLP + i) * WAVES + wave; };
@@ -238,8 +251,7 @@ gemv_w8a16_rows64_kernel(const Args a) {
         const int line = min(line_of(r, i), lines - 1);  // a slot past the last line is not used
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-            xr[i][q] = *reinterpret_cast<const v4i32 *>(
-                xbytes + tile_src(lane, q & 1, c * ROWS, a.M - 1, (size_t)a.K * 2, line * 256 + (q >> 1) * 128));
+            xr[i][q] = load_x<TAIL>(xbytes, lane, q & 1, c * ROWS, a.M - 1, (size_t)a.K * 2, line * 256 + (q >> 1) * 128);
     };
 #pragma unroll
     for (int i = 0; i < NLP; ++i) request_x(0, 0, i);
@@ -253,7 +265,7 @@ gemv_w8a16_rows64_kernel(const Args a) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
                     wr[t][r * NLP + i][h] = __builtin_nontemporal_load(reinterpret_cast<const v4i32 *>(
-                        a.wq + tile_src(lane, h, n0 + t * ROWS, a.N - 1, a.K, line * LINE)));
+                        a.wq + tile_src<TAIL>(lane, h, n0 + t * ROWS, a.N - 1, a.K, line * LINE)));
             }
     // the row scales of the outputs this thread will finish (n depends on the thread and the tile only),
     // requested behind the operands instead of cold at the end
@@ -338,27 +350,140 @@ gemv_w8a16_rows64_kernel(const Args a) {
 template <int NLP, int WAVES, int ROUNDS = 1, int T = 1>
 int launch64(const Args &a, hipStream_t st) {
     constexpr int LDS_MAX = MAX_CHUNKS * T * WAVES * 1024 + WAVES * (PATCH_BYTES + XPATCH_BYTES);
-    static std::atomic<uint64_t> devices{0};
-    if (const int rc = reserve_lds(reinterpret_cast<const void *>(gemv_w8a16_rows64_kernel<NLP, WAVES, ROUNDS, T>),
-                                   LDS_MAX, devices, "cmi_gemv_w8a16_mfma"))
-        return rc;
+    static std::atomic<uint64_t> devices[2];
     const int chunks = (a.M + ROWS - 1) / ROWS;
     const int lds_bytes = chunks * T * WAVES * 1024 + WAVES * (PATCH_BYTES + XPATCH_BYTES);
-    const dim3 grid((a.N + T * ROWS - 1) / (T * ROWS));
-    gemv_w8a16_rows64_kernel<NLP, WAVES, ROUNDS, T><<<grid, dim3(WAVES * 64), lds_bytes, st>>>(a);
-    return check_launch("cmi_gemv_w8a16_mfma");
+    const auto run = [&](auto kernel, std::atomic<uint64_t> &done) {
+        if (const int rc = reserve_lds(reinterpret_cast<const void *>(kernel), LDS_MAX, done, "cmi_gemv_w8a16_mfma")) return rc;
+        kernel<<<dim3((a.N + T * ROWS - 1) / (T * ROWS)), dim3(WAVES * 64), lds_bytes, st>>>(a);
+        return check_launch("cmi_gemv_w8a16_mfma");
+    };
+    return a.K % LINE == 0 ? run(gemv_w8a16_rows64_kernel<NLP, WAVES, ROUNDS, T, false>, devices[0])
+                           : run(gemv_w8a16_rows64_kernel<NLP, WAVES, ROUNDS, T, true>, devices[1]);
+}
+
+// 17..64 rows of more than 80 lines: the weight is asked for once, a round of NLP lines per wavefront at a time, and each
+// round's lines meet every chunk of 16 activation rows before the next round's take their registers, so a row's bits are those of a
+// 16-row call (its lines in the same order).  A launch per 16 rows, which this replaces, read the weight up to four
+// times: 13824 -> 5120, 17 rows 51.6 -> 46.6 us, 32 rows 58.4 -> 47.3, 63 rows 114.5 -> 69.3.
+template <int NLP, int WAVES, int CHUNKS, bool TAIL>
+__global__ void __launch_bounds__(WAVES * 64)
+gemv_w8a16_rows64_long_kernel(const Args a) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    float(*partial)[64][4] = reinterpret_cast<float(*)[64][4]>(lds);  // [CHUNKS * WAVES][64][4]
+    uint8_t *patches = lds + CHUNKS * WAVES * 1024;
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kq = lane >> 4;
+    const int n0 = blockIdx.x * ROWS;
+    const int lines = (a.K + LINE - 1) / LINE, rounds = (lines + NLP * WAVES - 1) / (NLP * WAVES);
+    uint8_t *wpatch = patches + wave * (PATCH_BYTES + XPATCH_BYTES), *xpatch = wpatch + PATCH_BYTES;
+    const uint8_t *xbytes = reinterpret_cast<const uint8_t *>(a.x);
+    auto line_of = [&](int r, int i) { return (r * NLP + i) * WAVES + wave; };
+
+    v4i32 xr[NLP][4], wr[NLP][2];
+    auto request_x = [&](int c, int r, int i) {
+        const int line = min(line_of(r, i), lines - 1);  // a slot past the last line is not used
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            xr[i][q] = load_x<TAIL>(xbytes, lane, q & 1, c * ROWS, a.M - 1, (size_t)a.K * 2, line * 256 + (q >> 1) * 128);
+    };
+    auto request_w = [&](int r, int i) {
+        const int line = min(line_of(r, i), lines - 1);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            wr[i][h] = __builtin_nontemporal_load(
+                reinterpret_cast<const v4i32 *>(a.wq + tile_src<TAIL>(lane, h, n0, a.N - 1, a.K, line * LINE)));
+    };
+#pragma unroll
+    for (int i = 0; i < NLP; ++i) request_x(0, 0, i);
+#pragma unroll
+    for (int i = 0; i < NLP; ++i) request_w(0, i);
+    const float ws_out = a.ws[min(n0 + (int)((threadIdx.x >> 2) & 15), a.N - 1)];
+
+    v4f32 acc[CHUNKS];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) acc[c] = v4f32{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int r = 0; r < rounds; ++r) {
+#pragma unroll
+        for (int i = 0; i < NLP; ++i) {  // weights into the MFMA arrangement, once
+            tile_park(wpatch, lane, wr[i][0], wr[i][1]);
+            wr[i][0] = tile_take(wpatch, lane, 2 * kq);
+            wr[i][1] = tile_take(wpatch, lane, 2 * kq + 1);
+        }
+#pragma unroll
+        for (int c = 0; c < CHUNKS; ++c) {
+#pragma unroll
+            for (int i = 0; i < NLP; ++i) {
+                uint8_t *p = xpatch + (lane >> 3) * XPITCH + (lane & 7) * 16;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) *reinterpret_cast<v4i32 *>(p + (q & 1) * 8 * XPITCH + (q >> 1) * 128) = xr[i][q];
+                const uint8_t *t = xpatch + (lane & 15) * XPITCH + kq * 64;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) xr[i][q] = *reinterpret_cast<const v4i32 *>(t + q * 16);
+            }
+#pragma unroll
+            for (int i = 0; i < NLP; ++i) {
+                if (line_of(r, i) < lines) {  // uniform per wavefront
+                    v4i32 w0 = wr[i][0], w1 = wr[i][1];
+                    asm volatile("" : "+v"(w0), "+v"(w1));  // widened for each chunk: all copies at once would spill
+                    const uint32_t d[8] = {(uint32_t)w0.x, (uint32_t)w0.y, (uint32_t)w0.z, (uint32_t)w0.w,
+                                           (uint32_t)w1.x, (uint32_t)w1.y, (uint32_t)w1.z, (uint32_t)w1.w};
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        uint32_t b[4];
+                        widen4(d[2 * s], b[0], b[1]);
+                        widen4(d[2 * s + 1], b[2], b[3]);
+                        const v4i32 bw = {(int)b[0], (int)b[1], (int)b[2], (int)b[3]};
+                        acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xr[i][s]),
+                                                                         __builtin_bit_cast(bf16x8, bw), acc[c], 0, 0, 0);
+                    }
+                }
+                if (c + 1 < CHUNKS) {
+                    request_x(c + 1, r, i);
+                } else if (r + 1 < rounds) {
+                    request_x(0, r + 1, i);
+                    request_w(r + 1, i);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) *reinterpret_cast<v4f32 *>(&partial[c * WAVES + wave][lane][0]) = acc[c];
+    __syncthreads();
+
+    for (int o = threadIdx.x; o < CHUNKS * 256; o += WAVES * 64) {
+        const int c = o >> 8, l = (o >> 2) & 63, v = o & 3;
+        const int n = n0 + (l & 15), m = c * ROWS + 4 * (l >> 4) + v;
+        if (n < a.N && m < a.M) {
+            float total = partial[c * WAVES][l][v];
+#pragma unroll
+            for (int wv = 1; wv < WAVES; ++wv) total += partial[c * WAVES + wv][l][v];
+            a.y[(size_t)m * a.N + n] = (uint16_t)f32_to_bf16_bits(total * ws_out);
+        }
+    }
+}
+
+template <int CHUNKS>
+int launch64_long(const Args &a, hipStream_t st) {
+    constexpr int NLP = 5, WAVES = 8, LDS_BYTES = CHUNKS * WAVES * 1024 + WAVES * (PATCH_BYTES + XPATCH_BYTES);
+    static std::atomic<uint64_t> devices[2];
+    const auto run = [&](auto kernel, std::atomic<uint64_t> &done) {
+        if (const int rc = reserve_lds(reinterpret_cast<const void *>(kernel), LDS_BYTES, done, "cmi_gemv_w8a16_mfma")) return rc;
+        kernel<<<dim3((a.N + ROWS - 1) / ROWS), dim3(WAVES * 64), LDS_BYTES, st>>>(a);
+        return check_launch("cmi_gemv_w8a16_mfma");
+    };
+    return a.K % LINE == 0 ? run(gemv_w8a16_rows64_long_kernel<NLP, WAVES, CHUNKS, false>, devices[0])
+                           : run(gemv_w8a16_rows64_long_kernel<NLP, WAVES, CHUNKS, true>, devices[1]);
 }
 
 }  // namespace
 
-extern "C" int cmi_gemv_w8a16_mfma(const int8_t *wq, const float *ws, const void *x, void *y, int M, int N,
-                                   int K, void *stream) {
-    CMI_REQUIRE(wq && ws && x && y, CMI_E_ARG, "cmi_gemv_w8a16_mfma: null pointer");
-    CMI_REQUIRE(M >= 1 && M <= MAX_CHUNKS * ROWS, CMI_E_UNSUPPORTED, "cmi_gemv_w8a16_mfma: M=%d outside 1..64", M);
-    CMI_REQUIRE(N >= 1 && K >= 1, CMI_E_ARG, "cmi_gemv_w8a16_mfma: bad shape N=%d K=%d", N, K);
-    CMI_REQUIRE(K % LINE == 0, CMI_E_UNSUPPORTED, "cmi_gemv_w8a16_mfma: K=%d is not a multiple of 128 (use cmi_gemv_w8a16)", K);
-    CMI_REQUIRE(aligned(wq, 16) && aligned(x, 16) && aligned(y, 2) && aligned(ws, 4), CMI_E_ARG,
-                "cmi_gemv_w8a16_mfma: wq and x must be 16-byte aligned");
+namespace {
+
+int run_mfma(const int8_t *wq, const float *ws, const void *x, void *y, int M, int N, int K, void *stream) {
     Args a;
     a.wq = wq;
     a.ws = ws;
@@ -368,19 +493,10 @@ extern "C" int cmi_gemv_w8a16_mfma(const int8_t *wq, const float *ws, const void
     a.N = N;
     a.K = K;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const int lines = K / LINE;
+    const int lines = (K + LINE - 1) / LINE;
     if (lines > 80) {
-        // rows longer than two rounds of registers hold: the 16-row kernel with a round count read at
-        // run time, 16 activation rows per launch (a row's bits are those of a 16-row call, as in the
-        // 64-row kernel; the weight is read once per 16 rows)
-        for (int lo = 0; lo < M; lo += ROWS) {
-            Args part = a;
-            part.x = a.x + (size_t)lo * K;
-            part.y = a.y + (size_t)lo * N;
-            part.M = M - lo < ROWS ? M - lo : ROWS;
-            if (const int rc = launch<5, 8, 0>(part, st)) return rc;
-        }
-        return CMI_OK;
+        // rows longer than two rounds of registers hold: as many rounds as it takes
+        return M <= 16 ? launch<5, 8, 0>(a, st) : M <= 32 ? launch64_long<2>(a, st) : M <= 48 ? launch64_long<3>(a, st) : launch64_long<4>(a, st);
     }
     if (M > ROWS) {
         if (lines <= 8) return launch64<2, 4>(a, st);
@@ -413,4 +529,33 @@ extern "C" int cmi_gemv_w8a16_mfma(const int8_t *wq, const float *ws, const void
     if (lines <= 24) return two ? launch<3, 8, 1, 2>(a, st) : launch<3, 8>(a, st);
     if (lines <= 40) return two ? launch<5, 8, 1, 2>(a, st) : launch<5, 8>(a, st);
     return launch<5, 8, 2>(a, st);
+}
+
+}  // namespace
+
+extern "C" int cmi_gemv_w8a16_mfma(const int8_t *wq, const float *ws, const void *x, void *y, int M, int N,
+                                   int K, void *stream) {
+    CMI_REQUIRE(wq && ws && x && y, CMI_E_ARG, "cmi_gemv_w8a16_mfma: null pointer");
+    CMI_REQUIRE(M >= 1 && M <= MAX_CHUNKS * ROWS, CMI_E_UNSUPPORTED, "cmi_gemv_w8a16_mfma: M=%d outside 1..64", M);
+    CMI_REQUIRE(N >= 1 && K >= 1, CMI_E_ARG, "cmi_gemv_w8a16_mfma: bad shape N=%d K=%d", N, K);
+    CMI_REQUIRE(K % LINE == 0, CMI_E_UNSUPPORTED, "cmi_gemv_w8a16_mfma: K=%d is not a multiple of 128 (use cmi_gemv_w8a16)", K);
+    CMI_REQUIRE(aligned(wq, 16) && aligned(x, 16) && aligned(y, 2) && aligned(ws, 4), CMI_E_ARG,
+                "cmi_gemv_w8a16_mfma: wq and x must be 16-byte aligned");
+    return run_mfma(wq, ws, x, y, M, N, K, stream);
+}
+
+extern "C" int cmi_linear_w8a16_rows(const int8_t *wq, const float *ws, const void *x, void *y, int M, int N, int K, void *stream) {
+    CMI_REQUIRE(M >= 0 && N >= 1 && K >= LINE, CMI_E_ARG, "cmi_linear_w8a16_rows: bad shape M=%d N=%d K=%d", M, N, K);
+    CMI_REQUIRE(K % 16 == 0 && K < 1 << 29, CMI_E_UNSUPPORTED, "cmi_linear_w8a16_rows: K=%d is not a multiple of 16 below 2^29", K);
+    if (M == 0) return CMI_OK;
+    CMI_REQUIRE(wq && ws && x && y, CMI_E_ARG, "cmi_linear_w8a16_rows: null pointer");
+    CMI_REQUIRE(aligned(wq, 16) && aligned(x, 16) && aligned(y, 2) && aligned(ws, 4), CMI_E_ARG,
+                "cmi_linear_w8a16_rows: wq and x must be 16-byte aligned");
+    const uint16_t *xr = static_cast<const uint16_t *>(x);
+    uint16_t *yr = static_cast<uint16_t *>(y);
+    for (int lo = 0; lo < M; lo += MAX_CHUNKS * ROWS) {
+        const int m = M - lo < MAX_CHUNKS * ROWS ? M - lo : MAX_CHUNKS * ROWS;
+        if (const int rc = run_mfma(wq, ws, xr + (size_t)lo * K, yr + (size_t)lo * N, m, N, K, stream)) return rc;
+    }
+    return CMI_OK;
 }

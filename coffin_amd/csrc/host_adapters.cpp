@@ -36,7 +36,7 @@ long long g_handed_uses[2];   // projections that took handed rows: int4 weights
 
 struct Names {
     PyObject *wq, *packed, *scale, *records, *kind, *src, *src2, *a, *b, *n, *k, *kd, *gs, *dev, *family, *index, *device;
-    PyObject *prefill_min, *mfma_min, *batch_mfma, *w8a8_verify, *w4a16, *handover, *handover_min, *handover_max, *seen, *handed;
+    PyObject *prefill_min, *mfma_min, *ragged_min, *batch_mfma, *w8a8_verify, *w4a16, *handover, *handover_min, *handover_max, *seen, *handed;
     PyObject *workspace, *handover_arena, *take, *resolve;
 } N;
 
@@ -426,8 +426,10 @@ PyObject *project(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     at::Tensor y = new_bf16(nd == 1 ? c10::IntArrayRef(size + 1, 1) : c10::IntArrayRef(size, 2), here);
     void *yp = y.mutable_data_ptr();
     const void *xd = x.const_data_ptr();
-    const bool fast = !quantised && K % 128 == 0 &&
-                      ((e.family >= 0 ? e.family == 1 : truth(N.batch_mfma)) || ((flags & MFMA) && rows >= number(N.mfma_min)));
+    const bool whole = e.family >= 0 ? e.family == 1 : truth(N.batch_mfma);
+    const bool fast = !quantised && K % 128 == 0 && (whole || ((flags & MFMA) && rows >= number(N.mfma_min)));
+    // rows that end inside a line of 128
+    const bool ragged = !quantised && !whole && K % 128 != 0 && K % 16 == 0 && K >= 128 && (flags & MFMA) && rows >= number(N.ragged_min);
     int rc;
     const char *what;
     {
@@ -452,7 +454,7 @@ PyObject *project(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
                 rc = cmi_linear_w8a8_bf16(xd, wq, e.b, yp, M, Nn, K, Nn, work, need, stream);
             } else {
                 what = "linear_w8a16";
-                rc = cmi_linear_w8a16(wq, e.b, xd, yp, M, Nn, K, fast ? CMI_FAMILY_MFMA : CMI_FAMILY_DOT, stream);
+                rc = ragged ? cmi_linear_w8a16_rows(wq, e.b, xd, yp, M, Nn, K, stream) : cmi_linear_w8a16(wq, e.b, xd, yp, M, Nn, K, fast ? CMI_FAMILY_MFMA : CMI_FAMILY_DOT, stream);
             }
         }
     }
@@ -671,7 +673,7 @@ PyMODINIT_FUNC PyInit__host(void) {
     } const all[] = {{&N.wq, "wq"}, {&N.packed, "packed"}, {&N.scale, "scale"}, {&N.records, "_RECORDS"}, {&N.kind, "kind"},
                      {&N.src, "src"}, {&N.src2, "src2"}, {&N.a, "a"}, {&N.b, "b"}, {&N.n, "n"}, {&N.k, "k"}, {&N.kd, "kd"},
                      {&N.gs, "gs"}, {&N.dev, "dev"}, {&N.family, "family"}, {&N.index, "index"}, {&N.device, "device"},
-                     {&N.prefill_min, "PREFILL_MIN_ROWS"}, {&N.mfma_min, "MFMA_MIN_ROWS"}, {&N.batch_mfma, "BATCH_MFMA"}, {&N.w8a8_verify, "W8A8_VERIFY"}, {&N.w4a16, "W4A16"},
+                     {&N.prefill_min, "PREFILL_MIN_ROWS"}, {&N.mfma_min, "MFMA_MIN_ROWS"}, {&N.ragged_min, "RAGGED_MFMA_MIN_ROWS"}, {&N.batch_mfma, "BATCH_MFMA"}, {&N.w8a8_verify, "W8A8_VERIFY"}, {&N.w4a16, "W4A16"},
                      {&N.handover, "HANDOVER"}, {&N.handover_min, "HANDOVER_MIN_ROWS"}, {&N.handover_max, "HANDOVER_MAX_BYTES"},
                      {&N.seen, "_QUANT_CONSUMER_SEEN"}, {&N.handed, "_HANDED"},
                      {&N.workspace, "_WORKSPACE"}, {&N.handover_arena, "_HANDOVER_ARENA"}, {&N.take, "take"}, {&N.resolve, "_resolve"}};

@@ -352,3 +352,57 @@ def test_w8a8_rows_are_handed_over_where_k_is_not_split(monkeypatch, rows, k, n,
     taken = len(used) + _native.load_host().handed_uses()[1] - before
     assert taken == (0 if backend._splits_k(rows, n, k, x.device) else 1)
     assert torch.equal(y.view(torch.int16), backend.linear_prefill(w, h.clone()).view(torch.int16))
+
+
+@pytest.mark.parametrize("m,n,k", [(5, 24, 128), (3, 40, 144), (16, 33, 1040), (17, 48, 1104), (33, 100, 2576), (64, 70, 2624), (63, 4808, 2624), (9, 4808, 2672),
+                                   (50, 32784, 1296), (6, 32784, 1296), (49, 60, 5008), (17, 60, 5136), (64, 60, 10192), (16, 40, 10288), (20, 40, 10256),
+                                   (40, 33, 13888), (64, 33, 13824), (65, 20, 20496), (1, 24, 2624)])
+def test_matrix_pipe_rows_that_end_inside_a_line(m, n, k):
+    """Every arrangement of the kernel, with what lies behind a row -- the next row, or NaN behind the last -- kept out of its sums;
+    a row's bits are those of a call of sixteen."""
+    g = synth.generator(m + n + k)
+    q = synth.int8_weight(n, k, g)
+    x = synth.activations(m, k, g, outliers=True)
+    buf = torch.full((m * k + 256,), float("nan"), dtype=torch.bfloat16, device=G.DEV)
+    xd = buf[:m * k].view(m, k)
+    xd.copy_(x)
+    wd, wsd = q.wq.to(G.DEV), q.scale.to(G.DEV)
+    lib = _native.load()
+
+    def call(rows):
+        y = torch.full((rows.shape[0], n), float("nan"), dtype=torch.bfloat16, device=G.DEV)
+        _native.check(lib.cmi_linear_w8a16_rows(G.ptr(wd), G.ptr(wsd), G.ptr(rows), G.ptr(y), rows.shape[0], n, k, G.stream()), "rows")
+        return y
+
+    y = call(xd)
+    exact = (x.double() @ q.wq.double().t()) * q.scale.double()
+    # fp32 sums of K exact products, then bf16: K eps of the sum of magnitudes, half a bf16 step of the result
+    slack = (x.double().abs() @ q.wq.double().abs().t()) * q.scale.double() * (k * 2.0 ** -24)
+    assert ((y.cpu().double() - exact).abs() <= slack + exact.abs() * 2.0 ** -8).all()
+    lo = max(0, m - 16)
+    assert torch.equal(call(xd[lo:])[:, :].view(torch.int16), y[lo:].view(torch.int16))
+    if k % 128 == 0 and m <= 64:
+        ref = torch.empty_like(y)
+        _native.check(lib.cmi_linear_w8a16(G.ptr(wd), G.ptr(wsd), G.ptr(xd), G.ptr(ref), m, n, k, 1, G.stream()), "mfma")
+        assert torch.equal(ref.view(torch.int16), y.view(torch.int16))
+
+
+@pytest.mark.parametrize("path", ["compiled", "adapters"])
+def test_ragged_rows_take_the_matrix_pipe_where_the_call_site_may(monkeypatch, path):
+    if path == "adapters":
+        for name in backend._HOST_CALLS:
+            monkeypatch.setattr(backend, "_host_" + name, lambda *args: None)
+    g = synth.generator(3)
+    k, n = 1344, 200
+    q = synth.int8_weight(n, k, g)
+    w = QWeight(q.wq.to(G.DEV), q.scale.to(G.DEV))
+    lib = _native.load()
+    for rows in (4, 5, 40):
+        x = synth.activations(rows, k, g).to(G.DEV)
+        dot, pipe = (torch.empty((rows, n), dtype=torch.bfloat16, device=G.DEV) for _ in range(2))
+        _native.check(lib.cmi_linear_w8a16(G.ptr(w.wq), G.ptr(w.scale), G.ptr(x), G.ptr(dot), rows, n, k, 0, G.stream()), "dot")
+        _native.check(lib.cmi_linear_w8a16_rows(G.ptr(w.wq), G.ptr(w.scale), G.ptr(x), G.ptr(pipe), rows, n, k, G.stream()), "rows")
+        want = pipe if rows >= 5 else dot
+        assert torch.equal(backend.linear_m_verify(w, x).view(torch.int16), want.view(torch.int16))
+        assert torch.equal(backend.linear_prefill(w, x).view(torch.int16), want.view(torch.int16))
+        assert torch.equal(backend.linear_m(w, x).view(torch.int16), dot.view(torch.int16))
