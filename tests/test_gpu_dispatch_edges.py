@@ -333,8 +333,9 @@ def test_w8a8_rows_that_end_inside_a_step(orc, m, n, k):
 @pytest.mark.parametrize("path", ["compiled", "adapters"])
 @pytest.mark.parametrize("rows,k,n", [(64, 2560, 512), (65, 9728, 512), (100, 9728, 2560), (256, 4096, 512), (257, 9728, 2560), (500, 9728, 2560), (500, 2560, 6144),
                                       (1024, 2048, 256), (1025, 2048, 256)])
-def test_w8a8_rows_are_handed_over_where_k_is_not_split(monkeypatch, rows, k, n, path):
+def test_w8a8_rows_are_handed_over_where_k_is_not_split(request, monkeypatch, rows, k, n, path):
     """Both sides of the rule at its edges: the bits of the call that quantises the bf16 rows."""
+    request.addfinalizer(backend._drop_handed)                     # the adapters' rows are not for the compiled path
     g = synth.generator(rows + k)
     if path == "adapters":
         for name in backend._HOST_CALLS:
