@@ -546,7 +546,8 @@ extern "C" int cmi_gemv_w8a16_mfma(const int8_t *wq, const float *ws, const void
 
 extern "C" int cmi_linear_w8a16_rows(const int8_t *wq, const float *ws, const void *x, void *y, int M, int N, int K, void *stream) {
     CMI_REQUIRE(M >= 0 && N >= 1 && K >= LINE, CMI_E_ARG, "cmi_linear_w8a16_rows: bad shape M=%d N=%d K=%d", M, N, K);
-    CMI_REQUIRE(K % 16 == 0 && K < 1 << 29, CMI_E_UNSUPPORTED, "cmi_linear_w8a16_rows: K=%d is not a multiple of 16 below 2^29", K);
+    // (the bound of cmi_gemv_w8a16, which takes such rows one by one)
+    CMI_REQUIRE(K % 16 == 0 && K <= 1 << 18, CMI_E_UNSUPPORTED, "cmi_linear_w8a16_rows: K=%d is not a multiple of 16 up to 262144", K);
     if (M == 0) return CMI_OK;
     CMI_REQUIRE(wq && ws && x && y, CMI_E_ARG, "cmi_linear_w8a16_rows: null pointer");
     CMI_REQUIRE(aligned(wq, 16) && aligned(x, 16) && aligned(y, 2) && aligned(ws, 4), CMI_E_ARG,
