@@ -26,8 +26,8 @@
 //
 // TAIL: rows that end inside a line.  Of the last line the activations past K are zeros that are not read, so what
 // the weight's pieces hold there (bytes of the row again) does not matter.  Against the dot-product kernel, which such rows
-// took at every count, cold weights: 9 rows of 2624 -> 9728 20.9 -> 11.6 us, 63 rows 98 -> 21.5; 16 rows of 9792 -> 2560 36.2 -> 13.9; 50
-// rows of 1344 -> 1000 22.7 -> 9.9; 63 rows of 13888 -> 5120 710 -> 74.
+// took at every count, cold weights: 9 rows of 2624 -> 9728 21.0 -> 11.7 us, 63 rows 98.9 -> 22.3; 16 rows of 9792 -> 2560 35.2 ->
+// 14.2; 50 rows of 1344 -> 1000 22.1 -> 8.6; 63 rows of 13888 -> 5120 691 -> 78.
 #include "rows16_tile.hpp"
 
 namespace {
@@ -62,6 +62,38 @@ __device__ __forceinline__ void widen4(uint32_t w, uint32_t &lo, uint32_t &hi) {
     hi = __builtin_amdgcn_perm(__float_as_uint(f3), __float_as_uint(f2), 0x07060302u);
 }
 
+// How the sums of a row's lines meet.  A chain of MFMAs is less exact than the dot-product kernel, which the rows that end inside a
+// line left, and which sums in short chains: so for those the MFMAs of a line start from zero and their sums meet in pairs, and where
+// a wavefront has many lines (LOW) what the additions round off is kept and added at the end.  Root mean square error of sums that
+// cancel, in 2^-24 of the sum of magnitudes, K = 960 / 2624 / 9664 / 25536: dot-product kernel 0.053 / 0.046 / 0.031 / 0.021, a chain
+// 0.061 / 0.054 / 0.053 / 0.058, these 0.053 / 0.046 / 0.025 / 0.015 (a kept sum over up to three lines as well: 0.045 at 2624, and 63 rows of 2624 ->
+// 9728 24.9 us instead of 22.1).
+enum Sum { CHAIN, PAIRS, LOW };
+constexpr Sum sum_of(bool tail, int nlp, int rounds) { return !tail ? CHAIN : rounds == 1 && nlp <= 3 ? PAIRS : LOW; }
+
+// The 128 products of a line onto acc: x holds the activations, w0 and w1 the codes in the MFMA arrangement.
+template <Sum S>
+__device__ __forceinline__ void add_line(v4f32 &acc, v4f32 &low, const v4i32 (&x)[4], v4i32 w0, v4i32 w1) {
+    const uint32_t d[8] = {(uint32_t)w0.x, (uint32_t)w0.y, (uint32_t)w0.z, (uint32_t)w0.w,
+                           (uint32_t)w1.x, (uint32_t)w1.y, (uint32_t)w1.z, (uint32_t)w1.w};
+    v4f32 sum[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {  // k = 32*kq + 8*s .. +7 of the line
+        uint32_t b[4];
+        widen4(d[2 * s], b[0], b[1]);
+        widen4(d[2 * s + 1], b[2], b[3]);
+        const v4i32 bw = {(int)b[0], (int)b[1], (int)b[2], (int)b[3]};
+        const v4f32 from = S == CHAIN ? acc : v4f32{0.f, 0.f, 0.f, 0.f};
+        sum[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x[s]), __builtin_bit_cast(bf16x8, bw), from, 0, 0, 0);
+        if (S == CHAIN) acc = sum[s];
+    }
+    if constexpr (S != CHAIN) {
+        const v4f32 line = (sum[0] + sum[1]) + (sum[2] + sum[3]), next = acc + line;
+        if (S == LOW) low += line - (next - acc);
+        acc = next;
+    }
+}
+
 // Sixteen bytes of an activation row: zeros past the row's end (TAIL).
 template <bool TAIL>
 __device__ __forceinline__ v4i32 load_x(const uint8_t *x, int lane, int half, int first_row, int last_row, size_t row_bytes, int byte) {
@@ -80,6 +112,7 @@ template <int NLP, int WAVES, int ROUNDS, int T, bool TAIL>
 __global__ void __launch_bounds__(WAVES * 64)
 gemv_w8a16_rows16_kernel(const Args a) {
     static_assert(T == 1 || ROUNDS == 1, "several tiles only in the single-round arrangement");
+    constexpr Sum SUM = sum_of(TAIL, NLP, ROUNDS);
     extern __shared__ __align__(16) uint8_t lds[];
     float(*partial)[64][4] = reinterpret_cast<float(*)[64][4]>(lds);  // [T * WAVES][64][4]
     uint8_t *patches = lds + T * WAVES * 1024;                            // per wavefront: weights, activations
@@ -137,9 +170,9 @@ gemv_w8a16_rows16_kernel(const Args a) {
     for (int t = 0; t < T; ++t) ws_out[t] = a.ws[min(n0 + t * ROWS + (int)((threadIdx.x >> 2) & 15), a.N - 1)];
 
     // the accumulator of lane l holds (n = l%16, m = 4*kq + v), v = 0..3, per tile
-    v4f32 acc[T];
+    v4f32 acc[T], low[T];
 #pragma unroll
-    for (int t = 0; t < T; ++t) acc[t] = v4f32{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < T; ++t) acc[t] = low[t] = v4f32{0.f, 0.f, 0.f, 0.f};
     const int rounds = ROUNDS > 0 ? ROUNDS : (lines + NLP * WAVES - 1) / (NLP * WAVES);
     constexpr int UNROLL = ROUNDS > 0 ? ROUNDS : 1;
 #pragma unroll UNROLL
@@ -164,17 +197,7 @@ gemv_w8a16_rows16_kernel(const Args a) {
             for (int t = 0; t < T; ++t) {
                 tile_park(wpatch, lane, wr[t][i][0], wr[t][i][1]);
                 const v4i32 w0 = tile_take(wpatch, lane, 2 * kq), w1 = tile_take(wpatch, lane, 2 * kq + 1);
-                const uint32_t d[8] = {(uint32_t)w0.x, (uint32_t)w0.y, (uint32_t)w0.z, (uint32_t)w0.w,
-                                       (uint32_t)w1.x, (uint32_t)w1.y, (uint32_t)w1.z, (uint32_t)w1.w};
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {  // k = 32*kq + 8*s .. +7 of the line
-                    uint32_t b[4];
-                    widen4(d[2 * s], b[0], b[1]);
-                    widen4(d[2 * s + 1], b[2], b[3]);
-                    const v4i32 bw = {(int)b[0], (int)b[1], (int)b[2], (int)b[3]};
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xr[i][s]),
-                                                                     __builtin_bit_cast(bf16x8, bw), acc[t], 0, 0, 0);
-                }
+                add_line<SUM>(acc[t], low[t], xr[i], w0, w1);
             }
             if (r + 1 < rounds) {
                 request_x(r + 1, i);
@@ -183,7 +206,7 @@ gemv_w8a16_rows16_kernel(const Args a) {
         }
     }
 #pragma unroll
-    for (int t = 0; t < T; ++t) *reinterpret_cast<v4f32 *>(&partial[t * WAVES + wave][lane][0]) = acc[t];
+    for (int t = 0; t < T; ++t) *reinterpret_cast<v4f32 *>(&partial[t * WAVES + wave][lane][0]) = SUM == LOW ? acc[t] + low[t] : acc[t];
     __syncthreads();
 
     if (threadIdx.x < 256) {
@@ -232,6 +255,7 @@ template <int NLP, int WAVES, int ROUNDS, int T, bool TAIL>
 __global__ void __launch_bounds__(WAVES * 64)
 gemv_w8a16_rows64_kernel(const Args a) {
     static_assert(T == 1 || ROUNDS == 1, "several tiles only in the single-round arrangement");
+    constexpr Sum SUM = sum_of(TAIL, NLP, ROUNDS);
     extern __shared__ __align__(16) uint8_t lds[];
     float(*partial)[64][4] = reinterpret_cast<float(*)[64][4]>(lds);  // [(chunk * T + tile) * WAVES + wave][64][4]
     const int chunks = (a.M + ROWS - 1) / ROWS;
@@ -284,9 +308,9 @@ gemv_w8a16_rows64_kernel(const Args a) {
 
 #pragma unroll 1
     for (int c = 0; c < chunks; ++c) {
-        v4f32 acc[T];
+        v4f32 acc[T], low[T];
 #pragma unroll
-        for (int t = 0; t < T; ++t) acc[t] = v4f32{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < T; ++t) acc[t] = low[t] = v4f32{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int r = 0; r < ROUNDS; ++r) {
             // this batch of activation lines into the MFMA arrangement: row lane%16, bytes 64*kq .. +63
@@ -309,17 +333,7 @@ gemv_w8a16_rows64_kernel(const Args a) {
                         // with two rounds or several tiles of weight registers the widened copies must
                         // not be kept across chunks (the compiler would hoist them out of the loop and spill)
                         if (ROUNDS > 1 || T > 1) asm volatile("" : "+v"(w0), "+v"(w1));
-                        const uint32_t d[8] = {(uint32_t)w0.x, (uint32_t)w0.y, (uint32_t)w0.z, (uint32_t)w0.w,
-                                               (uint32_t)w1.x, (uint32_t)w1.y, (uint32_t)w1.z, (uint32_t)w1.w};
-#pragma unroll
-                        for (int s = 0; s < 4; ++s) {
-                            uint32_t b[4];
-                            widen4(d[2 * s], b[0], b[1]);
-                            widen4(d[2 * s + 1], b[2], b[3]);
-                            const v4i32 bw = {(int)b[0], (int)b[1], (int)b[2], (int)b[3]};
-                            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xr[i][s]),
-                                                                             __builtin_bit_cast(bf16x8, bw), acc[t], 0, 0, 0);
-                        }
+                        add_line<SUM>(acc[t], low[t], xr[i], w0, w1);
                     }
                 }
                 // this line's activation registers are free: ask for the same slot of the next batch
@@ -328,7 +342,7 @@ gemv_w8a16_rows64_kernel(const Args a) {
             }
         }
 #pragma unroll
-        for (int t = 0; t < T; ++t) *reinterpret_cast<v4f32 *>(&partial[(c * T + t) * WAVES + wave][lane][0]) = acc[t];
+        for (int t = 0; t < T; ++t) *reinterpret_cast<v4f32 *>(&partial[(c * T + t) * WAVES + wave][lane][0]) = SUM == LOW ? acc[t] + low[t] : acc[t];
     }
     __syncthreads();
 
@@ -365,10 +379,11 @@ int launch64(const Args &a, hipStream_t st) {
 // 17..64 rows of more than 80 lines: the weight is asked for once, a round of NLP lines per wavefront at a time, and each
 // round's lines meet every chunk of 16 activation rows before the next round's take their registers, so a row's bits are those of a
 // 16-row call (its lines in the same order).  A launch per 16 rows, which this replaces, read the weight up to four
-// times: 13824 -> 5120, 17 rows 51.6 -> 46.6 us, 32 rows 58.4 -> 47.3, 63 rows 114.5 -> 69.3.
+// times: 13824 -> 5120, 17 rows 50.2 -> 46.1 us, 32 rows 56.8 -> 46.8, 63 rows 112 -> 69.
 template <int NLP, int WAVES, int CHUNKS, bool TAIL>
 __global__ void __launch_bounds__(WAVES * 64)
 gemv_w8a16_rows64_long_kernel(const Args a) {
+    constexpr Sum SUM = sum_of(TAIL, NLP, 0);
     extern __shared__ __align__(16) uint8_t lds[];
     float(*partial)[64][4] = reinterpret_cast<float(*)[64][4]>(lds);  // [CHUNKS * WAVES][64][4]
     uint8_t *patches = lds + CHUNKS * WAVES * 1024;
@@ -402,9 +417,9 @@ gemv_w8a16_rows64_long_kernel(const Args a) {
     for (int i = 0; i < NLP; ++i) request_w(0, i);
     const float ws_out = a.ws[min(n0 + (int)((threadIdx.x >> 2) & 15), a.N - 1)];
 
-    v4f32 acc[CHUNKS];
+    v4f32 acc[CHUNKS], low[CHUNKS];
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) acc[c] = v4f32{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < CHUNKS; ++c) acc[c] = low[c] = v4f32{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
     for (int r = 0; r < rounds; ++r) {
 #pragma unroll
@@ -429,17 +444,7 @@ gemv_w8a16_rows64_long_kernel(const Args a) {
                 if (line_of(r, i) < lines) {  // uniform per wavefront
                     v4i32 w0 = wr[i][0], w1 = wr[i][1];
                     asm volatile("" : "+v"(w0), "+v"(w1));  // widened for each chunk: all copies at once would spill
-                    const uint32_t d[8] = {(uint32_t)w0.x, (uint32_t)w0.y, (uint32_t)w0.z, (uint32_t)w0.w,
-                                           (uint32_t)w1.x, (uint32_t)w1.y, (uint32_t)w1.z, (uint32_t)w1.w};
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        uint32_t b[4];
-                        widen4(d[2 * s], b[0], b[1]);
-                        widen4(d[2 * s + 1], b[2], b[3]);
-                        const v4i32 bw = {(int)b[0], (int)b[1], (int)b[2], (int)b[3]};
-                        acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xr[i][s]),
-                                                                         __builtin_bit_cast(bf16x8, bw), acc[c], 0, 0, 0);
-                    }
+                    add_line<SUM>(acc[c], low[c], xr[i], w0, w1);
                 }
                 if (c + 1 < CHUNKS) {
                     request_x(c + 1, r, i);
@@ -451,7 +456,7 @@ gemv_w8a16_rows64_long_kernel(const Args a) {
         }
     }
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) *reinterpret_cast<v4f32 *>(&partial[c * WAVES + wave][lane][0]) = acc[c];
+    for (int c = 0; c < CHUNKS; ++c) *reinterpret_cast<v4f32 *>(&partial[c * WAVES + wave][lane][0]) = SUM == LOW ? acc[c] + low[c] : acc[c];
     __syncthreads();
 
     for (int o = threadIdx.x; o < CHUNKS * 256; o += WAVES * 64) {
