@@ -94,6 +94,16 @@ __device__ __forceinline__ void add_line(v4f32 &acc, v4f32 &low, const v4i32 (&x
     }
 }
 
+// A wavefront's share of its sums.  One that is infinite stays that: what was kept beside it is a difference of infinities.
+template <Sum S>
+__device__ __forceinline__ v4f32 whole_sum(v4f32 acc, v4f32 low) {
+    if constexpr (S == LOW) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[v] = fabsf(acc[v]) < INFINITY ? acc[v] + low[v] : acc[v];
+    }
+    return acc;
+}
+
 // Sixteen bytes of an activation row: zeros past the row's end (TAIL).
 template <bool TAIL>
 __device__ __forceinline__ v4i32 load_x(const uint8_t *x, int lane, int half, int first_row, int last_row, size_t row_bytes, int byte) {
@@ -206,7 +216,7 @@ gemv_w8a16_rows16_kernel(const Args a) {
         }
     }
 #pragma unroll
-    for (int t = 0; t < T; ++t) *reinterpret_cast<v4f32 *>(&partial[t * WAVES + wave][lane][0]) = SUM == LOW ? acc[t] + low[t] : acc[t];
+    for (int t = 0; t < T; ++t) *reinterpret_cast<v4f32 *>(&partial[t * WAVES + wave][lane][0]) = whole_sum<SUM>(acc[t], low[t]);
     __syncthreads();
 
     if (threadIdx.x < 256) {
@@ -342,7 +352,7 @@ gemv_w8a16_rows64_kernel(const Args a) {
             }
         }
 #pragma unroll
-        for (int t = 0; t < T; ++t) *reinterpret_cast<v4f32 *>(&partial[(c * T + t) * WAVES + wave][lane][0]) = SUM == LOW ? acc[t] + low[t] : acc[t];
+        for (int t = 0; t < T; ++t) *reinterpret_cast<v4f32 *>(&partial[(c * T + t) * WAVES + wave][lane][0]) = whole_sum<SUM>(acc[t], low[t]);
     }
     __syncthreads();
 
@@ -456,7 +466,7 @@ gemv_w8a16_rows64_long_kernel(const Args a) {
         }
     }
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) *reinterpret_cast<v4f32 *>(&partial[c * WAVES + wave][lane][0]) = SUM == LOW ? acc[c] + low[c] : acc[c];
+    for (int c = 0; c < CHUNKS; ++c) *reinterpret_cast<v4f32 *>(&partial[c * WAVES + wave][lane][0]) = whole_sum<SUM>(acc[c], low[c]);
     __syncthreads();
 
     for (int o = threadIdx.x; o < CHUNKS * 256; o += WAVES * 64) {

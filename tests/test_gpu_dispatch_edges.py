@@ -410,6 +410,31 @@ def test_matrix_pipe_sums_of_rows_that_end_inside_a_line_are_as_exact_as_the_dot
     assert rms[1] <= 1.05 * rms[0], rms
 
 
+@pytest.mark.parametrize("m,k", [(9, 2640), (16, 5200), (40, 9664), (9, 13888), (40, 13888)])
+def test_matrix_pipe_sums_of_rows_that_end_inside_a_line_that_are_infinite(m, k):
+    """Infinite activations, and finite ones whose products or sums leave the range, with a NaN row beside them: the infinities,
+    signs and NaN of the dot-product kernel."""
+    n = 48
+    gen = torch.Generator(device=G.DEV).manual_seed(m + k)
+    wq = torch.randint(1, 128, (n, k), dtype=torch.int8, device=G.DEV, generator=gen)
+    wq[1::2] = -wq[1::2]
+    x = torch.randn((m, k), device=G.DEV, generator=gen).to(torch.bfloat16)
+    x[0, 5], x[1, k - 1], x[2, k // 2] = float("inf"), float("-inf"), 3e38
+    x[3, 7::128] = 2e36                                            # a sum that overflows on the way
+    x[4, 3], x[5, 3], x[5, k - 3] = float("nan"), float("inf"), float("-inf")
+    wq[:, 7::128] = wq[:, 7:8]
+    wq[:, 3], wq[:, k // 2] = wq[:, 5], wq[:, 5]
+    wq[:, k - 3] = wq[:, 3]
+    ws = torch.rand(n, device=G.DEV, generator=gen) * 0.01 + 1e-3
+    lib = _native.load()
+    dot, rows = (torch.empty((m, n), dtype=torch.bfloat16, device=G.DEV) for _ in range(2))
+    _native.check(lib.cmi_linear_w8a16(G.ptr(wq), G.ptr(ws), G.ptr(x), G.ptr(dot), m, n, k, 0, G.stream()), "dot")
+    _native.check(lib.cmi_linear_w8a16_rows(G.ptr(wq), G.ptr(ws), G.ptr(x), G.ptr(rows), m, n, k, G.stream()), "rows")
+    assert dot[:2].isinf().all() and dot[4:6].isnan().all() and dot[6:].isfinite().all()
+    for kind in (torch.isposinf, torch.isneginf, torch.isnan):
+        assert torch.equal(kind(rows), kind(dot)), kind
+
+
 @pytest.mark.parametrize("path", ["compiled", "adapters"])
 def test_ragged_rows_take_the_matrix_pipe_where_the_call_site_may(monkeypatch, path):
     if path == "adapters":
