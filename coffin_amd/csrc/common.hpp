@@ -74,6 +74,8 @@ int gemv_w4a8_rows16(const uint8_t *w4, const float *ws, const int8_t *xq, const
 double gemm_w4a8_tile_us(int M, int N, int K, int gs, int *tile);
 double gemm_w4a8_deep_us(int M, int N, int K, int *tile);
 int gemm_w4a8_forced_tile(int option, int gs);
+// gemv_w4a8.hip: whether cmi_gemv_w4a8 gives rows of groups of 128 to a tile of four groups a step, and which.
+bool w4a8_rows_take_tiles(int M, int N, int K, int *tile);
 bool gemm_w4a8_deep_code(int code);
 int gemm_w4a8_tile(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs, void *y, int M, int N,
                    int K, int gs, int tile, void *stream);
