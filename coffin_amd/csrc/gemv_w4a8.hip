@@ -384,16 +384,17 @@ double rows16_us(int M, int N, int K, int gs) {
 
 }  // namespace
 
-// 3..16 rows: the tile GEMM of four groups a step where it is modelled to gain 10 % on the matrix-pipe GEMV, at many outputs or long
-// rows (it splits neither K nor a tile's rows among more workgroups than tiles).  Both models are within 9 % of nine in ten
-// sizes, so a smaller gain is none: of 304 sizes (38 shapes x 3..16 rows, rows quantised in front, every weight cold) some twenty take the tile, 4375 us ->
-// 4295 in all, none slower; asked for 5 % 40 do, 4273 us, up to 7 % slower (16 rows of 1536 -> 20235 9.3 -> 9.9, of 2560 -> 19456 12.4 -> 12.6).
+// 3..16 rows: the tile GEMM of four groups a step where it is modelled to gain 10 % on the matrix-pipe GEMV (5 % at rows of several passes,
+// whose GEMV takes 1.1 times its model: 14 rows of 12672 -> 6358 22.7 -> 20.7 us), at many outputs or long rows (it splits neither K nor a
+// tile's rows among more workgroups than tiles).  Both models are within 9 % of nine in ten sizes, so a smaller gain is none: of 304
+// sizes (38 shapes x 3..16 rows, rows quantised in front, every weight cold) 21 take the tile, 4375 us -> 4295 in all, none slower; asked
+// for 5 % throughout 40 do, 4273 us, up to 7 % slower (16 rows of 1536 -> 20235 9.3 -> 9.9, of 2560 -> 19456 12.4 -> 12.6).
 bool cmi::w4a8_rows_take_tiles(int M, int N, int K, int *tile) {
     if (M < 3 || M > 16) return false;
     const double mb = N * 0.5e-6 * K, k = K * 1e-3, share = M / 16.0, rounds = ceil(N / 4096.0);
     const double t_gemv = K <= 10240 ? 2.64 + mb * (0.1737 + 0.0734 * share) + k * (0.3668 + 0.0093 * share) + 0.048 * rounds
                                      : mb * (0.0997 + 0.0168 * share) + k * (0.4413 + 0.0397 * share) + 3.54 * rounds;
-    return gemm_w4a8_deep_us(M, N, K, tile) < 0.9 * t_gemv;
+    return gemm_w4a8_deep_us(M, N, K, tile) < (K <= 10240 ? 0.9 : 0.95) * t_gemv;
 }
 
 extern "C" int cmi_gemv_w4a8(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs,
