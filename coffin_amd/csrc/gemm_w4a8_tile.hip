@@ -658,16 +658,32 @@ const Cost COSTS[D16x64] = {
 
 // The same for the tiles of four groups a step: fixed part, per step a share of every tile the CU holds, of every round
 // of the workgroups it can hold at a time and of the cold weight, and what a tile and a round cost beside their steps.  Fitted to
-// cold-weight sweeps on fifteen layer shapes x 21 batch sizes (17..1024 rows) and twenty x five (2..16).
+// cold-weight sweeps on fifteen layer shapes x 21 batch sizes (17..1024 rows) and twenty x five (2..16).  A third workgroup
+// fits beside two of the smallest tiles, but takes as long as a round of its own (256 rows of 11008 -> 2700, 680 tiles of 32 x 32: 41.5
+// us, modelled 23.6 with three to a round; 38.8 on 64-row tiles).
 struct DeepCost {
     int bm, bn, per_cu, code;  // code: cmi_set_option("w4_gemm_deep"), rows x 100 + columns, one more for more stages
     double fixed, tile, round, n, tiles, rounds;
 };
 const DeepCost DEEP_COSTS[TILES - D16x64] = {
-    {16, 64, 3, 1664, 1.84, 0.196, 0.297, 0.289, 0.41, 0.28}, {16, 64, 1, 1665, 1.40, 0.463, 0.0, 0.219, 0.0, 1.57},
-    {32, 32, 3, 3232, 1.84, 0.198, 0.273, 0.222, 0.28, 0.52}, {32, 32, 1, 3233, 1.47, 0.452, 0.0, 0.121, 0.0, 1.53},
+    {16, 64, 2, 1664, 1.84, 0.196, 0.297, 0.289, 0.41, 0.28}, {16, 64, 1, 1665, 1.40, 0.463, 0.0, 0.219, 0.0, 1.57},
+    {32, 32, 2, 3232, 1.84, 0.198, 0.273, 0.222, 0.28, 0.52}, {32, 32, 1, 3233, 1.47, 0.452, 0.0, 0.121, 0.0, 1.53},
     {32, 64, 2, 3264, 1.64, 0.266, 0.412, 0.203, 0.31, 0.93}, {32, 64, 1, 3265, 1.41, 0.420, 0.188, 0.165, 0.0, 1.65},
     {48, 64, 1, 4864, 1.37, 0.865, 0.0, 0.180, 0.0, 1.88},
+};
+
+// Both for groups of 256, beyond 16 rows: they flush half as often, which shortens the steps of the wide tiles of one 128 more than the
+// others.  Fitted to sweeps of 52 layer shapes x 16 batch sizes (17..1024 rows, rows quantised in front, every weight cold).
+constexpr int ANY_GROUP = 4;
+const struct { Tile tile; Cost cost; } COSTS_256[ANY_GROUP] = {
+    {T64x128, {64, 128, 4.7938, 0.0351, 0.3903, 0.0588, 0.0133, true}}, {T64x64, {64, 64, 3.9387, 0.0301, 0.2420, 0.0552, 0.0144, true}},
+    {T32x64, {32, 64, 3.3359, 0.0639, 0.1595, 0.0522, 0.0380, true}},   {T16x32, {16, 32, 2.8913, 0.0966, 0.0642, 0.0302, 0.0699, true}},
+};
+const DeepCost DEEP_COSTS_256[TILES - D16x64] = {
+    {16, 64, 3, 1664, 2.048, 0.158, 0.565, 0.347, 0.558, 0.0}, {16, 64, 1, 1665, 1.568, 0.0, 0.520, 0.196, 0.719, 0.948},
+    {32, 32, 2, 3232, 2.469, 0.070, 0.618, 0.179, 0.365, 0.0}, {32, 32, 1, 3233, 1.575, 0.0, 0.491, 0.076, 1.499, 0.194},
+    {32, 64, 2, 3264, 2.101, 0.181, 0.674, 0.170, 0.973, 0.0}, {32, 64, 1, 3265, 1.590, 0.0, 0.681, 0.142, 1.742, 0.0},
+    {48, 64, 1, 4864, 1.385, 0.366, 0.561, 0.079, 2.233, 0.0},
 };
 
 Tile deep_tile(int code) {
@@ -693,19 +709,21 @@ double cost(const Cost &c, int M, int N, int K) {
 
 namespace cmi {
 
-double gemm_w4a8_deep_us(int M, int N, int K, int *tile) {
+static double deep_us(const DeepCost *costs, int tiles, int M, int N, int K, int *tile) {
     const int option = option_w4_gemm_deep();
     if (option > 1) {
         *tile = deep_tile(option);
         return 0.0;
     }
     double best = 1e30;
-    for (int t = 0; option == 0 && K <= 1 << 24 && t < TILES - D16x64; ++t) {  // (longer rows: the tile's offsets are 32-bit)
-        const double us = cost(DEEP_COSTS[t], M, N, K);
+    for (int t = 0; option == 0 && K <= 1 << 24 && t < tiles; ++t) {  // (longer rows: the tile's offsets are 32-bit)
+        const double us = cost(costs[t], M, N, K);
         if (us < best) best = us, *tile = D16x64 + t;
     }
     return best;
 }
+
+double gemm_w4a8_deep_us(int M, int N, int K, int *tile) { return deep_us(DEEP_COSTS, TILES - D16x64, M, N, K, tile); }
 
 double gemm_w4a8_tile_us(int M, int N, int K, int gs, int *tile) {
     double best = 1e30;
@@ -714,15 +732,24 @@ double gemm_w4a8_tile_us(int M, int N, int K, int gs, int *tile) {
         const double us = cost(COSTS[t], M, N, K);
         if (us < best) best = us, *tile = t;
     }
-    // Four groups a step where they are modelled to gain at least 3 %: 315 sizes of 17..1024 rows 6678 -> 5997 us in all (5908
-    // with the best of every size; the worst loss 9 %, 40 rows of 8960 -> 1536 6.0 -> 6.6 us).  The same with groups of 256 (twelve
-    // shapes x fourteen batch sizes; 24 rows of 14336 -> 4096 28.0 -> 16.5 us, 100 rows of 9728 -> 2560 21.6 -> 15.0).  Groups of 64
+    // Four groups a step where they are modelled to gain at least 5 %: of 480 sizes (24 layer shapes x 17..1024 rows, rows
+    // quantised in front, every weight cold) 205 take them, 19128 -> 17972 us in all (17749 with the best of every size), none
+    // more than 2 % slower.  Groups of 256 by costs of their own, with 3 % up to 200 rows and 7 % beyond (416 sizes 20221 -> 18180, 18000
+    // with the best of every size; by the costs above 19067 and up to 30 % slower, 80 rows of 2048 -> 11008 13.5 -> 17.5).  Groups of 64
     // flush twice as often, which costs these tiles 1.35 times their model and the others 1.17: up to 16 rows, where they
     // are modelled to gain more than that (1106 us in all, 1095 with the best of every size, 1230 without them; 16 rows of
     // 5120 -> 32768 28.3 -> 21.1); beyond, the gain is 2 % in all and the model does not find it.
     int deep = 0;
+    if (gs == 256 && M > 16) {
+        for (const auto &c : COSTS_256)
+            if (c.tile == *tile) best = cost(c.cost, M, N, K);
+        // (48 x 64, the last: beyond 150 rows up to 21 % slower than modelled where rows are long, 300 rows of 17920 -> 6617)
+        const double us = deep_us(DEEP_COSTS_256, TILES - D16x64 - (M > 150), M, N, K, &deep);
+        if (us < (M <= 200 ? 0.97 : 0.93) * best) best = us, *tile = deep;
+        return best;
+    }
     const double us = gs == 64 && M > 16 && option_w4_gemm_deep() == 0 ? 1e30 : gemm_w4a8_deep_us(M, N, K, &deep);
-    if (us < (gs == 64 ? 0.82 : 0.97) * best) best = us, *tile = deep;
+    if (us < (gs == 64 ? 0.82 : 0.95) * best) best = us, *tile = deep;
     return best;
 }
 
