@@ -559,6 +559,21 @@ extern "C" int cmi_gemv_w8a16_mfma(const int8_t *wq, const float *ws, const void
     return run_mfma(wq, ws, x, y, M, N, K, stream);
 }
 
+namespace {
+
+// Few outputs of long rows that end inside a line: rows below this go to the dot-product kernel.  A wavefront of this file takes every
+// eighth line of its 16 weight rows, a chain that grows with K alone, while the other kernel has a wavefront for every two weight rows
+// and 4096 k and, up to 16384, the activations of eight rows in LDS.  Cold weights, dot-product against this file's: 5 rows of
+// 12304 -> 300 10.9 us against 15.6, of 16368 -> 800 17.1 / 19.4; 8 rows of 12304 -> 300 15.1 / 15.9, of 9200 -> 300 13.7 / 12.1; 5 rows of
+// 32784 -> 64 29.3 / 33.5; the other way at 5 rows of 16400 -> 300 21.7 / 19.0, of 12304 -> 1200 19.3 / 16.3, of 7184 -> 64 10.0 / 9.7.
+int rows_from(int N, int K) {
+    if (K % LINE == 0 || K <= 8192) return 1;
+    if (K <= 16384) return N <= 512 ? (K >= 12288 ? 9 : 7) : N <= 832 ? 7 : N <= 1024 ? 6 : 1;
+    return K > 20480 && N <= 512 ? 6 : 1;
+}
+
+}  // namespace
+
 extern "C" int cmi_linear_w8a16_rows(const int8_t *wq, const float *ws, const void *x, void *y, int M, int N, int K, void *stream) {
     CMI_REQUIRE(M >= 0 && N >= 1 && K >= LINE, CMI_E_ARG, "cmi_linear_w8a16_rows: bad shape M=%d N=%d K=%d", M, N, K);
     // (the bound of cmi_gemv_w8a16, which takes such rows one by one)
@@ -567,6 +582,7 @@ extern "C" int cmi_linear_w8a16_rows(const int8_t *wq, const float *ws, const vo
     CMI_REQUIRE(wq && ws && x && y, CMI_E_ARG, "cmi_linear_w8a16_rows: null pointer");
     CMI_REQUIRE(aligned(wq, 16) && aligned(x, 16) && aligned(y, 2) && aligned(ws, 4), CMI_E_ARG,
                 "cmi_linear_w8a16_rows: wq and x must be 16-byte aligned");
+    if (M < rows_from(N, K)) return cmi_gemv_w8a16(wq, ws, x, y, M, N, K, stream);
     const uint16_t *xr = static_cast<const uint16_t *>(x);
     uint16_t *yr = static_cast<uint16_t *>(y);
     for (int lo = 0; lo < M; lo += MAX_CHUNKS * ROWS) {

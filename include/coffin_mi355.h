@@ -116,7 +116,9 @@ int cmi_gemv_w8a16_mfma(const int8_t *wq, const float *ws, const void *x, void *
 int cmi_linear_w8a16(const int8_t *wq, const float *ws, const void *x, void *y, int M, int N, int K,
                      int family, void *stream);
 /* The matrix-pipe family for rows that need not be whole lines (K % 16 == 0, 128 <= K <= 262144; the bits of
- * CMI_FAMILY_MFMA where it takes K): what the adapters issue for several rows without the single-row rule (verify, short prefill chunks). */
+ * CMI_FAMILY_MFMA where it takes K): what the adapters issue for several rows without the single-row rule (verify, short prefill
+ * chunks).  Up to 8 rows of at most 1024 outputs whose K is above 8192 and not whole lines go to cmi_gemv_w8a16's kernel where that is
+ * the faster. */
 int cmi_linear_w8a16_rows(const int8_t *wq, const float *ws, const void *x, void *y, int M, int N, int K,
                           void *stream);
 

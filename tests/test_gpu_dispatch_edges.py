@@ -435,6 +435,26 @@ def test_matrix_pipe_sums_of_rows_that_end_inside_a_line_that_are_infinite(m, k)
         assert torch.equal(kind(rows), kind(dot)), kind
 
 
+@pytest.mark.parametrize("m,n,k,dot", [(5, 300, 12304, True), (8, 512, 16368, True), (9, 300, 12304, False), (8, 300, 9200, False), (6, 300, 8208, True),
+                                       (6, 832, 9200, True), (7, 832, 9200, False), (5, 1024, 16368, True), (5, 1025, 16368, False),
+                                       (5, 300, 8176, False), (5, 300, 16400, False), (5, 512, 20496, True), (6, 512, 20496, False)])
+def test_few_outputs_of_long_rows_that_end_inside_a_line(m, n, k, dot):
+    """Both sides of the rule at its edges.  The products cancel to zero, so that a result is what its sum rounded off and the bits say
+    which kernel formed it; at most K eps of the sum of magnitudes."""
+    gen = torch.Generator(device=G.DEV).manual_seed(m + n + k)
+    wq = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=G.DEV, generator=gen)
+    ws = torch.ones(n, device=G.DEV)
+    x = torch.randn((m, k), device=G.DEV, generator=gen).to(torch.bfloat16)
+    order = torch.randperm(k, device=G.DEV, generator=gen)
+    wq[:, order[k // 2:]], x[:, order[k // 2:]] = wq[:, order[:k // 2]], -x[:, order[:k // 2]]
+    lib = _native.load()
+    one, rows = (torch.empty((m, n), dtype=torch.bfloat16, device=G.DEV) for _ in range(2))
+    _native.check(lib.cmi_linear_w8a16(G.ptr(wq), G.ptr(ws), G.ptr(x), G.ptr(one), m, n, k, 0, G.stream()), "dot")
+    _native.check(lib.cmi_linear_w8a16_rows(G.ptr(wq), G.ptr(ws), G.ptr(x), G.ptr(rows), m, n, k, G.stream()), "rows")
+    assert torch.equal(one.view(torch.int16), rows.view(torch.int16)) == dot
+    assert (rows.double().abs() <= (x.double().abs() @ wq.double().abs().t()) * (k * 2.0 ** -24)).all()
+
+
 @pytest.mark.parametrize("path", ["compiled", "adapters"])
 def test_ragged_rows_take_the_matrix_pipe_where_the_call_site_may(monkeypatch, path):
     if path == "adapters":
