@@ -25,10 +25,12 @@ __device__ __forceinline__ float block_max(float v, float *smem) {
     return r;
 }
 
-// How a row of K elements is read, eight at a time.  Whole: K % 8 == 0, rows 16-byte aligned.  Ragged: any K, any
-// alignment of two bytes (a vector load needs no more on gfx950); the elements past K of the last vector are zeros and
+// How a row of K elements is read, eight at a time.  Whole: K % 8 == 0, rows 16-byte aligned (PADDED: rows of q are longer).
+// Ragged: any K, any alignment of two bytes (a vector load needs no more on gfx950); the elements past K of the last vector are zeros and
 // are not read.
+template <bool P>
 struct Whole {
+    static constexpr bool PADDED = P;
     const uint4 *x;
     int nvec;
     __device__ __forceinline__ uint4 load(int row, int idx) const {
@@ -37,6 +39,7 @@ struct Whole {
     __device__ __forceinline__ int vecs() const { return nvec; }
 };
 struct Ragged {
+    static constexpr bool PADDED = true;
     const uint16_t *x;
     int K;
     __device__ __forceinline__ uint4 load(int row, int idx) const {
@@ -57,18 +60,19 @@ struct Ragged {
 };
 
 // VPT > 0: the row fits in VPT vectors per thread and stays in registers; VPT == 0: generic, second pass re-reads.
-// Rows of q have pvec vectors; past the row's own they are zeros, as quant8 makes of zeros under every scale (rows
-// padded to whole groups of an int4 weight).
+// Rows of q have q_vecs vectors where they are padded; past the row's own they are zeros, as quant8 makes of zeros under every scale
+// (rows padded to whole groups of an int4 weight).  Rows that are not know one count: with two in registers every launch took 0.04 us longer
+// (16 x 2560 2.49 -> 2.53).
 // zero / n_zero: a few ints of the caller's that the first workgroup clears on the way (the
 // arrival counters of a split-K GEMM that follows in the stream), or null / 0.
 template <int VPT, typename SRC>
 __global__ void __launch_bounds__(QUANT_THREADS)
-quant_act_i8_vec(const SRC x, uint2 *__restrict__ q, float *__restrict__ s, int pvec, int *__restrict__ zero, int n_zero) {
+quant_act_i8_vec(const SRC x, uint2 *__restrict__ q, float *__restrict__ s, int q_vecs, int *__restrict__ zero, int n_zero) {
     __shared__ float smem[QUANT_THREADS / 64];
     const int row = blockIdx.x;
     if (row == 0)
         for (int i = threadIdx.x; i < n_zero; i += QUANT_THREADS) zero[i] = 0;
-    const int nvec = x.vecs();
+    const int nvec = x.vecs(), pvec = SRC::PADDED ? q_vecs : nvec;
     uint2 *qr = q + (size_t)row * pvec;
     float amax = 0.f;
     if constexpr (VPT > 0) {
@@ -123,9 +127,10 @@ __device__ __forceinline__ float group_max(float v) {
 // 45.9 -> 7.8 us (3.2 TB/s), 8192 x 512 9.0 -> 5.6 us, 3000 x 1024 6.1 -> 4.5 us.  Same arithmetic, same bits.
 template <int LANES, int VPT, int R, typename SRC>
 __global__ void __launch_bounds__(QUANT_THREADS)
-quant_act_i8_rows(const SRC x, uint2 *__restrict__ q, float *__restrict__ s, int pvec, int rows,
+quant_act_i8_rows(const SRC x, uint2 *__restrict__ q, float *__restrict__ s, int q_vecs, int rows,
                   int *__restrict__ zero, int n_zero) {
     constexpr int STEP = QUANT_THREADS / LANES;
+    const int pvec = SRC::PADDED ? q_vecs : x.vecs();
     if (blockIdx.x == 0)
         for (int i = threadIdx.x; i < n_zero; i += QUANT_THREADS) zero[i] = 0;
     const int l = threadIdx.x % LANES;
@@ -213,7 +218,7 @@ int cmi::quant_act_i8_and_clear(const void *x, int8_t *q, float *s, int M, int K
     CMI_REQUIRE(x && q && s, CMI_E_ARG, "cmi_quant_act_i8: null pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (K % 8 == 0 && aligned(x, 16) && aligned(q, 8))
-        launch_vectors(Whole{static_cast<const uint4 *>(x), K / 8}, q, s, M, K / 8, zero, n_zero, st);
+        launch_vectors(Whole<false>{static_cast<const uint4 *>(x), K / 8}, q, s, M, K / 8, zero, n_zero, st);
     else
         quant_act_i8_scalar<<<dim3(M), dim3(QUANT_THREADS), 0, st>>>(static_cast<const uint16_t *>(x), q, s, K, zero, n_zero);
     return check_launch("cmi_quant_act_i8");
@@ -229,7 +234,7 @@ int cmi::quant_act_i8_padded(const void *x, int8_t *q, float *s, int M, int K, i
     CMI_REQUIRE(x && q && s, CMI_E_ARG, "cmi_quant_act_i8: null pointer");
     CMI_REQUIRE(aligned(q, 8), CMI_E_ARG, "cmi_quant_act_i8: rows must be 8-byte aligned");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (K % 8 == 0 && aligned(x, 16)) launch_vectors(Whole{static_cast<const uint4 *>(x), K / 8}, q, s, M, ldq / 8, nullptr, 0, st);
+    if (K % 8 == 0 && aligned(x, 16)) launch_vectors(Whole<true>{static_cast<const uint4 *>(x), K / 8}, q, s, M, ldq / 8, nullptr, 0, st);
     else launch_vectors(Ragged{static_cast<const uint16_t *>(x), K}, q, s, M, ldq / 8, nullptr, 0, st);
     return check_launch("cmi_quant_act_i8");
 }
