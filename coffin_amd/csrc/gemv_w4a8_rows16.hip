@@ -353,7 +353,7 @@ gemv_w4a8_rows16_long_kernel(const Args a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kq = lane >> 4;
     const int n0 = blockIdx.x * ROWS;
-    const int lines = (a.H + 1) / 2;
+    const int halves = LG == 2 ? a.G : a.H, lines = (halves + 1) / 2;
     const int passes = (a.G + LONG_GP - 1) / LONG_GP;
     const int nrows = min(ROWS, a.N - n0);
     uint8_t *patch = patches + wave * PATCH_BYTES;
@@ -369,7 +369,7 @@ gemv_w4a8_rows16_long_kernel(const Args a) {
             if (line >= lines) break;  // uniform per wavefront
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int g = min(2 * line + h, a.H - 1);
+                const int g = min(2 * line + h, halves - 1);
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
                     xa[i][h][j] =
@@ -429,7 +429,7 @@ gemv_w4a8_rows16_long_kernel(const Args a) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int half = 2 * line + h;
-                if (half >= a.H) break;  // uniform per wavefront
+                if (half >= halves) break;  // uniform per wavefront
                 half_sums<LG>(patch, lane, h, xa[i][h], acc, reinterpret_cast<v4i32 *>(sums), half - pass * LONG_HP);
             }
         }
