@@ -585,8 +585,9 @@ int launch_deep(Args &a, hipStream_t st) {
         kernel<<<dim3(a.tiles_m * a.tiles_n), dim3(C::THREADS), C::LDS_BYTES, st>>>(a);
         return check_launch("cmi_gemm_w4a8");
     };
-    return a.tiles_m == 1 ? run(gemm_w4a8_deep_kernel<WM, WN, TM, TN, NST, LG, true>, devices[1])
-                          : run(gemm_w4a8_deep_kernel<WM, WN, TM, TN, NST, LG, false>, devices[0]);
+    if (a.tiles_m == 1) return run(gemm_w4a8_deep_kernel<WM, WN, TM, TN, NST, LG, true>, devices[1]);
+    if constexpr (LG != 1) return run(gemm_w4a8_deep_kernel<WM, WN, TM, TN, NST, LG, false>, devices[0]);
+    return fail(CMI_E_UNSUPPORTED, "cmi_gemm_w4a8: internal dispatch");  // groups of 64: up to 16 rows (gemm_w4a8_tile_us)
 }
 
 template <int WM, int WN, int TM, int TN, int NST, int LG>
@@ -748,7 +749,7 @@ double gemm_w4a8_tile_us(int M, int N, int K, int gs, int *tile) {
         if (us < (M <= 200 ? 0.97 : 0.93) * best) best = us, *tile = deep;
         return best;
     }
-    const double us = gs == 64 && M > 16 && option_w4_gemm_deep() == 0 ? 1e30 : gemm_w4a8_deep_us(M, N, K, &deep);
+    const double us = gs == 64 && M > 16 ? 1e30 : gemm_w4a8_deep_us(M, N, K, &deep);
     if (us < (gs == 64 ? 0.82 : 0.95) * best) best = us, *tile = deep;
     return best;
 }
