@@ -74,6 +74,10 @@ int gemv_w4a8_rows16(const uint8_t *w4, const float *ws, const int8_t *xq, const
 double gemm_w4a8_tile_us(int M, int N, int K, int gs, int *tile);
 double gemm_w4a8_deep_us(int M, int N, int K, int *tile);
 int gemm_w4a8_forced_tile(int option, int gs);
+// gemm_w4a8.hip: the two-stage kernel, which also writes the group sums where they are asked for; K whole steps of 128 and whole
+// groups, arguments already checked, without the sums groups of 64 only.
+int gemm_w4a8_two_stage(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs, void *y, int32_t *group_acc, int M, int N,
+                        int K, int gs, void *stream);
 // gemv_w4a8.hip: whether cmi_gemv_w4a8 gives rows of groups of 128 to a tile of four groups a step, and which.
 bool w4a8_rows_take_tiles(int M, int N, int K, int *tile);
 bool gemm_w4a8_deep_code(int code);

@@ -302,6 +302,33 @@ double two_stage_us(int M, int N, int K) {
 
 }  // namespace
 
+int cmi::gemm_w4a8_two_stage(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs, void *y, int32_t *group_acc, int M,
+                             int N, int K, int gs, void *stream) {
+    Args a;
+    a.xq = xq;
+    a.w4 = w4;
+    a.xs = xs;
+    a.ws = ws;
+    a.y = static_cast<uint16_t *>(y);
+    a.group_acc = group_acc;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.G = K / gs;
+    a.tiles_m = (M + BM - 1) / BM;
+    a.tiles_n = (N + BN - 1) / BN;
+    static std::atomic<uint64_t> devices[4];
+    auto run = [&](auto kernel, int slot) {
+        if (const int rc = reserve_lds(reinterpret_cast<const void *>(kernel), LDS_BYTES, devices[slot], "cmi_gemm_w4a8"))
+            return rc;
+        kernel<<<dim3(a.tiles_m * a.tiles_n), dim3(THREADS), LDS_BYTES, static_cast<hipStream_t>(stream)>>>(a);
+        return check_launch("cmi_gemm_w4a8");
+    };
+    if (!group_acc) return run(gemm_w4a8_two_stage_kernel<1, false>, 0);
+    if (gs == 64) return run(gemm_w4a8_two_stage_kernel<1, true>, 1);
+    return gs == 256 ? run(gemm_w4a8_two_stage_kernel<3, true>, 2) : run(gemm_w4a8_two_stage_kernel<2, true>, 3);
+}
+
 extern "C" int cmi_gemm_w4a8(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs,
                              void *y, int32_t *group_acc, int M, int N, int K, int gs,
                              void *stream) {
@@ -351,27 +378,5 @@ extern "C" int cmi_gemm_w4a8(const uint8_t *w4, const float *ws, const int8_t *x
     const bool two_stage = gs == 64 && (forced ? forced == 128 : two_stage_us(M, N, K) < longer * t_tile);
     if (!group_acc && !two_stage)
         return gemm_w4a8_tile(w4, ws, xq, xs, y, M, N, K, gs, forced ? gemm_w4a8_forced_tile(forced, gs) : tile, stream);
-    Args a;
-    a.xq = xq;
-    a.w4 = w4;
-    a.xs = xs;
-    a.ws = ws;
-    a.y = static_cast<uint16_t *>(y);
-    a.group_acc = group_acc;
-    a.M = M;
-    a.N = N;
-    a.K = K;
-    a.G = K / gs;
-    a.tiles_m = (M + BM - 1) / BM;
-    a.tiles_n = (N + BN - 1) / BN;
-    static std::atomic<uint64_t> devices[4];
-    auto run = [&](auto kernel, int slot) {
-        if (const int rc = reserve_lds(reinterpret_cast<const void *>(kernel), LDS_BYTES, devices[slot], "cmi_gemm_w4a8"))
-            return rc;
-        kernel<<<dim3(a.tiles_m * a.tiles_n), dim3(THREADS), LDS_BYTES, static_cast<hipStream_t>(stream)>>>(a);
-        return check_launch("cmi_gemm_w4a8");
-    };
-    if (!group_acc) return run(gemm_w4a8_two_stage_kernel<1, false>, 0);
-    if (gs == 64) return run(gemm_w4a8_two_stage_kernel<1, true>, 1);
-    return gs == 256 ? run(gemm_w4a8_two_stage_kernel<3, true>, 2) : run(gemm_w4a8_two_stage_kernel<2, true>, 3);
+    return gemm_w4a8_two_stage(w4, ws, xq, xs, y, group_acc, M, N, K, gs, stream);
 }

@@ -24,7 +24,7 @@ using namespace cmi;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int GS = 128;  // group size the fast kernels are built for; the general kernel below also takes 64 and 256
+constexpr int GS = 128;  // group size the fast kernels are built for; the general kernel below also takes 64
 constexpr int FUSED_MAX_ROWS = 4;  // activation rows the fused-quantiser variant takes
 
 struct W4Args {
@@ -48,14 +48,14 @@ struct W4Args {
 // 16-byte vectors per thread and row -- with the arithmetic of the stand-alone
 // quantiser; the bf16 loads are issued before anything else and the weight
 // stream hides the work.  Saves a launch and the int8 round trip through memory.
-// LG: log2(group size / 32) -- 1, 2, 3 for groups of 64, 128, 256: a lane's 16-byte load is 32 k,
-// so 2, 4 or 8 adjacent lanes own a group and their partial sums meet in one, two or three DPP steps.
+// LG: log2(group size / 32) -- 1, 2 for groups of 64, 128: a lane's 16-byte load is 32 k,
+// so 2 or 4 adjacent lanes own a group and their partial sums meet in one or two DPP steps.
 template <int M, int R2, int CH, int XV, int LG = 2>
 __global__ void __launch_bounds__(256)
 gemv_w4a8_kernel(const W4Args a) {
     constexpr int ROWS = 2 * R2;
     constexpr int GPH = 32 >> LG;  // groups per half-wavefront load (32 chunks of 32 k)
-    static_assert(LG >= 1 && LG <= 3 && (LG == 2 || XV == 0), "group sizes 64, 128, 256; the fused quantiser only with 128");
+    static_assert(LG == 2 || (LG == 1 && XV == 0), "group sizes 64 and 128; the fused quantiser only with 128");
     extern __shared__ int32_t sums_base[];  // [fused: M*K int8, M scales, M*4 partial maxima] [teams][groups][ROWS*M]
     int8_t *xq_lds = reinterpret_cast<int8_t *>(sums_base);
     float *xs_lds = reinterpret_cast<float *>(xq_lds + (XV ? (size_t)M * a.K : 0));
@@ -188,7 +188,6 @@ gemv_w4a8_kernel(const W4Args a) {
                         acc = __builtin_amdgcn_sdot4((int)op[i], (int)xv[i], acc, false);
                     acc += dpp_i32<0xB1, 0xf>(acc);                           // quad_perm [1,0,3,2]
                     if constexpr (LG >= 2) acc += dpp_i32<0x4E, 0xf>(acc);    // quad_perm [2,3,0,1]
-                    if constexpr (LG >= 3) acc += dpp_i32<0x141, 0xf>(acc);   // row_half_mirror: the other quad of 8 lanes
                     if ((hl & ((1 << LG) - 1)) == 0 && live[j])
                         team_sums[group * (ROWS * M) + (2 * rr + half) * M + m] = acc;
                 }
@@ -217,7 +216,7 @@ struct Plan {
     int mt, r2, ch, kw, teams, iters;
 };
 
-// lg: log2(group size / 32).  Group sizes other than 128 are served by fewer instantiations (one
+// lg: log2(group size / 32).  Groups of 64 are served by fewer instantiations (one
 // row pair per wavefront, at most two chunks per trip).
 Plan make_plan(int M, int N, int K, int lg) {
     Plan p;
@@ -271,13 +270,13 @@ int launch_xv(const W4Args &a, hipStream_t st) {
     return check_launch("cmi_gemv_w4a8");
 }
 
-// Groups of 64 or 256: quantised activations only, one row pair per wavefront, one or two chunks per trip.
+// Groups of 64: quantised activations only, one row pair per wavefront, one or two chunks per trip.
 template <int M>
-int launch_other_group(const W4Args &a, int ch, int lg, hipStream_t st) {
+int launch_groups_of_64(const W4Args &a, int ch, hipStream_t st) {
     if constexpr (M <= 8) {
-        if (ch == 2) return lg == 1 ? launch_xv<M, 1, 2, 0, 1>(a, st) : launch_xv<M, 1, 2, 0, 3>(a, st);
+        if (ch == 2) return launch_xv<M, 1, 2, 0, 1>(a, st);
     }
-    return lg == 1 ? launch_xv<M, 1, 1, 0, 1>(a, st) : launch_xv<M, 1, 1, 0, 3>(a, st);
+    return launch_xv<M, 1, 1, 0, 1>(a, st);
 }
 
 template <int M, int R2, int CH>
@@ -327,7 +326,7 @@ int run_gemv_w4a8(const char *who, const uint8_t *w4, const float *ws, const int
     CMI_REQUIRE(N >= 1 && K >= gs, CMI_E_ARG, "%s: bad shape N=%d K=%d", who, N, K);
     CMI_REQUIRE(K % gs == 0, CMI_E_UNSUPPORTED, "%s: K=%d is not a multiple of the group size %d (pad the rows with zeros)", who, K, gs);
     CMI_REQUIRE(gs == GS || !xb, CMI_E_UNSUPPORTED, "%s: group size %d takes quantised rows only", who, gs);
-    const int lg = gs == 64 ? 1 : gs == 128 ? 2 : 3;
+    const int lg = gs == 64 ? 1 : 2;  // groups of 256 are whole steps of 128, which cmi_gemv_w4a8 gives to other kernels
     const Plan p = make_plan(M, N, K, lg);
     W4Args a;
     a.w4 = w4;
@@ -350,11 +349,11 @@ int run_gemv_w4a8(const char *who, const uint8_t *w4, const float *ws, const int
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (lg != 2) {
         switch (p.mt) {
-            case 1: return launch_other_group<1>(a, p.ch, lg, st);
-            case 2: return launch_other_group<2>(a, p.ch, lg, st);
-            case 4: return launch_other_group<4>(a, p.ch, lg, st);
-            case 8: return launch_other_group<8>(a, p.ch, lg, st);
-            default: return launch_other_group<16>(a, p.ch, lg, st);
+            case 1: return launch_groups_of_64<1>(a, p.ch, st);
+            case 2: return launch_groups_of_64<2>(a, p.ch, st);
+            case 4: return launch_groups_of_64<4>(a, p.ch, st);
+            case 8: return launch_groups_of_64<8>(a, p.ch, st);
+            default: return launch_groups_of_64<16>(a, p.ch, st);
         }
     }
     switch (p.mt) {
@@ -429,19 +428,18 @@ extern "C" int cmi_gemv_w4a8(const uint8_t *w4, const float *ws, const int8_t *x
     }
     // Groups of 64 and 256.  One row: the dot-product kernel with the chain in registers.  Up to 16: the matrix-pipe GEMV or the tile
     // GEMM, whichever is modelled to be faster (groups of 64: 0.9 for the tiles' model, which is fitted to groups of 128; of
-    // 180 sizes the choice is 7 and 1 % above the best).  The general kernel below keeps calls that ask for
-    // the group sums of several rows and rows that are not whole steps of 128; cold weights, the projection with its quantiser: one
+    // 180 sizes the choice is 7 and 1 % above the best).  The group sums of several rows come from the two-stage GEMM, the general
+    // kernel below keeps rows of groups of 64 that are not whole steps of 128; cold weights, the projection with its quantiser: one
     // row of 2560 -> 19456 17.2 -> 8.4 us (64), 12.9 -> 7.4 (256); 4 rows 27.2 -> 14.3, 23.3 -> 11.4; 16 rows 62.9 -> 14.7, 62.1 ->
     // 13.3; 16 rows of 2560 -> 151936 451 -> 60, 432 -> 51; of 9728 -> 2560 37.6 -> 14.7, 31.9 -> 12.2.
     if ((gs == 64 || gs == 256) && K >= gs && K % GS == 0 && K % gs == 0 && N >= 1 && M >= 1 && M <= 16) {
         int rc = CMI_E_UNSUPPORTED, tile = 0;
         if (M == 1) rc = gemv_w4a8_decode(w4, ws, nullptr, xq, xs, y, group_acc, nullptr, nullptr, M, N, K, gs, stream);
         if (rc != CMI_E_UNSUPPORTED) return rc;
-        if (!group_acc) {
-            if (rows16_us(M, N, K, gs) * (gs == 64 ? 0.9 : 1.0) <= gemm_w4a8_tile_us(M, N, K, gs, &tile))
-                return gemv_w4a8_rows16(w4, ws, xq, xs, nullptr, y, nullptr, nullptr, nullptr, M, N, K, gs, stream);
-            return gemm_w4a8_tile(w4, ws, xq, xs, y, M, N, K, gs, tile, stream);
-        }
+        if (group_acc) return gemm_w4a8_two_stage(w4, ws, xq, xs, y, group_acc, M, N, K, gs, stream);
+        if (rows16_us(M, N, K, gs) * (gs == 64 ? 0.9 : 1.0) <= gemm_w4a8_tile_us(M, N, K, gs, &tile))
+            return gemv_w4a8_rows16(w4, ws, xq, xs, nullptr, y, nullptr, nullptr, nullptr, M, N, K, gs, stream);
+        return gemm_w4a8_tile(w4, ws, xq, xs, y, M, N, K, gs, tile, stream);
     }
     return run_gemv_w4a8("cmi_gemv_w4a8", w4, ws, xq, xs, nullptr, nullptr, nullptr, y, group_acc, M, N, K, gs,
                          stream);
