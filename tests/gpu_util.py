@@ -121,3 +121,13 @@ def gemv_w4a16(w4, ws, x, k, gs=128):
     y = torch.empty(n, dtype=torch.bfloat16, device=DEV)
     _native.check(_native.load().cmi_gemv_w4a16(ptr(w4), ptr(ws), ptr(x), ptr(y), n, k, gs, stream()), "gemv_w4a16")
     return y
+
+
+def chosen_tile(symbol: str, *size: int):
+    """Result and tile of one of the library's own choices between int4 kernels (plain host functions of its C++ side, which run
+    without a GPU); tiles of four groups a step count from 8."""
+    tile = ctypes.c_int(-1)
+    fn = getattr(_native.load(), symbol)
+    fn.argtypes = [ctypes.c_int] * len(size) + [ctypes.POINTER(ctypes.c_int)]
+    fn.restype = ctypes.c_bool if "take" in symbol else ctypes.c_double
+    return fn(*size, ctypes.byref(tile)), tile.value

@@ -249,9 +249,13 @@ def test_one_row_of_other_groups_off_a_16_byte_boundary(orc, gs):
     assert (G.bits(y) == y_ref).all()
 
 
-@pytest.mark.parametrize("m,n,k", [(16, 12288, 4096), (4, 24000, 768), (9, 5120, 25600), (40, 2560, 9728), (70, 6144, 2560), (200, 2560, 9728)])
+@pytest.mark.parametrize("m,n,k", [(16, 12288, 4096), (16, 32768, 5120), (12, 4273, 11264), (40, 2560, 9728), (70, 6144, 2560), (200, 2560, 9728)])
 def test_w4a8_rows_through_the_chosen_tile(m, n, k):
     """Sizes where the choice is a tile of four groups a step: the results of the kernels without them."""
+    if m <= 16:
+        assert G.chosen_tile("_ZN3cmi20w4a8_rows_take_tilesEiiiPi", m, n, k)[0]
+    else:
+        assert G.chosen_tile("_ZN3cmi17gemm_w4a8_tile_usEiiiiPi", m, n, k, 128)[1] >= 8
     gen = torch.Generator(device=G.DEV).manual_seed(m + n + k)
     w4 = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=G.DEV, generator=gen)
     ws = torch.rand((n, k // 128), device=G.DEV, generator=gen) * 0.01 + 1e-4
@@ -306,10 +310,11 @@ def _with_neighbours(a: torch.Tensor) -> torch.Tensor:
 
 
 @pytest.mark.parametrize("m,n,k", [(3, 40, 144), (16, 33, 2064), (17, 8, 240), (31, 530, 1232), (70, 200, 9664), (100, 300, 10256), (129, 161, 208),
-                                   (200, 520, 192), (260, 264, 1040), (300, 2560, 2496), (577, 650, 320)])
+                                   (200, 520, 192), (260, 264, 1040), (300, 2560, 2496), (577, 650, 320), (200, 2560, 9664), (300, 2560, 9664)])
 def test_w8a8_rows_that_end_inside_a_step(orc, m, n, k):
-    """K of 16 .. 112 more than whole steps of 128: the library's choice (up to 16 rows, 17..256, beyond), then every tile,
-    with and without room to split K; beyond a row's end lie other rows' values."""
+    """K of 16 .. 112 more than whole steps of 128: the library's choice (up to 16 rows, 17..256, beyond), then every tile (320 names
+    the 256 x 256 one at such K), then with room to split K, which each of the three split tiles does at one size: 64 x 64, 128 x 64
+    and 128 x 128.  Beyond a row's end lie other rows' values."""
     g = synth.generator(m + n + k)
     q = synth.int8_weight(n, k, g)
     x = synth.activations(m, k, g, outliers=True)
@@ -328,6 +333,8 @@ def test_w8a8_rows_that_end_inside_a_step(orc, m, n, k):
     xb, y = x.to(G.DEV), torch.empty((m, n), dtype=torch.bfloat16, device=G.DEV)
     _native.check(lib.cmi_linear_w8a8_bf16(G.ptr(xb), G.ptr(wd), G.ptr(wsd), G.ptr(y), m, n, k, n, G.ptr(work), nbytes, G.stream()), "linear")
     assert (G.bits(y) == y_ref).all()
+    partials = work[int(lib.cmi_linear_workspace_bytes(m, k)) + 1024:]         # behind the rows, their scales and the arrival counters
+    assert bool((partials != 0xA5).any()) == ((m, n, k) in ((100, 300, 10256), (200, 2560, 9664), (300, 2560, 9664)))
 
 
 @pytest.mark.parametrize("path", ["compiled", "adapters"])
@@ -380,8 +387,11 @@ def test_matrix_pipe_rows_that_end_inside_a_line(m, n, k):
     # fp32 sums of K exact products, then bf16: K eps of the sum of magnitudes, half a bf16 step of the result
     slack = (x.double().abs() @ q.wq.double().abs().t()) * q.scale.double() * (k * 2.0 ** -24)
     assert ((y.cpu().double() - exact).abs() <= slack + exact.abs() * 2.0 ** -8).all()
-    lo = max(0, m - 16)
-    assert torch.equal(call(xd[lo:])[:, :].view(torch.int16), y[lo:].view(torch.int16))
+    if m < 16:
+        more = synth.activations(16 - m, k, g).to(G.DEV)
+        assert torch.equal(call(torch.cat([xd, more]))[:m].view(torch.int16), y.view(torch.int16))
+    for lo in {*range(0, m - 15, 16), m - 16} if m > 16 else ():
+        assert torch.equal(call(xd[lo:lo + 16].contiguous()).view(torch.int16), y[lo:lo + 16].view(torch.int16)), lo
     if k % 128 == 0 and m <= 64:
         ref = torch.empty_like(y)
         _native.check(lib.cmi_linear_w8a16(G.ptr(wd), G.ptr(wsd), G.ptr(xd), G.ptr(ref), m, n, k, 1, G.stream()), "mfma")

@@ -16,6 +16,7 @@ import torch
 from coffin_amd import _native, backend, contract, embed, gemv, synth
 from coffin_amd.weights import (QWeight, W4A8Weight, dequantize_projection,
                                 quantize_projection)
+from tests import gpu_util as G
 
 ROOT = Path(__file__).resolve().parent.parent
 
@@ -419,22 +420,13 @@ def test_entry_points_reject_bad_arguments_before_touching_the_device():
         _native.check(lib.cmi_gemv_w8a16(one, one, one, one, 0, 8, 16, null), "gemv")
 
 
-def _chosen_tile(symbol: str, *size: int):
-    """Result and tile of one of the library's own choices between int4 kernels (plain host functions of its C++ side)."""
-    tile = ctypes.c_int(-1)
-    fn = getattr(_native.load(), symbol)
-    fn.argtypes = [ctypes.c_int] * len(size) + [ctypes.POINTER(ctypes.c_int)]
-    fn.restype = ctypes.c_bool if "take" in symbol else ctypes.c_double
-    return fn(*size, ctypes.byref(tile)), tile.value
-
-
 @pytest.mark.parametrize("m,n,k,tiles", [(16, 19456, 2560, False), (14, 19456, 2560, False), (12, 20235, 1536, False), (16, 7793, 512, False),
                                          (14, 47028, 1280, False), (9, 5120, 25600, False), (4, 24000, 768, False), (16, 2560, 9728, False),
                                          (2, 151936, 2560, False), (17, 151936, 2560, False), (16, 151936, 2560, True), (16, 12288, 4096, True),
                                          (16, 32768, 5120, True)])
 def test_int4_rows_take_tiles_only_where_they_gain_more_than_the_models_err(m, n, k, tiles):
     """Sizes measured a few per cent either way stay on the GEMV."""
-    assert _chosen_tile("_ZN3cmi20w4a8_rows_take_tilesEiiiPi", m, n, k)[0] == tiles
+    assert G.chosen_tile("_ZN3cmi20w4a8_rows_take_tilesEiiiPi", m, n, k)[0] == tiles
 
 
 @pytest.mark.parametrize("m,n,k,gs,tile", [(256, 2700, 11008, 128, 12), (150, 4245, 3840, 128, 12), (64, 9393, 3328, 128, 0), (80, 11008, 2048, 256, 0),
@@ -444,5 +436,5 @@ def test_int4_rows_take_tiles_only_where_they_gain_more_than_the_models_err(m, n
 def test_int4_tiles_of_four_groups_a_step_where_they_are_the_faster_ones(m, n, k, gs, tile):
     """Sizes measured at least 4 % in favour of the side they are on: a tile of one group a step (the first eight: 0 here), or the
     one of four groups that was the fastest or within 5 % of it."""
-    chosen = _chosen_tile("_ZN3cmi17gemm_w4a8_tile_usEiiiiPi", m, n, k, gs)[1]
+    chosen = G.chosen_tile("_ZN3cmi17gemm_w4a8_tile_usEiiiiPi", m, n, k, gs)[1]
     assert (chosen if chosen >= 8 else 0) == tile
