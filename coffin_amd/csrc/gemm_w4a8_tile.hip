@@ -659,16 +659,14 @@ const Cost COSTS[D16x64] = {
 
 // The same for the tiles of four groups a step: fixed part, per step a share of every tile the CU holds, of every round
 // of the workgroups it can hold at a time and of the cold weight, and what a tile and a round cost beside their steps.  Fitted to
-// cold-weight sweeps on fifteen layer shapes x 21 batch sizes (17..1024 rows) and twenty x five (2..16).  A third workgroup
-// fits beside two of the smallest tiles, but takes as long as a round of its own (256 rows of 11008 -> 2700, 680 tiles of 32 x 32: 41.5
-// us, modelled 23.6 with three to a round; 38.8 on 64-row tiles).
+// cold-weight sweeps on fifteen layer shapes x 21 batch sizes (17..1024 rows) and twenty x five (2..16).
 struct DeepCost {
     int bm, bn, per_cu, code;  // code: cmi_set_option("w4_gemm_deep"), rows x 100 + columns, one more for more stages
     double fixed, tile, round, n, tiles, rounds;
 };
 const DeepCost DEEP_COSTS[TILES - D16x64] = {
-    {16, 64, 2, 1664, 1.84, 0.196, 0.297, 0.289, 0.41, 0.28}, {16, 64, 1, 1665, 1.40, 0.463, 0.0, 0.219, 0.0, 1.57},
-    {32, 32, 2, 3232, 1.84, 0.198, 0.273, 0.222, 0.28, 0.52}, {32, 32, 1, 3233, 1.47, 0.452, 0.0, 0.121, 0.0, 1.53},
+    {16, 64, 3, 1664, 1.84, 0.196, 0.297, 0.289, 0.41, 0.28}, {16, 64, 1, 1665, 1.40, 0.463, 0.0, 0.219, 0.0, 1.57},
+    {32, 32, 3, 3232, 1.84, 0.198, 0.273, 0.222, 0.28, 0.52}, {32, 32, 1, 3233, 1.47, 0.452, 0.0, 0.121, 0.0, 1.53},
     {32, 64, 2, 3264, 1.64, 0.266, 0.412, 0.203, 0.31, 0.93}, {32, 64, 1, 3265, 1.41, 0.420, 0.188, 0.165, 0.0, 1.65},
     {48, 64, 1, 4864, 1.37, 0.865, 0.0, 0.180, 0.0, 1.88},
 };
@@ -693,9 +691,12 @@ Tile deep_tile(int code) {
     return static_cast<Tile>(D16x64 + t);
 }
 
+// (Beyond 16 rows a third workgroup of the smallest tiles fits beside two, but between two and three tiles to a CU it takes as long as a round
+// of its own: 256 rows of 11008 -> 2700, 680 tiles of 32 x 32, 41.5 us, modelled 23.6 with three to a round, 38.8 on 64-row tiles.  Up to 16
+// rows it does so at some sizes and not at others -- 9 rows of 4096 -> 37022 20.2 us as modelled, of 7296 -> 34372 43 (GEMV 25 and 39).)
 double cost(const DeepCost &c, int M, int N, int K) {
     const double steps = (K + U * BK - 1) / (U * BK), r = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) / 256.0;
-    const double held = r <= 6 ? ceil(r) : r + 0.5, rounds = ceil(r / c.per_cu);
+    const double held = r <= 6 ? ceil(r) : r + 0.5, rounds = fmax(ceil(r / c.per_cu), M > 16 ? fmin(2.0, ceil(r / 2)) : 1.0);
     return c.fixed + steps * (c.tile * held + c.round * rounds + c.n * N * 1e-4) + c.tiles * held + c.rounds * rounds;
 }
 
@@ -733,9 +734,10 @@ double gemm_w4a8_tile_us(int M, int N, int K, int gs, int *tile) {
         const double us = cost(COSTS[t], M, N, K);
         if (us < best) best = us, *tile = t;
     }
-    // Four groups a step where they are modelled to gain at least 5 %: of 480 sizes (24 layer shapes x 17..1024 rows, rows
-    // quantised in front, every weight cold) 205 take them, 19128 -> 17972 us in all (17749 with the best of every size), none
-    // more than 2 % slower.  Groups of 256 by costs of their own, with 3 % up to 200 rows and 7 % beyond (416 sizes 20221 -> 18180, 18000
+    // Four groups a step where they are modelled to gain at least 5 %, or to lose at most 5 % on 16 x 32 tiles, which take up to 1.5
+    // times their model at long rows (35 rows of 17920 -> 1582 38.6 us against 25.1): of 480 sizes (24 layer shapes x 17..1024 rows, rows
+    // quantised in front, every weight cold) 19128 us without them, 17929 with, 17749 with the best of every size, none more than 2 %
+    // slower.  Groups of 256 by costs of their own, with 3 % up to 200 rows and 7 % beyond (416 sizes 20221 -> 18160, 17970
     // with the best of every size; by the costs above 19067 and up to 30 % slower, 80 rows of 2048 -> 11008 13.5 -> 17.5).  Groups of 64
     // flush twice as often, which costs these tiles 1.35 times their model and the others 1.17: up to 16 rows, where they
     // are modelled to gain more than that (1106 us in all, 1095 with the best of every size, 1230 without them; 16 rows of
@@ -745,12 +747,12 @@ double gemm_w4a8_tile_us(int M, int N, int K, int gs, int *tile) {
         for (const auto &c : COSTS_256)
             if (c.tile == *tile) best = cost(c.cost, M, N, K);
         // (48 x 64, the last: beyond 150 rows up to 21 % slower than modelled where rows are long, 300 rows of 17920 -> 6617)
-        const double us = deep_us(DEEP_COSTS_256, TILES - D16x64 - (M > 150), M, N, K, &deep);
+        const double us = deep_us(DEEP_COSTS_256, TILES - D16x64 - (M > 150 && K > 10240), M, N, K, &deep);
         if (us < (M <= 200 ? 0.97 : 0.93) * best) best = us, *tile = deep;
         return best;
     }
     const double us = gs == 64 && M > 16 ? 1e30 : gemm_w4a8_deep_us(M, N, K, &deep);
-    if (us < (gs == 64 ? 0.82 : 0.95) * best) best = us, *tile = deep;
+    if (us < (gs == 64 ? 0.82 : M > 16 && *tile == T16x32 ? 1.05 : 0.95) * best) best = us, *tile = deep;
     return best;
 }
 

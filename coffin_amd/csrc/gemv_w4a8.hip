@@ -383,17 +383,25 @@ double rows16_us(int M, int N, int K, int gs) {
 
 }  // namespace
 
-// 3..16 rows: the tile GEMM of four groups a step where it is modelled to gain 10 % on the matrix-pipe GEMV (5 % at rows of several passes,
-// whose GEMV takes 1.1 times its model: 14 rows of 12672 -> 6358 22.7 -> 20.7 us), at many outputs or long rows (it splits neither K nor a
-// tile's rows among more workgroups than tiles).  Both models are within 9 % of nine in ten sizes, so a smaller gain is none: of 304
-// sizes (38 shapes x 3..16 rows, rows quantised in front, every weight cold) 21 take the tile, 4375 us -> 4295 in all, none slower; asked
-// for 5 % throughout 40 do, 4273 us, up to 7 % slower (16 rows of 1536 -> 20235 9.3 -> 9.9, of 2560 -> 19456 12.4 -> 12.6).
+// 3..16 rows: the tile GEMM of four groups a step where it is modelled to gain 5 % on the matrix-pipe GEMV (10 % up to 2560, where a tile
+// takes 1.1 times its model; to lose 10 % beyond 10240, where the GEMV takes up to 1.15 times its own: 15 rows of 10496 -> 5633 19.3 us against
+// 17.5), at many outputs or long rows: it splits neither K nor a tile's rows among more workgroups than tiles, and
+// the GEMV's workgroups hold a row's group sums in LDS, which leaves a CU one or two of them at long rows.  The GEMV's model is fitted to
+// 744 sizes (126 shapes x 3..16 rows, rows quantised in front, every weight cold), nine in ten within 10 %; the choice takes 10464 us in
+// all, the GEMV alone 10966, the better of the two 10423, with up to 8 % lost at one size in a hundred.  By 5 % throughout and a model
+// without the LDS it was 10618: 16 rows of 1536 -> 20235 9.9 us on tiles (GEMV 9.3), of 2560 -> 19456 12.6 (12.4).
 bool cmi::w4a8_rows_take_tiles(int M, int N, int K, int *tile) {
     if (M < 3 || M > 16) return false;
-    const double mb = N * 0.5e-6 * K, k = K * 1e-3, share = M / 16.0, rounds = ceil(N / 4096.0);
-    const double t_gemv = K <= 10240 ? 2.64 + mb * (0.1737 + 0.0734 * share) + k * (0.3668 + 0.0093 * share) + 0.048 * rounds
-                                     : mb * (0.0997 + 0.0168 * share) + k * (0.4413 + 0.0397 * share) + 3.54 * rounds;
-    return gemm_w4a8_deep_us(M, N, K, tile) < (K <= 10240 ? 0.9 : 0.95) * t_gemv;
+    const double mb = N * 0.5e-6 * K, k = K * 1e-3, share = M / 16.0, wgs = (N + 15) / 16;
+    double t_gemv;
+    if (K <= 10240) {
+        const int lines = (K / 128 + 1) / 2, waves = lines > 20 || (wgs <= 640 && lines >= 8) ? 8 : 4;
+        const int by_lds = 163840 / (K / 128 * 1088 + waves * 2304), per_cu = by_lds < 32 / waves ? by_lds : 32 / waves;
+        t_gemv = 2.73 + fmax(1.0, wgs / (256.0 * per_cu)) * 0.1494 * k + 0.2402 * k + mb * (0.1824 + 0.0667 * share);
+    } else {
+        t_gemv = 1.43 + ceil(wgs / 512) * ceil(K / 6144.0) * 0.8303 + 0.3437 * k + mb * (0.1787 + 0.0466 * share);
+    }
+    return gemm_w4a8_deep_us(M, N, K, tile) < (K <= 2560 ? 0.9 : K <= 10240 ? 0.95 : 1.1) * t_gemv;
 }
 
 extern "C" int cmi_gemv_w4a8(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs,

@@ -249,7 +249,7 @@ def test_one_row_of_other_groups_off_a_16_byte_boundary(orc, gs):
     assert (G.bits(y) == y_ref).all()
 
 
-@pytest.mark.parametrize("m,n,k", [(16, 12288, 4096), (16, 32768, 5120), (12, 4273, 11264), (40, 2560, 9728), (70, 6144, 2560), (200, 2560, 9728)])
+@pytest.mark.parametrize("m,n,k", [(16, 12288, 4096), (16, 32768, 5120), (5, 24238, 9728), (40, 2560, 9728), (70, 6144, 2560), (200, 2560, 9728)])
 def test_w4a8_rows_through_the_chosen_tile(m, n, k):
     """Sizes where the choice is a tile of four groups a step: the results of the kernels without them."""
     if m <= 16:
