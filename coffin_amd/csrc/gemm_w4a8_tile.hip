@@ -373,7 +373,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_tile_kernel(const A
 // What bounds it.  With a tile or two per CU the kernel above is a chain of K / 128 steps of 0.27 us whatever is in them:
 // the barrier, the trip to LDS for the next fragments and one wavefront per SIMD with 40 vector instructions to issue.
 // Here a barrier buys four groups: 0.6 .. 0.9 us per step of 512 k, of which, taken apart for 100 rows of 9728 -> 2560 (32
-// x 64 tiles, 20.6 us in all with the quantiser), the operands' way from L2 to LDS takes 10 us (62 B/ns per CU of the 75 that
+// x 64 tiles, 20.1 us in all with the quantiser), the operands' way from L2 to LDS takes 10 us (62 B/ns per CU of the 75 that
 // such loads reach) and fragments and arithmetic 10, half of it hidden under the other.
 //
 // A row's 512 (activations) or 256 (packed weight) bytes of a step are requested together and lie together in LDS, 16-byte
@@ -389,9 +389,10 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_w4a8_tile_kernel(const A
 //
 // ONCE: a single tile of rows, so that every weight byte is read by one workgroup and need not stay in the caches.
 //
-// Cold weights, with the quantiser: 100 rows of 9728 -> 2560 29.2 -> 20.6 us, 40 rows 23.8 -> 16.7, 200 rows 34.6 ->
-// 27.1; 100 rows of 4096 -> 2560 14.3 -> 10.8; 40 rows of 25600 -> 5120 60.7 -> 39.6; 16 rows of 2560 -> 151936 54.3 -> 48.7,
-// of 4096 -> 12288 12.1 -> 9.2 (both against the matrix-pipe GEMV).
+// Cold weights, with the quantiser in front (2.5 us at 16 x 4096, 4.7 at 100 x 9728): 100 rows of 9728 -> 2560 28.7 -> 20.1 us, 40
+// rows 23.3 -> 16.3, 200 rows 33.7 -> 26.4; 100 rows of 4096 -> 2560 15.1 -> 11.6; 40 rows of 25600 -> 5120 59.5 -> 38.4; 16 rows of
+// 2560 -> 151936 54.6 -> 51.3, of 4096 -> 12288 14.6 -> 12.9 (both against the matrix-pipe GEMV); groups of 256, 100 rows of 9728 ->
+// 2560 28.4 -> 19.8, 24 rows of 14336 -> 4096 32.1 -> 21.0.
 constexpr int NT = 2;  // cache policy of a load: nontemporal
 constexpr int U = 4, X_ROW = U * BK, P_ROW = U * BK / 2;  // 128s of a stage; bytes of a row in it: 512 and 256
 

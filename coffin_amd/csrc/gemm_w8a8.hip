@@ -132,8 +132,8 @@ __device__ __forceinline__ void stage_scales(const Args &a, float *dst, int n0, 
 //
 // K need not be whole steps of 128: in the last one the chunks past K belong to the next row.  Those of the activations
 // are asked for past the resource's end and read as zeros, so what the weight's hold does not matter.  Two vector
-// instructions a step; on the register-staged kernel such rows took, 9664 -> 2560, 100 rows 98.8 us against 19.8 now,
-// 1000 rows 100.7 / 51.5, 8000 rows 377 / 187, 200 rows of 2496 -> 9000 34.2 / 20.6.
+// instructions a step; on the register-staged kernel such rows took, 9664 -> 2560, 100 rows 98.2 us against 19.2 now,
+// 1000 rows 99.5 / 51.0, 8000 rows 364 / 188, 200 rows of 2496 -> 9000 33.5 / 20.4 (quantiser in front).
 struct Operand {
     static constexpr uint32_t PAST = 1u << 30;  // beyond any tile: launches keep rows x K below it
     __amdgpu_buffer_rsrc_t res;

@@ -438,8 +438,8 @@ extern "C" int cmi_gemv_w4a8(const uint8_t *w4, const float *ws, const int8_t *x
     // GEMM, whichever is modelled to be faster (groups of 64: 0.9 for the tiles' model, which is fitted to groups of 128; of
     // 180 sizes the choice is 7 and 1 % above the best).  The group sums of several rows come from the two-stage GEMM, the general
     // kernel below keeps rows of groups of 64 that are not whole steps of 128; cold weights, the projection with its quantiser: one
-    // row of 2560 -> 19456 17.2 -> 8.4 us (64), 12.9 -> 7.4 (256); 4 rows 27.2 -> 14.3, 23.3 -> 11.4; 16 rows 62.9 -> 14.7, 62.1 ->
-    // 13.3; 16 rows of 2560 -> 151936 451 -> 60, 432 -> 51; of 9728 -> 2560 37.6 -> 14.7, 31.9 -> 12.2.
+    // row of 2560 -> 19456 16.5 -> 7.7 us (64), 12.4 -> 7.0 (256); 4 rows 26.1 -> 14.0, 22.2 -> 10.6; 16 rows 61.5 -> 14.5, 58.7 ->
+    // 12.2; 16 rows of 2560 -> 151936 428 -> 57, 411 -> 48; of 9728 -> 2560 35.8 -> 13.8, 29.9 -> 11.6.
     if ((gs == 64 || gs == 256) && K >= gs && K % GS == 0 && K % gs == 0 && N >= 1 && M >= 1 && M <= 16) {
         int rc = CMI_E_UNSUPPORTED, tile = 0;
         if (M == 1) rc = gemv_w4a8_decode(w4, ws, nullptr, xq, xs, y, group_acc, nullptr, nullptr, M, N, K, gs, stream);

@@ -26,7 +26,7 @@
 //   and cannot reach -0).
 // * Groups of 64 and 256 (one row): a group is two or eight lanes, so one or three DPP steps form its sum and a load
 //   instruction covers LPR/2 or LPR/8 groups.  Against the kernel that kept a row's sums in LDS and walked them serially,
-//   cold weights, quantised here instead of in a launch before: 2560 -> 19456 17.2 -> 8.4 us (64), 12.9 -> 7.4 (256); 2560 -> 151936 97 -> 39,
+//   cold weights, quantised here instead of in a launch before: 2560 -> 19456 16.5 -> 7.7 us (64), 12.4 -> 7.0 (256); 2560 -> 151936 97 -> 39,
 //   67 -> 35; 9728 -> 2560 21.3 -> 9.8, 11.4 -> 7.4; 4096 -> 2560 8.8 -> 4.6, 6.8 -> 3.7.
 // * Longer rows are shared by S wavefronts of a workgroup, each a contiguous run of loads: every
 //   wavefront forms and converts its integer sums as its bytes arrive, then the chain passes

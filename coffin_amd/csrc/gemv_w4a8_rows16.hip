@@ -30,7 +30,7 @@
 // Groups of 64 and 256 (up to 16 quantised rows).  256: the two halves of a line go into one sum.  64: an MFMA has to stay
 // inside a group, so lane l takes half l/16 % 2 of piece 2e + l/32 of the packed half line for group e of its two: eight
 // bytes, whose nibbles are 16 consecutive k, against 16 consecutive activation bytes.  The dot-product kernel that took
-// these rows forms 16 rows' products in the vector ALU: 16 rows of 9728 -> 2560 32.7 -> 10.9 us (64), 26.8 -> 8.5 (256), of 14336 ->
+// these rows forms 16 rows' products in the vector ALU: 16 rows of 9728 -> 2560 31.8 -> 9.9 us (64), 25.8 -> 7.7 (256), of 14336 ->
 // 4096 69.4 -> 15.5, 54.0 -> 12.4; 4 rows of 2560 -> 6144 9.4 -> 5.8, 7.9 -> 5.1.  The sums of 64s take twice the LDS, so K = 5120 leaves
 // room for one workgroup per CU (5120 -> 32768 51 us): the tile GEMM takes such sizes.
 #include "quant_math.hpp"

@@ -226,7 +226,7 @@ int cmi::quant_act_i8_and_clear(const void *x, int8_t *q, float *s, int M, int K
 
 // Rows of an int4 weight whose K is not whole groups: the vector kernels as well, whatever K is, since the padded rows
 // of q are whole vectors.  Element by element, each read twice, the projection behind it included: 9664 -> 2560, one
-// row 15.7 -> 9.0 us, 16 rows 24.6 -> 12.9, 8000 rows 395 -> 308; 100 rows of 2497 -> 9000 21.7 -> 17.5.
+// row 15.2 -> 8.9 us, 16 rows 18.8 -> 12.5, 8000 rows 359 -> 280; 100 rows of 2497 -> 9000 21.7 -> 17.5.
 int cmi::quant_act_i8_padded(const void *x, int8_t *q, float *s, int M, int K, int ldq, void *stream) {
     if (ldq == K) return quant_act_i8_and_clear(x, q, s, M, K, nullptr, 0, stream);
     CMI_REQUIRE(M >= 0 && K > 0 && ldq > K && ldq % 8 == 0, CMI_E_ARG, "cmi_quant_act_i8: bad shape M=%d K=%d pitch=%d", M, K, ldq);
