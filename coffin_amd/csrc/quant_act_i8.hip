@@ -31,6 +31,7 @@ __device__ __forceinline__ float block_max(float v, float *smem) {
 template <bool P>
 struct Whole {
     static constexpr bool PADDED = P;
+    typedef uint4 T;
     const uint4 *x;
     int nvec;
     __device__ __forceinline__ uint4 load(int row, int idx) const {
@@ -40,6 +41,7 @@ struct Whole {
 };
 struct Ragged {
     static constexpr bool PADDED = true;
+    typedef uint16_t T;
     const uint16_t *x;
     int K;
     __device__ __forceinline__ uint4 load(int row, int idx) const {
@@ -61,13 +63,16 @@ struct Ragged {
 
 // VPT > 0: the row fits in VPT vectors per thread and stays in registers; VPT == 0: generic, second pass re-reads.
 // Rows of q have q_vecs vectors where they are padded; past the row's own they are zeros, as quant8 makes of zeros under every scale
-// (rows padded to whole groups of an int4 weight).  Rows that are not know one count: with two in registers every launch took 0.04 us longer
-// (16 x 2560 2.49 -> 2.53).
+// (rows padded to whole groups of an int4 weight).  Rows that are not know one count, and it and the row pointer are arguments of
+// their own: with two counts, and a struct among the arguments, every launch took 1 .. 3 % longer (16 x 2560 2.49 -> 2.51 us, 65536 x 128
+// 6.95 -> 7.15).  n: SRC's second member.
 // zero / n_zero: a few ints of the caller's that the first workgroup clears on the way (the
 // arrival counters of a split-K GEMM that follows in the stream), or null / 0.
 template <int VPT, typename SRC>
 __global__ void __launch_bounds__(QUANT_THREADS)
-quant_act_i8_vec(const SRC x, uint2 *__restrict__ q, float *__restrict__ s, int q_vecs, int *__restrict__ zero, int n_zero) {
+quant_act_i8_vec(const typename SRC::T *__restrict__ x_rows, uint2 *__restrict__ q, float *__restrict__ s, int n, int *__restrict__ zero,
+                 int n_zero, int q_vecs) {
+    const SRC x{x_rows, n};
     __shared__ float smem[QUANT_THREADS / 64];
     const int row = blockIdx.x;
     if (row == 0)
@@ -127,8 +132,9 @@ __device__ __forceinline__ float group_max(float v) {
 // 45.9 -> 7.8 us (3.2 TB/s), 8192 x 512 9.0 -> 5.6 us, 3000 x 1024 6.1 -> 4.5 us.  Same arithmetic, same bits.
 template <int LANES, int VPT, int R, typename SRC>
 __global__ void __launch_bounds__(QUANT_THREADS)
-quant_act_i8_rows(const SRC x, uint2 *__restrict__ q, float *__restrict__ s, int q_vecs, int rows,
-                  int *__restrict__ zero, int n_zero) {
+quant_act_i8_rows(const typename SRC::T *__restrict__ x_rows, uint2 *__restrict__ q, float *__restrict__ s, int n, int rows,
+                  int *__restrict__ zero, int n_zero, int q_vecs) {
+    const SRC x{x_rows, n};
     constexpr int STEP = QUANT_THREADS / LANES;
     const int pvec = SRC::PADDED ? q_vecs : x.vecs();
     if (blockIdx.x == 0)
@@ -182,14 +188,15 @@ quant_act_i8_scalar(const uint16_t *__restrict__ x, int8_t *__restrict__ q,
 
 // The vector kernels' launch: rows of pvec vectors in q.
 template <typename SRC>
-void launch_vectors(const SRC &x, int8_t *q, float *s, int M, int pvec, int *zero, int n_zero, hipStream_t st) {
+void launch_vectors(const void *x_rows, int n, int8_t *q, float *s, int M, int pvec, int *zero, int n_zero, hipStream_t st) {
     const dim3 grid(M), block(QUANT_THREADS);
+    const auto *x = static_cast<const typename SRC::T *>(x_rows);
     uint2 *qv = reinterpret_cast<uint2 *>(q);
     const int vpt = (pvec + QUANT_THREADS - 1) / QUANT_THREADS;
     const auto rows_launch = [&](auto kernel, int rows_per_block) {
-        kernel<<<dim3((M + rows_per_block - 1) / rows_per_block), block, 0, st>>>(x, qv, s, pvec, M, zero, n_zero);
+        kernel<<<dim3((M + rows_per_block - 1) / rows_per_block), block, 0, st>>>(x, qv, s, n, M, zero, n_zero, pvec);
     };
-    const auto row_launch = [&](auto kernel) { kernel<<<grid, block, 0, st>>>(x, qv, s, pvec, zero, n_zero); };
+    const auto row_launch = [&](auto kernel) { kernel<<<grid, block, 0, st>>>(x, qv, s, n, zero, n_zero, pvec); };
     // Up to 1024 elements a wavefront or less owns a row.  Two rows per lane group once one each would
     // be more than two workgroups per CU: twice the bytes in flight per wavefront (65536 x 128: 9.8 ->
     // 7.8 us; below that the second row only lengthens the launch, 2048 x 576: 3.3 -> 3.9 us).
@@ -218,7 +225,7 @@ int cmi::quant_act_i8_and_clear(const void *x, int8_t *q, float *s, int M, int K
     CMI_REQUIRE(x && q && s, CMI_E_ARG, "cmi_quant_act_i8: null pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (K % 8 == 0 && aligned(x, 16) && aligned(q, 8))
-        launch_vectors(Whole<false>{static_cast<const uint4 *>(x), K / 8}, q, s, M, K / 8, zero, n_zero, st);
+        launch_vectors<Whole<false>>(x, K / 8, q, s, M, K / 8, zero, n_zero, st);
     else
         quant_act_i8_scalar<<<dim3(M), dim3(QUANT_THREADS), 0, st>>>(static_cast<const uint16_t *>(x), q, s, K, zero, n_zero);
     return check_launch("cmi_quant_act_i8");
@@ -234,8 +241,8 @@ int cmi::quant_act_i8_padded(const void *x, int8_t *q, float *s, int M, int K, i
     CMI_REQUIRE(x && q && s, CMI_E_ARG, "cmi_quant_act_i8: null pointer");
     CMI_REQUIRE(aligned(q, 8), CMI_E_ARG, "cmi_quant_act_i8: rows must be 8-byte aligned");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (K % 8 == 0 && aligned(x, 16)) launch_vectors(Whole<true>{static_cast<const uint4 *>(x), K / 8}, q, s, M, ldq / 8, nullptr, 0, st);
-    else launch_vectors(Ragged{static_cast<const uint16_t *>(x), K}, q, s, M, ldq / 8, nullptr, 0, st);
+    if (K % 8 == 0 && aligned(x, 16)) launch_vectors<Whole<true>>(x, K / 8, q, s, M, ldq / 8, nullptr, 0, st);
+    else launch_vectors<Ragged>(x, K, q, s, M, ldq / 8, nullptr, 0, st);
     return check_launch("cmi_quant_act_i8");
 }
 
