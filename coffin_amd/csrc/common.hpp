@@ -51,6 +51,9 @@ int quant_act_i8_padded(const void *x, int8_t *q, float *s, int M, int K, int ld
 // 16-row weight tiles per workgroup (1 or 2) that gemm_w8a8_rows16 uses for 17..128 rows.
 int gemm_w8a8_rows_tiles(int N);
 
+// gemv_w8a16_batch.hip: cmi_gemv_w8a16 for 2..16 rows; arguments already checked.
+int gemv_w8a16_batch(const int8_t *wq, const float *ws, const void *x, void *y, int M, int N, int K, void *stream);
+
 // gemv_w4a8_decode.hip: W4A8 GEMV for 1..4 rows, K <= 10240, from bf16 activations (x) or
 // quantised ones (xq, xs), groups of 64 and 256 for one row; returns CMI_E_UNSUPPORTED (no error text) for other shapes.
 int gemv_w4a8_decode(const uint8_t *w4, const float *ws, const void *x, const int8_t *xq, const float *xs,
@@ -138,26 +141,8 @@ __device__ __forceinline__ float wave_sum_to_lane63(float v) {
     return v;
 }
 
-// The wave sums of NV per-lane values (NV = 8, 16 or 32) with the pairing of wave_sum_to_lane63 --
-// lanes l^1, l^2, then quads, half rows, rows, halves; fp32 addition commutes, so the totals have
-// the same bits -- as a transposing reduction: at each level a lane forms the pair sums of only half
-// of the values it still holds and its partner those of the other half, so the work halves per
-// level (NV + NV/2 + .. adds instead of 6 NV) and the NV totals end in NV different lanes.
-// Which half a lane keeps at levels 1..4 is chosen so that the partner of the *next* levels
-// (l^2, l^7, l^15: the DPP controls of the plain tree) holds the same values: bits
-// b0^b2, b1^b2, b2^b3, b3 of the lane number; the row and half levels swap whole rows
-// (v_permlane16_swap, v_permlane32_swap).  Returns the total of value wave_sum_transposed_index<NV>(lane);
-// lanes 0..NV-1 cover every value once.
-template <int NV>
-__device__ __forceinline__ int wave_sum_transposed_index(int lane) {
-    static_assert(NV == 8 || NV == 16 || NV == 32, "8, 16 or 32 values per lane");
-    const int s1 = (lane ^ (lane >> 2)) & 1, s2 = ((lane >> 1) ^ (lane >> 2)) & 1;
-    const int s3 = ((lane >> 2) ^ (lane >> 3)) & 1, s4 = (lane >> 3) & 1, s5 = (lane >> 4) & 1;
-    if constexpr (NV == 8) return s1 * 4 + s2 * 2 + s3;
-    else if constexpr (NV == 16) return s1 * 8 + s2 * 4 + s3 * 2 + s4;
-    else return s1 * 16 + s2 * 8 + s3 * 4 + s4 * 2 + s5;
-}
-
+// One level of a transposing reduction: of 2 H values a lane forms the sums with its partner (a DPP control) of one half and the
+// partner those of the other, so the work halves per level.  The pairing is a plain tree's, and fp32 addition commutes: same bits.
 template <int CTRL, int H>
 __device__ __forceinline__ void transposed_level(const float (&in)[2 * H], float (&out)[H], bool upper) {
 #pragma unroll
@@ -166,36 +151,6 @@ __device__ __forceinline__ void transposed_level(const float (&in)[2 * H], float
         const float hi = in[i + H] + dpp_f32<CTRL, 0xf>(in[i + H]);
         out[i] = upper ? hi : lo;
     }
-}
-
-template <int NV>
-__device__ __forceinline__ float wave_sum_transposed(const float (&v)[NV], int lane) {
-    static_assert(NV == 8 || NV == 16 || NV == 32, "8, 16 or 32 values per lane");
-    typedef unsigned u32x2_swap __attribute__((ext_vector_type(2)));
-    float a1[NV / 2], a2[NV / 4], a3[NV / 8];
-    transposed_level<0xB1, NV / 2>(v, a1, ((lane ^ (lane >> 2)) & 1) != 0);          // l ^ 1
-    transposed_level<0x4E, NV / 4>(a1, a2, (((lane >> 1) ^ (lane >> 2)) & 1) != 0);  // l ^ 2
-    transposed_level<0x141, NV / 8>(a2, a3, (((lane >> 2) ^ (lane >> 3)) & 1) != 0); // other quad of the half row
-    float t;
-    if constexpr (NV == 8) {
-        t = a3[0] + dpp_f32<0x140, 0xf>(a3[0]);                                      // other half of the row
-    } else {
-        float a4[NV / 16];
-        transposed_level<0x140, NV / 16>(a3, a4, ((lane >> 3) & 1) != 0);
-        if constexpr (NV == 32) {
-            // rows 0+1 and 2+3: even rows end with value 0, odd rows with value 1
-            const u32x2_swap r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a4[0]), __float_as_uint(a4[1]), false, false);
-            t = __uint_as_float(r.x) + __uint_as_float(r.y);
-        } else {
-            t = a4[0];
-        }
-    }
-    if constexpr (NV != 32) {
-        const u32x2_swap r = __builtin_amdgcn_permlane16_swap(__float_as_uint(t), __float_as_uint(t), false, false);
-        t = __uint_as_float(r.x) + __uint_as_float(r.y);                              // rows 0+1, 2+3
-    }
-    const u32x2_swap h = __builtin_amdgcn_permlane32_swap(__float_as_uint(t), __float_as_uint(t), false, false);
-    return __uint_as_float(h.x) + __uint_as_float(h.y);                               // the two halves
 }
 
 // Max over the 64 lanes; every lane of row 3 ends with the wave maximum, lane

@@ -1,5 +1,5 @@
 // Arithmetic shared by the int8 weight-only GEMV kernels: the canonical summation order's
-// blocking of K and the exact int8 -> packed-bf16 widening.  Every kernel that includes this
+// blocking of K, the exact int8 -> packed-bf16 widening and the MFMA steps of a chain.  Every kernel that includes this
 // produces the same bits for the same (weight row, activation row).
 #pragma once
 
@@ -32,19 +32,42 @@ __device__ __forceinline__ void widen4(uint32_t w, bf16x2_t &lo, bf16x2_t &hi) {
     hi = __builtin_bit_cast(bf16x2_t, p1);
 }
 
+typedef short bf16x4_t __attribute__((ext_vector_type(4)));
+typedef float v4f32 __attribute__((ext_vector_type(4)));
 
-// One 16-element chunk of a lane's chain: eight chained two-element dot products, k ascending.
-__device__ __forceinline__ float chain_chunk(float v, const u32x4 &w, const uint4 &x0, const uint4 &x1) {
-    bf16x2_t wb[8];
-    widen4(w.x, wb[0], wb[1]);
-    widen4(w.y, wb[2], wb[3]);
-    widen4(w.z, wb[4], wb[5]);
-    widen4(w.w, wb[6], wb[7]);
-    const uint32_t xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+// Sixteen codes of a weight row as the four MFMA steps take them, four k each.
+struct Chunk {
+    bf16x4_t step[4];
+};
+
+__device__ __forceinline__ bf16x4_t pair_bits(uint32_t lo, uint32_t hi) { return __builtin_bit_cast(bf16x4_t, make_uint2(lo, hi)); }
+
+__device__ __forceinline__ Chunk widen_chunk(const u32x4 &w) {
+    Chunk c;
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-        v = __builtin_amdgcn_fdot2_f32_bf16(wb[i], __builtin_bit_cast(bf16x2_t, xv[i]), v, false);
+    for (int i = 0; i < 4; ++i) {
+        bf16x2_t lo, hi;
+        widen4(w[i], lo, hi);
+        c.step[i] = pair_bits(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+    }
+    return c;
+}
+
+// One 16-element chunk of a lane's chain, k ascending: v_mfma_f32_4x4x4_16b_bf16 works on 16 blocks of four lanes; for block b and
+// lane 4b + j, register i of v gains the four products of the codes in lane 4b + i with the activations in lane 4b + j, exact
+// products summed with what v held and rounded once.
+__device__ __forceinline__ v4f32 chain_chunk(v4f32 v, const Chunk &w, const uint4 &x0, const uint4 &x1) {
+    v = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(w.step[0], pair_bits(x0.x, x0.y), v, 0, 0, 0);
+    v = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(w.step[1], pair_bits(x0.z, x0.w), v, 0, 0, 0);
+    v = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(w.step[2], pair_bits(x1.x, x1.y), v, 0, 0, 0);
+    v = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(w.step[3], pair_bits(x1.z, x1.w), v, 0, 0, 0);
     return v;
+}
+
+// The chain of the lane's own codes with its own activations: the diagonal of its block.
+__device__ __forceinline__ float own_chain(v4f32 v, int lane) {
+    const float a = (lane & 1) ? v.y : v.x, b = (lane & 1) ? v.w : v.z;
+    return (lane & 2) ? b : a;
 }
 
 }  // namespace cmi

@@ -484,3 +484,35 @@ def test_ragged_rows_take_the_matrix_pipe_where_the_call_site_may(monkeypatch, p
         assert torch.equal(backend.linear_m_verify(w, x).view(torch.int16), want.view(torch.int16))
         assert torch.equal(backend.linear_prefill(w, x).view(torch.int16), want.view(torch.int16))
         assert torch.equal(backend.linear_m(w, x).view(torch.int16), dot.view(torch.int16))
+
+
+@pytest.mark.parametrize("m,n,k", [(2, 1, 16), (3, 5, 1040), (4, 1023, 2560), (16, 1024, 2576), (4, 300, 9744), (8, 700, 9728),
+                                   (7, 2047, 4096), (5, 2561, 4112), (2, 9000, 6416),
+                                   (3, 200, 20496), (6, 500, 12304), (7, 2000, 33024), (16, 300, 9728), (12, 5000, 6160), (9, 9300, 12304),
+                                   (4, 5001, 2560), (8, 7000, 5136), (16, 8192, 1024), (2, 6000, 16), (13, 3333, 3072),
+                                   (4, 32773, 4112), (5, 16385, 1040), (16, 9217, 2576), (15, 9301, 4096), (11, 4100, 5120),
+                                   (3, 20000, 5136), (8, 8193, 6160), (16, 16400, 6160)])
+def test_batches_of_weight_only_rows_carry_the_single_row_bits(m, n, k):
+    """Every kernel that 2..16 rows of cmi_gemv_w8a16 take, at odd counts of rows, outputs and chunks: few outputs by quarters of a row
+    (units dealt to wavefronts, one block or two a wavefront), long rows in windows, many outputs streamed, sixteen rows in two halves.
+    Infinite and NaN activations stay in their rows; nothing is written past the outputs."""
+    gen = torch.Generator(device=G.DEV).manual_seed(m + n + k)
+    wq = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=G.DEV, generator=gen)
+    ws = torch.rand(n, device=G.DEV, generator=gen) * 0.01 + 1e-3
+    x = torch.randn((m, k), device=G.DEV, generator=gen).to(torch.bfloat16)
+    x[0, k - 1] = float("inf")
+    x[m // 2, k // 2] = float("nan")
+    lib = _native.load()
+    y = torch.full((m * n + 64,), -77.0, dtype=torch.bfloat16, device=G.DEV)
+    _native.check(lib.cmi_gemv_w8a16(G.ptr(wq), G.ptr(ws), G.ptr(x), G.ptr(y), m, n, k, G.stream()), "gemv")
+    single = torch.cat([G.gemv_w8a16(wq, ws, x[r:r + 1].contiguous()) for r in range(m)])
+    finite = [r for r in range(m) if r not in (0, m // 2)]
+    got = y[:m * n].view(m, n)
+    assert torch.equal(got[finite].view(torch.int16), single[finite].view(torch.int16)) and (y[m * n:] == -77.0).all()
+    for kind in (torch.isposinf, torch.isneginf, torch.isnan):
+        assert torch.equal(kind(got), kind(single)), kind
+    if finite:
+        xd, wd = x[finite[0]].double(), wq.double()
+        exact = (wd @ xd) * ws.double()
+        bound = exact.abs() * 2.0 ** -8 + (wd.abs() @ xd.abs()) * ws.double() * (k * 2.0 ** -24)
+        assert ((got[finite[0]].double() - exact).abs() <= bound).all()

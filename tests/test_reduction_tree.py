@@ -1,10 +1,12 @@
-"""The transposing wave reduction of the 4..16-row GEMV against the plain DPP tree, symbolically.
+"""Transposing wave reductions against the plain DPP tree, symbolically.
 
 coffin_amd/csrc/common.hpp sums the 64 lane chains of a unit with a fixed tree
 (wave_sum_to_lane63: lanes l^1, l^2, quads, half rows, rows, halves); a batched row must have the
-bits of the single-row call (reference contract: models/qwen35/batch.py:19-22), so
-wave_sum_transposed -- which reduces 8, 16 or 32 values per lane together, each lane keeping half
-of its values per level -- has to build exactly that tree for every value.  Here both are run on
+bits of the single-row call (reference contract: models/qwen35/batch.py:19-22), so a
+transposing reduction -- several values per lane together, each lane keeping half
+of its values per level -- has to build exactly that tree for every value: over whole wavefronts
+(wave_sum_transposed below), and over the 16 blocks of four lanes that the batch kernels' MFMA
+steps work on (quarter_sum of gemv_w8a16_batch.hip).  Here both are run on
 symbols, with fp32 addition modelled as an unordered pair (it commutes bit for bit and does not
 associate), the cross-lane moves modelled after the ISA (DPP quad_perm / row_half_mirror /
 row_mirror / row_bcast, v_permlane16_swap, v_permlane32_swap).  The GPU parity tests check the
@@ -146,3 +148,57 @@ def test_a_different_choice_of_halves_is_caught():
     x, y = swap32(t, t)
     got = [add(x[l], y[l]) for l in range(64)]
     assert any(got[lane] not in want for lane in range(64))
+
+
+def batch(mg, vals):
+    """quarter_sum<mg> of gemv_w8a16_batch.hip: 4 mg values a lane over the 16 blocks of four lanes."""
+    nv = 4 * mg
+    a = level(vals, 0x141, nv // 2, lambda l: ((l >> 2) ^ (l >> 3)) & 1)
+    b = level(a, 0x140, nv // 4, lambda l: (l >> 3) & 1)
+
+    def swapped(swap, x, y):
+        p, q = swap(x, y)
+        return [add(p[lane], q[lane]) for lane in range(64)]
+
+    if mg == 4:
+        return swapped(swap32, swapped(swap16, b[0], b[2]), swapped(swap16, b[1], b[3]))
+    c = swapped(swap16, b[0], b[1] if mg == 2 else b[0])
+    return swapped(swap32, c, c)
+
+
+@pytest.mark.parametrize("mg", [1, 2, 4])
+def test_batch_reduction_continues_the_single_row_tree(mg):
+    """Blocks b ^ 1, b ^ 2, b ^ 4, b ^ 8 in this order: the levels of wave_sum_to_lane63 between chunks that differ in one bit.  The
+    activation rows of a block's four lanes are reversed in odd blocks (lane_row)."""
+    def act(lane):
+        return 3 - (lane & 3) if lane & 4 else lane & 3
+
+    def tree(i, j):
+        def leaf(b):
+            return [(i, lane) for lane in range(4 * b, 4 * b + 4) if act(lane) == j][0]
+
+        cur = [leaf(b) for b in range(16)]
+        while len(cur) > 1:
+            cur = [add(cur[2 * b], cur[2 * b + 1]) for b in range(len(cur) // 2)]
+        return cur[0]
+
+    vals = [[(i, lane) for lane in range(64)] for i in range(4 * mg)]
+    got = batch(mg, vals)
+    held = set()
+    for lane in range(64):
+        s1, s2, b4, b5 = ((lane >> 2) ^ (lane >> 3)) & 1, (lane >> 3) & 1, (lane >> 4) & 1, (lane >> 5) & 1
+        i = {4: s1 * 8 + s2 * 4 + b4 * 2 + b5, 2: s1 * 4 + s2 * 2 + b4, 1: s1 * 2 + s2}[mg]
+        assert got[lane] == tree(i, act(lane)), (mg, lane)
+        if mg == 4 or not lane & (32 if mg == 2 else 48):
+            held.add((i, act(lane)))
+    # the lanes that store cover every output exactly once
+    assert held == {(i, j) for i in range(4 * mg) for j in range(4)}
+
+
+def test_single_row_tree_pairs_chunks_by_one_bit():
+    """wave_sum_to_lane63 on symbols equals the tree over lane numbers, lowest bit first."""
+    cur = [(0, lane) for lane in range(64)]
+    want = list(cur)
+    while len(want) > 1:
+        want = [add(want[2 * b], want[2 * b + 1]) for b in range(len(want) // 2)]
+    assert original(cur) == want[0]
