@@ -71,6 +71,9 @@ int gemv_w4a8_chain(const uint8_t *w4, const float *ws, const void *x, const int
 int gemv_w4a8_rows16(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs, const void *x,
                      void *y, int32_t *group_acc, int8_t *xq_out, float *xs_out, int M, int N, int K, int gs,
                      void *stream);
+// gemv_w4a8_stream.hip: W4A8 GEMV of groups of 128 for the quantised rows of a large weight, and whether it is the one for a shape.
+bool gemv_w4a8_streams(int M, int N, int K);
+int gemv_w4a8_stream(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs, void *y, int M, int N, int K, void *stream);
 // gemm_w4a8_tile.hip: W4A8 tile GEMM, arguments already checked by cmi_gemm_w4a8 / cmi_gemv_w4a8.  The cheapest tile for a
 // shape and its modelled time (us), of all tiles and of those of four groups a step; the tile a gemm_tile
 // option names; whether a w4_gemm_deep option names one; the launch.

@@ -516,3 +516,28 @@ def test_batches_of_weight_only_rows_carry_the_single_row_bits(m, n, k):
         exact = (wd @ xd) * ws.double()
         bound = exact.abs() * 2.0 ** -8 + (wd.abs() @ xd.abs()) * ws.double() * (k * 2.0 ** -24)
         assert ((got[finite[0]].double() - exact).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(3, 655361, 256), (16, 145637, 1152), (9, 65543, 2560), (5, 62425, 2688), (4, 32768, 5120), (13, 33333, 5120)])
+def test_rows_of_a_large_int4_weight_carry_the_small_weights_bits(m, n, k):
+    """One line to the longest rows, odd counts of groups, rows and outputs, at the rule's edge: the bits of the kernels
+    that the first and the last outputs take alone."""
+    gen = torch.Generator(device=G.DEV).manual_seed(m + n + k)
+    w4 = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=G.DEV, generator=gen)
+    ws = torch.rand((n, k // 128), device=G.DEV, generator=gen) * 0.01 + 1e-3
+    xq = torch.randint(-127, 128, (m, k), dtype=torch.int8, device=G.DEV, generator=gen)
+    xs = torch.rand(m, device=G.DEV, generator=gen) + 0.1
+    lib = _native.load()
+    y = torch.full((m * n + 64,), -77.0, dtype=torch.bfloat16, device=G.DEV)
+    _native.check(lib.cmi_gemv_w4a8(G.ptr(w4), G.ptr(ws), G.ptr(xq), G.ptr(xs), G.ptr(y), None, m, n, k, 128, G.stream()), "gemv_w4a8")
+    got = y[:m * n].view(m, n)
+    assert (y[m * n:] == -77.0).all()
+    cut = n - 16 * 2048                                    # few enough outputs for the other kernels
+    part = torch.empty((m, n - cut), dtype=torch.bfloat16, device=G.DEV)
+    sums = torch.empty((m, k // 128, n - cut), dtype=torch.int32, device=G.DEV)
+    _native.check(lib.cmi_gemv_w4a8(G.ptr(w4[cut:]), G.ptr(ws[cut:]), G.ptr(xq), G.ptr(xs), G.ptr(part), G.ptr(sums), m, n - cut, k, 128,
+                                    G.stream()), "gemv_w4a8")
+    assert torch.equal(got[:, cut:].contiguous().view(torch.int16), part.view(torch.int16))
+    head = torch.empty((m, 4096), dtype=torch.bfloat16, device=G.DEV)
+    _native.check(lib.cmi_gemv_w4a8(G.ptr(w4), G.ptr(ws), G.ptr(xq), G.ptr(xs), G.ptr(head), None, m, 4096, k, 128, G.stream()), "gemv_w4a8")
+    assert torch.equal(got[:, :4096].contiguous().view(torch.int16), head.view(torch.int16))
