@@ -13,7 +13,7 @@ Routing, by storage type first (never by op name), then by row count:
 =================  ==========================  =================================
 weight             rows                        kernel
 =================  ==========================  =================================
-QWeight (int8)     linear, linear_m            int8 weight-only dot-product GEMV, 16
+QWeight (int8)     linear, linear_m            int8 weight-only GEMV, 16
                                                rows at a time (row r == linear(x[r]))
 QWeight            >= 3, linear_m_verify and   weight-only GEMV on the matrix pipe,
                    linear_prefill below 64     16 rows at a time
@@ -63,14 +63,15 @@ PREFILL_MIN_ROWS = 64
 W8A8_VERIFY = os.environ.get("COFFIN_AMD_W8A8_VERIFY", "0").strip() == "1"
 #: Static-batch decode owes its users "row r of a batch equals the single-row call on x[r]", bit
 #: for bit (models/qwen35/batch.py:19-22: a batched and an unbatched request must give the same
-#: numbers), so ``linear`` and ``linear_m`` on int8 weights stay on the dot-product GEMV, whose
+#: numbers), so ``linear`` and ``linear_m`` on int8 weights stay on the GEMV of the single-row order, whose
 #: summation order depends on K only.  ``linear_m_verify`` (which may use a path of its own,
 #: backends/protocol.py:152-155) and short ``linear_prefill`` chunks do not carry that obligation
-#: and take the matrix-pipe GEMV from three rows up: 1.5-2.8 times faster at 8-16 rows, same
+#: and take the matrix-pipe GEMV from three rows up: up to 1.6 times faster at 16 rows, up to 1.5 times
+#: slower at three to eight of a large weight, a row's bits the same in a window of any length; same
 #: weight-only arithmetic, last-place differences from fp32 summation order.
 #: ``COFFIN_AMD_BATCH_MFMA=1`` moves *every* int8 weight-only call -- ``linear`` included, one row
 #: included -- to the matrix-pipe GEMV: the contract holds again (one kernel family, a row's bits
-#: independent of its batch), static batches of 4-16 requests run 1.05-2.8 times faster, and
+#: independent of its batch), and
 #: single-stream decode pays for it (7.9 us instead of 6.3 us for 2560 -> 9728).  A deployment choice.
 BATCH_MFMA = os.environ.get("COFFIN_AMD_BATCH_MFMA", "0").strip() == "1"
 #: int4 weights are answered with W4A8 arithmetic (per-token int8 activations), which is what coffin
@@ -81,7 +82,7 @@ BATCH_MFMA = os.environ.get("COFFIN_AMD_BATCH_MFMA", "0").strip() == "1"
 W4A16 = os.environ.get("COFFIN_AMD_W4A16", "0").strip() == "1"
 W4A16_MAX_ROWS = 4
 W4A16_MAX_K = 32768
-#: Rows from which the matrix-pipe GEMV beats the dot-product one (measured on every layer shape).
+#: Rows from which verify windows and short chunks take the matrix-pipe GEMV (when this was chosen, the faster one on every layer shape).
 MFMA_MIN_ROWS = 3
 #: The same for K that is not whole lines of 128 (2624 -> 9728: the dot-product kernel takes four rows in 8.7 us, the
 #: matrix-pipe one five in 11.4; five take the former 12.0, nine 20.2 against 11.5).  A weight whose family is "mfma" keeps such
@@ -114,9 +115,9 @@ def configure(*, batch_family: str | None = None, w8a8_verify: bool | None = Non
     """Process-wide switches of this backend, settable after import (the environment variables
     above give the initial values).  Returns the settings in force.
 
-    ``batch_family``: ``"dot"`` -- ``linear`` / ``linear_m`` on int8 weights run the dot-product
-    GEMV (fastest single row; 4-16 rows are vector-ALU bound) -- or ``"mfma"`` -- every int8
-    weight-only call, single rows included, runs the matrix-pipe GEMV (4-16 rows 1.05-2.8 times
+    ``batch_family``: ``"dot"`` -- ``linear`` / ``linear_m`` on int8 weights run the GEMV of the
+    single-row order (fastest single row) -- or ``"mfma"`` -- every int8
+    weight-only call, single rows included, runs the 16-row matrix-pipe GEMV (16 rows up to 1.6 times
     faster, a single row slower).  Either way row r of a batch carries the bits of the single-row
     call (models/qwen35/batch.py:19-22): the rule needs one family per weight, not a particular
     one.  A weight object may carry its own choice in an attribute ``batch_family`` (read when the

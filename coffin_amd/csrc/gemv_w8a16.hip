@@ -423,6 +423,15 @@ bool x_fits_lds(int M, int K, int units, int segs) {
     return lds <= XLDS_MAX_BYTES && (size_t)M * K * 2 <= 16 * (size_t)xstage_vectors(M) * (64 * uw * teams);
 }
 
+// Two rows that this file's kernel, which has a wavefront for every two weight rows and unit, takes faster than the batch kernels: K of several units and outputs too few
+// for those to stream (5120 -> 10000 13.0 against 14.3 us, 6400 -> 9000 14.9 against 17.0), or so few that a wavefront of theirs walks
+// several units (12800 -> 512 4.4 against 5.5, 9728 -> 256 3.8 against 4.6, 16384 -> 300 4.4 against 5.7; the other way 9728 -> 1024 5.4 against 5.2, 16384 -> 1024 6.8 either
+// way, 14336 -> 2560 13.0 against 10.5).
+bool two_rows_stay(int N, int K, int units, int segs) {
+    if (units == 1 || !x_fits_lds(2, K, units, segs)) return false;
+    return (N > 8192 && (size_t)N * K < ((size_t)96 << 20)) || (units > 2 && N <= 384 * (units - 1));
+}
+
 template <int M, int R, int CHT, bool MULTI>
 int launch(GemvArgs &a, hipStream_t st) {
     a.nblocks = (a.N + R - 1) / R;
@@ -477,9 +486,7 @@ extern "C" int cmi_gemv_w8a16(const int8_t *wq, const float *ws, const void *x, 
     CMI_REQUIRE(a.units <= MAX_UNITS, CMI_E_UNSUPPORTED, "cmi_gemv_w8a16: K=%d above %d", K,
                 MAX_UNITS * 4096);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // Two rows of a K of several units and a few to many outputs that still are too few wavefronts for the streaming kernel stay here
-    // (5120 -> 10000 13.0 against 14.3 us, 6400 -> 9000 14.9 against 17.0); every other batch is the other file's.
-    if (M > 2 || (M == 2 && !(a.units > 1 && N > 8192 && (size_t)N * K < ((size_t)96 << 20) && x_fits_lds(2, K, a.units, a.units * a.unit))))
+    if (M > 2 || (M == 2 && !two_rows_stay(N, K, a.units, a.units * a.unit)))
         return gemv_w8a16_batch(wq, ws, x, y, M, N, K, stream);
     // One row of a long K (two or three units), or of a mid-sized weight with K in one unit: a
     // wavefront per weight row.  CMI_GEMV_WHOLEROW=0 keeps the general kernel (the tests compare

@@ -3,10 +3,8 @@
 //
 //   y[m,n] = bf16( (sum_k x[m,k] * (float)wq[n,k]) * ws[n] )        fp32 sums
 //
-// With one row the kernel is a stream of weight bytes and a few dot-product
-// instructions per 16 of them; with 16 rows the dot products alone (8 per row
-// and 16 weight bytes) run at a quarter of memory speed.  int8 -> bf16 is exact
-// and bf16 x bf16 products are exact in fp32, so here v_mfma_f32_16x16x32_bf16
+// int8 -> bf16 is exact
+// and bf16 x bf16 products are exact in fp32, so v_mfma_f32_16x16x32_bf16
 // forms the sums -- 16 weight rows x 16 activation rows x 32 k per instruction
 // -- and the vector ALU only widens the weight bytes.  The kernel stays a GEMV
 // in every other respect: the weight is read once, straight into registers, all
@@ -19,7 +17,7 @@
 // lines and rearranged through private LDS patches.  The fp32 partial tiles of
 // the wavefronts are added in wavefront order through LDS, so a row's result
 // depends on K only, not on the batch it came in -- but it is not the bit
-// pattern of the dot-product kernel behind cmi_gemv_w8a16 (different fp32
+// pattern of the kernels behind cmi_gemv_w8a16 (different fp32
 // summation order), which is why this kernel has an entry point of its own:
 // callers that owe their users "a batched row equals the single-row call"
 // (static-batch decode) stay on cmi_gemv_w8a16.

@@ -1,6 +1,6 @@
 // int8 weight-only projection of any number of bf16 rows in one call, with the kernel family as
-// an argument: the dot-product GEMV (a row's bits are those of the single-row call) or the
-// matrix-pipe GEMV (a row's bits depend on K only, not on the dot-product kernel's).  The batch is
+// an argument: the GEMV of the single-row order (a row's bits are those of the single-row call) or the
+// 16-row matrix-pipe GEMV (a row's bits depend on K only, and are not the other family's).  The batch is
 // cut into the launches the family takes; every piece goes to the same family, so a row's bits
 // never depend on where the batch was cut.
 #include "common.hpp"

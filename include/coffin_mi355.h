@@ -90,7 +90,7 @@ int cmi_gemv_w8a16(const int8_t *wq, const float *ws, const void *x, void *y,
  * K % 128 == 0 (else CMI_E_UNSUPPORTED: use cmi_gemv_w8a16); also
  * up to 64 rows (up to K = 10240 the weight is still read once, the rows go through in chunks
  * of 16 with the 16-row arithmetic; longer weight rows are read once per 16 activation rows).
- * 2-3 times faster than cmi_gemv_w8a16 at 8-16 rows.  A row's bits depend on K
+ * Up to 1.6 times faster than cmi_gemv_w8a16 at 16 rows.  A row's bits depend on K
  * only, not on the rows it travels with, but differ from cmi_gemv_w8a16's in
  * the last place (fp32 summation order): for callers without the
  * "batched row == single-row call" obligation of static-batch decode
