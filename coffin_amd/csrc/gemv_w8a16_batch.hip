@@ -15,8 +15,8 @@
 //   quarters  a wavefront holds a quarter of the chunks of a row block, so a block is four wavefronts (more where units of K are
 //             dealt to several sets of four): few outputs then still are many wavefronts with few instructions each, which is what
 //             a launch of under 10 us is made of.  2560 -> 6144 at 4 / 16 rows 6.3 -> 5.5 / 13.7 -> 7.8, 4096 -> 2560 5.6 -> 4.4 / 10.8 -> 7.5,
-//             9728 -> 2560 9.1 -> 9.0 / 35 -> 17, 1024 outputs of 2560 3.4 -> 3.0 / 8.5 -> 4.7.
-// Rows of K that do not fit LDS go through it in windows of whole units (25600 -> 5120 at 4 / 16 rows 107 -> 41 / 403 -> 77; the
+//             9728 -> 2560 9.1 -> 9.0 / 35 -> 15, 1024 outputs of 2560 3.4 -> 3.0 / 8.5 -> 4.7.
+// Rows of K that do not fit LDS go through it in windows of whole units (25600 -> 5120 at 4 / 16 rows 107 -> 37 / 403 -> 62; the
 // dot-product kernel split the batch until each part fit and read the weight once for each).
 
 #include "gemv_w8a16_math.hpp"
@@ -279,6 +279,9 @@ __global__ void __launch_bounds__(1024)
 gemv_w8a16_quarters_kernel(const BatchArgs a) {
     extern __shared__ uint4 smem[];
     constexpr int OUT = 16 * MG;  // outputs of four weight rows
+    // The next unit's weights are asked for behind this one's sums: segment by segment as registers free up measured 5..20 % slower
+    // (two rows of 5120 -> 7168 12.4 against 10.3 us, 16 of 25600 -> 5120 77 against 62) except between windows with two blocks (41 against 39).
+    constexpr bool AS_FREED = WINDOW && RG == 2;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int sets = SETS ? SETS : a.sets, threads = a.teams * sets * 256;
@@ -340,20 +343,19 @@ gemv_w8a16_quarters_kernel(const BatchArgs a) {
 #pragma unroll
                 for (int r = 0; r < RG; ++r) add_step<MG>(acc[r], w[s][r], x, false);
             }
-            if constexpr (WINDOW)
-                if (more) load_seg(u + SETS, s);
+            if constexpr (AS_FREED)
+                if (more) load_seg(u + sets, s);
         }
 #pragma unroll
         for (int r = 0; r < RG; ++r) {
             const float t = quarter_sum<MG>(acc[r], lane);
             if (mine && (WINDOW || u < units)) totals[((r * kept + (WINDOW ? set : u)) * 4 + q) * OUT + vi * 4 + xrow] = t;
         }
-        if constexpr (!WINDOW) {
-            if (more) {
+        if (!AS_FREED && more) {
 #pragma unroll
-                for (int s = 0; s < U; ++s) load_seg(u + sets, s);
-            }
-        } else {
+            for (int s = 0; s < U; ++s) load_seg(u + sets, s);
+        }
+        if constexpr (WINDOW) {
             __syncthreads();  // every wavefront has read its part of the window and left its totals
             for (int v = trip; v < trip + SETS && v < units; ++v) add_unit(v);
             if (more) {
@@ -451,11 +453,13 @@ int run(BatchArgs &a, bool streamed, hipStream_t st) {
     // wavefront (4096 -> 2560 at four rows 4.4 us, two blocks 4.9); above, two share the activation fragments.  Short rows and pairs of
     // rows want small workgroups (1024 -> 8192 at four rows 3.9 with two blocks, 4.3 with eight; two rows of 2560 -> 6144 5.2 against 5.5), and so
     // does everything beyond 32 rows a CU, where workgroups follow each other (2560 -> 19456 12.0 with four blocks, 13.9 with eight).
+    // Up to sixteen rows a CU of many units: four teams of one block (14336 -> 4096 at 4 / 8 rows 14.6 / 17.9 us, two of two 16.8 / 22.8; 9728 -> 3800
+    // at four rows 11.0 against 10.7, at eight 12.6 against 17.2).
     int rg = 2;
     if (rows <= 12) rg = 1, a.teams = (rows + 3) / 4;
     else if (MG <= 2 && a.K <= 1024) a.teams = MG;
     else if (a.M <= 2 && a.units == 1 && rows <= 32) a.teams = 1;
-    else if (rows <= 16) rg = MG == 4 ? 1 : 2, a.teams = MG == 4 ? 4 : 2;
+    else if (rows <= 16) rg = MG == 4 || a.units > (MG == 1 ? 3 : 2) ? 1 : 2, a.teams = 4 / rg;
     else if (rows <= 32) a.teams = rows <= 24 ? 3 : 4;
     else a.teams = MG == 4 ? 4 : 2;
     // wavefronts left in a workgroup of sixteen share the units of a long K (12800 -> 1000 at four rows 11 -> 6.7 us)

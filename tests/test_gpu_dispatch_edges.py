@@ -488,7 +488,7 @@ def test_ragged_rows_take_the_matrix_pipe_where_the_call_site_may(monkeypatch, p
 
 @pytest.mark.parametrize("m,n,k", [(2, 1, 16), (3, 5, 1040), (4, 1023, 2560), (16, 1024, 2576), (4, 300, 9744), (8, 700, 9728),
                                    (7, 2047, 4096), (5, 2561, 4112), (2, 9000, 6416), (2, 1152, 16384), (2, 1153, 16384),
-                                   (3, 200, 20496), (6, 500, 12304), (7, 2000, 33024), (16, 300, 9728), (12, 5000, 6160), (9, 9300, 12304),
+                                   (3, 200, 20496), (6, 500, 12304), (7, 2000, 33024), (4, 4096, 14336), (8, 3900, 9728), (6, 5000, 20496), (16, 300, 9728), (12, 5000, 6160), (9, 9300, 12304),
                                    (4, 5001, 2560), (8, 7000, 5136), (16, 8192, 1024), (2, 6000, 16), (13, 3333, 3072),
                                    (4, 32773, 4112), (5, 16385, 1040), (16, 9217, 2576), (15, 9301, 4096), (11, 4100, 5120),
                                    (3, 20000, 5136), (8, 8193, 6160), (16, 16400, 6160)])
