@@ -184,6 +184,7 @@ int launch(const Args &a, hipStream_t st) {
 }  // namespace
 
 bool cmi::gemv_w4a8_streams(int M, int N, int K) {
+    if (option_w4_gemm_deep() != 0) return false;  // the caller names the tile of 3..16 rows, or the GEMV
     return M >= 3 && M <= 16 && K % GS == 0 && K >= 2 * GS && K <= 5120 && (size_t)N * K >= (size_t)160 << 20;
 }
 

@@ -52,7 +52,8 @@ int cmi_abi_version(void);
  *                   decode GEMV (one bf16 or quantised row);
  *   "w4_gemm_deep"  0 (the library chooses) | 1 (never) | 1664 | 1665 | 3232 | 3233 | 3264 | 3265 | 4864: the tiles of
  *                   cmi_gemm_w4a8 and cmi_gemv_w4a8 that take four groups of 128 a step (rows x 100 + columns, one more: more
- *                   stages in flight; groups of 64: up to 16 rows);
+ *                   stages in flight; groups of 64: up to 16 rows).  3..16 rows of cmi_gemv_w4a8 take the named tile whatever
+ *                   the weight, with 1 the GEMV of the smaller weights;
  *   "w4_decode_chain" 0 (the library chooses) | 1 (never) | lanes + 100 * split + 10000 * waves: the
  *                   W4A8 decode kernel that keeps the fp32 chain in registers, with `lanes` (8, 16)
  *                   lanes per weight row, `split` (1, 2, 4, 8) wavefronts sharing a row and `waves`

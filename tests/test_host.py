@@ -429,6 +429,22 @@ def test_int4_rows_take_tiles_only_where_they_gain_more_than_the_models_err(m, n
     assert G.chosen_tile("_ZN3cmi20w4a8_rows_take_tilesEiiiPi", m, n, k)[0] == tiles
 
 
+@pytest.mark.parametrize("m,n,k", [(3, 32768, 5120), (16, 151936, 2560)])
+def test_a_named_int4_tile_decides_the_rows_of_a_large_weight(m, n, k):
+    """w4_gemm_deep names the tile of 3..16 rows, or none, whatever the library would choose for the size."""
+    lib = _native.load()
+    streams = lib._ZN3cmi17gemv_w4a8_streamsEiii
+    streams.restype = ctypes.c_bool
+    try:
+        assert streams(m, n, k)
+        for option, tiles in ((1, False), (1664, True), (4864, True)):
+            assert lib.cmi_set_option(b"w4_gemm_deep", option) == _native.OK
+            assert not streams(m, n, k), option
+            assert G.chosen_tile("_ZN3cmi20w4a8_rows_take_tilesEiiiPi", m, n, k)[0] == tiles, option
+    finally:
+        lib.cmi_set_option(b"w4_gemm_deep", 0)
+
+
 @pytest.mark.parametrize("m,n,k,gs,tile", [(256, 2700, 11008, 128, 12), (150, 4245, 3840, 128, 12), (64, 9393, 3328, 128, 0), (80, 11008, 2048, 256, 0),
                                            (200, 4805, 13568, 256, 0), (1024, 2560, 9728, 256, 0), (300, 6617, 17920, 256, 0),
                                            (40, 2560, 9728, 64, 0), (35, 1582, 17920, 128, 11), (40, 2560, 9728, 128, 11), (100, 2560, 9728, 128, 13),
