@@ -156,6 +156,30 @@ __device__ __forceinline__ void transposed_level(const float (&in)[2 * H], float
     }
 }
 
+// Rows 0 + 1 and 2 + 3 of the wavefront: even rows hold the sums of a, odd ones those of b.
+__device__ __forceinline__ float swap16_add(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// The two halves of the wavefront, likewise.
+__device__ __forceinline__ float swap32_add(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// The wave sums of two values in one tree, with the pairing of wave_sum_to_lane63: lanes 0 and 1 end with the totals of a and b.
+// Which of the two a lane keeps (bits 0 and 2 of its number differ: b) is the same for its partners of all later levels.
+__device__ __forceinline__ float wave_sum_pair(float a, float b, int lane) {
+    const float v[2] = {a, b};
+    float t[1];
+    transposed_level<0xB1, 1>(v, t, ((lane ^ (lane >> 2)) & 1) != 0);  // quad_perm [1,0,3,2]
+    t[0] += dpp_f32<0x4E, 0xf>(t[0]);                                   // quad_perm [2,3,0,1]
+    t[0] += dpp_f32<0x141, 0xf>(t[0]);                                  // row_half_mirror
+    t[0] += dpp_f32<0x140, 0xf>(t[0]);                                  // row_mirror
+    t[0] = swap16_add(t[0], t[0]);
+    return swap32_add(t[0], t[0]);
+}
+
 // Max over the 64 lanes; every lane of row 3 ends with the wave maximum, lane
 // 63 included.  Inputs must be >= 0 (masked lanes contribute 0).
 __device__ __forceinline__ float wave_max_to_lane63(float v) {

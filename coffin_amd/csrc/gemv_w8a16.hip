@@ -19,9 +19,10 @@
 //     total (not from 0.f);
 //   - the per-row weight scale multiplies that sum once, then one bf16 rounding.
 //
-// The MFMA's 16 blocks of 4 x 4 outputs cost what the eight v_dot2 did that they replace (one row: every shape within 1 %,
-// 2560 -> 151936 54.6 -> 54.2 us) though only the diagonal is wanted here; with several activation rows every output is, and
-// the kernels for those read the weight at the speed of one row.  (v_dot2 rounds after two products, so
+// Of the MFMA's 16 blocks of 4 x 4 outputs only the diagonal is wanted here, and it costs about what eight v_dot2 would (one
+// row, chains of v_dot2 -> these: 2560 -> 151936 58.9 -> 58.7 us, 4096 -> 128256 78.1 -> 78.5, 3584 -> 120000 64.8 -> 65.5, and
+// 1-2 % more where a launch is one round of latencies: 4608 -> 340 2.76 -> 2.82); with several activation rows every output is, and the
+// kernels for those read the weight at the speed of one row.  (v_dot2 rounds after two products, so
 // chains of both kinds cannot be mixed: the order is the MFMA's for every count.)
 //
 // Execution: one wavefront = (block of R weight rows, one unit of K).  All of a
@@ -36,9 +37,11 @@
 // returns data in issue order -- and every wavefront reads its fragments from
 // there.  When K spans several units the wavefronts of a team each take units
 // of the same rows and the unit totals meet in LDS (summed in unit order by one
-// lane per output); otherwise lane 63, which holds the tree result, scales and
-// stores.  A single activation row against a K of two or three units (and against a
-// mid-sized weight with K in one unit) takes gemv_w8a16_wholerow_kernel instead: one
+// lane per output); otherwise the lanes that hold the tree results scale and
+// store them.  Two weight rows share one tree (wave_sum_pair) and one store: what a wavefront does after its last bytes have
+// arrived is time in which it has none in flight (1024 -> 151936 28.7 -> 27.3 us).
+// A single activation row against a K of two or three units (and against a
+// mid-sized weight with K in one unit, from 2305 on) takes gemv_w8a16_wholerow_kernel instead: one
 // wavefront per weight row, all units.
 
 #include "gemv_w8a16_math.hpp"
@@ -68,6 +71,10 @@ struct GemvArgs {
 // stages the whole activation row for two weight rows; workgroups of 6, 9 and 12 wavefronts stage
 // less and measured 8.6, 9.3 and 9.7 us against 7.3.)
 constexpr int BLOCK_WAVES = 4;
+
+// Wavefronts per SIMD the compiler is to leave room for.  No kernel here needs more than 128 registers; told so, the compiler
+// forms the MFMA sums in the ordinary ones instead of accumulation registers that each sum has to be copied out of.
+constexpr int MIN_SIMD_WAVES = 4;
 
 // uint4 vectors of the LDS copy of the activations.
 //   K one unit: [row][segment][lane][half], i.e. a row as it is in memory, padded
@@ -99,7 +106,7 @@ struct WStage {
 //       reads them from global memory (only when they do not fit).
 // XV: 16-byte vectors of activations each thread carries from global memory to LDS.
 template <int M, int R, int CHT, bool MULTI, bool XLDS, int XV>
-__global__ void __launch_bounds__(64 * BLOCK_WAVES)
+__global__ void __launch_bounds__(64 * BLOCK_WAVES, MIN_SIMD_WAVES)
 gemv_w8a16_kernel(const GemvArgs a) {
     extern __shared__ uint4 smem[];  // staged activations (XLDS, see xlds_vectors), then unit totals
     const int lane = threadIdx.x & 63;
@@ -176,9 +183,9 @@ gemv_w8a16_kernel(const GemvArgs a) {
 #pragma unroll
             for (int m = 0; m < M; ++m) acc[r][m] = v4f32{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int r = 0; r < R; ++r)
+        for (int j = 0; j < CHT; ++j)
 #pragma unroll
-            for (int j = 0; j < CHT; ++j) {
+            for (int r = 0; r < R; ++r) {
                 const Chunk w = widen_chunk(ws_.w[r][j]);
 #pragma unroll
                 for (int m = 0; m < M; ++m) acc[r][m] = chain_chunk(acc[r][m], w, xs_.x[m][j][0], xs_.x[m][j][1]);
@@ -203,21 +210,12 @@ gemv_w8a16_kernel(const GemvArgs a) {
     }
     WStage<R, CHT> w0;
     load_w(w0, min(u, a.units - 1));
-    // Row scales: uniform per wavefront, but fetched as vector loads behind the weights (the
+    // The scale of the output that this lane stores, requested behind the weights and by vector loads (with one weight row the
     // opaque zero keeps the address in a vector register).  As scalar loads they would share the
     // LDS counter and sit in front of the barrier of the activation hand-over.
-    int vzero = 0;
-    asm volatile("" : "+v"(vzero));
-    float scale[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int n = rb * R + r;
-        scale[r] = a.ws[(n < a.N ? n : a.N - 1) + vzero];
-    }
-    // several units: the lane that adds the unit totals of output (r, m) = (lane / M, lane % M)
-    // scales it; its scale is requested here, not cold at the end
-    float scale_fin = 0.f;
-    if constexpr (MULTI) scale_fin = a.ws[min(rb * R + min(lane / M, R - 1), a.N - 1)];
+    int srow = MULTI ? min(lane / M, R - 1) : R == 2 ? lane & 1 : 0;
+    asm volatile("" : "+v"(srow));
+    const float scale = a.ws[min(rb * R + srow, a.N - 1)];
     if constexpr (XLDS) {
 #pragma unroll
         for (int j = 0; j < XV; ++j) {
@@ -239,7 +237,10 @@ gemv_w8a16_kernel(const GemvArgs a) {
         __syncthreads();
     }
 
-    float tot[R][M];
+    // the lanes that hold the totals, one weight row each (wave_sum_pair: lanes 0 and 1)
+    const bool holds = R == 2 ? lane < 2 : lane == 63;
+    const int hrow = R == 2 ? lane & 1 : 0;
+    float tot[M];
 #pragma unroll 1
     for (; u < a.units; u += a.uw) {
         if (idle) break;
@@ -248,31 +249,24 @@ gemv_w8a16_kernel(const GemvArgs a) {
         compute(w0, x0);
         if (MULTI && u + a.uw < a.units) load_w(w0, u + a.uw);  // next unit of this wavefront
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int m = 0; m < M; ++m) tot[r][m] = wave_sum_to_lane63(own_chain(acc[r][m], lane));
+        for (int m = 0; m < M; ++m) {
+            if constexpr (R == 2) tot[m] = wave_sum_pair(own_chain(acc[0][m], lane), own_chain(acc[1][m], lane), lane);
+            else tot[m] = wave_sum_to_lane63(own_chain(acc[0][m], lane));
+        }
         if constexpr (!MULTI) break;
         // unit totals meet in LDS; one lane per output adds them in unit order below
-        if (lane == 63) {
+        if (holds) {
 #pragma unroll
-            for (int r = 0; r < R; ++r)
-#pragma unroll
-                for (int m = 0; m < M; ++m) unit_total[u * (R * M) + r * M + m] = tot[r][m];
+            for (int m = 0; m < M; ++m) unit_total[u * (R * M) + hrow * M + m] = tot[m];
         }
     }
 
     if constexpr (!MULTI) {
-        if (!idle && lane == 63) {
+        const int n = rb * R + hrow;
+        if (!idle && holds && n < a.N) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int n = rb * R + r;
-                if (n < a.N) {
-#pragma unroll
-                    for (int m = 0; m < M; ++m)
-                        if (m < a.M)
-                            a.y[(size_t)m * a.N + n] = (uint16_t)f32_to_bf16_bits(scale[r] * tot[r][m]);
-                }
-            }
+            for (int m = 0; m < M; ++m)
+                if (m < a.M) a.y[(size_t)m * a.N + n] = (uint16_t)f32_to_bf16_bits(scale * tot[m]);
         }
     } else {
         __syncthreads();
@@ -282,7 +276,7 @@ gemv_w8a16_kernel(const GemvArgs a) {
             if (n < a.N && m < a.M) {
                 float total = unit_total[lane];
                 for (int v = 1; v < a.units; ++v) total += unit_total[v * (R * M) + lane];
-                a.y[(size_t)m * a.N + n] = (uint16_t)f32_to_bf16_bits(scale_fin * total);
+                a.y[(size_t)m * a.N + n] = (uint16_t)f32_to_bf16_bits(scale * total);
             }
         }
     }
@@ -294,7 +288,7 @@ gemv_w8a16_kernel(const GemvArgs a) {
 // workgroup of W wavefronts stages the activation row once for W weight rows (the team
 // arrangement of the general kernel stages it once per two rows).  Same bits.
 template <int CHT, int NU, int XV>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, MIN_SIMD_WAVES)
 gemv_w8a16_wholerow_kernel(const GemvArgs a) {
     extern __shared__ uint4 smem[];  // the activation row, then one zeroed 32-byte slot
     const int lane = threadIdx.x & 63;
@@ -372,14 +366,13 @@ int dispatch_wholerow(const GemvArgs &a, hipStream_t st) {
     if (a.units == 1) {
         // K in one unit: the general kernel is as good or better for small launches (one weight row per
         // wavefront there too, padded activation copy without selects: 4096 -> 2560 3.85 against 3.91 us)
-        // and for very tall weights; in between this kernel is 2-4 % faster (2560 -> 19456 9.7 -> 9.4 us,
-        // 2560 -> 9728 6.03 -> 5.81 us; two weight rows per wavefront here measured slower again).
+        // and for very tall weights; in between this kernel is 1-4 % faster (2560 -> 19456 10.1 -> 9.7 us, 3072 -> 40000 21.1 -> 20.4)
+        // while a row is long enough to keep the memory busy by itself.  Up to 2304 the general kernel's two rows a wavefront are
+        // (2048 -> 40000 16.4 -> 14.6 us, 1536 -> 60000 20.3 -> 16.4, 1040 -> 126030 34.3 -> 25.3, 2112 -> 39718 16.3 -> 15.2;
+        // 2304 -> 56888 23.6 -> 23.1, 2432 -> 53894 22.5 against 23.2).
         const size_t wbytes = (size_t)a.N * a.K;
-        if (wbytes <= ((size_t)20 << 20) || wbytes > ((size_t)128 << 20)) return CMI_E_UNSUPPORTED;
-        if (a.unit == 4) return launch_wholerow<4, 1>(a, st);
-        if (a.unit == 3) return launch_wholerow<3, 1>(a, st);
-        if (a.unit == 2) return launch_wholerow<2, 1>(a, st);
-        return CMI_E_UNSUPPORTED;
+        if (a.K <= 2304 || wbytes <= ((size_t)20 << 20) || wbytes > ((size_t)128 << 20)) return CMI_E_UNSUPPORTED;
+        return a.unit == 4 ? launch_wholerow<4, 1>(a, st) : launch_wholerow<3, 1>(a, st);
     }
     if (a.units == 2) {
         if (a.unit == 4) return launch_wholerow<4, 2>(a, st);

@@ -95,16 +95,6 @@ __device__ __forceinline__ void quad_transpose(u32x4 (&w)[4]) {
     }
 }
 
-typedef unsigned u32x2_swap __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float swap32_add(float a, float b) {
-    const u32x2_swap r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r.x) + __uint_as_float(r.y);
-}
-__device__ __forceinline__ float swap16_add(float a, float b) {
-    const u32x2_swap r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r.x) + __uint_as_float(r.y);
-}
-
 // Sums over the 16 blocks of a wavefront of 4 MG values a lane (value 4 * group + weight row), pairing blocks b ^ 1, b ^ 2, b ^ 4,
 // b ^ 8 in this order.  Lanes l ^ 7 and l ^ 15 are the pairs of the first two levels (see lane_row; the half that a lane keeps is chosen
 // so that its partner at the next level keeps the same one), then rows and halves of the wavefront.  While values are left to

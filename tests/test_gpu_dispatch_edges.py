@@ -518,6 +518,24 @@ def test_batches_of_weight_only_rows_carry_the_single_row_bits(m, n, k):
         assert ((got[finite[0]].double() - exact).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("n,k", [(20479, 1024), (20481, 1024), (131, 1040), (20301, 1040), (130001, 1040), (9103, 2304), (9041, 2320), (52429, 2560),
+                                 (32769, 4096), (7, 16400), (1025, 20496)])
+def test_one_weight_only_row_where_two_weight_rows_share_a_tree(n, k):
+    """Both sides of the rules for one or two weight rows a wavefront and for a wavefront a whole row, odd outputs, several units: the bits of
+    the batch kernels' rows, and the exact sum."""
+    gen = torch.Generator(device=G.DEV).manual_seed(n + k)
+    wq = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=G.DEV, generator=gen)
+    ws = torch.rand(n, device=G.DEV, generator=gen) * 0.01 + 1e-3
+    x = torch.randn((1, k), device=G.DEV, generator=gen).to(torch.bfloat16)
+    y = torch.full((n + 64,), -77.0, dtype=torch.bfloat16, device=G.DEV)
+    _native.check(_native.load().cmi_gemv_w8a16(G.ptr(wq), G.ptr(ws), G.ptr(x), G.ptr(y), 1, n, k, G.stream()), "gemv")
+    assert torch.equal(y[:n].view(torch.int16), G.gemv_w8a16(wq, ws, x.expand(4, k).contiguous())[3].view(torch.int16)) and (y[n:] == -77.0).all()
+    xd, wd = x[0].double(), wq.double()
+    exact = (wd @ xd) * ws.double()
+    bound = exact.abs() * 2.0 ** -8 + (wd.abs() @ xd.abs()) * ws.double() * (k * 2.0 ** -24)
+    assert ((y[:n].double() - exact).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("m,n,k", [(3, 655361, 256), (16, 145637, 1152), (9, 65543, 2560), (5, 62425, 2688), (4, 32768, 5120), (13, 33333, 5120)])
 def test_rows_of_a_large_int4_weight_carry_the_small_weights_bits(m, n, k):
     """One line to the longest rows, odd counts of groups, rows and outputs, at the rule's edge: the bits of the kernels

@@ -5,7 +5,7 @@ coffin_amd/csrc/common.hpp sums the 64 lane chains of a unit with a fixed tree
 bits of the single-row call (reference contract: models/qwen35/batch.py:19-22), so a
 transposing reduction -- several values per lane together, each lane keeping half
 of its values per level -- has to build exactly that tree for every value: over whole wavefronts
-(wave_sum_transposed below), and over the 16 blocks of four lanes that the batch kernels' MFMA
+(wave_sum_pair), and over the 16 blocks of four lanes that the batch kernels' MFMA
 steps work on (quarter_sum of gemv_w8a16_batch.hip).  Here both are run on
 symbols, with fp32 addition modelled as an unordered pair (it commutes bit for bit and does not
 associate), the cross-lane moves modelled after the ISA (DPP quad_perm / row_half_mirror /
@@ -87,67 +87,26 @@ def level(vals, ctrl, half, upper):
     return out
 
 
-def transposed(nv, vals):
-    """wave_sum_transposed<nv>: what every lane ends with."""
-    a1 = level(vals, 0xB1, nv // 2, lambda l: (l ^ (l >> 2)) & 1)
-    a2 = level(a1, 0x4E, nv // 4, lambda l: ((l >> 1) ^ (l >> 2)) & 1)
-    a3 = level(a2, 0x141, nv // 8, lambda l: ((l >> 2) ^ (l >> 3)) & 1)
-    if nv == 8:
-        d = dpp(a3[0], 0x140)
-        t = [add(a3[0][lane], d[lane]) for lane in range(64)]
-    else:
-        a4 = level(a3, 0x140, nv // 16, lambda l: (l >> 3) & 1)
-        if nv == 32:
-            x, y = swap16(a4[0], a4[1])
-            t = [add(x[lane], y[lane]) for lane in range(64)]
-        else:
-            t = a4[0]
-    if nv != 32:
-        x, y = swap16(t, t)
+def pair(vals, upper=lambda l: (l ^ (l >> 2)) & 1):
+    """wave_sum_pair of two values: what every lane ends with."""
+    t = level(vals, 0xB1, 1, upper)[0]
+    for ctrl in (0x4E, 0x141, 0x140):
+        d = dpp(t, ctrl)
+        t = [add(t[lane], d[lane]) for lane in range(64)]
+    for swap in (swap16, swap32):
+        x, y = swap(t, t)
         t = [add(x[lane], y[lane]) for lane in range(64)]
-    x, y = swap32(t, t)
-    return [add(x[lane], y[lane]) for lane in range(64)]
+    return t
 
 
-def index(nv, lane):
-    """wave_sum_transposed_index<nv>."""
-    s1 = (lane ^ (lane >> 2)) & 1
-    s2 = ((lane >> 1) ^ (lane >> 2)) & 1
-    s3 = ((lane >> 2) ^ (lane >> 3)) & 1
-    s4 = (lane >> 3) & 1
-    s5 = (lane >> 4) & 1
-    return {8: s1 * 4 + s2 * 2 + s3,
-            16: s1 * 8 + s2 * 4 + s3 * 2 + s4,
-            32: s1 * 16 + s2 * 8 + s3 * 4 + s4 * 2 + s5}[nv]
-
-
-@pytest.mark.parametrize("nv", [8, 16, 32])
-def test_transposing_reduction_builds_the_plain_tree(nv):
-    vals = [[(i, lane) for lane in range(64)] for i in range(nv)]
-    want = [original(vals[i]) for i in range(nv)]
-    got = transposed(nv, vals)
+def test_two_rows_of_one_tree_are_the_plain_trees():
+    vals = [[(i, lane) for lane in range(64)] for i in range(2)]
+    got = pair(vals)
     for lane in range(64):
-        assert got[lane] == want[index(nv, lane)], (nv, lane)
-    # the lanes that store cover every value exactly once
-    assert sorted(index(nv, lane) for lane in range(nv)) == list(range(nv))
-
-
-def test_a_different_choice_of_halves_is_caught():
-    """Keeping halves by the plain lane bit at the quad level pairs lanes that hold different
-    values at the next level: the model must tell the two apart."""
-    nv = 8
-    vals = [[(i, lane) for lane in range(64)] for i in range(nv)]
-    a1 = level(vals, 0xB1, 4, lambda l: l & 1)          # plain bit 0 instead of b0 ^ b2
-    a2 = level(a1, 0x4E, 2, lambda l: (l >> 1) & 1)
-    a3 = level(a2, 0x141, 1, lambda l: (l >> 2) & 1)
-    want = [original(vals[i]) for i in range(nv)]
-    d = dpp(a3[0], 0x140)
-    t = [add(a3[0][l], d[l]) for l in range(64)]
-    x, y = swap16(t, t)
-    t = [add(x[l], y[l]) for l in range(64)]
-    x, y = swap32(t, t)
-    got = [add(x[l], y[l]) for l in range(64)]
-    assert any(got[lane] not in want for lane in range(64))
+        assert got[lane] == original(vals[(lane ^ (lane >> 2)) & 1]), lane
+    assert got[0] == original(vals[0]) and got[1] == original(vals[1])    # the lanes that store
+    # chosen by the plain bit, a lane and its partner of the half row hold different values
+    assert original(vals[0]) not in pair(vals, lambda l: l & 1)
 
 
 def batch(mg, vals):
