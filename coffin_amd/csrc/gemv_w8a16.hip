@@ -416,13 +416,19 @@ bool x_fits_lds(int M, int K, int units, int segs) {
     return lds <= XLDS_MAX_BYTES && (size_t)M * K * 2 <= 16 * (size_t)xstage_vectors(M) * (64 * uw * teams);
 }
 
-// Two rows that this file's kernel, which has a wavefront for every two weight rows and unit, takes faster than the batch kernels: K of several units and outputs too few
-// for those to stream (5120 -> 10000 13.0 against 14.3 us, 6400 -> 9000 14.9 against 17.0), or so few that a wavefront of theirs walks
-// several units (12800 -> 512 4.4 against 5.5, 9728 -> 256 3.8 against 4.6, 16384 -> 300 4.4 against 5.7; the other way 9728 -> 1024 5.4 against 5.2, 16384 -> 1024 6.8 either
-// way, 14336 -> 2560 13.0 against 10.5).
+// Two rows that this file's kernel, which has a wavefront for every two weight rows and unit, takes faster than the batch kernels (us, batch
+// kernel -> this one).
+//   One unit: more outputs than fit the chip's workgroups of the batch kernel at once, K > 1024 (1280 -> 8400 5.5 -> 4.7, 2560 -> 10000
+//   8.1 -> 7.1, 4096 -> 10000 11.3 -> 10.0, 2560 -> 151936 79.6 -> 63.4; 1728 -> 6000 4.1 against 4.3, 1024 -> 20000 5.9 against 6.8).  Short rows
+//   that do not start on whole lines only up to 16384 (1088 -> 12000 5.3 -> 5.2, 1088 -> 50000 14.8 against 15.5, 1152 -> 50000 17.6 -> 15.7).
+//   Several units: outputs too few for the batch kernel to stream (5120 -> 10000 14.3 -> 13.0, 6400 -> 9000 17.0 -> 14.9), or so few that a
+//   wavefront of it walks several units: 768 of three, 1152 of four (12800 -> 512 5.5 -> 4.4, 16384 -> 300 5.7 -> 4.4), and where it then has one
+//   workgroup for two CUs (1025..1536: 8320 -> 1200 6.4 -> 5.4, 9728 -> 1100 7.3 -> 6.0, 14336 -> 1300 8.5 -> 7.8;
+//   8320 -> 900 4.3 against 4.5, 9728 -> 1800 8.0 -> 7.4 but 11264 -> 1800 8.25 against 8.3, 16384 -> 1600 9.3 against 10.3).
 bool two_rows_stay(int N, int K, int units, int segs) {
-    if (units == 1 || !x_fits_lds(2, K, units, segs)) return false;
-    return (N > 8192 && (size_t)N * K < ((size_t)96 << 20)) || (units > 2 && N <= 384 * (units - 1));
+    if (units == 1) return K > 1024 && N > 8192 && (N <= 16384 || K % 128 == 0 || K > 2048);
+    if (!x_fits_lds(2, K, units, segs)) return false;
+    return (N > 8192 && (size_t)N * K < ((size_t)96 << 20)) || (units > 2 && (N <= 384 * (units - 1) || (N > 1024 && N <= 1536)));
 }
 
 template <int M, int R, int CHT, bool MULTI>

@@ -441,12 +441,13 @@ int run(BatchArgs &a, bool streamed, hipStream_t st) {
     const int rows = (a.N - 1) / 256 + 1;  // of a CU
     // Row blocks for every CU at once: 4 rg weight rows a team, up to four teams a workgroup.  Twelve rows a CU go one block a
     // wavefront (4096 -> 2560 at four rows 4.4 us, two blocks 4.9); above, two share the activation fragments.  Short rows and pairs of
-    // rows want small workgroups (1024 -> 8192 at four rows 3.9 with two blocks, 4.3 with eight; two rows of 2560 -> 6144 5.2 against 5.5), and so
-    // does everything beyond 32 rows a CU, where workgroups follow each other (2560 -> 19456 12.0 with four blocks, 13.9 with eight).
+    // rows want small workgroups (1024 -> 8192 at four rows 3.9 with two blocks, 4.3 with eight; 896 -> 1030 at three 2.62 with one
+    // block, 2.73 with two; two rows of 2560 -> 6144 5.2 against 5.5), and so does everything beyond 32 rows a CU, where workgroups
+    // follow each other (2560 -> 19456 12.0 with four blocks, 13.9 with eight).
     // Up to sixteen rows a CU of many units: four teams of one block (14336 -> 4096 at 4 / 8 rows 14.6 / 17.9 us, two of two 16.8 / 22.8; 9728 -> 3800
     // at four rows 11.0 against 10.7, at eight 12.6 against 17.2).
     int rg = 2;
-    if (rows <= 12) rg = 1, a.teams = (rows + 3) / 4;
+    if (rows <= 12) rg = 1, a.teams = MG == 1 && a.K <= 1024 ? 1 : (rows + 3) / 4;
     else if (MG <= 2 && a.K <= 1024) a.teams = MG;
     else if (a.M <= 2 && a.units == 1 && rows <= 32) a.teams = 1;
     else if (rows <= 16) rg = MG == 4 || a.units > (MG == 1 ? 3 : 2) ? 1 : 2, a.teams = 4 / rg;

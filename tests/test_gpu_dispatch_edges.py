@@ -491,7 +491,9 @@ def test_ragged_rows_take_the_matrix_pipe_where_the_call_site_may(monkeypatch, p
                                    (3, 200, 20496), (6, 500, 12304), (7, 2000, 33024), (4, 4096, 14336), (8, 3900, 9728), (6, 5000, 20496), (16, 300, 9728), (12, 5000, 6160), (9, 9300, 12304),
                                    (4, 5001, 2560), (8, 7000, 5136), (16, 8192, 1024), (2, 6000, 16), (13, 3333, 3072),
                                    (4, 32773, 4112), (5, 16385, 1040), (16, 9217, 2576), (15, 9301, 4096), (11, 4100, 5120),
-                                   (3, 20000, 5136), (8, 8193, 6160), (16, 16400, 6160)])
+                                   (3, 20000, 5136), (8, 8193, 6160), (16, 16400, 6160),
+                                   (2, 8192, 1040), (2, 8193, 1040), (2, 16385, 1040), (2, 16385, 1152), (2, 16387, 2064), (2, 9001, 4096), (2, 8200, 1024),
+                                   (2, 1025, 9744), (2, 1536, 12304), (2, 1537, 9744), (3, 1025, 1024), (4, 3072, 784)])
 def test_batches_of_weight_only_rows_carry_the_single_row_bits(m, n, k):
     """Every kernel that 2..16 rows of cmi_gemv_w8a16 take, at odd counts of rows, outputs and chunks: few outputs by quarters of a row
     (units dealt to wavefronts, one block or two a wavefront), long rows in windows, many outputs streamed, sixteen rows in two halves.
