@@ -423,8 +423,6 @@ extern "C" int cmi_gemv_w4a8(const uint8_t *w4, const float *ws, const int8_t *x
         const bool forced = option_w4_decode_chain() > 1 && M <= 2;  // a variant named by the caller
         int rc = CMI_E_UNSUPPORTED;
         int tile = 0;
-        // 80 MiB of codes and more: 5120 -> 32768 at 3 / 16 rows 18.5 against 18.9 / 19.3 against 19.9 us, 4096 -> 28672 (56 MiB) 14.6 against
-        // 14.0 / 15.3 against 15.3.
         if (!group_acc && gemv_w4a8_streams(M, N, K)) return gemv_w4a8_stream(w4, ws, xq, xs, y, M, N, K, stream);
         if (K >= GS && K % GS == 0 && !group_acc && w4a8_rows_take_tiles(M, N, K, &tile))
             return gemm_w4a8_tile(w4, ws, xq, xs, y, M, N, K, gs, tile, stream);

@@ -176,8 +176,9 @@ int launch(const Args &a, hipStream_t st) {
     static std::atomic<uint64_t> devices{0};
     if (const int rc = reserve_lds(reinterpret_cast<const void *>(k), shared_bytes(MAX_G) + WAVES * wave_bytes(MAX_G), devices, "cmi_gemv_w4a8"))
         return rc;
-    const int blocks = (a.tiles + WAVES - 1) / WAVES;
-    k<<<dim3(blocks < 256 ? blocks : 256), dim3(WAVES * 64), shared_bytes(a.G) + WAVES * wave_bytes(a.G), st>>>(a);
+    // One workgroup per CU although some wavefronts of each then have no tile: as few workgroups as the tiles fill left 5120 -> 32768 to 128 CUs
+    // (18.8 us, 23.6 so; 3968 -> 42281 21.8, 26.1).
+    k<<<dim3(a.tiles < 256 ? a.tiles : 256), dim3(WAVES * 64), shared_bytes(a.G) + WAVES * wave_bytes(a.G), st>>>(a);
     return check_launch("cmi_gemv_w4a8");
 }
 
@@ -185,7 +186,15 @@ int launch(const Args &a, hipStream_t st) {
 
 bool cmi::gemv_w4a8_streams(int M, int N, int K) {
     if (option_w4_gemm_deep() != 0) return false;  // the caller names the tile of 3..16 rows, or the GEMV
-    return M >= 3 && M <= 16 && K % GS == 0 && K >= 2 * GS && K <= 5120 && (size_t)N * K >= (size_t)160 << 20;
+    if (M < 3 || M > 16 || K % GS != 0 || K < 2 * GS || K > 5120) return false;
+    // From 80 MiB of codes; us, the kernels of the smaller weights against this one at 3 / 16 rows: 5120 -> 32768 18.7, 18.8 / 20.1, 19.8, 3072 -> 54613
+    // 21.3, 19.6 / 26.1, 20.6, 512 -> 327680 24.8, 21.2 / 29.4, 22.9.  The others stay longer for few rows of few lines, each a
+    // larger share of a tile's fixed steps: up to four rows to 88 MiB below K = 2560 (2048 -> 82432 at 3 rows 19.9, 20.7, 2304 -> 81920 23.3, 21.6),
+    // up to eight to 112 at K = 1024 (184320 outputs at 3 rows 21.1, 22.7, 276480 30.1, 29.8), and where besides the last line is half empty always
+    // (896 -> 315977 33.4, 35.9; 1152 -> 245760 34.0, 34.3, from five rows on 35.5, 34.8).
+    const size_t codes = (size_t)N * K / 2, mib = (size_t)1 << 20;
+    if (M <= 8 && K > 768 && K < 1280) return K % (2 * GS) == 0 ? codes >= 112 * mib : K > 1024 && M > 4 && codes >= 80 * mib;
+    return codes >= (M <= 4 && K > 768 && K < 2560 ? 88 : 80) * mib;
 }
 
 int cmi::gemv_w4a8_stream(const uint8_t *w4, const float *ws, const int8_t *xq, const float *xs, void *y, int M, int N, int K, void *stream) {

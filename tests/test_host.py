@@ -429,6 +429,18 @@ def test_int4_rows_take_tiles_only_where_they_gain_more_than_the_models_err(m, n
     assert G.chosen_tile("_ZN3cmi20w4a8_rows_take_tilesEiiiPi", m, n, k)[0] == tiles
 
 
+@pytest.mark.parametrize("m,n,k,streams", [(16, 32768, 5120, True), (16, 32767, 5120, False), (3, 54613, 3072, False), (3, 54614, 3072, True),
+                                           (3, 82432, 2048, False), (3, 92160, 2048, True), (9, 82432, 2048, True), (3, 184320, 1024, False),
+                                           (4, 276480, 1024, True), (16, 164864, 1024, True), (4, 1000000, 896, False), (8, 315977, 896, False),
+                                           (12, 234057, 896, True), (3, 245760, 1152, False), (6, 163840, 1152, True), (5, 82432, 2048, True), (3, 327680, 512, True), (3, 163840, 1280, True),
+                                           (2, 151936, 2560, False), (17, 151936, 2560, False), (3, 151936, 5248, False), (3, 1400000, 128, False)])
+def test_int4_rows_of_large_weights_stream_where_that_is_the_faster_kernel(m, n, k, streams):
+    """Both sides of the rule; inside it, sizes measured to be at most 3 % faster on the other side."""
+    fn = _native.load()._ZN3cmi17gemv_w4a8_streamsEiii
+    fn.restype = ctypes.c_bool
+    assert fn(m, n, k) == streams
+
+
 @pytest.mark.parametrize("m,n,k", [(3, 32768, 5120), (16, 151936, 2560)])
 def test_a_named_int4_tile_decides_the_rows_of_a_large_weight(m, n, k):
     """w4_gemm_deep names the tile of 3..16 rows, or none, whatever the library would choose for the size."""
