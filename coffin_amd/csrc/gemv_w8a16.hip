@@ -86,10 +86,8 @@ __host__ __device__ constexpr int xlds_vectors(int rows, int K, int segs, bool o
     return one_unit ? rows * segs * 128 : rows * (K / 8) + 2;
 }
 
-// 16-byte vectors of activations each thread can carry from global memory to LDS, and the
-// short variant that covers the decode shapes (e.g. K up to 4096 for one row).
-constexpr int xstage_vectors(int m) { return m <= 1 ? 8 : 16; }
-constexpr int xstage_short(int m) { return m <= 1 ? 2 : 4; }
+// 16-byte vectors of activations each thread can carry from global memory to LDS: K of one unit is at most 4096, and 256 threads carry it.
+constexpr int xstage_vectors(int m, bool multi) { return (multi ? 8 : 2) * m; }
 
 template <int M, int CHT>
 struct XStage {
@@ -104,8 +102,7 @@ struct WStage {
 // MULTI: several units (totals via LDS); else K is one unit.  A unit is CHT segments, all its loads up front.
 // XLDS: the workgroup stages the activations in LDS; otherwise each wavefront
 //       reads them from global memory (only when they do not fit).
-// XV: 16-byte vectors of activations each thread carries from global memory to LDS.
-template <int M, int R, int CHT, bool MULTI, bool XLDS, int XV>
+template <int M, int R, int CHT, bool MULTI, bool XLDS>
 __global__ void __launch_bounds__(64 * BLOCK_WAVES, MIN_SIMD_WAVES)
 gemv_w8a16_kernel(const GemvArgs a) {
     extern __shared__ uint4 smem[];  // staged activations (XLDS, see xlds_vectors), then unit totals
@@ -196,6 +193,7 @@ gemv_w8a16_kernel(const GemvArgs a) {
     // wavefront waits for must have been requested before the long weight
     // stream), then all first-trip weights, then the LDS hand-over: the copy and
     // its barrier run in the shadow of the weight latency.
+    constexpr int XV = xstage_vectors(M, MULTI);
     uint4 xstage[XV];
     const int xtotal = a.M * xvecs;
     if constexpr (XLDS) {
@@ -397,13 +395,13 @@ int weight_rows(int M, int N, int K, int units) {
     return M == 1 && units == 1 && (size_t)N * K <= ((size_t)20 << 20) ? 1 : 2;
 }
 
-template <int M, int R, int CHT, bool MULTI, bool XLDS, int XV>
-int launch_xv(const GemvArgs &a, const dim3 grid, const dim3 block, size_t lds, hipStream_t st) {
+template <int M, int R, int CHT, bool MULTI, bool XLDS>
+int launch_x(const GemvArgs &a, const dim3 grid, const dim3 block, size_t lds, hipStream_t st) {
     static std::atomic<uint64_t> devices{0};
-    if (const int rc = reserve_lds(reinterpret_cast<const void *>(gemv_w8a16_kernel<M, R, CHT, MULTI, XLDS, XV>),
-                                   128 * 1024, devices, "cmi_gemv_w8a16"))
+    if (const int rc = reserve_lds(reinterpret_cast<const void *>(gemv_w8a16_kernel<M, R, CHT, MULTI, XLDS>), 128 * 1024, devices,
+                                   "cmi_gemv_w8a16"))
         return rc;
-    gemv_w8a16_kernel<M, R, CHT, MULTI, XLDS, XV><<<grid, block, lds, st>>>(a);
+    gemv_w8a16_kernel<M, R, CHT, MULTI, XLDS><<<grid, block, lds, st>>>(a);
     return check_launch("cmi_gemv_w8a16");
 }
 
@@ -413,7 +411,7 @@ bool x_fits_lds(int M, int K, int units, int segs) {
     const int teams = BLOCK_WAVES / uw;
     // the unit totals share the allocation: one float per (team, unit, weight row, activation row)
     const size_t lds = 16 * (size_t)xlds_vectors(M, K, segs, units == 1) + (units > 1 ? sizeof(float) * teams * units * 4 * M : 0);
-    return lds <= XLDS_MAX_BYTES && (size_t)M * K * 2 <= 16 * (size_t)xstage_vectors(M) * (64 * uw * teams);
+    return lds <= XLDS_MAX_BYTES && (size_t)M * K * 2 <= 16 * (size_t)xstage_vectors(M, units > 1) * (64 * uw * teams);
 }
 
 // Two rows that this file's kernel, which has a wavefront for every two weight rows and unit, takes faster than the batch kernels (us, batch
@@ -441,11 +439,9 @@ int launch(GemvArgs &a, hipStream_t st) {
     const dim3 block(64 * a.uw * a.teams);
     const size_t totals = MULTI ? sizeof(float) * a.teams * a.units * R * M : 0;
     const int segs = a.units * a.unit;
-    if (!x_fits_lds(a.M, a.K, a.units, segs)) return launch_xv<M, R, CHT, MULTI, false, 1>(a, grid, block, totals, st);
-    const size_t lds = 16 * (size_t)xlds_vectors(a.M, a.K, segs, !MULTI) + totals;
-    if ((size_t)a.M * (a.K / 8) <= (size_t)xstage_short(M) * block.x)
-        return launch_xv<M, R, CHT, MULTI, true, xstage_short(M)>(a, grid, block, lds, st);
-    return launch_xv<M, R, CHT, MULTI, true, xstage_vectors(M)>(a, grid, block, lds, st);
+    if constexpr (MULTI && M == 1 && CHT == 4)  // (units of three segments fit, and two rows that do not are the batch kernels')
+        if (!x_fits_lds(a.M, a.K, a.units, segs)) return launch_x<M, R, CHT, MULTI, false>(a, grid, block, totals, st);
+    return launch_x<M, R, CHT, MULTI, true>(a, grid, block, 16 * (size_t)xlds_vectors(a.M, a.K, segs, !MULTI) + totals, st);
 }
 
 template <int M, int R>
@@ -454,7 +450,8 @@ int by_unit(GemvArgs &a, hipStream_t st) {
         if constexpr (R == 2) return a.unit == 3 ? launch<M, R, 3, true>(a, st) : launch<M, R, 4, true>(a, st);
         return fail(CMI_E_UNSUPPORTED, "cmi_gemv_w8a16: no kernel for %d weight rows and several units", R);
     }
-    if (a.unit == 1) return launch<M, R, 1, false>(a, st);
+    if constexpr (M == 1)  // (two rows that short are the batch kernels')
+        if (a.unit == 1) return launch<M, R, 1, false>(a, st);
     if (a.unit == 2) return launch<M, R, 2, false>(a, st);
     if (a.unit == 3) return launch<M, R, 3, false>(a, st);
     return launch<M, R, 4, false>(a, st);

@@ -388,51 +388,83 @@ int launch_quarters(BatchArgs &a, hipStream_t st) {
 // Whether every activation row fits LDS as the stream kernel holds it.
 bool stream_fits(int mg, int segs) { return (size_t)segs * mg * 8192 <= LDS_BYTES; }
 
+constexpr int up(int v, int d) { return (v + d - 1) / d; }
+
+// Only forms that some row count and K reach are built: with U segments a unit K is above (U - 1) * 1024, one unit is at most U * 1024, and
+// units of three (unit_segments) are of 5, 6 or 9 segments.  A count outside what a form was built for is an error, never a short copy.
+template <int MG>
+constexpr int least_rows() { return MG == 1 ? 1 : MG == 2 ? 5 : 9; }
+
+int unbuilt(const BatchArgs &a) { return fail(CMI_E_UNSUPPORTED, "cmi_gemv_w8a16: no kernel for %d rows of %d", a.M, a.K); }
+
 template <int MG, int U>
 int stream(const BatchArgs &a, hipStream_t st) {
     if constexpr (MG == 1)
         if (a.segs <= 6 && a.M * (a.K / 8) <= 8 * 512) return launch_stream<MG, U, 8, 8, 2>(a, st);
-    constexpr int WAVES = MG == 4 && U == 4 ? 8 : 12;  // 16 rows and four segments in flight take more than 168 registers
-    const int need = (a.M * (a.K / 8) + 64 * WAVES - 1) / (64 * WAVES);
-    if (need <= 3) return launch_stream<MG, U, 3, WAVES, 1>(a, st);
-    if (need <= 7) return launch_stream<MG, U, 7, WAVES, 1>(a, st);
-    return launch_stream<MG, U, WAVES == 8 ? 20 : 14, WAVES, 1>(a, st);
+    if constexpr (MG > 1 || U >= 3) {
+        constexpr int WAVES = MG == 4 && U == 4 ? 8 : 12;  // 16 rows and four segments in flight take more than 168 registers
+        constexpr int LAST = WAVES == 8 ? 20 : 14;
+        constexpr int LONGEST = U <= 2 ? U * 1024 : U == 3 && MG < 4 ? 9216 : 20480 / MG;  // stream_fits
+        constexpr int LEAST = up(least_rows<MG>() * ((U - 1) * 128 + 2), 64 * WAVES), MOST = up(4 * MG * (LONGEST / 8), 64 * WAVES);
+        const int need = up(a.M * (a.K / 8), 64 * WAVES);
+        if constexpr (LEAST <= 3)
+            if (need <= 3) return launch_stream<MG, U, 3, WAVES, 1>(a, st);
+        if constexpr (MOST > 3)
+            if (need <= 7) return launch_stream<MG, U, 7, WAVES, 1>(a, st);
+        if constexpr (MOST > 7)
+            if (need <= LAST) return launch_stream<MG, U, LAST, WAVES, 1>(a, st);
+    }
+    return unbuilt(a);
 }
 
 template <int MG, int RG, int U, bool ONE>
 int by_vectors(BatchArgs &a, int need, hipStream_t st) {
-    if (need <= 4) return launch_quarters<MG, RG, U, 1, ONE, false, 4>(a, st);
-    if (need <= 8) return launch_quarters<MG, RG, U, 1, ONE, false, 8>(a, st);
-    if (need <= 12) return launch_quarters<MG, RG, U, 1, ONE, false, 12>(a, st);
-    return launch_quarters<MG, RG, U, 1, ONE, false, 16>(a, st);
+    // most of one unit: of the smallest workgroup (run); of several: of three teams, as fewer have sets, or of sixteen wavefronts.  Least of several: of
+    // sixteen wavefronts, which one block a wavefront at eight rows has above K = 8192
+    constexpr int THREADS = 256 * (RG == 1 ? 1 : MG == 4 ? 3 : 2);
+    constexpr int LEAST = ONE ? 1 : up(least_rows<MG>() * (U == 3 ? 514 : MG == 2 && RG == 1 ? 1026 : 770), 1024);
+    constexpr int MOST = ONE ? up(MG * U * 512, THREADS) : MG == 1 && RG == 1 && U == 3 ? up(4 * 1152, 768) : 12;
+    if constexpr (LEAST <= 4)
+        if (need <= 4) return launch_quarters<MG, RG, U, 1, ONE, false, 4>(a, st);
+    if constexpr (MOST > 4)
+        if (need <= 8) return launch_quarters<MG, RG, U, 1, ONE, false, 8>(a, st);
+    if constexpr (MOST > 8)
+        if (need <= 12) return launch_quarters<MG, RG, U, 1, ONE, false, 12>(a, st);
+    return unbuilt(a);
 }
 
 template <int MG, int U, int RG>
 int quarters(BatchArgs &a, hipStream_t st) {
-    constexpr int XMAX = 16;
-    auto need = [&] { return (a.M * (a.K / 8) + 256 * a.teams * a.sets - 1) / (256 * a.teams * a.sets); };
+    auto need = [&] { return up(a.M * (a.K / 8), 256 * a.teams * a.sets); };
     const int rows = 4 * RG * a.teams;
     while (a.teams * a.sets < 4 && need() > 12) ++a.teams, a.sets = 1;
     if (a.sets > 1 && need() > 12) a.teams = 4, a.sets = 1;
     const size_t totals = (size_t)a.teams * a.units * (RG * MG * 256);
-    if (need() <= XMAX && (size_t)a.quarters * MG * 2048 + totals <= LDS_BYTES) {
-        if constexpr (RG == 1 && U >= 3)
-            if (a.sets > 1) return need() <= 4 ? launch_quarters<MG, RG, U, 0, false, false, 4>(a, st) : launch_quarters<MG, RG, U, 0, false, false, 12>(a, st);
-        if constexpr (U >= 3)
+    // (what fits LDS is at most ten vectors a thread of sixteen wavefronts)
+    if ((size_t)a.quarters * MG * 2048 + totals <= LDS_BYTES) {
+        if constexpr (U == 3 || (U == 4 && MG < 4)) {  // (16 rows of several units of four segments do not fit)
+            if constexpr (RG == 1) {
+                if constexpr (MG < 4)
+                    if (a.sets > 1 && need() <= 4) return launch_quarters<MG, RG, U, 0, false, false, 4>(a, st);
+                if (a.sets > 1) return launch_quarters<MG, RG, U, 0, false, false, 12>(a, st);
+            }
             if (a.units > 1) return by_vectors<MG, RG, U, false>(a, need(), st);
+        }
         return by_vectors<MG, RG, U, true>(a, need(), st);
     }
-    // long rows: windows of as many units as LDS takes and the row blocks leave wavefronts for
-    constexpr int XV = (MG * U * 512 + 1023) / 1024;
-    if constexpr (U >= 3 && RG == 1) {
+    // long rows: windows of as many units as LDS takes and the row blocks leave wavefronts for (units of four segments: the only
+    // longer rows of units of three are sixteen)
+    constexpr bool LONG = U == 4 || (U == 3 && MG == 4);
+    constexpr int XV = up(MG * U * 512, 1024);
+    if constexpr (LONG && RG == 1) {
         if constexpr (MG == 1)
             if (rows <= 4) return a.teams = 1, a.sets = 4, launch_quarters<MG, RG, U, 4, false, true, 4 * XV>(a, st);
         if constexpr (MG <= 2)
             if (rows <= 8) return a.teams = 2, a.sets = 2, launch_quarters<MG, RG, U, 2, false, true, 2 * XV>(a, st);
     }
     a.teams = 4, a.sets = 1;
-    if constexpr (U >= 3 && (RG == 1 || MG <= 2)) return launch_quarters<MG, RG, U, 1, false, true, XV>(a, st);
-    return fail(CMI_E_UNSUPPORTED, "cmi_gemv_w8a16: no kernel for %d rows of %d", a.M, a.K);
+    if constexpr (LONG && (RG == 1 || MG <= 2)) return launch_quarters<MG, RG, U, 1, false, true, XV>(a, st);
+    return unbuilt(a);
 }
 
 template <int MG, int U>
@@ -458,7 +490,7 @@ int run(BatchArgs &a, bool streamed, hipStream_t st) {
     if (a.sets > a.units) a.sets = a.units;
     // four groups whose rows go through LDS in windows have registers for one block
     const size_t whole = (size_t)a.quarters * MG * 2048 + (size_t)4 * a.units * (2 * MG * 256);
-    if (MG == 4 && (whole > LDS_BYTES || a.M * (a.K / 8) > 16 * 1024)) rg = 1;
+    if (MG == 4 && whole > LDS_BYTES) rg = 1;
     return rg == 1 ? quarters<MG, U, 1>(a, st) : quarters<MG, U, 2>(a, st);
 }
 
