@@ -270,8 +270,8 @@ def test_w4a8_rows_through_the_chosen_tile(m, n, k):
 @pytest.mark.parametrize("n,k", [(65535, 2064), (65536, 1040), (65537, 3072), (70001, 4096), (65536, 1024), (65600, 4112), (65537, 1664), (65539, 2560), (300, 2560),
                                  (4096, 4096), (4097, 4096), (33, 9728)])
 def test_weight_only_rows_keep_the_single_row_s_bits_at_the_edges_of_the_row_blocks(n, k):
-    """Four weight rows per wavefront for very tall weights at 3..4 rows, one at 9..16 rows and few outputs, three
-    tiles of activation rows at 9..12: integers of both signs, every row against the call with that row alone."""
+    """Tall weights that are streamed or whose workgroups follow each other, and few outputs; last segments nearly empty, half full and
+    full: integers of both signs, every row against the call with that row alone."""
     gen = torch.Generator(device=G.DEV).manual_seed(n + k)
     wq = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=G.DEV, generator=gen)
     ws = torch.rand(n, device=G.DEV, generator=gen) * 0.01
@@ -486,6 +486,27 @@ def test_ragged_rows_take_the_matrix_pipe_where_the_call_site_may(monkeypatch, p
         assert torch.equal(backend.linear_m(w, x).view(torch.int16), dot.view(torch.int16))
 
 
+#: Rows: (outputs, K), one for each kernel of gemv_w8a16_batch.hip (groups of four activation rows, row blocks a wavefront, segments a unit, sets of
+#: wavefronts, windows, vectors carried to LDS) that the shapes at the test itself do not take.
+_BATCH_KERNELS = {
+    2: [(131, 2064), (131, 3088), (131, 4112), (131, 8208), (1027, 19984), (2051, 4112), (2051, 6160), (2051, 19984), (3075, 3088),
+        (3075, 4112), (3075, 6160), (3075, 8208), (3075, 9232), (4099, 19472), (8195, 12288), (12001, 8720), (16387, 6160)],
+    3: [(131, 3088), (2051, 8208), (2051, 16400), (3075, 11280), (6151, 16384), (12001, 8720)],
+    4: [(131, 4112), (3075, 8208), (5121, 25600), (33001, 4096), (66001, 2048), (131075, 1024)],
+    5: [(131, 16), (131, 1040), (131, 2064), (131, 3344), (131, 4112), (131, 6160), (1027, 2064), (1027, 3088), (1027, 4112),
+        (1027, 6160), (2051, 6160), (2051, 9744), (3075, 16), (3075, 1040), (3075, 2064), (3075, 3088), (3075, 3344), (3075, 6160),
+        (3075, 7184), (4099, 4112), (6151, 6160), (8195, 4112), (8195, 6160), (16387, 16), (16387, 2064), (16387, 3088)],
+    6: [(2051, 4112), (2051, 8208)],
+    8: [(131, 1040), (131, 2064), (3075, 2064), (3075, 4112), (8195, 5392)],
+    9: [(131, 16), (131, 1040), (131, 3088), (131, 4112), (131, 4880), (1027, 1040), (2051, 2064), (2051, 4112), (3075, 3088),
+        (4099, 1040), (4099, 2064), (4099, 3088), (4099, 4112), (6151, 3088), (9217, 16), (9217, 1040), (9217, 3088), (16385, 5136),
+        (20001, 6160)],
+    10: [(131, 3344)],
+    12: [(131, 4112), (4099, 2064), (4099, 4112), (9217, 1552)],
+    16: [(131, 528), (131, 1040), (701, 25600), (4099, 1552), (4099, 3088)],
+}
+
+
 @pytest.mark.parametrize("m,n,k", [(2, 1, 16), (3, 5, 1040), (4, 1023, 2560), (16, 1024, 2576), (4, 300, 9744), (8, 700, 9728),
                                    (7, 2047, 4096), (5, 2561, 4112), (2, 9000, 6416), (2, 1152, 16384), (2, 1153, 16384),
                                    (3, 200, 20496), (6, 500, 12304), (7, 2000, 33024), (4, 4096, 14336), (8, 3900, 9728), (6, 5000, 20496), (16, 300, 9728), (12, 5000, 6160), (9, 9300, 12304),
@@ -493,10 +514,12 @@ def test_ragged_rows_take_the_matrix_pipe_where_the_call_site_may(monkeypatch, p
                                    (4, 32773, 4112), (5, 16385, 1040), (16, 9217, 2576), (15, 9301, 4096), (11, 4100, 5120),
                                    (3, 20000, 5136), (8, 8193, 6160), (16, 16400, 6160),
                                    (2, 8192, 1040), (2, 8193, 1040), (2, 16385, 1040), (2, 16385, 1152), (2, 16387, 2064), (2, 9001, 4096), (2, 8200, 1024),
-                                   (2, 1025, 9744), (2, 1536, 12304), (2, 1537, 9744), (3, 1025, 1024), (4, 3072, 784)])
+                                   (2, 1025, 9744), (2, 1536, 12304), (2, 1537, 9744), (3, 1025, 1024), (4, 3072, 784)]
+                         + [(m, n, k) for m, shapes in _BATCH_KERNELS.items() for n, k in shapes])
 def test_batches_of_weight_only_rows_carry_the_single_row_bits(m, n, k):
     """Every kernel that 2..16 rows of cmi_gemv_w8a16 take, at odd counts of rows, outputs and chunks: few outputs by quarters of a row
-    (units dealt to wavefronts, one block or two a wavefront), long rows in windows, many outputs streamed, sixteen rows in two halves.
+    (units dealt to wavefronts, one block or two a wavefront), long rows in windows, many outputs streamed, sixteen rows in two halves
+    (the second of one row, too), two rows that share a tree.
     Infinite and NaN activations stay in their rows; nothing is written past the outputs."""
     gen = torch.Generator(device=G.DEV).manual_seed(m + n + k)
     wq = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=G.DEV, generator=gen)
