@@ -109,10 +109,10 @@ def test_two_rows_of_one_tree_are_the_plain_trees():
     assert original(vals[0]) not in pair(vals, lambda l: l & 1)
 
 
-def batch(mg, vals):
+def batch(mg, vals, first=lambda l: ((l >> 2) ^ (l >> 3)) & 1):
     """quarter_sum<mg> of gemv_w8a16_batch.hip: 4 mg values a lane over the 16 blocks of four lanes."""
     nv = 4 * mg
-    a = level(vals, 0x141, nv // 2, lambda l: ((l >> 2) ^ (l >> 3)) & 1)
+    a = level(vals, 0x141, nv // 2, first)
     b = level(a, 0x140, nv // 4, lambda l: (l >> 3) & 1)
 
     def swapped(swap, x, y):
@@ -125,33 +125,45 @@ def batch(mg, vals):
     return swapped(swap32, c, c)
 
 
-@pytest.mark.parametrize("mg", [1, 2, 4])
-def test_batch_reduction_continues_the_single_row_tree(mg):
-    """Blocks b ^ 1, b ^ 2, b ^ 4, b ^ 8 in this order: the levels of wave_sum_to_lane63 between chunks that differ in one bit.  The
-    activation rows of a block's four lanes are reversed in odd blocks (lane_row)."""
-    def act(lane):
-        return 3 - (lane & 3) if lane & 4 else lane & 3
+def reversed_in_odd_blocks(lane):
+    """lane_row: the activation row that a lane of a block holds."""
+    return 3 - (lane & 3) if lane & 4 else lane & 3
 
+
+def wrong_lanes(mg, got, act):
+    """Lanes whose value is not the plain tree over the blocks, b ^ 1, b ^ 2, b ^ 4, b ^ 8 in this order, of value quarter_index and
+    the lane's activation row; and the outputs of the lanes that store."""
     def tree(i, j):
-        def leaf(b):
-            return [(i, lane) for lane in range(4 * b, 4 * b + 4) if act(lane) == j][0]
-
-        cur = [leaf(b) for b in range(16)]
+        cur = [[(i, lane) for lane in range(4 * b, 4 * b + 4) if act(lane) == j][0] for b in range(16)]
         while len(cur) > 1:
             cur = [add(cur[2 * b], cur[2 * b + 1]) for b in range(len(cur) // 2)]
         return cur[0]
 
-    vals = [[(i, lane) for lane in range(64)] for i in range(4 * mg)]
-    got = batch(mg, vals)
-    held = set()
+    wrong, held = [], set()
     for lane in range(64):
         s1, s2, b4, b5 = ((lane >> 2) ^ (lane >> 3)) & 1, (lane >> 3) & 1, (lane >> 4) & 1, (lane >> 5) & 1
         i = {4: s1 * 8 + s2 * 4 + b4 * 2 + b5, 2: s1 * 4 + s2 * 2 + b4, 1: s1 * 2 + s2}[mg]
-        assert got[lane] == tree(i, act(lane)), (mg, lane)
+        if got[lane] != tree(i, act(lane)):
+            wrong.append(lane)
         if mg == 4 or not lane & (32 if mg == 2 else 48):
             held.add((i, act(lane)))
-    # the lanes that store cover every output exactly once
-    assert held == {(i, j) for i in range(4 * mg) for j in range(4)}
+    return wrong, held
+
+
+@pytest.mark.parametrize("mg", [1, 2, 4])
+def test_batch_reduction_continues_the_single_row_tree(mg):
+    """The levels of wave_sum_to_lane63 between chunks that differ in one bit; the lanes that store cover every output exactly once."""
+    vals = [[(i, lane) for lane in range(64)] for i in range(4 * mg)]
+    wrong, held = wrong_lanes(mg, batch(mg, vals), reversed_in_odd_blocks)
+    assert not wrong and held == {(i, j) for i in range(4 * mg) for j in range(4)}
+
+
+@pytest.mark.parametrize("mg", [1, 2, 4])
+def test_batch_reduction_with_other_halves_or_rows_is_caught(mg):
+    """Halves kept by the plain lane bit, and activation rows that are not reversed in odd blocks: sums of what does not belong together."""
+    vals = [[(i, lane) for lane in range(64)] for i in range(4 * mg)]
+    assert wrong_lanes(mg, batch(mg, vals, lambda l: (l >> 2) & 1), reversed_in_odd_blocks)[0]
+    assert wrong_lanes(mg, batch(mg, vals), lambda l: l & 3)[0]
 
 
 def test_single_row_tree_pairs_chunks_by_one_bit():
