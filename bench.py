@@ -148,7 +148,7 @@ def parse_args():
     ap.add_argument("--rows", type=int, default=1, help="activation rows M of the headline workload")
     ap.add_argument("--mfma", action="store_true",
                     help="headline workload through cmi_gemv_w8a16_mfma (the verify / short-prefill kernel) "
-                         "instead of the dot-product GEMV; meant for --rows 3..16")
+                         "instead of the GEMV of the single-row order; meant for --rows 3..16")
     ap.add_argument("--no-graph", action="store_true", help="launch eagerly instead of replaying a HIP graph")
     ap.add_argument("--no-extra", action="store_true", help="skip the secondary configurations")
     ap.add_argument("--cpu-seconds", type=float, default=10.0, help="budget of the CPU baseline leg (0 = skip)")
@@ -503,7 +503,7 @@ def main() -> int:
     def run_step(m, mfma=False):
         # mfma: the matrix-pipe GEMV that verify and short prefill chunks take (rows of a batch
         # independent of each other, not bit-identical to the single-row call); otherwise the
-        # dot-product GEMV of linear / linear_m
+        # GEMV of linear / linear_m
         st = cur_stream()
         fn = lib.cmi_gemv_w8a16_mfma if mfma else lib.cmi_gemv_w8a16
         for wq, sc, x, y, n_, k_ in launches:

@@ -15,7 +15,7 @@ weight             rows                        kernel
 =================  ==========================  =================================
 QWeight (int8)     linear, linear_m            int8 weight-only GEMV, 16
                                                rows at a time (row r == linear(x[r]))
-QWeight            >= 3, linear_m_verify and   weight-only GEMV on the matrix pipe,
+QWeight            >= 3, linear_m_verify and   16-row matrix-pipe GEMV, weight-only,
                    linear_prefill below 64     16 rows at a time
 QWeight            >= 64, linear_prefill       per-token quant + W8A8 MFMA GEMM
 QWeight            >= 2, linear_m_verify with  per-token quant + W8A8 (weight read
@@ -66,9 +66,9 @@ W8A8_VERIFY = os.environ.get("COFFIN_AMD_W8A8_VERIFY", "0").strip() == "1"
 #: numbers), so ``linear`` and ``linear_m`` on int8 weights stay on the GEMV of the single-row order, whose
 #: summation order depends on K only.  ``linear_m_verify`` (which may use a path of its own,
 #: backends/protocol.py:152-155) and short ``linear_prefill`` chunks do not carry that obligation
-#: and take the matrix-pipe GEMV from three rows up: up to 1.6 times faster at 16 rows, up to 1.5 times
-#: slower at three to eight of a large weight, a row's bits the same in a window of any length; same
-#: weight-only arithmetic, last-place differences from fp32 summation order.
+#: and take the matrix-pipe GEMV from ``MFMA_MIN_ROWS`` rows up: same weight-only arithmetic, last-place
+#: differences from fp32 summation order, so a row's bits are the same in all windows from there on, and
+#: those of decode in shorter ones.
 #: ``COFFIN_AMD_BATCH_MFMA=1`` moves *every* int8 weight-only call -- ``linear`` included, one row
 #: included -- to the matrix-pipe GEMV: the contract holds again (one kernel family, a row's bits
 #: independent of its batch), and
@@ -82,11 +82,15 @@ BATCH_MFMA = os.environ.get("COFFIN_AMD_BATCH_MFMA", "0").strip() == "1"
 W4A16 = os.environ.get("COFFIN_AMD_W4A16", "0").strip() == "1"
 W4A16_MAX_ROWS = 4
 W4A16_MAX_K = 32768
-#: Rows from which verify windows and short chunks take the matrix-pipe GEMV (when this was chosen, the faster one on every layer shape).
+#: Rows from which verify windows and short chunks take the matrix-pipe GEMV.  Chosen against kernels of the single-row order that
+#: are gone.  Those of today are the faster ones up to eight rows: over eleven layer shapes, large weights among them, they take 0.79 of its
+#: time at three rows, 0.83 at four, 0.94 at eight and 1.1 at nine to sixteen (three rows of 2560 -> 9728 8.3 against 9.1 us, of
+#: 4096 -> 128256 82 / 140; sixteen of 9728 -> 2560 15.2 / 11.0).  The line stays: windows of three rows and more agree in
+#: their bits with one of sixteen, which one at nine would end.
 MFMA_MIN_ROWS = 3
-#: The same for K that is not whole lines of 128 (2624 -> 9728: the dot-product kernel takes four rows in 8.7 us, the
-#: matrix-pipe one five in 11.4; five take the former 12.0, nine 20.2 against 11.5).  A weight whose family is "mfma" keeps such
-#: rows on the dot-product kernel, single rows included.
+#: The same for K that is not whole lines of 128 (2624 -> 9728, single-row order against matrix pipe: five rows 9.1 / 11.5 us, eight
+#: 9.8 / 11.5, nine 12.5 / 11.7): likewise where it was.  A weight whose family is "mfma" keeps such
+#: rows in the single-row order, single rows included.
 RAGGED_MFMA_MIN_ROWS = 5
 #: ``rms_norm`` / ``add_rms_norm`` / ``silu_mul`` also leave their output rows quantised (int8 +
 #: scale) in private scratch, and a ``linear*`` call on that very output -- W4A8 at any row count,
@@ -117,7 +121,7 @@ def configure(*, batch_family: str | None = None, w8a8_verify: bool | None = Non
 
     ``batch_family``: ``"dot"`` -- ``linear`` / ``linear_m`` on int8 weights run the GEMV of the
     single-row order (fastest single row) -- or ``"mfma"`` -- every int8
-    weight-only call, single rows included, runs the 16-row matrix-pipe GEMV (16 rows up to 1.6 times
+    weight-only call, single rows included, runs the 16-row matrix-pipe GEMV (16 rows up to 1.4 times
     faster, a single row slower).  Either way row r of a batch carries the bits of the single-row
     call (models/qwen35/batch.py:19-22): the rule needs one family per weight, not a particular
     one.  A weight object may carry its own choice in an attribute ``batch_family`` (read when the

@@ -12,7 +12,7 @@
 //   - K is cut into segments of 1024 (64 chunks of 16 elements);
 //   - U consecutive segments form a unit (U = unit_segments(K), 1..4);
 //   - chunk c of a unit's segments owns one fp32 chain that starts at 0.f: segments ascending, a
-//     segment's sixteen products as four MFMA steps of four k each (one rounding per step);
+//     segment's sixteen products as four MFMA steps of four k each (what a step rounds off: chain_chunk);
 //   - the 64 chains of a unit are summed by a fixed tree: chunks c ^ 1, c ^ 2, c ^ 4, c ^ 8, c ^ 16, c ^ 32
 //     (wave_sum_to_lane63 where lane l holds chunk l);
 //   - unit totals are added in ascending unit order, starting from unit 0's
@@ -22,7 +22,7 @@
 // Of the MFMA's 16 blocks of 4 x 4 outputs only the diagonal is wanted here, and it costs about what eight v_dot2 would (one
 // row, chains of v_dot2 -> these: 2560 -> 151936 58.9 -> 58.7 us, 4096 -> 128256 78.1 -> 78.5, 3584 -> 120000 64.8 -> 65.5, and
 // 1-2 % more where a launch is one round of latencies: 4608 -> 340 2.76 -> 2.82); with several activation rows every output is, and the
-// kernels for those read the weight at the speed of one row.  (v_dot2 rounds after two products, so
+// kernels for those read the weight at the speed of one row.  (v_dot2 does the same with two products, so
 // chains of both kinds cannot be mixed: the order is the MFMA's for every count.)
 //
 // Execution: one wavefront = (block of R weight rows, one unit of K).  All of a

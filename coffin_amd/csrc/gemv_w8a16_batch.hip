@@ -476,8 +476,9 @@ int run(BatchArgs &a, bool streamed, hipStream_t st) {
     // rows want small workgroups (1024 -> 8192 at four rows 3.9 with two blocks, 4.3 with eight; 896 -> 1030 at three 2.62 with one
     // block, 2.73 with two; two rows of 2560 -> 6144 5.2 against 5.5), and so does everything beyond 32 rows a CU, where workgroups
     // follow each other (2560 -> 19456 12.0 with four blocks, 13.9 with eight).
-    // Up to sixteen rows a CU of many units: four teams of one block (14336 -> 4096 at 4 / 8 rows 14.6 / 17.9 us, two of two 16.8 / 22.8; 9728 -> 3800
-    // at four rows 11.0 against 10.7, at eight 12.6 against 17.2).
+    // Up to sixteen rows a CU of many units: four teams of one block (14336 -> 4096 at 4 / 8 rows 16.0 / 17.9 us, two of two 18.8 / 22.8, at two and
+    // three rows 1 % the other way; 20480 -> 3600 at three rows 20.5, 29.8).  Of three units only from five rows on (9728 -> 3800 at eight rows
+    // 12.6, 17.2; at four 11.5 against 11.2, 10240 -> 3800 12.3 against 11.8).
     int rg = 2;
     if (rows <= 12) rg = 1, a.teams = MG == 1 && a.K <= 1024 ? 1 : (rows + 3) / 4;
     else if (MG <= 2 && a.K <= 1024) a.teams = MG;
@@ -527,7 +528,7 @@ int gemv_w8a16_batch(const int8_t *wq, const float *ws, const void *x, void *y, 
     // outputs (16 rows of 2560 -> 9728 12.0 against 13.3 us, 2560 -> 6144 9.7 against 7.6); two: 16384 (2560 -> 19456 14.5 against 15.8, 4096 -> 14336 17.1
     // against 16.4); one: four rows of 128 MiB and more (2560 -> 151936 67 against 72; three rows of 3072 -> 100000 53.6
     // against 50.4).  K of several units: 8192 outputs at two groups (6400 -> 9000 19.1 against 21.2), 96 MiB at one (5120 -> 51200 44.6 against 56, 5120 ->
-    // 10000 16.7 against 15.2).  Four groups whose copy leaves the quarters kernel no room (K of 4097..5120): from 4096 outputs (5120 -> 5120 14.2 against 18.8).
+    // 10000 16.7 against 15.2).  Four groups whose copy leaves the quarters kernel no room (K of 4609..5120): from 4096 outputs (5120 -> 5120 14.2 against 18.8).
     const size_t bytes = (size_t)N * K;
     const bool many = mg == 4   ? N >= 9216 || (a.quarters * 4 * 2048 + 16384 > (int)LDS_BYTES && N >= 4096)
                       : mg == 2 ? N >= (a.units > 1 ? 8193 : 16384)

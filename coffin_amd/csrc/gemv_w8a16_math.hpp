@@ -54,8 +54,8 @@ __device__ __forceinline__ Chunk widen_chunk(const u32x4 &w) {
 }
 
 // One 16-element chunk of a lane's chain, k ascending: v_mfma_f32_4x4x4_16b_bf16 works on 16 blocks of four lanes; for block b and
-// lane 4b + j, register i of v gains the four products of the codes in lane 4b + i with the activations in lane 4b + j, exact
-// products summed with what v held and rounded once.
+// lane 4b + j, register i of v gains the four products of the codes in lane 4b + i with the activations in lane 4b + j.  The products
+// are exact; they and what v held are cut off 26 bits below the largest of their exponents, summed, and rounded once (probed on the device).
 __device__ __forceinline__ v4f32 chain_chunk(v4f32 v, const Chunk &w, const uint4 &x0, const uint4 &x1) {
     v = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(w.step[0], pair_bits(x0.x, x0.y), v, 0, 0, 0);
     v = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(w.step[1], pair_bits(x0.z, x0.w), v, 0, 0, 0);

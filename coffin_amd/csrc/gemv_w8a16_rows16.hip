@@ -23,9 +23,9 @@
 // (static-batch decode) stay on cmi_gemv_w8a16.
 //
 // TAIL: rows that end inside a line.  Of the last line the activations past K are zeros that are not read, so what
-// the weight's pieces hold there (bytes of the row again) does not matter.  Against the dot-product kernel, which such rows
-// took at every count, cold weights: 9 rows of 2624 -> 9728 21.0 -> 11.7 us, 63 rows 98.9 -> 22.3; 16 rows of 9792 -> 2560 35.2 ->
-// 14.2; 50 rows of 1344 -> 1000 22.1 -> 8.6; 63 rows of 13888 -> 5120 691 -> 78.
+// the weight's pieces hold there (bytes of the row again) does not matter.  Cold weights, against the kernels of cmi_gemv_w8a16, 16 rows a
+// launch: 9 rows of 2624 -> 9728 11.4 us, 12.5 there; 63 rows 22.0, 47.2; 16 rows of 9792 -> 2560 14.3, 14.5; 50 rows of 1344 -> 1000 8.6, 14.2;
+// 63 rows of 13888 -> 5120 80, 141.
 #include "rows16_tile.hpp"
 
 namespace {
@@ -60,11 +60,11 @@ __device__ __forceinline__ void widen4(uint32_t w, uint32_t &lo, uint32_t &hi) {
     hi = __builtin_amdgcn_perm(__float_as_uint(f3), __float_as_uint(f2), 0x07060302u);
 }
 
-// How the sums of a row's lines meet.  A chain of MFMAs is less exact than the dot-product kernel, which the rows that end inside a
+// How the sums of a row's lines meet.  A chain of MFMAs is less exact than the single-row order, which the rows that end inside a
 // line left, and which sums in short chains: so for those the MFMAs of a line start from zero and their sums meet in pairs, and where
 // a wavefront has many lines (LOW) what the additions round off is kept and added at the end.  Root mean square error of sums that
-// cancel, in 2^-24 of the sum of magnitudes, K = 960 / 2624 / 9664 / 25536: dot-product kernel 0.053 / 0.046 / 0.031 / 0.021, a chain
-// 0.061 / 0.054 / 0.053 / 0.058, these 0.053 / 0.046 / 0.025 / 0.015 (a kept sum over up to three lines as well: 0.045 at 2624, and 63 rows of 2624 ->
+// cancel (activations N(0, 1), 1 % of them 20 times larger, weights N(0, 30)), in 2^-24 of the sum of magnitudes, K = 960 / 2624 / 9664 / 25536:
+// single-row order 0.054 / 0.046 / 0.031 / 0.022, a chain 0.061 / 0.054 / 0.053 / 0.058, these 0.054 / 0.046 / 0.025 / 0.015 (a kept sum over up to three lines as well: 0.045 at 2624, and 63 rows of 2624 ->
 // 9728 24.9 us instead of 22.1).
 enum Sum { CHAIN, PAIRS, LOW };
 constexpr Sum sum_of(bool tail, int nlp, int rounds) { return !tail ? CHAIN : rounds == 1 && nlp <= 3 ? PAIRS : LOW; }
@@ -575,11 +575,12 @@ extern "C" int cmi_gemv_w8a16_mfma(const int8_t *wq, const float *ws, const void
 
 namespace {
 
-// Few outputs of long rows that end inside a line: rows below this go to the dot-product kernel.  A wavefront of this file takes every
-// eighth line of its 16 weight rows, a chain that grows with K alone, while the other kernel has a wavefront for every two weight rows
-// and 4096 k and, up to 16384, the activations of eight rows in LDS.  Cold weights, dot-product against this file's: 5 rows of
-// 12304 -> 300 10.9 us against 15.6, of 16368 -> 800 17.1 / 19.4; 8 rows of 12304 -> 300 15.1 / 15.9, of 9200 -> 300 13.7 / 12.1; 5 rows of
-// 32784 -> 64 29.3 / 33.5; the other way at 5 rows of 16400 -> 300 21.7 / 19.0, of 12304 -> 1200 19.3 / 16.3, of 7184 -> 64 10.0 / 9.7.
+// Few outputs of long rows that end inside a line: rows below this go to the kernels of cmi_gemv_w8a16.  A wavefront of this file takes every
+// eighth line of its 16 weight rows, a chain that grows with K alone.  The line was measured against a kernel that is gone (5 rows of 12304 -> 300
+// 10.9 us, 15.6 here).  The batch kernels in its place are the faster ones up to eight rows on both sides of it (5 rows of 12304 -> 1200
+// 8.9 us, 16.4 here, of 16400 -> 300 10.4 / 19.0; 8 rows of 9200 -> 300 6.1 / 12.3, of 16368 -> 800 10.5 / 19.9; 9 rows of 12304 -> 300
+// 15.5 / 16.1, of 2624 -> 9728 12.5 / 11.7); it stays: rows beyond it agree in their bits with
+// those of a call of sixteen.
 int rows_from(int N, int K) {
     if (K % LINE == 0 || K <= 8192) return 1;
     if (K <= 16384) return N <= 512 ? (K >= 12288 ? 9 : 7) : N <= 832 ? 7 : N <= 1024 ? 6 : 1;

@@ -91,7 +91,7 @@ int cmi_gemv_w8a16(const int8_t *wq, const float *ws, const void *x, void *y,
  * K % 128 == 0 (else CMI_E_UNSUPPORTED: use cmi_gemv_w8a16); also
  * up to 64 rows (up to K = 10240 the weight is still read once, the rows go through in chunks
  * of 16 with the 16-row arithmetic; longer weight rows are read once per 16 activation rows).
- * Up to 1.6 times faster than cmi_gemv_w8a16 at 16 rows.  A row's bits depend on K
+ * Up to 1.4 times faster than cmi_gemv_w8a16 at 16 rows, slower up to 8.  A row's bits depend on K
  * only, not on the rows it travels with, but differ from cmi_gemv_w8a16's in
  * the last place (fp32 summation order): for callers without the
  * "batched row == single-row call" obligation of static-batch decode
@@ -106,8 +106,8 @@ int cmi_gemv_w8a16_mfma(const int8_t *wq, const float *ws, const void *x, void *
  *   CMI_FAMILY_DOT   cmi_gemv_w8a16, 16 rows per launch: row m carries the bits of the single-row call
  *                    (what static-batch decode owes its users, models/qwen35/batch.py:19-22);
  *   CMI_FAMILY_MFMA  cmi_gemv_w8a16_mfma, 64 rows per launch (K % 128 == 0, else
- *                    CMI_E_UNSUPPORTED and nothing is launched): 1.5-2.8 times faster at 4-16 rows,
- *                    slower at one row; a row's bits depend on K only.
+ *                    CMI_E_UNSUPPORTED and nothing is launched): up to 1.4 times faster at 9-16 rows,
+ *                    slower at fewer; a row's bits depend on K only.
  * The rule holds inside either family as long as every call on a weight -- single rows included --
  * names the same one, so the family is a property of a weight (or of a deployment), not of a call
  * site.  Stands where linear / linear_m / linear_m_verify reach gemv_nk_i8 / gemv_nk_i8_m
@@ -118,8 +118,8 @@ int cmi_linear_w8a16(const int8_t *wq, const float *ws, const void *x, void *y, 
                      int family, void *stream);
 /* The matrix-pipe family for rows that need not be whole lines (K % 16 == 0, 128 <= K <= 262144; the bits of
  * CMI_FAMILY_MFMA where it takes K): what the adapters issue for several rows without the single-row rule (verify, short prefill
- * chunks).  Up to 8 rows of at most 1024 outputs whose K is above 8192 and not whole lines go to cmi_gemv_w8a16's kernel where that is
- * the faster. */
+ * chunks).  Up to 8 rows of at most 1024 outputs whose K is above 8192 and not whole lines go to cmi_gemv_w8a16's kernels (rows_from in
+ * gemv_w8a16_rows16.hip). */
 int cmi_linear_w8a16_rows(const int8_t *wq, const float *ws, const void *x, void *y, int M, int N, int K,
                           void *stream);
 

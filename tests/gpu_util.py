@@ -46,7 +46,7 @@ def quant(x: torch.Tensor):
 
 
 def gemv_w8a16(wq, ws, x, mfma: bool = False):
-    """The dot-product GEMV, or (mfma) the matrix-pipe one for batches."""
+    """The GEMV of the single-row order, or (mfma) the 16-row matrix-pipe one."""
     m, k = x.shape
     n = wq.shape[0]
     y = torch.empty((m, n), dtype=torch.bfloat16, device=DEV)

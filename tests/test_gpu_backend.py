@@ -673,7 +673,7 @@ def test_scratch_captured_by_a_graph_survives_forty_other_shapes():
 
 def test_family_is_a_property_of_the_weight_or_the_process():
     """Static-batch decode is owed "row r == single-row call" (models/qwen35/batch.py:19-22).  It
-    holds in the dot-product family (default) and in the matrix-pipe family, chosen per weight
+    holds in the family of the single-row order (default) and in the matrix-pipe family, chosen per weight
     (attribute ``batch_family``) or per process (``configure``) -- every entry switches together."""
     g = synth.generator(10)
     k, n = 2560, 1536

@@ -401,7 +401,7 @@ def test_matrix_pipe_rows_that_end_inside_a_line(m, n, k):
 @pytest.mark.parametrize("m,k", [(16, 5200), (63, 9664), (16, 13888), (40, 25536)])
 def test_matrix_pipe_sums_of_rows_that_end_inside_a_line_are_as_exact_as_the_dot_product_s(m, k):
     """Rows whose products cancel to zero, so that a result is the error of its sum: in the root mean square no larger than the
-    dot-product kernel's (5 % for the sample: m x 2048 sums, and a ratio of 0.93 at 5200, 0.65 at 25536)."""
+    single-row order's (5 % for the sample: m x 2048 sums, and a ratio of 0.93 at 5200, 0.65 at 25536)."""
     n = 2048
     gen = torch.Generator(device=G.DEV).manual_seed(k)
     wq = (torch.randn((n, k), device=G.DEV, generator=gen) * 30).round().clamp(-127, 127).to(torch.int8)
@@ -423,7 +423,7 @@ def test_matrix_pipe_sums_of_rows_that_end_inside_a_line_are_as_exact_as_the_dot
 @pytest.mark.parametrize("m,k", [(9, 2640), (16, 5200), (40, 9664), (9, 13888), (40, 13888)])
 def test_matrix_pipe_sums_of_rows_that_end_inside_a_line_that_are_infinite(m, k):
     """Infinite activations, and finite ones whose products or sums leave the range, with a NaN row beside them: the infinities,
-    signs and NaN of the dot-product kernel."""
+    signs and NaN of the single-row order."""
     n = 48
     gen = torch.Generator(device=G.DEV).manual_seed(m + k)
     wq = torch.randint(1, 128, (n, k), dtype=torch.int8, device=G.DEV, generator=gen)

@@ -157,7 +157,7 @@ def test_gemv_w8a16_whole_row_kernel_gives_the_general_kernels_bits(orc, n, k):
                                    # rows longer than two rounds of registers: the round count read at run time
                                    (16, 64, 10368), (5, 5120, 25600), (16, 100, 12800), (1, 77, 16384), (9, 40, 65536)])
 def test_gemv_w8a16_mfma_within_tolerance(orc, m, n, k):
-    """The matrix-pipe GEMV: same tolerance bars as the dot-product kernel, every
+    """The matrix-pipe GEMV: same tolerance bars as the single-row order's kernels, every
     lines-per-wavefront variant, one, two and more rounds, ragged N."""
     wq, ws, x, y = _w8a16_case(orc, m, n, k, seeded(), mfma=True)
     _assert_weight_only_tolerance(orc, wq, ws, x, y)
@@ -209,7 +209,7 @@ def test_gemv_w8a16_batched_row_equals_single_row(n, k):
 @pytest.mark.parametrize("n,k", [(4096, 2560), (2560, 9728), (512, 5120), (300, 6656), (64, 128), (200, 25600)])
 def test_gemv_w8a16_mfma_rows_do_not_depend_on_the_batch(n, k):
     """The matrix-pipe GEMV makes the weaker promise: a row's bits depend on K only, not on
-    the rows it travels with (also one row alone); against the dot-product kernel the
+    the rows it travels with (also one row alone); against the single-row order the
     difference is fp32 summation noise."""
     g = seeded()
     q = synth.int8_weight(n, k, g)
@@ -782,7 +782,7 @@ def test_random_shapes_every_kernel_against_the_oracle(orc):
         q, s = G.quant(x.to(G.DEV))
         q_ref, s_ref = orc.quant_act_i8(G.bits(x))
         assert (q.cpu().numpy() == q_ref).all() and (s.cpu().numpy() == s_ref).all(), ("quant", m, k)
-    # int8 weight-only: dot-product kernel (K % 16) and matrix-pipe kernel (K % 128)
+    # int8 weight-only: single-row order (K % 16) and matrix-pipe kernel (K % 128)
     for mfma, shapes in ((False, _rand_shapes(3, 10, 16, 200, 16, 4096)),
                          (True, _rand_shapes(4, 10, 16, 200, 128, 10240))):
         for m, n, k in shapes:
