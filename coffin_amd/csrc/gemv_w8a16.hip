@@ -20,7 +20,7 @@
 //   - the per-row weight scale multiplies that sum once, then one bf16 rounding.
 //
 // Of the MFMA's 16 blocks of 4 x 4 outputs only the diagonal is wanted here, and it costs about what eight v_dot2 would (one
-// row, chains of v_dot2 -> these: 2560 -> 151936 58.9 -> 58.7 us, 4096 -> 128256 78.1 -> 78.5, 3584 -> 120000 64.8 -> 65.5, and
+// row, chains of v_dot2 -> these: 2560 -> 151936 57.4 -> 56.8 us, 4096 -> 128256 78.2 -> 77.9, 3584 -> 120000 62.8 -> 62.7, and
 // 1-2 % more where a launch is one round of latencies: 4608 -> 340 2.76 -> 2.82); with several activation rows every output is, and the
 // kernels for those read the weight at the speed of one row.  (v_dot2 does the same with two products, so
 // chains of both kinds cannot be mixed: the order is the MFMA's for every count.)
@@ -38,8 +38,8 @@
 // there.  When K spans several units the wavefronts of a team each take units
 // of the same rows and the unit totals meet in LDS (summed in unit order by one
 // lane per output); otherwise the lanes that hold the tree results scale and
-// store them.  Two weight rows share one tree (wave_sum_pair) and one store: what a wavefront does after its last bytes have
-// arrived is time in which it has none in flight (1024 -> 151936 28.7 -> 27.3 us).
+// store them.  What a wavefront does after its last bytes have arrived is time in which it has none in flight: where that is a large
+// share, two weight rows go through one tree and one store (pairs below).
 // A single activation row against a K of two or three units (and against a
 // mid-sized weight with K in one unit, from 2305 on) takes gemv_w8a16_wholerow_kernel instead: one
 // wavefront per weight row, all units.
@@ -72,9 +72,14 @@ struct GemvArgs {
 // less and measured 8.6, 9.3 and 9.7 us against 7.3.)
 constexpr int BLOCK_WAVES = 4;
 
-// Wavefronts per SIMD the compiler is to leave room for.  No kernel here needs more than 128 registers; told so, the compiler
-// forms the MFMA sums in the ordinary ones instead of accumulation registers that each sum has to be copied out of.
-constexpr int MIN_SIMD_WAVES = 4;
+// Wavefronts per SIMD the compiler is to leave room for.  Told of four, it forms the MFMA sums in ordinary registers instead of accumulation registers
+// that each sum has to be copied out of: two activation rows of 6400 -> 9000 14.7 -> 13.8 us, of 2560 -> 151936 65.5 -> 61.1.  One row has no use for it
+// (2560 -> 151936 57.2 -> 57.7: an eighth wavefront a SIMD does not help a stream).
+constexpr int simd_waves(int m) { return m == 2 ? 4 : 1; }
+
+// Whether two weight rows go through one tree (wave_sum_pair) and end in two lanes that store together: two activation rows, where it halves four trees,
+// and short rows, of which the tail is a large share (one row of 1024 -> 151936 28.4 -> 26.7 us; 2560 -> 151936 56.8 against 57.2).
+constexpr bool pairs(int m, int r, int cht) { return r == 2 && (m == 2 || cht <= 2); }
 
 // uint4 vectors of the LDS copy of the activations.
 //   K one unit: [row][segment][lane][half], i.e. a row as it is in memory, padded
@@ -103,7 +108,7 @@ struct WStage {
 // XLDS: the workgroup stages the activations in LDS; otherwise each wavefront
 //       reads them from global memory (only when they do not fit).
 template <int M, int R, int CHT, bool MULTI, bool XLDS>
-__global__ void __launch_bounds__(64 * BLOCK_WAVES, MIN_SIMD_WAVES)
+__global__ void __launch_bounds__(64 * BLOCK_WAVES, simd_waves(M))
 gemv_w8a16_kernel(const GemvArgs a) {
     extern __shared__ uint4 smem[];  // staged activations (XLDS, see xlds_vectors), then unit totals
     const int lane = threadIdx.x & 63;
@@ -179,14 +184,14 @@ gemv_w8a16_kernel(const GemvArgs a) {
         for (int r = 0; r < R; ++r)
 #pragma unroll
             for (int m = 0; m < M; ++m) acc[r][m] = v4f32{0.f, 0.f, 0.f, 0.f};
+        // two activation rows: the weight rows' chains side by side (one row: no faster)
 #pragma unroll
-        for (int j = 0; j < CHT; ++j)
+        for (int i = 0; i < R * CHT; ++i) {
+            const int r = M == 2 ? i % R : i / CHT, j = M == 2 ? i / R : i % CHT;
+            const Chunk w = widen_chunk(ws_.w[r][j]);
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const Chunk w = widen_chunk(ws_.w[r][j]);
-#pragma unroll
-                for (int m = 0; m < M; ++m) acc[r][m] = chain_chunk(acc[r][m], w, xs_.x[m][j][0], xs_.x[m][j][1]);
-            }
+            for (int m = 0; m < M; ++m) acc[r][m] = chain_chunk(acc[r][m], w, xs_.x[m][j][0], xs_.x[m][j][1]);
+        }
     };
 
     // Activation fetch first (memory returns data in issue order, so whatever a
@@ -208,12 +213,18 @@ gemv_w8a16_kernel(const GemvArgs a) {
     }
     WStage<R, CHT> w0;
     load_w(w0, min(u, a.units - 1));
-    // The scale of the output that this lane stores, requested behind the weights and by vector loads (with one weight row the
-    // opaque zero keeps the address in a vector register).  As scalar loads they would share the
+    // The scales of the outputs that this lane stores, requested behind the weights and by vector loads (where they are uniform,
+    // an opaque value keeps the address in a vector register).  As scalar loads they would share the
     // LDS counter and sit in front of the barrier of the activation hand-over.
-    int srow = MULTI ? min(lane / M, R - 1) : R == 2 ? lane & 1 : 0;
-    asm volatile("" : "+v"(srow));
-    const float scale = a.ws[min(rb * R + srow, a.N - 1)];
+    constexpr bool PAIR = pairs(M, R, CHT);
+    constexpr int ROWS = PAIR ? 1 : R;  // weight rows of a lane that holds totals: lanes 0 and 1 (PAIR), or lane 63
+    float scale[MULTI ? 1 : ROWS];
+#pragma unroll
+    for (int i = 0; i < (MULTI ? 1 : ROWS); ++i) {
+        int row = MULTI ? min(lane / M, R - 1) : PAIR ? lane & 1 : i;
+        asm volatile("" : "+v"(row));
+        scale[i] = a.ws[min(rb * R + row, a.N - 1)];
+    }
     if constexpr (XLDS) {
 #pragma unroll
         for (int j = 0; j < XV; ++j) {
@@ -235,10 +246,8 @@ gemv_w8a16_kernel(const GemvArgs a) {
         __syncthreads();
     }
 
-    // the lanes that hold the totals, one weight row each (wave_sum_pair: lanes 0 and 1)
-    const bool holds = R == 2 ? lane < 2 : lane == 63;
-    const int hrow = R == 2 ? lane & 1 : 0;
-    float tot[M];
+    const bool holds = PAIR ? lane < 2 : lane == 63;
+    float tot[ROWS][M];
 #pragma unroll 1
     for (; u < a.units; u += a.uw) {
         if (idle) break;
@@ -248,23 +257,32 @@ gemv_w8a16_kernel(const GemvArgs a) {
         if (MULTI && u + a.uw < a.units) load_w(w0, u + a.uw);  // next unit of this wavefront
 #pragma unroll
         for (int m = 0; m < M; ++m) {
-            if constexpr (R == 2) tot[m] = wave_sum_pair(own_chain(acc[0][m], lane), own_chain(acc[1][m], lane), lane);
-            else tot[m] = wave_sum_to_lane63(own_chain(acc[0][m], lane));
+            if constexpr (PAIR) tot[0][m] = wave_sum_pair(own_chain(acc[0][m], lane), own_chain(acc[1][m], lane), lane);
+            else
+#pragma unroll
+                for (int i = 0; i < ROWS; ++i) tot[i][m] = wave_sum_to_lane63(own_chain(acc[i][m], lane));
         }
         if constexpr (!MULTI) break;
         // unit totals meet in LDS; one lane per output adds them in unit order below
         if (holds) {
 #pragma unroll
-            for (int m = 0; m < M; ++m) unit_total[u * (R * M) + hrow * M + m] = tot[m];
+            for (int i = 0; i < ROWS; ++i)
+#pragma unroll
+                for (int m = 0; m < M; ++m) unit_total[u * (R * M) + (PAIR ? lane : i) * M + m] = tot[i][m];
         }
     }
 
     if constexpr (!MULTI) {
-        const int n = rb * R + hrow;
-        if (!idle && holds && n < a.N) {
+        if (!idle && holds) {
 #pragma unroll
-            for (int m = 0; m < M; ++m)
-                if (m < a.M) a.y[(size_t)m * a.N + n] = (uint16_t)f32_to_bf16_bits(scale * tot[m]);
+            for (int i = 0; i < ROWS; ++i) {
+                const int n = rb * R + (PAIR ? lane : i);
+                if (n < a.N) {
+#pragma unroll
+                    for (int m = 0; m < M; ++m)
+                        if (m < a.M) a.y[(size_t)m * a.N + n] = (uint16_t)f32_to_bf16_bits(scale[i] * tot[i][m]);
+                }
+            }
         }
     } else {
         __syncthreads();
@@ -274,7 +292,7 @@ gemv_w8a16_kernel(const GemvArgs a) {
             if (n < a.N && m < a.M) {
                 float total = unit_total[lane];
                 for (int v = 1; v < a.units; ++v) total += unit_total[v * (R * M) + lane];
-                a.y[(size_t)m * a.N + n] = (uint16_t)f32_to_bf16_bits(scale * total);
+                a.y[(size_t)m * a.N + n] = (uint16_t)f32_to_bf16_bits(scale[0] * total);
             }
         }
     }
@@ -286,7 +304,7 @@ gemv_w8a16_kernel(const GemvArgs a) {
 // workgroup of W wavefronts stages the activation row once for W weight rows (the team
 // arrangement of the general kernel stages it once per two rows).  Same bits.
 template <int CHT, int NU, int XV>
-__global__ void __launch_bounds__(256, MIN_SIMD_WAVES)
+__global__ void __launch_bounds__(256)
 gemv_w8a16_wholerow_kernel(const GemvArgs a) {
     extern __shared__ uint4 smem[];  // the activation row, then one zeroed 32-byte slot
     const int lane = threadIdx.x & 63;
@@ -384,6 +402,8 @@ int dispatch_wholerow(const GemvArgs &a, hipStream_t st) {
 
 //: Most K-units one launch handles (LDS holds one total per unit and output).
 constexpr int MAX_UNITS = 64;
+//: LDS of a workgroup of which a CU holds six.
+constexpr size_t SIX_PER_CU = 26 * 1024;
 //: Activations up to this many bytes are staged in LDS.
 constexpr size_t XLDS_MAX_BYTES = 128 * 1024;
 
@@ -441,7 +461,13 @@ int launch(GemvArgs &a, hipStream_t st) {
     const int segs = a.units * a.unit;
     if constexpr (MULTI && M == 1 && CHT == 4)  // (units of three segments fit, and two rows that do not are the batch kernels')
         if (!x_fits_lds(a.M, a.K, a.units, segs)) return launch_x<M, R, CHT, MULTI, false>(a, grid, block, totals, st);
-    return launch_x<M, R, CHT, MULTI, true>(a, grid, block, 16 * (size_t)xlds_vectors(a.M, a.K, segs, !MULTI) + totals, st);
+    size_t lds = 16 * (size_t)xlds_vectors(a.M, a.K, segs, !MULTI) + totals;
+    // One row of a large weight of several segments, mostly full: six workgroups a CU have 100..200 KB in flight, and a seventh only takes turns with them.
+    // Seven or eight -> six: 2048 -> 151936 48.6 -> 47.4 us, 3584 -> 120000 65.4 -> 64.9, 4096 -> 151936 92.1 -> 91.4, 2560 -> 151936 58.8 -> 58.6 (five 59.7);
+    // 2176 -> 128256, its third segment an eighth full, 43.9 against 45.1, 1024 -> 151936 27.3 / 28.4.  Up to 128 MiB it makes no difference.
+    if constexpr (M == 1 && R == 2 && CHT >= 2 && !MULTI)
+        if ((size_t)a.N * a.K > (size_t)128 << 20 && a.nchunks * 5 >= segs * 256) lds = lds < SIX_PER_CU ? SIX_PER_CU : lds;
+    return launch_x<M, R, CHT, MULTI, true>(a, grid, block, lds, st);
 }
 
 template <int M, int R>
