@@ -201,6 +201,18 @@ __device__ __forceinline__ int xcd_contiguous_block(int b, int nb) {
     return x * q + min(x, r) + (b >> 3);
 }
 
+// Items walked by wavefronts that stay: those of this XCD are one contiguous run, dealt to its workgroups in turn, a wavefront of each at a
+// time (few items are spread over all workgroups).
+struct XcdItems {
+    int next, end, step;
+};
+__device__ __forceinline__ XcdItems xcd_items(int items, int wave, int waves) {
+    const int xcd = blockIdx.x & 7, nq = gridDim.x >> 3, nr = gridDim.x & 7;
+    const int nb = nq + (xcd < nr), before = xcd * nq + min(xcd, nr);
+    const int first = (int)((uint64_t)items * before / gridDim.x), end = (int)((uint64_t)items * (before + nb) / gridDim.x);
+    return {first + wave * nb + (int)(blockIdx.x >> 3), end, waves * nb};
+}
+
 __device__ __forceinline__ float lane63(float v) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }

@@ -67,12 +67,9 @@ gemv_w4a8_stream_kernel(const Args a) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) xs[v] = a.xs[min(4 * kq + v, a.M - 1)];
 
-    // tiles of this XCD: one contiguous run, dealt to its wavefronts in turn
-    const int xcd = blockIdx.x & 7, nq = gridDim.x >> 3, nr = gridDim.x & 7;
-    const int nb = nq + (xcd < nr), before = xcd * nq + min(xcd, nr);
-    const int first = (int)((uint64_t)a.tiles * before / gridDim.x), end = (int)((uint64_t)a.tiles * (before + nb) / gridDim.x);
-    const int step = WAVES * nb;
-    int tile = first + wave * nb + (blockIdx.x >> 3), line = 0;
+    const XcdItems tiles = xcd_items(a.tiles, wave, WAVES);
+    const int end = tiles.end, step = tiles.step;
+    int tile = tiles.next, line = 0;
     int ptile = tile, pline = 0;
 
     float wsr[WSN];

@@ -182,12 +182,9 @@ gemv_w8a16_stream_kernel(const BatchArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint4 xs[XV];
     request_x(xs, a, 64 * WAVES);
-    // row blocks (four weight rows each) of this XCD: one contiguous run, dealt to its wavefronts in turn
-    const int xcd = blockIdx.x & 7, nq = gridDim.x >> 3, nr = gridDim.x & 7;
-    const int nb = nq + (xcd < nr), before = xcd * nq + min(xcd, nr);
-    const int first = (int)((uint64_t)a.items * before / gridDim.x), end = (int)((uint64_t)a.items * (before + nb) / gridDim.x);
-    const int step = WAVES * nb;
-    int item = first + wave * nb + (blockIdx.x >> 3), u = 0;
+    const XcdItems blocks = xcd_items(a.items, wave, WAVES);  // of four weight rows
+    const int end = blocks.end, step = blocks.step;
+    int item = blocks.next, u = 0;
 
     u32x4 w[U][4];
     auto load_seg = [&](int it, int unit, int s) {
