@@ -213,17 +213,18 @@ gemv_w8a16_kernel(const GemvArgs a) {
     }
     WStage<R, CHT> w0;
     load_w(w0, min(u, a.units - 1));
-    // The scales of the outputs that this lane stores, requested behind the weights and by vector loads (where they are uniform,
-    // an opaque value keeps the address in a vector register).  As scalar loads they would share the
+    // The scales of the outputs that this lane stores, requested behind the weights and by vector loads (the
+    // opaque zero keeps a uniform address in a vector register).  As scalar loads they would share the
     // LDS counter and sit in front of the barrier of the activation hand-over.
     constexpr bool PAIR = pairs(M, R, CHT);
     constexpr int ROWS = PAIR ? 1 : R;  // weight rows of a lane that holds totals: lanes 0 and 1 (PAIR), or lane 63
+    int vzero = 0;
+    asm volatile("" : "+v"(vzero));
     float scale[MULTI ? 1 : ROWS];
 #pragma unroll
     for (int i = 0; i < (MULTI ? 1 : ROWS); ++i) {
-        int row = MULTI ? min(lane / M, R - 1) : PAIR ? lane & 1 : i;
-        asm volatile("" : "+v"(row));
-        scale[i] = a.ws[min(rb * R + row, a.N - 1)];
+        const int row = MULTI ? min(lane / M, R - 1) : PAIR ? lane & 1 : i;
+        scale[i] = a.ws[min(rb * R + row, a.N - 1) + (MULTI ? 0 : vzero)];
     }
     if constexpr (XLDS) {
 #pragma unroll
@@ -246,7 +247,7 @@ gemv_w8a16_kernel(const GemvArgs a) {
         __syncthreads();
     }
 
-    const bool holds = PAIR ? lane < 2 : lane == 63;
+    auto holds = [&] { return PAIR ? lane < 2 : lane == 63; };
     float tot[ROWS][M];
 #pragma unroll 1
     for (; u < a.units; u += a.uw) {
@@ -264,7 +265,7 @@ gemv_w8a16_kernel(const GemvArgs a) {
         }
         if constexpr (!MULTI) break;
         // unit totals meet in LDS; one lane per output adds them in unit order below
-        if (holds) {
+        if (holds()) {
 #pragma unroll
             for (int i = 0; i < ROWS; ++i)
 #pragma unroll
@@ -273,7 +274,7 @@ gemv_w8a16_kernel(const GemvArgs a) {
     }
 
     if constexpr (!MULTI) {
-        if (!idle && holds) {
+        if (!idle && holds()) {
 #pragma unroll
             for (int i = 0; i < ROWS; ++i) {
                 const int n = rb * R + (PAIR ? lane : i);
